@@ -37,6 +37,7 @@ template <typename T> T *jfm_alloc(jfm_ctx *ctx, int64_t count) {
     return (T *)p;
 }
 template uint16_t *jfm_alloc<uint16_t>(jfm_ctx *, int64_t);
+template uint64_t *jfm_alloc<uint64_t>(jfm_ctx *, int64_t);
 
 void jfm_free(jfm_ctx *ctx, void *p) {
     if (!p) return;
@@ -197,6 +198,7 @@ static void release_mesh(jfm_ctx *ctx) {
     ctx->has_state = ctx->minv_tangent = false;
     jfem_coarse_release(ctx);
     jfem_patch_release(ctx);
+    jfem_cells_release(ctx);
     release_heat(ctx);
     ctx->h_X.clear();
     ctx->has_user = false;
@@ -919,11 +921,29 @@ static int pcg_run(jfm_ctx *ctx, int op, const T *Minv, double rtol, int maxit, 
     T *x = (T *)w.x, *r = (T *)w.r, *z = (T *)w.z, *p = (T *)w.p, *q = (T *)w.q, *b = (T *)w.b;
     const int64_t n = ctx->ndof;
     hipStream_t s = ctx->stream;
+    int np = 0;
+    bool resident = false;
+    if (!coarse)
+        if (int rc = jfem_persist_ready<T>(ctx, op, &resident)) return rc;
+    if (resident) {
+        const bool from_x = warm && sizeof(T) == 8;
+        if (from_x) {
+            CHECK_LAUNCH(ctx, op_apply<T>(ctx, op, x, q, nullptr, nullptr, nullptr, nullptr));
+            CHECK_LAUNCH(ctx, launch_residual(ctx, (const double *)b, (const double *)q, ctx->fixed, (double *)r, n, &np));
+        }
+        CHECK_LAUNCH(ctx, launch_pcg_persist<T>(ctx, Minv, b, from_x ? r : nullptr, x, rtol, maxit));
+        if (int rc = read_scalars(ctx)) return rc;
+        if (!ctx->S_host->fail) {
+            *iters = ctx->S_host->iter;
+            *status = ctx->S_host->done[0];
+            return JFM_OK;
+        }
+        ctx->persist_off = true;  // launched below, and from now on
+    }
     std::memset(ctx->S_host, 0, sizeof(PcgScalars));
     ctx->S_host->rtol2 = rtol * rtol;
     ctx->S_host->maxit = maxit;
     if (int rc = write_scalars(ctx)) return rc;
-    int np = 0;
     if (warm && sizeof(T) == 8) {
         // restart from the current x with the true residual r = b - K x
         CHECK_LAUNCH(ctx, op_apply<T>(ctx, op, x, q, nullptr, nullptr, nullptr, nullptr));

@@ -124,6 +124,7 @@ struct PcgScalars {
     double rr0;         // r.r at the PCG start
     int done[2];        // 0 running, DONE_* otherwise, by parity
     int iter, maxit;
+    int fail;           // the resident PCG gave up waiting
 };
 // done codes
 enum { DONE_RUNNING = 0, DONE_CONVERGED = 1, DONE_BREAKDOWN = 2, DONE_MAXIT = 3 };
@@ -314,6 +315,21 @@ struct jfm_ctx {
     int hf_nfn = 0;
     int32_t *hf_conn = nullptr, *hf_ptr = nullptr, *hf_inc = nullptr;
     double *hf_h = nullptr, *hf_g = nullptr, *hf_text = nullptr, *hf_fe = nullptr;
+    // patches of the resident PCG (persist.hip): smaller ones, with per patch
+    // node its id, partial slot, slot range and incidences
+    struct Cells {
+        bool ready = false, usable = false;
+        int npatch = 0;
+        float rho32 = 0.0f;
+        int32_t *eperm = nullptr, *pn_ptr = nullptr, *pn_node = nullptr, *pn_slot = nullptr, *pn_sh = nullptr;
+        int32_t *pn_inc = nullptr;
+        uint16_t *connL = nullptr, *pn_cnt = nullptr, *lin = nullptr;
+        double *gf64 = nullptr, *part = nullptr;  // part: 4 values per slot (FP32 or FP64 view)
+        float *gf32 = nullptr, *gfQ32 = nullptr;
+        uint64_t *words = nullptr;
+        int nslot = 0;
+    } cells;
+    bool persist_off = false;      // a resident solve gave up waiting: this context launches its iterations
     double *Muser64 = nullptr;     // N x 9 user blocks (JFM_PREC_USER)
     float *Muser32 = nullptr;
     bool has_user = false;
@@ -401,6 +417,23 @@ hipError_t launch_patch_apply(jfm_ctx *ctx, int op, const T *x, T *y, const T *d
 // (JFEM_DEFER_SHARED=0 turns it off).
 int jfem_patch_qsrc(jfm_ctx *ctx);
 bool jfem_patch_defer_shared(const jfm_ctx *ctx, int op);
+// persist.hip: the whole PCG in one resident kernel, one workgroup per patch
+// (meshes of up to kPersistPatches patches).
+constexpr int kPersistPatches = 256;
+constexpr int kPersistWords = 6;  // exchange words per workgroup (and 256 more)
+// elements of a patch, its workgroup's threads (and most nodes), the row
+// stride of its LDS image of the element terms
+struct PersistGeometry { int elems = 0, threads = 0, stride = 0; };
+int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g);
+void jfem_cells_release(jfm_ctx *ctx);
+// Whether the PCG on `op` runs resident on this context (builds its patches
+// on first use); JFEM_PERSIST=0 turns it off.
+template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, bool *yes);
+// Solves K x = b (r0 null) or continues from x with its residual r0; the
+// scalars are in ctx->S afterwards (S->fail set when a wait gave up, x then
+// untouched).
+template <typename T>
+hipError_t launch_pcg_persist(jfm_ctx *ctx, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit);
 // coarse.hip
 // With learned_beside, the learned blocks start on the second stream
 // (jfem_learned_launch) once A_c is formed, beside its inversion.

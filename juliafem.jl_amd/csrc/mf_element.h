@@ -32,9 +32,9 @@ namespace jfem {
 // the same for every element; then G and sigma carry a factor sqrt(cm) and
 // 1 / sqrt(cm), and P = invJ' sigma is unchanged (two fewer loads and
 // multiplications per element).
-template <typename T, bool FOLD = false, typename XL, typename Out>
-__host__ __device__ __forceinline__ void mf_element_tet10_affine(int n_el, int e, const T *__restrict__ gf, XL &&xl,
-                                                                 Out &&out, T rho = T(0)) {
+// gl(q, k) gives factor k of factor set q (set 0 here).
+template <typename T, bool FOLD = false, typename GL, typename XL, typename Out>
+__host__ __device__ __forceinline__ void mf_element_tet10_affine(GL &&gl, XL &&xl, Out &&out, T rho = T(0)) {
     constexpr int EDG[4][4] = {{-1, 4, 6, 7}, {4, -1, 5, 8}, {6, 5, -1, 9}, {7, 8, 9, -1}};
     T u[10][3];
     T v0[3];
@@ -49,13 +49,9 @@ __host__ __device__ __forceinline__ void mf_element_tet10_affine(int n_el, int e
         for (int c = 0; c < 3; ++c) u[i][c] = v[c] - v0[c];   // translation removed (FP32)
     }
     T Ji[9];
-    auto gld = [&](int k) -> T {
-        return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(gf) +
-                                            (uint32_t)sizeof(T) * (uint32_t)(k * n_el + e));
-    };
 #pragma unroll
-    for (int k = 0; k < 9; ++k) Ji[k] = gld(k);
-    const T cl = FOLD ? rho : T(0.2) * gld(9), cm = FOLD ? T(1) : T(0.2) * gld(10);
+    for (int k = 0; k < 9; ++k) Ji[k] = gl(0, k);
+    const T cl = FOLD ? rho : T(0.2) * gl(0, 9), cm = FOLD ? T(1) : T(0.2) * gl(0, 10);
     T P[4][9];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -111,24 +107,39 @@ __host__ __device__ __forceinline__ void mf_element_tet10_affine(int n_el, int e
     }
 }
 
-// Element e with node values read through xl(i, v): v = x at local node i;
-// geometric factors gf[(q * GF + k) * n_el + e]; out(i, f0, f1, f2) receives
-// node i's terms.
-template <int NPE, typename T, bool AFF, typename XL, typename Out>
-__host__ __device__ __forceinline__ void mf_element_gp(int n_el, int e, const T *__restrict__ gf, XL &&xl, Out &&out);
+// The element with node values read through xl(i, v): v = x at local node i;
+// geometric factor k of set q (affine: set 0) through gl(q, k); out(i, f0,
+// f1, f2) receives node i's terms.
+template <int NPE, typename T, bool AFF, typename GL, typename XL, typename Out>
+__host__ __device__ __forceinline__ void mf_element_gp(GL &&gl, XL &&xl, Out &&out);
 
+template <int NPE, typename T, bool AFF, bool FOLD = false, typename GL, typename XL, typename Out>
+__host__ __device__ __forceinline__ void mf_element_f(GL &&gl, XL &&xl, Out &&out, T rho = T(0)) {
+    if constexpr (NPE == 10 && AFF)
+        mf_element_tet10_affine<T, FOLD>(gl, xl, out, rho);
+    else
+        mf_element_gp<NPE, T, AFF>(gl, xl, out);
+}
+
+// The same with the factors of element e read from gf[(q * GF + k) * n_el + e].
 template <int NPE, typename T, bool AFF, bool FOLD = false, typename XL, typename Out>
 __host__ __device__ __forceinline__ void mf_element_x(int n_el, int e, const T *__restrict__ gf, XL &&xl, Out &&out,
                                                       T rho = T(0)) {
-    if constexpr (NPE == 10 && AFF)
-        mf_element_tet10_affine<T, FOLD>(n_el, e, gf, xl, out, rho);
+    if constexpr (NPE == 10 && AFF)  // one set below 4 GiB: 32-bit offsets from the uniform base
+        mf_element_f<NPE, T, AFF, FOLD>(
+            [&](int, int k) -> T {
+                return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(gf) +
+                                                    (uint32_t)sizeof(T) * (uint32_t)(k * n_el + e));
+            },
+            xl, out, rho);
     else
-        mf_element_gp<NPE, T, AFF>(n_el, e, gf, xl, out);
+        mf_element_f<NPE, T, AFF, FOLD>(
+            [&](int q, int k) -> T { return gf[(size_t)(q * GF + k) * n_el + e]; }, xl, out, rho);
 }
 
 // The Gauss-point form: every element type, affine or not.
-template <int NPE, typename T, bool AFF, typename XL, typename Out>
-__host__ __device__ __forceinline__ void mf_element_gp(int n_el, int e, const T *__restrict__ gf, XL &&xl, Out &&out) {
+template <int NPE, typename T, bool AFF, typename GL, typename XL, typename Out>
+__host__ __device__ __forceinline__ void mf_element_gp(GL &&gl, XL &&xl, Out &&out) {
     using EL = Elem<NPE>;
     constexpr int NG = EL::NGP;
     T H[NG][9];
@@ -157,11 +168,10 @@ __host__ __device__ __forceinline__ void mf_element_gp(int n_el, int e, const T 
     }
     T Ji[9], cl, cm;
     auto load = [&](int q) {
-        const T *g = gf + (size_t)q * GF * n_el + e;
 #pragma unroll
-        for (int k = 0; k < 9; ++k) Ji[k] = g[(size_t)k * n_el];
-        cl = g[(size_t)9 * n_el];
-        cm = g[(size_t)10 * n_el];
+        for (int k = 0; k < 9; ++k) Ji[k] = gl(q, k);
+        cl = gl(q, 9);
+        cm = gl(q, 10);
     };
     if (AFF) load(0);
 #pragma unroll

@@ -386,13 +386,24 @@ void jfem_patch_release(jfm_ctx *ctx) {
 // not fit its type.
 struct PatchHost {
     int npatch = 0;
+    // with `cells`: patch nodes' ids, partial slots (-1: interior), first slot
+    // of the node << 5 | slots, local connectivity (position in the patch)
+    // and the incidences (i, e) of patch node l at lin[pn_inc[l]..]: 3 i stride
+    // + local element, ascending
+    std::vector<int32_t> pn_node, pn_slot, pn_sh, pn_inc;
+    std::vector<uint16_t> connL, lin;
+    int pn_max = 0, slots_max = 0;
+    bool orphans = false;  // a node of no element
     std::vector<int32_t> perm, connP, pn_ptr, pn_out, rstart, rbase, bnode, bptr, pbase;
     std::vector<uint16_t> connP16;  // empty when a patch spans more than 65,536 node ids
     std::vector<uint16_t> pn_cnt, linT;
 };
 
+// ps: elements per patch (and nodes per round); stride > 0: the form of the
+// resident PCG (cells), whose LDS rows have this stride.
 static bool build_patches(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int64_t N,
-                          int npe, PatchHost &P) {
+                          int npe, int ps, int stride, PatchHost &P) {
+    const bool cells = stride > 0;
     // Morton order of the element centroids (stable in element id)
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
     for (int64_t a = 0; a < N; ++a)
@@ -421,7 +432,7 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
     code.shrink_to_fit();
     std::vector<int32_t> val(N, 0);  // node valences
     for (int32_t v : conn) ++val[v];
-    const int npatch = (int)((n_el + kPatch - 1) / kPatch);
+    const int npatch = (int)((n_el + ps - 1) / ps);
     P.npatch = npatch;
     P.connP.assign((size_t)npe * n_el, 0);
     P.pn_ptr.assign(npatch + 1, 0);
@@ -430,51 +441,63 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
     P.pn_cnt.clear();
     P.rbase.clear();
     P.linT.clear();
+    if (cells) P.connL.assign((size_t)npe * n_el, 0);
     std::vector<std::vector<int32_t>> shared_l(N);  // per node: patch-node indices, ascending patch
-    std::vector<std::pair<int64_t, int32_t>> pairs;  // (node * kPatch + local element, i)
+    std::vector<std::pair<int64_t, int32_t>> pairs;  // (node * ps + local element, i)
     struct PNode { int32_t a, first, cnt; };
     std::vector<PNode> nodes;
     for (int p = 0; p < npatch; ++p) {
-        const int64_t k0 = (int64_t)p * kPatch, k1 = std::min<int64_t>(k0 + kPatch, n_el);
+        const int64_t k0 = (int64_t)p * ps, k1 = std::min<int64_t>(k0 + ps, n_el);
         pairs.clear();
         for (int64_t k = k0; k < k1; ++k) {
             const int32_t e = perm[k];
             for (int i = 0; i < npe; ++i) {
                 const int32_t a = conn[(size_t)e * npe + i];
                 P.connP[(size_t)i * n_el + k] = a;
-                pairs.emplace_back((int64_t)a * kPatch + (k - k0), i);
+                pairs.emplace_back((int64_t)a * ps + (k - k0), i);
             }
         }
         std::sort(pairs.begin(), pairs.end());  // by node, then local element
         nodes.clear();
         for (size_t r = 0; r < pairs.size();) {
-            const int32_t a = (int32_t)(pairs[r].first / kPatch);
+            const int32_t a = (int32_t)(pairs[r].first / ps);
             size_t r2 = r;
-            while (r2 < pairs.size() && pairs[r2].first / kPatch == a) ++r2;
+            while (r2 < pairs.size() && pairs[r2].first / ps == a) ++r2;
             nodes.push_back({a, (int32_t)r, (int32_t)(r2 - r)});
             r = r2;
         }
         // most incidences first, so that a round's counts are close
         std::stable_sort(nodes.begin(), nodes.end(), [](const PNode &u, const PNode &v) { return u.cnt > v.cnt; });
         const int64_t l0 = (int64_t)P.pn_out.size();
-        for (size_t u = 0; u < nodes.size(); u += kPatch) {
+        for (size_t u = 0; u < nodes.size() && !cells; u += ps) {
             const int cntmax = nodes[u].cnt;
             const int64_t base = (int64_t)P.linT.size();
             if (base > INT32_MAX) return false;
             P.rbase.push_back((int32_t)base);
-            P.linT.resize(base + (size_t)cntmax * kPatch, 0);
-            for (size_t t = 0; t < (size_t)kPatch && u + t < nodes.size(); ++t) {
+            P.linT.resize(base + (size_t)cntmax * ps, 0);
+            for (size_t t = 0; t < (size_t)ps && u + t < nodes.size(); ++t) {
                 const PNode &nd = nodes[u + t];
                 for (int j = 0; j < nd.cnt; ++j) {
                     const auto &pr = pairs[nd.first + j];
-                    const int kl = (int)(pr.first % kPatch), i = pr.second;
-                    P.linT[base + (size_t)j * kPatch + t] = (uint16_t)(3 * i * kPatch + kl);
+                    const int kl = (int)(pr.first % ps), i = pr.second;
+                    P.linT[base + (size_t)j * ps + t] = (uint16_t)(3 * i * ps + kl);
                 }
             }
         }
+        P.pn_max = std::max(P.pn_max, (int)nodes.size());
         for (size_t u = 0; u < nodes.size(); ++u) {
             const PNode &nd = nodes[u];
             if (nd.cnt > 65535) return false;
+            if (cells) {
+                P.pn_node.push_back(nd.a);
+                P.pn_inc.push_back((int32_t)P.lin.size());
+                for (int j = 0; j < nd.cnt; ++j) {
+                    const auto &pr = pairs[nd.first + j];
+                    const int kl = (int)(pr.first % ps);
+                    P.connL[(size_t)pr.second * n_el + k0 + kl] = (uint16_t)u;
+                    P.lin.push_back((uint16_t)(3 * pr.second * stride + kl));
+                }
+            }
             P.pn_cnt.push_back((uint16_t)nd.cnt);
             if (nd.cnt == val[nd.a]) {
                 P.pn_out.push_back(nd.a);  // interior
@@ -493,7 +516,10 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
         if (!shared_l[a].empty()) order.push_back((int32_t)a);
     std::sort(order.begin(), order.end(), [&](int32_t u, int32_t v) { return shared_l[u][0] < shared_l[v][0]; });
     for (int64_t a = 0; a < N; ++a)
-        if (val[a] == 0) order.push_back((int32_t)a);
+        if (val[a] == 0) {
+            order.push_back((int32_t)a);
+            P.orphans = true;
+        }
     P.bnode.clear();
     P.bptr.assign(1, 0);
     for (int32_t a : order) {
@@ -502,12 +528,26 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
         for (size_t j = 0; j < shared_l[a].size(); ++j) P.pn_out[shared_l[a][j]] = -(P.bptr.back() + (int32_t)j + 1);
         P.bptr.push_back(P.bptr.back() + (int32_t)shared_l[a].size());
     }
+    if (cells) {
+        P.pn_slot.assign(P.pn_out.size(), -1);
+        P.pn_sh.assign(P.pn_out.size(), 0);
+        for (size_t b = 0; b < P.bnode.size(); ++b) {
+            const int32_t first = P.bptr[b], n = P.bptr[b + 1] - first;
+            P.slots_max = std::max(P.slots_max, (int)n);
+            for (int j = 0; j < n; ++j) {
+                const int32_t l = shared_l[P.bnode[b]][j];
+                P.pn_slot[l] = first + j;
+                P.pn_sh[l] = first << 5 | (n & 31);
+            }
+        }
+        return 3 * npe * stride <= 65536 && (int64_t)P.pn_out.size() < INT32_MAX / 3;
+    }
     // 16-bit connectivity relative to each patch's lowest node id, when every
     // patch's ids span at most 65,536
     P.pbase.assign(npatch, 0);
     bool fits16 = true;
     for (int p = 0; p < npatch && fits16; ++p) {
-        const int64_t k0 = (int64_t)p * kPatch, k1 = std::min<int64_t>(k0 + kPatch, n_el);
+        const int64_t k0 = (int64_t)p * ps, k1 = std::min<int64_t>(k0 + ps, n_el);
         int32_t lo = INT32_MAX, hi = -1;
         for (int i = 0; i < npe; ++i)
             for (int64_t k = k0; k < k1; ++k) {
@@ -521,9 +561,9 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
         P.connP16.assign((size_t)npe * n_el, 0);
         for (int i = 0; i < npe; ++i)
             for (int64_t k = 0; k < n_el; ++k)
-                P.connP16[(size_t)i * n_el + k] = (uint16_t)(P.connP[(size_t)i * n_el + k] - P.pbase[k / kPatch]);
+                P.connP16[(size_t)i * n_el + k] = (uint16_t)(P.connP[(size_t)i * n_el + k] - P.pbase[k / ps]);
     }
-    return 3 * (npe - 1) * kPatch + kPatch <= 65536 && (int64_t)P.pn_out.size() < INT32_MAX / 3;
+    return 3 * (npe - 1) * ps + ps <= 65536 && (int64_t)P.pn_out.size() < INT32_MAX / 3;
 }
 
 // Builds the patch structure for the uploaded mesh (once per mesh).
@@ -535,7 +575,7 @@ int jfem_patch_setup(jfm_ctx *ctx) {
     if ((int64_t)ctx->h_conn.size() != n_el * npe || (int64_t)ctx->h_X.size() != 3 * N)
         return jfm_fail(ctx, JFM_ESTATE, "patch setup needs the host mesh");
     PatchHost P;
-    if (!build_patches(ctx->h_conn, ctx->h_X, n_el, N, npe, P))
+    if (!build_patches(ctx->h_conn, ctx->h_X, n_el, N, npe, kPatch, 0, P))
         return jfm_fail(ctx, JFM_EINVAL, "patch structure out of range");
     const int npatch = P.npatch;
     const int64_t npn = (int64_t)P.pn_out.size(), nb = (int64_t)P.bnode.size();
@@ -608,6 +648,62 @@ int jfem_patch_setup(jfm_ctx *ctx) {
     for (int64_t i = 0; i < nb; ++i) ctx->bmaxcnt = std::max(ctx->bmaxcnt, P.bptr[i + 1] - P.bptr[i]);
     ctx->patch_ready = true;
     return JFM_OK;
+}
+
+// The resident PCG's patches (persist.hip), once per mesh: the same structure
+// in that kernel's patch size, with local connectivity and, per patch node,
+// its id, slots and incidences.  cells.usable tells whether the mesh fits.
+int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g) {
+    auto &C = ctx->cells;
+    if (C.ready) return JFM_OK;
+    C.ready = true;
+    C.usable = false;
+    const int64_t n_el = ctx->n_el, N = ctx->N;
+    const int npe = ctx->npe;
+    if ((int64_t)ctx->h_conn.size() != n_el * npe || (int64_t)ctx->h_X.size() != 3 * N) return JFM_OK;
+    PatchHost P;
+    if (!build_patches(ctx->h_conn, ctx->h_X, n_el, N, npe, g.elems, g.stride, P)) return JFM_OK;
+    // pn_sh holds 26 bits of slot and 5 of count; a node of no element is in no patch
+    if (P.orphans || P.slots_max > 31 || P.bptr.back() >= (1 << 25) || P.pn_max > g.threads) return JFM_OK;
+    hipStream_t s = ctx->stream;
+    auto put = [&](auto *&dst, const auto &v) -> bool {
+        using V = std::decay_t<decltype(v[0])>;
+        dst = jfm_alloc<V>(ctx, std::max<int64_t>(1, (int64_t)v.size()));
+        return dst && (v.empty() || hipMemcpyAsync(dst, v.data(), sizeof(V) * v.size(), hipMemcpyHostToDevice, s) == hipSuccess);
+    };
+    const int64_t rows = (int64_t)ctx->ngf * GF;
+    bool ok = put(C.eperm, P.perm) && put(C.connL, P.connL) && put(C.pn_ptr, P.pn_ptr) && put(C.pn_cnt, P.pn_cnt) &&
+              put(C.pn_node, P.pn_node) && put(C.pn_slot, P.pn_slot) && put(C.pn_sh, P.pn_sh) &&
+              put(C.pn_inc, P.pn_inc) && put(C.lin, P.lin);
+    ok = ok && (C.gf64 = jfm_alloc<double>(ctx, rows * n_el)) && (C.gf32 = jfm_alloc<float>(ctx, rows * n_el)) &&
+         (C.part = jfm_alloc<double>(ctx, 4 * std::max<int64_t>(1, P.bptr.back()))) &&
+         (C.words = jfm_alloc<uint64_t>(ctx, kPersistWords * ((int64_t)P.npatch + 256)));
+    const bool fold = ctx->affine && npe == 10 && ctx->nu_uniform;
+    if (ok && fold) ok = (C.gfQ32 = jfm_alloc<float>(ctx, 9 * n_el)) != nullptr;
+    if (!ok) {
+        jfem_cells_release(ctx);
+        (void)hipStreamSynchronize(s);  // host vectors go out of scope
+        return jfm_fail(ctx, JFM_ENOMEM, "resident PCG allocation failed");
+    }
+    k_permute_gf<double><<<1024, 256, 0, s>>>(rows, (int)n_el, C.eperm, ctx->gf64, C.gf64);
+    k_permute_gf<float><<<1024, 256, 0, s>>>(rows, (int)n_el, C.eperm, ctx->gf32, C.gf32);
+    if (fold) k_fold_gf<<<1024, 256, 0, s>>>((int)n_el, C.gf64, C.gfQ32);
+    JFM_HIP(ctx, hipGetLastError());
+    JFM_HIP(ctx, hipStreamSynchronize(s));
+    C.npatch = P.npatch;
+    C.nslot = P.bptr.back();
+    C.rho32 = (float)(2.0 * ctx->nu0 / (1.0 - 2.0 * ctx->nu0));
+    C.usable = true;
+    return JFM_OK;
+}
+
+void jfem_cells_release(jfm_ctx *ctx) {
+    auto &C = ctx->cells;
+    for (void *p : {(void *)C.eperm, (void *)C.connL, (void *)C.pn_ptr, (void *)C.pn_cnt, (void *)C.pn_node, (void *)C.pn_slot,
+                    (void *)C.pn_sh, (void *)C.pn_inc, (void *)C.lin, (void *)C.gf64, (void *)C.gf32,
+                    (void *)C.gfQ32, (void *)C.part, (void *)C.words})
+        jfm_free(ctx, p);
+    C = {};
 }
 
 // qsrc for the update kernel of the two-level PCG (nodes in aggregate order)

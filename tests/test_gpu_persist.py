@@ -1,0 +1,116 @@
+"""The resident PCG (persist.hip), through the C ABI.
+
+Meshes at the edges of its patches (128 Tet10 or 512 Tet4 elements), of its
+groups of 16 workgroups and of its range (256 workgroups), against the oracle's
+direct solve, and against the launched iterations (JFEM_PERSIST=0, a child
+process): the FP64 iteration counts differ only by the order of the reductions
+(3% + 2; the FP32 inner solves restart at FP32's attainable residual, where
+rounding decides the count), the answers are bit-reproducible.  The bars follow from the solves'
+own tolerance: the residual 1e-10 (1e-11 is below what the FP64
+residual of such a cantilever can show) bounds the error at 1e-8 for these meshes
+(the direct solve itself is good to 1e-10).
+"""
+import json
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from jfem import mesh as M
+
+pytestmark = pytest.mark.gpu
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+# name -> (generator, grid); workgroups in the comments
+CASES = {
+    "tet10_6": ("box_tet10", (1, 1, 1)),        # 1, six elements
+    "tet10_126": ("box_tet10", (7, 3, 1)),      # 1, two elements short of a patch
+    "tet10_132": ("box_tet10", (11, 2, 1)),     # 2, four elements in the second
+    "tet10_2016": ("box_tet10", (14, 6, 4)),    # 16, one group
+    "tet10_2052": ("box_tet10", (19, 6, 3)),    # 17, two groups, the second of one
+    "tet4_510": ("box_tet4", (17, 5, 1)),       # 1
+    "tet4_10368": ("box_tet4", (24, 9, 8)),     # 21
+}
+_CHILD = r"""
+import json, sys
+sys.path[:0] = [{pkg!r}]
+import jfem
+from jfem import mesh as M
+out = {{}}
+for name, (gen, g) in json.loads({cases!r}).items():
+    m = getattr(M, gen)(*g, seed=5, jitter=0.1, E_sigma=0.4)
+    c = jfem.Context(0)
+    c.upload(m)
+    for meth in (0, 1):
+        print("launched", name, meth, flush=True)
+        out[f"{{name}}/{{meth}}"] = c.solve(method=meth, rtol=1e-10, inner_rtol=1e-2)[2]["iterations"]
+    c.close()
+json.dump(out, open({out!r}, "w"))
+"""
+
+
+def say(msg):
+    print(f"[gpu] {msg}", flush=True)
+
+
+@pytest.fixture(scope="module")
+def launched(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("launched") / "it.json")
+    code = _CHILD.format(pkg=os.path.join(ROOT, "juliafem.jl_amd"), cases=json.dumps(CASES), out=out)
+    subprocess.run([sys.executable, "-c", code], env=dict(os.environ, JFEM_PERSIST="0"), check=True, timeout=120)
+    return json.load(open(out))
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_resident_pcg(oracle, launched, name):
+    import jfem
+    gen, g = CASES[name]
+    m = getattr(M, gen)(*g, seed=5, jitter=0.1, E_sigma=0.4)
+    csr = oracle.assemble_csr(m)
+    ud, _, _ = oracle.solve_direct_lapack(csr, m.fixed_mask(), np.zeros(m.n_dofs), oracle.load_vector(m))
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    for meth in (0, 1):   # FP64 PCG; FP32 PCG in FP64 refinement
+        say(f"resident {name} method={meth} nodes={m.n_nodes} el={m.n_el}")
+        u, _, st = ctx.solve(method=meth, rtol=1e-10, inner_rtol=1e-2)
+        u2, _, _ = ctx.solve(method=meth, rtol=1e-10, inner_rtol=1e-2)
+        assert np.array_equal(u, u2)
+        assert np.linalg.norm(u - ud) <= 1e-8 * np.linalg.norm(ud)
+        it = launched[f"{name}/{meth}"]
+        if meth == 1 or it > m.n_dofs - 3 * len(m.clamp_nodes):
+            continue   # past CG's exact termination the count is rounding alone
+        assert abs(st["iterations"] - it) <= 2 + 0.03 * it
+    ctx.close()
+
+
+def test_resident_edges(oracle):
+    """Iteration cap, a zero load, prescribed displacements, user blocks and a
+    given right-hand side behave as in the launched form."""
+    import jfem
+    m = M.box_tet10(12, 3, 3, seed=8, jitter=0.1, E_sigma=0.4)
+    csr = oracle.assemble_csr(m)
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    say("iteration cap")
+    u, _, st = ctx.solve(rtol=1e-10, maxit=7, raise_on_noconv=False)
+    assert st["iterations"] == 7 and st["converged"] == 0 and np.all(np.isfinite(u))
+    say("zero load")
+    u, _, st = ctx.solve(f=np.zeros(m.n_dofs))
+    assert not np.any(u) and st["iterations"] == 0
+    say("user blocks")
+    blocks = np.tile(np.eye(3).ravel(), (m.n_nodes, 1)) * 1e-4
+    ctx.set_preconditioner_blocks(blocks)
+    f = oracle.load_vector(m) * 3.0
+    u, la, _ = ctx.solve(f=f, precond=2, rtol=1e-10, maxit=100000, want_la=True)
+    ud, lad, _ = oracle.solve_direct_lapack(csr, m.fixed_mask(), np.zeros(m.n_dofs), f)
+    assert np.linalg.norm(u - ud) <= 1e-8 * np.linalg.norm(ud)
+    say("prescribed displacements")
+    g = np.zeros(m.n_dofs)
+    g[3 * m.clamp_nodes + 2] = 1e-3
+    ctx.upload_bcs(m.fixed_mask(), g, m.faces, m.ftype, m.face_traction())
+    u, la, _ = ctx.solve(rtol=1e-10, want_la=True)
+    ud, lad, _ = oracle.solve_direct_lapack(csr, m.fixed_mask(), g, oracle.load_vector(m))
+    assert np.linalg.norm(u - ud) <= 1e-8 * np.linalg.norm(ud)
+    ctx.close()
