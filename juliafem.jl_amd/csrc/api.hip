@@ -169,6 +169,8 @@ static void release_heat(jfm_ctx *ctx) {
     free_ptr(ctx, ctx->heat_k); free_ptr(ctx, ctx->heat_fixed); free_ptr(ctx, ctx->heat_g); free_ptr(ctx, ctx->heat_Minv);
     free_ptr(ctx, ctx->hf_conn); free_ptr(ctx, ctx->hf_ptr); free_ptr(ctx, ctx->hf_inc); free_ptr(ctx, ctx->hf_h);
     free_ptr(ctx, ctx->hf_g); free_ptr(ctx, ctx->hf_text); free_ptr(ctx, ctx->hf_fe);
+    free_ptr(ctx, ctx->hf_first); free_ptr(ctx, ctx->hf_next); free_ptr(ctx, ctx->hf_map); free_ptr(ctx, ctx->hf_K);
+    ctx->heat_resident = false;
     ctx->hf_n = 0;
     ctx->hf_nfn = 0;
 }
@@ -922,8 +924,8 @@ static int pcg_run(jfm_ctx *ctx, int op, const T *Minv, double rtol, int maxit, 
     const int64_t n = ctx->ndof;
     hipStream_t s = ctx->stream;
     int np = 0;
-    bool resident = false;
-    if (!coarse)
+    int resident = coarse ? 0 : 1;
+    if (resident)
         if (int rc = jfem_persist_ready<T>(ctx, op, &resident)) return rc;
     if (resident) {
         const bool from_x = warm && sizeof(T) == 8;
@@ -931,7 +933,7 @@ static int pcg_run(jfm_ctx *ctx, int op, const T *Minv, double rtol, int maxit, 
             CHECK_LAUNCH(ctx, op_apply<T>(ctx, op, x, q, nullptr, nullptr, nullptr, nullptr));
             CHECK_LAUNCH(ctx, launch_residual(ctx, (const double *)b, (const double *)q, ctx->fixed, (double *)r, n, &np));
         }
-        CHECK_LAUNCH(ctx, launch_pcg_persist<T>(ctx, Minv, b, from_x ? r : nullptr, x, rtol, maxit));
+        CHECK_LAUNCH(ctx, launch_pcg_persist<T>(ctx, op, Minv, b, from_x ? r : nullptr, x, rtol, maxit));
         if (int rc = read_scalars(ctx)) return rc;
         if (!ctx->S_host->fail) {
             *iters = ctx->S_host->iter;
@@ -1507,6 +1509,36 @@ extern "C" int jfm_solve_nonlinear(jfm_ctx *ctx, const jfm_newton_opts *opts, do
 }
 
 // ========================================================= postprocessing ==
+// M x_k = b_k for the nsys right-hand sides at b + k n, x likewise (M the
+// consistent mass, Mm its inverse diagonal).
+static int mass_solves(jfm_ctx *ctx, const double *Mm, int nsys, const double *b, double *x) {
+    const int64_t n = ctx->ndof;
+    hipStream_t s = ctx->stream;
+    const double rtol = 1e-13;
+    const int maxit = 2000;
+    int beside = nsys;
+    if (int rc = jfem_persist_ready<double>(ctx, kOpMass, &beside)) return rc;
+    if (beside > 1) {
+        std::vector<PcgScalars> S(beside);
+        for (int k = 0; k < nsys && beside > 1; k += beside) {
+            CHECK_LAUNCH(ctx, launch_pcg_persist<double>(ctx, kOpMass, Mm, b + k * n, nullptr, x + k * n, rtol, maxit, beside, n));
+            JFM_HIP(ctx, hipMemcpyAsync(S.data(), ctx->cells.S, sizeof(PcgScalars) * beside, hipMemcpyDeviceToHost, s));
+            if (int rc = sync(ctx)) return rc;
+            for (const PcgScalars &v : S)
+                if (v.fail) ctx->persist_off = true;
+            if (ctx->persist_off) beside = 0;
+        }
+        if (beside) return JFM_OK;
+    }
+    for (int k = 0; k < nsys; ++k) {
+        JFM_HIP(ctx, hipMemcpyAsync(ctx->ws64.b, b + k * n, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
+        int it = 0, status = 0;
+        if (int rc = pcg_run<double>(ctx, kOpMass, Mm, rtol, maxit, 32, &it, &status)) return rc;
+        JFM_HIP(ctx, hipMemcpyAsync(x + k * n, ctx->ws64.x, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
+    }
+    return JFM_OK;
+}
+
 extern "C" int jfm_postprocess(jfm_ctx *ctx, const double *u, double *strain_gp, double *stress_gp,
                                double *strain_nodal, double *stress_nodal) {
     if (!ctx || !u) return JFM_EINVAL;
@@ -1545,22 +1577,25 @@ extern "C" int jfm_postprocess(jfm_ctx *ctx, const double *u, double *strain_gp,
     if (rc == JFM_OK && (strain_nodal || stress_nodal)) {
         e = launch_mass_diag(ctx, Mm);
         if (e != hipSuccess) fail_hip(e, "launch_mass_diag");
-        std::vector<double> part(n);
+        // the fits are one operator with two right-hand sides per field, all
+        // of them side by side where the resident PCG takes them
         double *outs[2] = {strain_nodal, stress_nodal};
-        for (int f = 0; f < 2 && rc == JFM_OK; ++f) {
-            if (!outs[f]) continue;
-            for (int comp0 = 0; comp0 < 6 && rc == JFM_OK; comp0 += 3) {
-                e = launch_post_rhs(ctx, du, f, comp0, (double *)ctx->ws64.b);
-                if (e != hipSuccess) { fail_hip(e, "launch_post_rhs"); break; }
-                int it = 0, status = 0;
-                if ((rc = pcg_run<double>(ctx, kOpMass, Mm, 1e-13, 2000, 32, &it, &status))) break;
-                e = hipMemcpyAsync(part.data(), ctx->ws64.x, sizeof(double) * n, hipMemcpyDeviceToHost, s);
-                if (e == hipSuccess) e = hipStreamSynchronize(s);
-                if (e != hipSuccess) { fail_hip(e, "nodal copy"); break; }
-                for (int64_t a = 0; a < N; ++a)
-                    for (int c = 0; c < 3; ++c) outs[f][6 * a + comp0 + c] = part[3 * a + c];
-            }
+        int nf = 0, field[2];
+        for (int f = 0; f < 2; ++f)
+            if (outs[f]) field[nf++] = f;
+        const int nsys = 2 * nf;
+        double *B = jfm_alloc<double>(ctx, nsys * n), *X = jfm_alloc<double>(ctx, nsys * n), *J = jfm_alloc<double>(ctx, 6 * N);
+        if (!B || !X || !J) rc = jfm_fail(ctx, JFM_ENOMEM, "device allocation failed in jfm_postprocess");
+        for (int k = 0; k < nsys && rc == JFM_OK; ++k)
+            if ((e = launch_post_rhs(ctx, du, field[k / 2], 3 * (k % 2), B + k * n)) != hipSuccess) fail_hip(e, "launch_post_rhs");
+        if (rc == JFM_OK) rc = mass_solves(ctx, Mm, nsys, B, X);
+        for (int f = 0; f < nf && rc == JFM_OK; ++f) {
+            e = launch_post_join(ctx, X + (2 * f) * n, X + (2 * f + 1) * n, J);
+            if (e == hipSuccess) e = hipMemcpyAsync(outs[field[f]], J, sizeof(double) * 6 * N, hipMemcpyDeviceToHost, s);
+            if (e != hipSuccess) fail_hip(e, "nodal copy");
         }
+        (void)hipStreamSynchronize(s);
+        for (void *p : {(void *)B, (void *)X, (void *)J}) jfm_free(ctx, p);
     }
     (void)hipStreamSynchronize(s);
     cleanup();
@@ -1638,6 +1673,7 @@ extern "C" int jfm_heat_solve(jfm_ctx *ctx, const double *k, const double *q, in
                 JFM_HIP(ctx, hipMemcpyAsync(*dst, v, sizeof(double) * n_faces, hipMemcpyHostToDevice, s));
             }
     }
+    if (int rc = jfem_heat_faces(ctx)) return rc;
     // the heat row mask stands in for the elasticity one for this solve
     struct MaskSwap {
         jfm_ctx *c;

@@ -140,6 +140,124 @@ __global__ __launch_bounds__(256) void k_heat_face(int nf, int nfn, const int32_
         for (int c = 0; c < 3; ++c) fe[((size_t)f * nfn + i) * 3 + c] = out[i][c];
 }
 
+// For the resident form: the element that holds all nodes of a face (the first
+// in the incidence order of the face's first node), the face's nodes in that
+// element's numbering (4 bits each), and its convection matrix sum_q w detJ h
+// N N' (6 x 6, zero padded).
+__global__ __launch_bounds__(256) void k_heat_owner(int nf, int nfn, int npe, int n_el, const int32_t *__restrict__ fconn,
+                                                   const int32_t *__restrict__ conn, const int32_t *__restrict__ ptr,
+                                                   const int32_t *__restrict__ inc, const double *__restrict__ X,
+                                                   const double *__restrict__ h, int32_t *__restrict__ owner,
+                                                   int32_t *__restrict__ map, double *__restrict__ K) {
+    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= nf) return;
+    int nd[6], found = -1, m = 0;
+    double Xf[6][3];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+        nd[i] = i < nfn ? fconn[(size_t)i * nf + f] : -1;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) Xf[i][c] = i < nfn ? X[3 * (size_t)nd[i] + c] : 0.0;
+    }
+    for (int k = ptr[nd[0]]; k < ptr[nd[0] + 1] && found < 0; ++k) {
+        const int e = inc[k] / npe;
+        int hit = 0;
+        m = 0;
+        for (int i = 0; i < npe; ++i) {
+            const int a = conn[(size_t)i * n_el + e];
+#pragma unroll
+            for (int j = 0; j < 6; ++j)
+                if (j < nfn && nd[j] == a) {
+                    m |= i << (4 * j);
+                    ++hit;
+                }
+        }
+        if (hit == nfn) found = e;
+    }
+    owner[f] = found;
+    map[f] = m;
+    double Kf[6][6];
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+        for (int j = 0; j < 6; ++j) Kf[i][j] = 0.0;
+    double w[4], pu[4], pv[4];
+    const int ng = surf_rule(nfn, w, pu, pv);
+    for (int q = 0; q < ng; ++q) {
+        double N[6] = {0, 0, 0, 0, 0, 0}, dN[6][2] = {};
+        surf_basis(nfn, pu[q], pv[q], N, dN);
+        double J[2][3] = {{0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int b = 0; b < 3; ++b) J[a][b] += dN[i][a] * Xf[i][b];
+        const double cx = J[0][1] * J[1][2] - J[0][2] * J[1][1];
+        const double cy = J[0][2] * J[1][0] - J[0][0] * J[1][2];
+        const double cz = J[0][0] * J[1][1] - J[0][1] * J[1][0];
+        const double wq = w[q] * sqrt(cx * cx + cy * cy + cz * cz) * h[f];
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+#pragma unroll
+            for (int j = 0; j < 6; ++j) Kf[i][j] += wq * N[i] * N[j];
+    }
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+        for (int j = 0; j < 6; ++j) K[(size_t)f * 36 + 6 * i + j] = Kf[i][j];
+}
+
+hipError_t launch_heat_owner(jfm_ctx *ctx, int32_t *owner, int32_t *map, double *K) {
+    const int nf = (int)ctx->hf_n;
+    k_heat_owner<<<nblk(nf), kBlock, 0, ctx->stream>>>(nf, ctx->hf_nfn, ctx->npe, (int)ctx->n_el, ctx->hf_conn, ctx->conn,
+                                                       ctx->inc_ptr, ctx->inc, ctx->X, ctx->hf_h, owner, map, K);
+    return hipGetLastError();
+}
+
+// Lists the convection faces by element for the resident PCG (persist.hip).  A
+// face whose nodes are in no one element leaves the launched form.
+int jfem_heat_faces(jfm_ctx *ctx) {
+    ctx->heat_resident = false;
+    if (ctx->hf_n == 0 || !ctx->hf_h) {
+        ctx->heat_resident = true;
+        return JFM_OK;
+    }
+    ctx->heat_resident = true;  // as far as the faces go, to learn whether the mesh fits
+    int one = 1;
+    if (int rc = jfem_persist_ready<double>(ctx, kOpHeat, &one)) return rc;
+    ctx->heat_resident = false;
+    if (!one) return JFM_OK;
+    const int nf = (int)ctx->hf_n;
+    const int64_t n_el = ctx->n_el;
+    int32_t *d_owner = jfm_alloc<int32_t>(ctx, nf);
+    ctx->hf_map = jfm_alloc<int32_t>(ctx, nf);
+    ctx->hf_next = jfm_alloc<int32_t>(ctx, nf);
+    ctx->hf_first = jfm_alloc<int32_t>(ctx, n_el);
+    ctx->hf_K = jfm_alloc<double>(ctx, 36 * (int64_t)nf);
+    if (!d_owner || !ctx->hf_map || !ctx->hf_next || !ctx->hf_first || !ctx->hf_K) {
+        jfm_free(ctx, d_owner);
+        return jfm_fail(ctx, JFM_ENOMEM, "device allocation failed in jfm_heat_solve");
+    }
+    std::vector<int32_t> owner(nf), first(n_el, -1), next(nf, -1);
+    hipError_t e = launch_heat_owner(ctx, d_owner, ctx->hf_map, ctx->hf_K);
+    if (e == hipSuccess) e = hipMemcpyAsync(owner.data(), d_owner, sizeof(int32_t) * nf, hipMemcpyDeviceToHost, ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    jfm_free(ctx, d_owner);
+    if (e != hipSuccess) return jfm_hip_fail(ctx, e, "convection faces");
+    for (int f = nf - 1; f >= 0; --f) {  // lists in ascending face order
+        if (owner[f] < 0) return JFM_OK;
+        int32_t &head = first[ctx->cells.epos[owner[f]]];
+        next[f] = head;
+        head = f;
+    }
+    JFM_HIP(ctx, hipMemcpyAsync(ctx->hf_first, first.data(), sizeof(int32_t) * n_el, hipMemcpyHostToDevice, ctx->stream));
+    JFM_HIP(ctx, hipMemcpyAsync(ctx->hf_next, next.data(), sizeof(int32_t) * nf, hipMemcpyHostToDevice, ctx->stream));
+    JFM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    ctx->heat_resident = true;
+    return JFM_OK;
+}
+
 // y_a = sum (element slots of a) + sum (face slots of a), rows masked;
 // optional partials of y . dotv.  The same fixed order as k_gather.
 __global__ __launch_bounds__(256) void k_heat_gather(int N, const int32_t *__restrict__ ptr, const double *__restrict__ yinc,

@@ -315,6 +315,11 @@ struct jfm_ctx {
     int hf_nfn = 0;
     int32_t *hf_conn = nullptr, *hf_ptr = nullptr, *hf_inc = nullptr;
     double *hf_h = nullptr, *hf_g = nullptr, *hf_text = nullptr, *hf_fe = nullptr;
+    // resident form: per element (patch order) its first convection face, per
+    // face the next one, its element-local nodes (4 bits each) and 6 x 6 matrix
+    bool heat_resident = false;
+    int32_t *hf_first = nullptr, *hf_next = nullptr, *hf_map = nullptr;
+    double *hf_K = nullptr;
     // patches of the resident PCG (persist.hip): smaller ones, with per patch
     // node its id, partial slot, slot range and incidences
     struct Cells {
@@ -327,7 +332,9 @@ struct jfm_ctx {
         double *gf64 = nullptr, *part = nullptr;  // part: 4 values per slot (FP32 or FP64 view)
         float *gf32 = nullptr, *gfQ32 = nullptr;
         uint64_t *words = nullptr;
-        int nslot = 0;
+        jfem::PcgScalars *S = nullptr;       // scalars of the systems solved side by side
+        int nslot = 0, systems = 0;          // systems that words, part and S hold
+        std::vector<int32_t> epos;           // element -> position in the patch order
     } cells;
     bool persist_off = false;      // a resident solve gave up waiting: this context launches its iterations
     double *Muser64 = nullptr;     // N x 9 user blocks (JFM_PREC_USER)
@@ -428,12 +435,19 @@ int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g);
 void jfem_cells_release(jfm_ctx *ctx);
 // Whether the PCG on `op` runs resident on this context (builds its patches
 // on first use); JFEM_PERSIST=0 turns it off.
-template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, bool *yes);
+// *nsys: the systems (right-hand sides of one operator) asked for; returns how
+// many of them can be solved side by side, 0: none, use the launched form.
+template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys);
+// makes room for m systems
+int jfem_cells_systems(jfm_ctx *ctx, int m);
+// heat: maps the convection faces to elements (ctx->heat_resident)
+int jfem_heat_faces(jfm_ctx *ctx);
 // Solves K x = b (r0 null) or continues from x with its residual r0; the
-// scalars are in ctx->S afterwards (S->fail set when a wait gave up, x then
-// untouched).
+// scalars are in ctx->S afterwards, for nsys > 1 (b and x of system s at + s
+// ss) in ctx->cells.S (fail set when a wait gave up, x then untouched).
 template <typename T>
-hipError_t launch_pcg_persist(jfm_ctx *ctx, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit);
+hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit,
+                              int nsys = 1, int64_t ss = 0);
 // coarse.hip
 // With learned_beside, the learned blocks start on the second stream
 // (jfem_learned_launch) once A_c is formed, beside its inversion.
@@ -468,12 +482,17 @@ hipError_t launch_heat_apply(jfm_ctx *ctx, const double *x, double *y, const dou
                              int *npart);
 hipError_t launch_heat_load(jfm_ctx *ctx, const double *src, double *f);
 hipError_t launch_heat_jacobi(jfm_ctx *ctx, double *Minv);
+// owner[f]: the first element (in the incidence order of its first node) that
+// holds all nodes of convection face f, or -1; map: its local nodes; K: 6 x 6
+hipError_t launch_heat_owner(jfm_ctx *ctx, int32_t *owner, int32_t *map, double *K);
 // postprocess.hip (kOpMass: consistent scalar mass, three components, no row mask)
 constexpr int kOpMass = 16;
 hipError_t launch_mass_elem(jfm_ctx *ctx, const double *x, const int *done);
 hipError_t launch_post_gp(jfm_ctx *ctx, const double *u, double *strain, double *stress);
 hipError_t launch_post_rhs(jfm_ctx *ctx, const double *u, int field, int comp0, double *b);
 hipError_t launch_mass_diag(jfm_ctx *ctx, double *Minv);
+// out[6 a + c] = x0[3 a + c], out[6 a + 3 + c] = x1[3 a + c]
+hipError_t launch_post_join(jfm_ctx *ctx, const double *x0, const double *x1, double *out);
 // linalg_kernels.hip
 template <typename T>
 hipError_t launch_bsr_spmv(jfm_ctx *ctx, const T *vals, const T *x, T *y, const T *dotv, double *part,

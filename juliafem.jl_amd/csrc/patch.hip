@@ -388,7 +388,7 @@ struct PatchHost {
     int npatch = 0;
     // with `cells`: patch nodes' ids, partial slots (-1: interior), first slot
     // of the node << 5 | slots, local connectivity (position in the patch)
-    // and the incidences (i, e) of patch node l at lin[pn_inc[l]..]: 3 i stride
+    // and the incidences (i, e) of patch node l at lin[pn_inc[l]..]: i stride
     // + local element, ascending
     std::vector<int32_t> pn_node, pn_slot, pn_sh, pn_inc;
     std::vector<uint16_t> connL, lin;
@@ -495,7 +495,7 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
                     const auto &pr = pairs[nd.first + j];
                     const int kl = (int)(pr.first % ps);
                     P.connL[(size_t)pr.second * n_el + k0 + kl] = (uint16_t)u;
-                    P.lin.push_back((uint16_t)(3 * pr.second * stride + kl));
+                    P.lin.push_back((uint16_t)(pr.second * stride + kl));
                 }
             }
             P.pn_cnt.push_back((uint16_t)nd.cnt);
@@ -540,7 +540,7 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
                 P.pn_sh[l] = first << 5 | (n & 31);
             }
         }
-        return 3 * npe * stride <= 65536 && (int64_t)P.pn_out.size() < INT32_MAX / 3;
+        return npe * stride <= 65536 && (int64_t)P.pn_out.size() < INT32_MAX / 3;
     }
     // 16-bit connectivity relative to each patch's lowest node id, when every
     // patch's ids span at most 65,536
@@ -675,9 +675,7 @@ int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g) {
     bool ok = put(C.eperm, P.perm) && put(C.connL, P.connL) && put(C.pn_ptr, P.pn_ptr) && put(C.pn_cnt, P.pn_cnt) &&
               put(C.pn_node, P.pn_node) && put(C.pn_slot, P.pn_slot) && put(C.pn_sh, P.pn_sh) &&
               put(C.pn_inc, P.pn_inc) && put(C.lin, P.lin);
-    ok = ok && (C.gf64 = jfm_alloc<double>(ctx, rows * n_el)) && (C.gf32 = jfm_alloc<float>(ctx, rows * n_el)) &&
-         (C.part = jfm_alloc<double>(ctx, 4 * std::max<int64_t>(1, P.bptr.back()))) &&
-         (C.words = jfm_alloc<uint64_t>(ctx, kPersistWords * ((int64_t)P.npatch + 256)));
+    ok = ok && (C.gf64 = jfm_alloc<double>(ctx, rows * n_el)) && (C.gf32 = jfm_alloc<float>(ctx, rows * n_el));
     const bool fold = ctx->affine && npe == 10 && ctx->nu_uniform;
     if (ok && fold) ok = (C.gfQ32 = jfm_alloc<float>(ctx, 9 * n_el)) != nullptr;
     if (!ok) {
@@ -692,8 +690,23 @@ int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g) {
     JFM_HIP(ctx, hipStreamSynchronize(s));
     C.npatch = P.npatch;
     C.nslot = P.bptr.back();
+    C.epos.resize(n_el);
+    for (int64_t k = 0; k < n_el; ++k) C.epos[P.perm[k]] = (int32_t)k;
     C.rho32 = (float)(2.0 * ctx->nu0 / (1.0 - 2.0 * ctx->nu0));
     C.usable = true;
+    return JFM_OK;
+}
+
+int jfem_cells_systems(jfm_ctx *ctx, int m) {
+    auto &C = ctx->cells;
+    if (m <= C.systems) return JFM_OK;
+    for (void *q : {(void *)C.part, (void *)C.words, (void *)C.S}) jfm_free(ctx, q);
+    C.systems = 0;
+    C.part = jfm_alloc<double>(ctx, (int64_t)m * 4 * std::max(1, C.nslot));
+    C.words = jfm_alloc<uint64_t>(ctx, (int64_t)m * kPersistWords * (C.npatch + 256));
+    C.S = jfm_alloc<PcgScalars>(ctx, m);
+    if (!C.part || !C.words || !C.S) return jfm_fail(ctx, JFM_ENOMEM, "resident PCG allocation failed");
+    C.systems = m;
     return JFM_OK;
 }
 
@@ -701,7 +714,7 @@ void jfem_cells_release(jfm_ctx *ctx) {
     auto &C = ctx->cells;
     for (void *p : {(void *)C.eperm, (void *)C.connL, (void *)C.pn_ptr, (void *)C.pn_cnt, (void *)C.pn_node, (void *)C.pn_slot,
                     (void *)C.pn_sh, (void *)C.pn_inc, (void *)C.lin, (void *)C.gf64, (void *)C.gf32,
-                    (void *)C.gfQ32, (void *)C.part, (void *)C.words})
+                    (void *)C.gfQ32, (void *)C.part, (void *)C.words, (void *)C.S})
         jfm_free(ctx, p);
     C = {};
 }

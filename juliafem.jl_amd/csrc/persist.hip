@@ -44,7 +44,7 @@
 // host repeats the solve with the launched form.
 #include <algorithm>
 #include <cstdlib>
-#include <vector>
+#include <type_traits>
 
 #include "jfem_device.h"
 #include "mf_element.h"
@@ -89,9 +89,13 @@ template <typename T> struct Partials {
     __amdgpu_buffer_rsrc_t rs;
     __device__ __forceinline__ Partials(void *p, int slots)
         : rs(__builtin_amdgcn_make_buffer_rsrc(p, 0, slots * 4 * (int)sizeof(T), 0x00027000)) {}
-    __device__ __forceinline__ void put(int slot, const T (&v)[3]) const {
+    template <int NC> __device__ __forceinline__ void put(int slot, const T (&v)[NC]) const {
         const int o = slot * 4 * (int)sizeof(T);
-        if constexpr (sizeof(T) == 8) {
+        if constexpr (NC == 1) {
+            u32x2 a;
+            __builtin_memcpy(&a, v, 8);
+            __builtin_amdgcn_raw_buffer_store_b64(a, rs, o, 0, kSc1);
+        } else if constexpr (sizeof(T) == 8) {
             u32x4 a;
             u32x2 b;
             __builtin_memcpy(&a, v, 16);
@@ -104,9 +108,13 @@ template <typename T> struct Partials {
             __builtin_amdgcn_raw_buffer_store_b96(a, rs, o, 0, kSc1);
         }
     }
-    __device__ __forceinline__ void get(int slot, T (&v)[3]) const {
+    template <int NC> __device__ __forceinline__ void get(int slot, T (&v)[NC]) const {
+        static_assert(NC == 3 || (NC == 1 && sizeof(T) == 8), "a node's values");
         const int o = slot * 4 * (int)sizeof(T);
-        if constexpr (sizeof(T) == 8) {
+        if constexpr (NC == 1) {
+            const u32x2 a = __builtin_amdgcn_raw_buffer_load_b64(rs, o, 0, kSc1);
+            __builtin_memcpy(v, &a, 8);
+        } else if constexpr (sizeof(T) == 8) {
             const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(rs, o, 0, kSc1);
             const u32x2 b = __builtin_amdgcn_raw_buffer_load_b64(rs, o + 16, 0, kSc1);
             __builtin_memcpy(v, &a, 16);
@@ -191,8 +199,8 @@ __device__ __forceinline__ void put_rows(uint64_t *words, int stride, int at, ui
 }
 
 template <int NV, int NT>
-__device__ __forceinline__ bool grid_sum(double (&v)[NV], uint64_t *words, int nwg, uint32_t epoch, GridSumLds<NV> &sh,
-                                         int *bad) {
+__device__ __forceinline__ bool grid_sum(double (&v)[NV], uint64_t *words, int wg, int nwg, uint32_t epoch,
+                                         GridSumLds<NV> &sh, int *bad) {
     static_assert(NV <= 2 && NT / 64 <= 16, "one row of 16 lanes per value");
     constexpr int kW = NT / 64;
     const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
@@ -203,7 +211,7 @@ __device__ __forceinline__ bool grid_sum(double (&v)[NV], uint64_t *words, int n
     }
     __syncthreads();
     if (wv == 0) {
-        const int k = lane >> 4, m = lane & 15, wg = (int)blockIdx.x;
+        const int k = lane >> 4, m = lane & 15;
         double s = row_sum(k < NV && m < kW ? sh.a[k < NV ? k : 0][m] : 0.0);  // row k: the block's value k
         if (nwg > 1) {
             put_rows<NV>(words, nwg, wg, epoch, s);
@@ -241,15 +249,21 @@ template <typename T> struct PersistArgs {
     int n_el, npatch;
     const uint16_t *connL;    // npe x n_el (patch order): the node's position in its patch
     const T *el;              // geometric factors, patch order
-    T rho;
+    T rho;                    // lambda / mu of the folded factors
+    int ngf;
+    const double *kc;         // heat: conductivities (element order) and the elements' order
+    const int32_t *eperm;
+    const int32_t *ef, *enext, *fmap;  // heat: the element's first convection face (or -1), the next
+    const double *fk;         // one, its element-local nodes (4 bits each) and its matrix
+    int nfn;
     const int32_t *pn_ptr;    // patch nodes: range per patch
     const int32_t *pn_node;   // patch node -> node
     const int32_t *pn_slot;   // its partial slot, or -1 (interior)
     const int32_t *pn_sh;     // shared: first slot of its node << 5 | slots
     const uint16_t *pn_cnt;   // its incidences in the patch
     const int32_t *pn_inc;    // their start in lin
-    const uint16_t *lin;      // incidences (i, e): 3 i kStride + e, ascending e
-    const uint8_t *fixed;
+    const uint16_t *lin;      // incidences (i, e): i stride + e, ascending e
+    const uint8_t *fixed;     // (null: no row mask)
     const T *Minv, *b, *r0;   // r0: the true residual at the x that is given (null: x = 0)
     T *x;
     T *part;                  // the shared nodes' partials, 4 values per slot
@@ -258,88 +272,22 @@ template <typename T> struct PersistArgs {
     double rtol2;
     int maxit;
     PcgScalars *S;
+    // nsys systems of one operator side by side: workgroups npatch s .. of the
+    // grid solve system s, its b and x ss values further, scalars at S + s
+    int nsys;
+    int64_t ss;
 };
 
-// A patch's threads and elements.  The affine Tet10 product runs on four
-// lanes per element, one per vertex (below), which shortens the longest
-// instruction stream of the iteration: with one thread per element and three
-// nodes per thread (256 threads) an iteration of a single patch took 7.5 us,
-// four waves each issuing some 4,300 instructions one after the other.  512
-// threads may hold 256 registers each, enough for a node's and a vertex's
+// A patch has 512 threads (one node each at most).  The affine Tet10 products
+// run on four lanes per element, one per vertex (below), which shortens the
+// longest instruction stream of the iteration: with one thread per element and
+// three nodes per thread (256 threads) an iteration of a single patch took 7.5
+// us, four waves each issuing some 4,300 instructions one after the other.
+// 512 threads may hold 256 registers each, enough for a node's and a vertex's
 // data; with 256 elements on 1,024 threads the FP64 kernel spilled 73
 // registers and an iteration took 9 us.
-template <int NPE> struct PersistShape {
-    static_assert(NPE == 10 || NPE == 4, "affine Tet10 and Tet4");
-    static constexpr bool kVertexLanes = NPE == 10;
-    static constexpr int kThreads = 512;  // also the most nodes of a patch
-    static constexpr int kEl = kVertexLanes ? kThreads / 4 : kThreads;
-    static constexpr int kStride = kEl + 1;                     // one zero column for padded incidences
-};
-
-// Affine Tet10 element product on the four lanes of a quad, lane k holding
-// vertex k.  With u relative to vertex k, the displacement gradient at vertex
-// k is sum_d h_d (x) g_d over the other vertices j = k ^ d, h_d = 4 u_kj - u_j,
-// g_d = grad L_j (mf_element.h writes the same sums in the reference frame of
-// vertex 0).  With sigma_k the stress there (0.2 w detJ folded in), S = sum
-// sigma_k, r_d = sigma_k g_d, s_d = S g_d and index 0 the vertex itself
-// (g_0 = -sum g_d):
-//     y_corner k = 4 r_0 - s_0,  y_edge kj = 4 ((r_d + r_d of lane j) + (s_0 + s_d)),
-// and the element's energy is the sum over its lanes of G_k : (sigma_k + S).
-// ex(v, d) returns lane (k ^ d)'s v.
-template <typename T, typename XL, typename Out>
-__device__ __forceinline__ T tet10_vertex(const T (&g)[9], T cl, T cm, int k, XL &&xl, Out &&out) {
-    T u0[3], h[3][3];
-    xl(0, u0);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        T ue[3], uv[3];
-        xl(1 + d, ue);   // mid node of edge (k, k ^ (d + 1))
-        xl(4 + d, uv);   // vertex k ^ (d + 1)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) h[d][c] = T(4) * (ue[c] - u0[c]) - (uv[c] - u0[c]);
-    }
-    T G[9];
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int b = 0; b < 3; ++b) G[a * 3 + b] = h[0][a] * g[b] + h[1][a] * g[3 + b] + h[2][a] * g[6 + b];
-    const T tr = cl * (G[0] + G[4] + G[8]);
-    // 11, 22, 33, 12, 23, 13
-    T s[6] = {tr + T(2) * cm * G[0], tr + T(2) * cm * G[4], tr + T(2) * cm * G[8], cm * (G[1] + G[3]), cm * (G[5] + G[7]),
-              cm * (G[2] + G[6])};
-    T S[6];
-#pragma unroll
-    for (int m = 0; m < 6; ++m) {
-        S[m] = s[m] + dpp_mov<kQuadXor1>(s[m]);
-        S[m] += dpp_mov<kQuadXor2>(S[m]);
-    }
-    const T en = G[0] * (s[0] + S[0]) + G[4] * (s[1] + S[1]) + G[8] * (s[2] + S[2]) + (G[1] + G[3]) * (s[3] + S[3]) +
-                 (G[5] + G[7]) * (s[4] + S[4]) + (G[2] + G[6]) * (s[5] + S[5]);
-    auto mul = [&](const T (&m)[6], const T *v, T (&o)[3]) {
-        o[0] = m[0] * v[0] + m[3] * v[1] + m[5] * v[2];
-        o[1] = m[3] * v[0] + m[1] * v[1] + m[4] * v[2];
-        o[2] = m[5] * v[0] + m[4] * v[1] + m[2] * v[2];
-    };
-    T g0[3], s0[3], r0[3];
-#pragma unroll
-    for (int b = 0; b < 3; ++b) g0[b] = -(g[b] + g[3 + b] + g[6 + b]);
-    mul(S, g0, s0);
-    mul(s, g0, r0);
-    out(0, T(4) * r0[0] - s0[0], T(4) * r0[1] - s0[1], T(4) * r0[2] - s0[2]);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        T r[3], sd[3], f[3];
-        mul(s, g + 3 * d, r);
-        mul(S, g + 3 * d, sd);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const T o = d == 0 ? dpp_mov<kQuadXor1>(r[c]) : (d == 1 ? dpp_mov<kQuadXor2>(r[c]) : dpp_mov<kQuadXor3>(r[c]));
-            f[c] = T(4) * ((r[c] + o) + (s0[c] + sd[c]));
-        }
-        if (k < (k ^ (d + 1))) out(1 + d, f[0], f[1], f[2]);  // one of the edge's two lanes
-    }
-    return en;
-}
+constexpr int kNT = 512;
+template <int NPE> constexpr int persist_elems() { return NPE == 10 ? 128 : (NPE == 8 ? 256 : 512); }
 
 // local node of lane k's slot m: itself, the mid nodes of its edges to
 // k ^ 1, k ^ 2, k ^ 3, and those vertices
@@ -347,62 +295,373 @@ __host__ __device__ constexpr int tet10_lane_node(int k, int m) {
     constexpr int EDG[4][4] = {{-1, 4, 6, 7}, {4, -1, 5, 8}, {6, 5, -1, 9}, {7, 8, 9, -1}};
     return m == 0 ? k : (m < 4 ? EDG[k][k ^ m] : k ^ (m - 3));
 }
+template <int D, typename T> __device__ __forceinline__ T quad_xor(T v) {
+    return dpp_mov<D == 1 ? kQuadXor1 : (D == 2 ? kQuadXor2 : kQuadXor3)>(v);
+}
+template <typename T> __device__ __forceinline__ T quad_sum(T v) {
+    v += quad_xor<1>(v);
+    return v + quad_xor<2>(v);
+}
+// grad L_j of the vertices j = kv ^ d from invJ: column j - 1, or minus the sum
+// of the columns for vertex 0
+template <typename T> __device__ __forceinline__ void lane_gradients(const T (&Ji)[9], int kv, T (&g)[9]) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int j = kv ^ (d + 1);
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+            g[3 * d + b] = j == 0 ? -(Ji[b * 3] + Ji[b * 3 + 1] + Ji[b * 3 + 2]) : (j == 1 ? Ji[b * 3] : (j == 2 ? Ji[b * 3 + 1] : Ji[b * 3 + 2]));
+    }
+}
+__device__ __forceinline__ double det_inv(const double (&A)[9]) {
+    return A[0] * (A[4] * A[8] - A[5] * A[7]) - A[1] * (A[3] * A[8] - A[5] * A[6]) + A[2] * (A[3] * A[7] - A[4] * A[6]);
+}
 
-template <int NPE, typename T, bool FOLD>
-__global__ __launch_bounds__(PersistShape<NPE>::kThreads) void k_pcg_persist(const PersistArgs<T> A) {
-    using SH = PersistShape<NPE>;
-    constexpr int kPP = SH::kEl, NT = SH::kThreads, ST = SH::kStride;
-    constexpr bool VL = SH::kVertexLanes;
-    __shared__ T ys[3 * NPE * ST];   // element terms: (3 i + c) ST + element; column kPP is zero
-    __shared__ T ps[3 * NT];         // p at the patch's nodes
+// An operator of the resident PCG: NC components per node, kLanes lanes per
+// element, kIn nodes that a lane reads and kOut that it writes; xc(m, c) is
+// component c of p at the lane's m-th node, oc(m, c, v) its term there.
+// product() returns the lane's share of p_e.K_e p_e.
+template <int N_, int C_, int L_, int I_, int O_, bool D_, int W_> struct OpShape {
+    static constexpr int NPE = N_, NC = C_, kLanes = L_, kIn = I_, kOut = O_, kWaves = W_;
+    static constexpr bool kDiag = D_;  // diagonal preconditioner (heat, mass)
+    static constexpr int kEl = persist_elems<N_>(), kStride = kEl + 1;  // one zero column for padded incidences
+    __device__ static int in_node(int kv, int m) { return L_ == 4 && I_ == 7 ? tet10_lane_node(kv, m) : m; }
+    template <typename A, typename D, typename X, typename O>
+    __device__ static double faces(const A &, const D &, int, const uint16_t *, X &&, O &&) { return 0.0; }
+};
+
+// Affine Tet10 elasticity on the four lanes of a quad, lane k holding vertex k.
+// With u relative to vertex k, the displacement gradient at vertex k is sum_d
+// h_d (x) g_d over the other vertices j = k ^ d, h_d = 4 u_kj - u_j, g_d = grad
+// L_j (mf_element.h writes the same sums in the reference frame of vertex 0).
+// With sigma_k the stress there (0.2 w detJ folded in), S = sum sigma_k, r_d =
+// sigma_k g_d, s_d = S g_d and index 0 the vertex itself (g_0 = -sum g_d):
+//     y_corner k = 4 r_0 - s_0,  y_edge kj = 4 ((r_d + r_d of lane j) + (s_0 + s_d)),
+// and the element's energy is the sum over its lanes of G_k : (sigma_k + S).
+template <typename T_, bool FOLD> struct ElasticTet10 : OpShape<10, 3, 4, 7, 4, false, 2> {
+    using T = T_;
+    struct Data { T g[9], cl, cm; };
+    __device__ static void load(const PersistArgs<T> &A, int k, int kv, bool has, Data &d) {
+        T Ji[9];
+#pragma unroll
+        for (int m = 0; m < 9; ++m) Ji[m] = has ? A.el[(size_t)m * A.n_el + k] : T(0);
+        lane_gradients<T>(Ji, kv, d.g);
+        d.cl = FOLD ? A.rho : (has ? T(0.2) * A.el[(size_t)9 * A.n_el + k] : T(0));
+        d.cm = FOLD ? T(1) : (has ? T(0.2) * A.el[(size_t)10 * A.n_el + k] : T(0));
+    }
+    template <typename XC, typename OC>
+    __device__ static double product(const PersistArgs<T> &, const Data &D, int, int k, bool has, XC &&xc, OC &&oc) {
+        const T *g = D.g, cl = D.cl, cm = D.cm;
+        T u0[3], h[3][3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) u0[c] = xc(0, c);
+#pragma unroll
+        for (int d = 0; d < 3; ++d)  // mid node of edge (k, k ^ (d + 1)), vertex k ^ (d + 1)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) h[d][c] = T(4) * (xc(1 + d, c) - u0[c]) - (xc(4 + d, c) - u0[c]);
+        T G[9];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int b = 0; b < 3; ++b) G[a * 3 + b] = h[0][a] * g[b] + h[1][a] * g[3 + b] + h[2][a] * g[6 + b];
+        const T tr = cl * (G[0] + G[4] + G[8]);
+        // 11, 22, 33, 12, 23, 13
+        const T s[6] = {tr + T(2) * cm * G[0], tr + T(2) * cm * G[4], tr + T(2) * cm * G[8], cm * (G[1] + G[3]),
+                        cm * (G[5] + G[7]), cm * (G[2] + G[6])};
+        T S[6];
+#pragma unroll
+        for (int m = 0; m < 6; ++m) S[m] = quad_sum(s[m]);
+        const T en = G[0] * (s[0] + S[0]) + G[4] * (s[1] + S[1]) + G[8] * (s[2] + S[2]) + (G[1] + G[3]) * (s[3] + S[3]) +
+                     (G[5] + G[7]) * (s[4] + S[4]) + (G[2] + G[6]) * (s[5] + S[5]);
+        auto mul = [&](const T (&m)[6], const T *v, T (&o)[3]) {
+            o[0] = m[0] * v[0] + m[3] * v[1] + m[5] * v[2];
+            o[1] = m[3] * v[0] + m[1] * v[1] + m[4] * v[2];
+            o[2] = m[5] * v[0] + m[4] * v[1] + m[2] * v[2];
+        };
+        T g0[3], s0[3], r0[3];
+#pragma unroll
+        for (int b = 0; b < 3; ++b) g0[b] = -(g[b] + g[3 + b] + g[6 + b]);
+        mul(S, g0, s0);
+        mul(s, g0, r0);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) oc(0, c, T(4) * r0[c] - s0[c]);
+        auto edge = [&](auto dc) {
+            constexpr int d = decltype(dc)::value;
+            T r[3], sd[3], f[3];
+            mul(s, g + 3 * (d - 1), r);
+            mul(S, g + 3 * (d - 1), sd);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) f[c] = T(4) * ((r[c] + quad_xor<d>(r[c])) + (s0[c] + sd[c]));
+            if (k < (k ^ d))  // one of the edge's two lanes
+#pragma unroll
+                for (int c = 0; c < 3; ++c) oc(d, c, f[c]);
+        };
+        edge(std::integral_constant<int, 1>{});
+        edge(std::integral_constant<int, 2>{});
+        edge(std::integral_constant<int, 3>{});
+        return has ? (double)en : 0.0;
+    }
+};
+
+template <typename T_> struct ElasticTet4 : OpShape<4, 3, 1, 4, 4, false, 2> {
+    using T = T_;
+    struct Data { T f[GF]; };
+    __device__ static void load(const PersistArgs<T> &A, int k, int, bool has, Data &d) {
+#pragma unroll
+        for (int m = 0; m < GF; ++m) d.f[m] = has ? A.el[(size_t)m * A.n_el + k] : T(0);
+    }
+    template <typename XC, typename OC>
+    __device__ static double product(const PersistArgs<T> &, const Data &D, int, int, bool has, XC &&xc, OC &&oc) {
+        double en = 0.0;
+        if (has)
+            mf_element_f<4, T, true>([&](int, int m) -> T { return D.f[m]; },
+                                     [&](int i, T (&v)[3]) { v[0] = xc(i, 0); v[1] = xc(i, 1); v[2] = xc(i, 2); },
+                                     [&](int i, T f0, T f1, T f2) {
+                                         oc(i, 0, f0);
+                                         oc(i, 1, f1);
+                                         oc(i, 2, f2);
+                                         if (i > 0)  // K_e annihilates translations
+                                             en += (double)((xc(i, 0) - xc(0, 0)) * f0 + (xc(i, 1) - xc(0, 1)) * f1 +
+                                                            (xc(i, 2) - xc(0, 2)) * f2);
+                                     });
+        return en;
+    }
+};
+
+// Conduction (heat.hip), one component.  The convection faces are faces of an
+// element each: the element's (first) lane adds their terms to its own.
+template <int NPE_, int L_, int I_, int O_> struct HeatShape : OpShape<NPE_, 1, L_, I_, O_, true, 2> {
+    using T = double;
+    template <typename D, typename X, typename O>
+    __device__ static double faces(const PersistArgs<double> &A, const D &d, int k, X &&xe, O &&ye) {
+        double en = 0.0;
+        for (int f = d.face; f >= 0; f = A.enext[f]) {
+            const int map = A.fmap[f];
+            const double *K = A.fk + (size_t)f * 36;
+            double v[6];
+#pragma unroll
+            for (int j = 0; j < 6; ++j) v[j] = j < A.nfn ? xe(map >> (4 * j) & 15) : 0.0;
+#pragma unroll
+            for (int j = 0; j < 6; ++j)
+                if (j < A.nfn) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int l = 0; l < 6; ++l) s += K[6 * j + l] * v[l];
+                    ye(map >> (4 * j) & 15, s);
+                    en += v[j] * s;
+                }
+        }
+        return en;
+    }
+};
+struct HeatTet10 : HeatShape<10, 4, 7, 4> {  // the vertex form of ElasticTet10, sigma = k grad T
+    struct Data { double g[9], c; int face; };
+    __device__ static void load(const PersistArgs<double> &A, int k, int kv, bool has, Data &d) {
+        double Ji[9];
+#pragma unroll
+        for (int m = 0; m < 9; ++m) Ji[m] = has ? A.el[(size_t)m * A.n_el + k] : (m % 4 == 0 ? 1.0 : 0.0);
+        lane_gradients<double>(Ji, kv, d.g);
+        d.c = has ? 0.2 * A.kc[A.eperm[k]] * Elem<10>::w(0) / det_inv(Ji) : 0.0;
+        d.face = has && kv == 0 && A.ef ? A.ef[k] : -1;
+    }
+    template <typename XC, typename OC>
+    __device__ static double product(const PersistArgs<double> &, const Data &D, int, int k, bool has, XC &&xc, OC &&oc) {
+        const double *g = D.g, u0 = xc(0, 0);
+        double h[3], G[3], s[3], S[3], s0 = 0.0, r0 = 0.0, en = 0.0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) h[d] = 4.0 * (xc(1 + d, 0) - u0) - (xc(4 + d, 0) - u0);
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            G[b] = h[0] * g[b] + h[1] * g[3 + b] + h[2] * g[6 + b];
+            s[b] = D.c * G[b];
+            S[b] = quad_sum(s[b]);
+            const double g0 = -(g[b] + g[3 + b] + g[6 + b]);
+            s0 += S[b] * g0;
+            r0 += s[b] * g0;
+            en += G[b] * (s[b] + S[b]);
+        }
+        oc(0, 0, 4.0 * r0 - s0);
+        auto edge = [&](auto dc) {
+            constexpr int d = decltype(dc)::value;
+            const double *gd = g + 3 * (d - 1);
+            const double r = s[0] * gd[0] + s[1] * gd[1] + s[2] * gd[2], sd = S[0] * gd[0] + S[1] * gd[1] + S[2] * gd[2];
+            const double f = 4.0 * ((r + quad_xor<d>(r)) + (s0 + sd));
+            if (k < (k ^ d)) oc(d, 0, f);
+        };
+        edge(std::integral_constant<int, 1>{});
+        edge(std::integral_constant<int, 2>{});
+        edge(std::integral_constant<int, 3>{});
+        return has ? en : 0.0;
+    }
+};
+template <int NPE_> struct HeatElem : HeatShape<NPE_, 1, NPE_, NPE_> {  // Tet4, Hex8: the Gauss-point form
+    struct Data { double kc; int face; };
+    __device__ static void load(const PersistArgs<double> &A, int k, int, bool has, Data &d) {
+        d.kc = has ? A.kc[A.eperm[k]] : 0.0;
+        d.face = has && A.ef ? A.ef[k] : -1;
+    }
+    template <typename XC, typename OC>
+    __device__ static double product(const PersistArgs<double> &A, const Data &D, int k, int, bool has, XC &&xc, OC &&oc) {
+        using EL = Elem<NPE_>;
+        if (!has) return 0.0;
+        double xe[NPE_], y[NPE_], Ji[9];
+        const double x0 = xc(0, 0);
+#pragma unroll
+        for (int i = 0; i < NPE_; ++i) {
+            xe[i] = xc(i, 0) - x0;  // sum grad N = 0
+            y[i] = 0.0;
+        }
+#pragma unroll 1  // (unrolled, the points' factors spill)
+        for (int q = 0; q < EL::NGP; ++q) {
+            if (q == 0 || A.ngf > 1)
+#pragma unroll
+                for (int m = 0; m < 9; ++m) Ji[m] = A.el[(size_t)(q * GF + m) * A.n_el + k];
+            const double w = D.kc * EL::w(q) / det_inv(Ji);
+            double h[3] = {0.0, 0.0, 0.0}, t[3], u[3];
+#pragma unroll
+            for (int i = 1; i < NPE_; ++i)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) h[c] += xe[i] * dn_rt<NPE_>(q, i, c);
+#pragma unroll
+            for (int b = 0; b < 3; ++b) t[b] = w * (Ji[b * 3] * h[0] + Ji[b * 3 + 1] * h[1] + Ji[b * 3 + 2] * h[2]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) u[c] = Ji[c] * t[0] + Ji[3 + c] * t[1] + Ji[6 + c] * t[2];
+#pragma unroll
+            for (int i = 0; i < NPE_; ++i) y[i] += u[0] * dn_rt<NPE_>(q, i, 0) + u[1] * dn_rt<NPE_>(q, i, 1) + u[2] * dn_rt<NPE_>(q, i, 2);
+        }
+        double en = 0.0;
+#pragma unroll
+        for (int i = 0; i < NPE_; ++i) {
+            oc(i, 0, y[i]);
+            en += xe[i] * y[i];
+        }
+        return en;
+    }
+};
+
+// Consistent mass of the nodal fit (postprocess.hip), three components.  An
+// affine Tet10's is detJ / 2520 times one constant matrix (6 on a corner's
+// diagonal, 1 between corners, -4 to the mid nodes at the corner, -6 to the
+// others; 32 on a mid node's diagonal, 8 to the opposite one, 16 to the rest),
+// applied through the sums over corners (Sc), mid nodes (Se) and the mid nodes
+// at a corner (A_i):
+//     corner i:  5 x_i + Sc + 2 A_i - 6 Se
+//     edge ab:   16 (x_ab + Se) - 8 x_opposite + 2 (x_a + x_b) - 6 Sc
+// about 70 operations per component against 36 points of the fit rule.
+struct MassTet10 : OpShape<10, 3, 4, 10, 10, true, 4> {  // lanes 0..2: one component each
+    using T = double;
+    struct Data { double w; };
+    __device__ static void load(const PersistArgs<double> &A, int k, int, bool has, Data &d) {
+        double Ji[9];
+#pragma unroll
+        for (int m = 0; m < 9; ++m) Ji[m] = has ? A.el[(size_t)m * A.n_el + k] : (m % 4 == 0 ? 1.0 : 0.0);
+        d.w = has ? 1.0 / (2520.0 * det_inv(Ji)) : 0.0;
+    }
+    template <typename XC, typename OC>
+    __device__ static double product(const PersistArgs<double> &, const Data &D, int, int kv, bool has, XC &&xc, OC &&oc) {
+        if (!has || kv == 3) return 0.0;
+        double x[10], en = 0.0;
+#pragma unroll
+        for (int i = 0; i < 10; ++i) x[i] = xc(i, kv);
+        const double Sc = (x[0] + x[1]) + (x[2] + x[3]), Se = ((x[4] + x[5]) + (x[6] + x[7])) + (x[8] + x[9]);
+        const double At[4] = {x[4] + x[6] + x[7], x[4] + x[5] + x[8], x[5] + x[6] + x[9], x[7] + x[8] + x[9]};
+        constexpr int EA[6] = {0, 1, 2, 0, 1, 2}, EB[6] = {1, 2, 0, 3, 3, 3}, EO[6] = {9, 7, 8, 5, 6, 4};
+        auto put = [&](int i, double v) {
+            const double y = D.w * v;
+            oc(i, kv, y);
+            en += x[i] * y;
+        };
+#pragma unroll
+        for (int i = 0; i < 4; ++i) put(i, 5.0 * x[i] + Sc + 2.0 * At[i] - 6.0 * Se);
+#pragma unroll
+        for (int m = 0; m < 6; ++m) put(4 + m, 16.0 * (x[4 + m] + Se) - 8.0 * x[EO[m]] + 2.0 * (x[EA[m]] + x[EB[m]]) - 6.0 * Sc);
+        return en;
+    }
+};
+template <int NPE_> struct MassElem : OpShape<NPE_, 3, 1, NPE_, NPE_, true, 2> {  // Tet4, Hex8
+    using T = double;
+    static constexpr int NW = NPE_ == 8 ? 8 : 1;
+    struct Data { double w[NW]; };  // w detJ at the rule's points
+    __device__ static void load(const PersistArgs<double> &A, int k, int, bool has, Data &d) {
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            double Ji[9];
+#pragma unroll
+            for (int m = 0; m < 9; ++m)
+                Ji[m] = has ? A.el[(size_t)((A.ngf > 1 ? q : 0) * GF + m) * A.n_el + k] : (m % 4 == 0 ? 1.0 : 0.0);
+            d.w[q] = has ? (NPE_ == 8 ? 1.0 : 1.0 / 120.0) / det_inv(Ji) : 0.0;
+        }
+    }
+    template <typename XC, typename OC>
+    __device__ static double product(const PersistArgs<double> &, const Data &D, int, int, bool has, XC &&xc, OC &&oc) {
+        if (!has) return 0.0;
+        double en = 0.0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            double x[NPE_], y[NPE_];
+#pragma unroll
+            for (int i = 0; i < NPE_; ++i) {
+                x[i] = xc(i, c);
+                y[i] = 0.0;
+            }
+            if constexpr (NPE_ == 4) {  // detJ / 120 (1 + delta)
+                const double s = (x[0] + x[1]) + (x[2] + x[3]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y[i] = D.w[0] * (s + x[i]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < NW; ++q) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int i = 0; i < NPE_; ++i) s += Elem<NPE_>::N(q, i) * x[i];
+                    s *= D.w[q];
+#pragma unroll
+                    for (int i = 0; i < NPE_; ++i) y[i] += Elem<NPE_>::N(q, i) * s;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < NPE_; ++i) {
+                oc(i, c, y[i]);
+                en += x[i] * y[i];
+            }
+        }
+        return en;
+    }
+};
+
+template <class Op>
+__global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistArgs<typename Op::T> A0) {
+    using T = typename Op::T;
+    constexpr int NPE = Op::NPE, NC = Op::NC, NL = Op::kLanes, EL = Op::kEl, ST = Op::kStride, NT = kNT, CS = NPE * ST;
+    __shared__ T ys[NC * CS];    // element terms: c CS + i ST + element; column EL of row 0 is zero
+    __shared__ T ps[NC * NT];    // p at the patch's nodes
     __shared__ GridSumLds<1> shB;
     __shared__ GridSumLds<2> shC;
     __shared__ int bad;
-    const int t = (int)threadIdx.x, p = (int)blockIdx.x, nwg = A.npatch;
-    const int el = VL ? t >> 2 : t, kv = t & 3;   // its element (and vertex)
-    const int k = p * kPP + el;
-    const bool has_el = el < kPP && k < A.n_el;
+    const PersistArgs<T> &A = A0;
+    const int nwg = A.npatch, sys = (int)blockIdx.x / nwg, p = (int)blockIdx.x - sys * nwg;
+    const int t = (int)threadIdx.x;
+    const int el = t / NL, kv = NL == 4 ? t & 3 : 0;   // its element (and vertex or component)
+    const int k = p * EL + el;
+    const bool has_el = el < EL && k < A.n_el;
     const int lb = A.pn_ptr[p], nn = A.pn_ptr[p + 1] - lb;
-    uint64_t *wordsB = A.words, *wordsC = A.words + 2 * (size_t)(nwg + kGroup * kGroup);
-    const Partials<T> part(A.part, A.nslot);
+    const int rows = nwg + kGroup * kGroup;
+    uint64_t *wordsB = A.words + (size_t)sys * kPersistWords * rows, *wordsC = wordsB + 2 * (size_t)rows;
+    PcgScalars *S = A.S + sys;
+    const Partials<T> part(A.part + (size_t)sys * 4 * A.nslot, A.nslot);
+    const T *bvec = A.b + sys * A.ss;
+    T *xvec = A.x + sys * A.ss;
     if (t == 0) bad = 0;
-    for (int i = t; i < 3 * NPE; i += NT) ys[i * ST + kPP] = T(0);
+    if (t < NC) ys[t * CS + EL] = T(0);
 
     // the element's data, held for the whole solve
-    constexpr int NC = VL ? 7 : NPE;
-    int cl[NC];
-    int row[4];   // lane's output rows (vertex lanes)
-    constexpr int NF = FOLD ? 9 : GF;
-    T fac[NF];
-    if constexpr (VL) {
+    int cl[Op::kIn], row[Op::kOut];
 #pragma unroll
-        for (int m = 0; m < 7; ++m) {
-            const int i = tet10_lane_node(kv, m);
-            cl[m] = has_el ? 3 * (int)A.connL[(size_t)i * A.n_el + k] : 0;
-            if (m < 4) row[m] = 3 * i * ST + el;
-        }
-        // grad L_j of the vertices j = kv ^ d from invJ: column j - 1, or
-        // minus the sum of the columns for vertex 0
-        T Ji[9];
+    for (int m = 0; m < Op::kIn; ++m) cl[m] = has_el ? NC * (int)A.connL[(size_t)Op::in_node(kv, m) * A.n_el + k] : 0;
 #pragma unroll
-        for (int m = 0; m < 9; ++m) Ji[m] = has_el ? A.el[(size_t)m * A.n_el + k] : T(0);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const int j = kv ^ (d + 1);
-#pragma unroll
-            for (int b = 0; b < 3; ++b)
-                fac[3 * d + b] = j == 0 ? -(Ji[b * 3] + Ji[b * 3 + 1] + Ji[b * 3 + 2]) : (j == 1 ? Ji[b * 3] : (j == 2 ? Ji[b * 3 + 1] : Ji[b * 3 + 2]));
-        }
-        if constexpr (!FOLD) {
-            fac[9] = has_el ? T(0.2) * A.el[(size_t)9 * A.n_el + k] : T(0);
-            fac[10] = has_el ? T(0.2) * A.el[(size_t)10 * A.n_el + k] : T(0);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < NPE; ++i) cl[i] = has_el ? 3 * (int)A.connL[(size_t)i * A.n_el + k] : 0;
-#pragma unroll
-        for (int m = 0; m < NF; ++m) fac[m] = has_el ? A.el[(size_t)m * A.n_el + k] : T(0);
-    }
+    for (int m = 0; m < Op::kOut; ++m) row[m] = Op::in_node(kv, m) * ST + el;
+    typename Op::Data data;
+    Op::load(A, k, kv, has_el, data);
     // the node's data (one node per thread)
     const bool in = t < nn;
     const int cnt = in ? (int)A.pn_cnt[lb + t] : 0, base = in ? A.pn_inc[lb + t] : 0;
@@ -414,32 +673,33 @@ __global__ __launch_bounds__(PersistShape<NPE>::kThreads) void k_pcg_persist(con
     uint32_t inc[kInc / 2];
 #pragma unroll
     for (int m = 0; m < kInc / 2; ++m) {
-        const uint32_t lo = 2 * m < cnt ? A.lin[base + 2 * m] : (uint32_t)kPP;
-        const uint32_t hi = 2 * m + 1 < cnt ? A.lin[base + 2 * m + 1] : (uint32_t)kPP;
+        const uint32_t lo = 2 * m < cnt ? A.lin[base + 2 * m] : (uint32_t)EL;
+        const uint32_t hi = 2 * m + 1 < cnt ? A.lin[base + 2 * m + 1] : (uint32_t)EL;
         inc[m] = lo | hi << 16;
     }
     // nodes are sorted by count, most first: the wave's first lane has the most
     const int cw = __builtin_amdgcn_readfirstlane(cnt);
     uint32_t fx = 0;
-    T r[3], z[3], pv[3], x[3];
-    Blk9<T> M;
+    T r[NC], z[NC], pv[NC], x[NC];
+    constexpr int NM = Op::kDiag ? NC : NC * NC;
+    T M[NM];
 #pragma unroll
-    for (int m = 0; m < 9; ++m) M.v[m] = in ? A.Minv[9 * (size_t)node + m] : T(0);
+    for (int m = 0; m < NM; ++m) M[m] = in ? A.Minv[9 * (size_t)node + (Op::kDiag ? 4 * m : m)] : T(0);
     double bb[1] = {0.0};
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
+    for (int c = 0; c < NC; ++c) {
         const size_t d = 3 * (size_t)node + c;
-        if (in && A.fixed[d]) fx |= 1u << c;
-        const T bv = in ? A.b[d] : T(0);
+        if (in && A.fixed && A.fixed[d]) fx |= 1u << c;
+        const T bv = in ? bvec[d] : T(0);
         if (own) bb[0] += (double)bv * (double)bv;
         r[c] = in && A.r0 ? A.r0[d] : bv;
-        x[c] = in && A.r0 ? A.x[d] : T(0);
+        x[c] = in && A.r0 ? xvec[d] : T(0);
         pv[c] = T(0);
     }
     __syncthreads();  // bad
     uint32_t epoch = 1;
-    if (!grid_sum<1, NT>(bb, wordsB, nwg, epoch, shB, &bad)) {
-        if (t == 0) A.S->fail = 1;
+    if (!grid_sum<1, NT>(bb, wordsB, p, nwg, epoch, shB, &bad)) {
+        if (t == 0) S->fail = 1;
         return;
     }
     const double tol2 = A.rtol2 * bb[0];
@@ -450,15 +710,18 @@ __global__ __launch_bounds__(PersistShape<NPE>::kThreads) void k_pcg_persist(con
         // z = M r and the partials of the owned nodes
         double s2[2] = {0.0, 0.0};
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            z[c] = M.v[3 * c] * r[0] + M.v[3 * c + 1] * r[1] + M.v[3 * c + 2] * r[2];
+        for (int c = 0; c < NC; ++c) {
+            if constexpr (Op::kDiag)
+                z[c] = M[c] * r[c];
+            else
+                z[c] = M[3 * c] * r[0] + M[3 * c + 1] * r[1] + M[3 * c + 2] * r[2];
             if (own) {
                 s2[0] += (double)r[c] * (double)z[c];
                 s2[1] += (double)r[c] * (double)r[c];
             }
         }
         ++epoch;
-        if (!grid_sum<2, NT>(s2, wordsC, nwg, epoch, shC, &bad)) break;
+        if (!grid_sum<2, NT>(s2, wordsC, p, nwg, epoch, shC, &bad)) break;
         rr = s2[1];
         if (epoch == 2) {  // the start
             rr0 = rr;
@@ -475,70 +738,54 @@ __global__ __launch_bounds__(PersistShape<NPE>::kThreads) void k_pcg_persist(con
         // p = z + beta p
         const T beta = (T)beta_d;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
+        for (int c = 0; c < NC; ++c) {
             pv[c] = z[c] + beta * pv[c];
-            ps[3 * t + c] = pv[c];
+            ps[NC * t + c] = pv[c];
         }
         __syncthreads();
         // element products; p.Kp as the sum of the elements' energies (p is
-        // zero on fixed DOFs and K_e annihilates translations)
-        double en[1] = {0.0};
-        auto xl = [&](int i, T (&v)[3]) {
-            v[0] = ps[cl[i]];
-            v[1] = ps[cl[i] + 1];
-            v[2] = ps[cl[i] + 2];
-        };
-        if constexpr (VL) {
-            const T cLa = FOLD ? A.rho : fac[NF > 9 ? 9 : 0], cMu = FOLD ? T(1) : fac[NF > 10 ? 10 : 0];
-            const T e = tet10_vertex<T>(reinterpret_cast<const T(&)[9]>(fac), cLa, cMu, kv, xl, [&](int m, T f0, T f1, T f2) {
-                ys[row[m]] = f0;
-                ys[row[m] + ST] = f1;
-                ys[row[m] + 2 * ST] = f2;
-            });
-            if (has_el) en[0] = (double)e;
-        } else if (has_el) {
-            T x0[3];
-            xl(0, x0);
-            auto out = [&](int i, T f0, T f1, T f2) {
-                ys[(3 * i) * ST + t] = f0;
-                ys[(3 * i + 1) * ST + t] = f1;
-                ys[(3 * i + 2) * ST + t] = f2;
-                if (i > 0) {
-                    T v[3];
-                    xl(i, v);
-                    en[0] += (double)((v[0] - x0[0]) * f0 + (v[1] - x0[1]) * f1 + (v[2] - x0[2]) * f2);
-                }
-            };
-            mf_element_f<NPE, T, true, FOLD>([&](int, int m) -> T { return fac[m]; }, xl, out, A.rho);
+        // zero on fixed DOFs)
+        double en[1] = {Op::product(
+            A, data, k, kv, has_el, [&](int m, int c) -> T { return ps[cl[m] + c]; },
+            [&](int m, int c, T v) { ys[c * CS + row[m]] = v; })};
+        if constexpr (NC == 1) {
+            if (data.face >= 0) {
+                wave_sync();  // after the quad's own terms (LDS accesses of one wave stay in order)
+                en[0] += Op::faces(
+                    A, data, k, [&](int i) -> T { return ps[A.connL[(size_t)i * A.n_el + k]]; },
+                    [&](int i, T v) { ys[i * ST + el] += v; });
+            }
         }
         __syncthreads();
-        // nodal sums in ascending local element order
-        T q[3] = {T(0), T(0), T(0)};
-        // four incidences' terms are in flight at a time
+        // nodal sums in ascending local element order, four incidences' terms
+        // in flight at a time
+        T q[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) q[c] = T(0);
 #pragma unroll
         for (int m0 = 0; m0 < kInc; m0 += 4)
             if (m0 < cw) {  // uniform in the wave
-                T v[4][3];
+                T v[4][NC];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
                     const uint32_t w = inc[(m0 + u) / 2];
                     const int m = (int)(u & 1 ? w >> 16 : w & 0xffffu);
 #pragma unroll
-                    for (int c = 0; c < 3; ++c) v[u][c] = ys[m + c * ST];
+                    for (int c = 0; c < NC; ++c) v[u][c] = ys[m + c * CS];
                 }
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
 #pragma unroll
-                    for (int c = 0; c < 3; ++c) q[c] += v[u][c];
+                    for (int c = 0; c < NC; ++c) q[c] += v[u][c];
             }
         for (int m = kInc; m < cnt; ++m) {
             const int o = (int)A.lin[base + m];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) q[c] += ys[o + c * ST];
+            for (int c = 0; c < NC; ++c) q[c] += ys[o + c * CS];
         }
-        if (slot >= 0) part.put(slot, q);
+        if (slot >= 0) part.template put<NC>(slot, q);
         stores_done();  // before the block barrier in grid_sum, hence before its words
-        if (!grid_sum<1, NT>(en, wordsB, nwg, epoch, shB, &bad)) break;
+        if (!grid_sum<1, NT>(en, wordsB, p, nwg, epoch, shB, &bad)) break;
         pq = en[0];
         alpha_d = (pq > 0.0 && finite(pq)) ? rz / pq : 0.0;
         const T alpha = (T)alpha_d;
@@ -547,42 +794,45 @@ __global__ __launch_bounds__(PersistShape<NPE>::kThreads) void k_pcg_persist(con
             // own from the registers), the first four in flight together
             constexpr int kS = 4;
             const int n = sh & 31, first = sh >> 5, me = slot - first;
-            T v[kS][3], s[3] = {T(0), T(0), T(0)};
+            T v[kS][NC], s[NC];
 #pragma unroll
             for (int u = 0; u < kS; ++u) {
 #pragma unroll
-                for (int c = 0; c < 3; ++c) v[u][c] = u == me ? q[c] : T(0);
-                if (u < n && u != me) part.get(first + u, v[u]);
+                for (int c = 0; c < NC; ++c) v[u][c] = u == me ? q[c] : T(0);
+                if (u < n && u != me) part.template get<NC>(first + u, v[u]);
             }
 #pragma unroll
-            for (int u = 0; u < kS; ++u)
+            for (int c = 0; c < NC; ++c) {
+                s[c] = v[0][c];
 #pragma unroll
-                for (int c = 0; c < 3; ++c) s[c] += v[u][c];
+                for (int u = 1; u < kS; ++u) s[c] += v[u][c];
+            }
             for (int u = kS; u < n; ++u) {
-                T w[3] = {q[0], q[1], q[2]};
-                if (u != me) part.get(first + u, w);
+                T w[NC];
 #pragma unroll
-                for (int c = 0; c < 3; ++c) s[c] += w[c];
+                for (int c = 0; c < NC; ++c) w[c] = q[c];
+                if (u != me) part.template get<NC>(first + u, w);
+#pragma unroll
+                for (int c = 0; c < NC; ++c) s[c] += w[c];
             }
 #pragma unroll
-            for (int c = 0; c < 3; ++c) q[c] = s[c];
+            for (int c = 0; c < NC; ++c) q[c] = s[c];
         }
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
+        for (int c = 0; c < NC; ++c) {
             if (fx >> c & 1u) q[c] = T(0);
             x[c] += alpha * pv[c];
             r[c] -= alpha * q[c];
         }
     }
     if (bad) {
-        if (t == 0) A.S->fail = 1;
+        if (t == 0) S->fail = 1;
         return;
     }
     if (own)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) A.x[3 * (size_t)node + c] = x[c];
+        for (int c = 0; c < 3; ++c) xvec[3 * (size_t)node + c] = c < NC ? x[c < NC ? c : 0] : T(0);
     if (p == 0 && t == 0) {
-        PcgScalars *S = A.S;
         S->rz[0] = S->rz[1] = rz;
         S->alpha = alpha_d;
         S->beta = beta_d;
@@ -597,34 +847,50 @@ __global__ __launch_bounds__(PersistShape<NPE>::kThreads) void k_pcg_persist(con
 }
 
 // no word of an earlier solve is taken for one of this
-__global__ __launch_bounds__(256) void k_persist_clear(int n, uint64_t *__restrict__ words, PcgScalars *S) {
+__global__ __launch_bounds__(256) void k_persist_clear(int n, uint64_t *__restrict__ words, int nsys, PcgScalars *S) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) words[i] = 0;
-    if (i == 0) S->fail = 0;
+    if (i < nsys) S[i].fail = 0;
 }
 
 // --------------------------------------------------------------- launchers ---
 struct PersistLaunch { const void *f = nullptr; PersistGeometry g; };
-template <int NPE, typename T, bool FOLD> static PersistLaunch persist_of() {
-    using SH = PersistShape<NPE>;
-    return {(const void *)k_pcg_persist<NPE, T, FOLD>, {SH::kEl, SH::kThreads, SH::kStride}};
+template <class Op> static PersistLaunch persist_of() {
+    return {(const void *)k_pcg_persist<Op>, {Op::kEl, kNT, Op::kStride}};
 }
-template <typename T> static PersistLaunch persist_kernel(const jfm_ctx *ctx) {
-    if (ctx->npe == 4) return persist_of<4, T, false>();
-    if (ctx->npe != 10 || !ctx->affine) return {};
-    if constexpr (sizeof(T) == 4)
-        if (ctx->nu_uniform) return persist_of<10, T, true>();
-    return persist_of<10, T, false>();
+// the kernel of an operator on this mesh; none: the launched form
+template <typename T> static PersistLaunch persist_kernel(const jfm_ctx *ctx, int op) {
+    const bool tet10 = ctx->npe == 10 && ctx->affine;
+    if (op == JFM_OP_MATFREE) {
+        if constexpr (sizeof(T) == 4)
+            if (tet10 && ctx->nu_uniform) return persist_of<ElasticTet10<T, true>>();
+        if (tet10) return persist_of<ElasticTet10<T, false>>();
+        if (ctx->npe == 4) return persist_of<ElasticTet4<T>>();
+    }
+    if constexpr (sizeof(T) == 8) {
+        if (op == kOpHeat) {
+            if (tet10) return persist_of<HeatTet10>();
+            if (ctx->npe == 4) return persist_of<HeatElem<4>>();
+            if (ctx->npe == 8) return persist_of<HeatElem<8>>();
+        }
+        if (op == kOpMass) {
+            if (tet10) return persist_of<MassTet10>();
+            if (ctx->npe == 4) return persist_of<MassElem<4>>();
+            if (ctx->npe == 8) return persist_of<MassElem<8>>();
+        }
+    }
+    return {};
 }
 
-template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, bool *yes) {
-    *yes = false;
+template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys) {
+    const int want = *nsys;
+    *nsys = 0;
     static const bool on = [] {
         const char *v = std::getenv("JFEM_PERSIST");
         return !(v && v[0] == '0');
     }();
-    if (!on || ctx->persist_off || op != JFM_OP_MATFREE || !jfem_patch_enabled() || ctx->n_el < 1) return JFM_OK;
-    const PersistLaunch L = persist_kernel<T>(ctx);
+    if (!on || ctx->persist_off || !jfem_patch_enabled() || ctx->n_el < 1) return JFM_OK;
+    const PersistLaunch L = persist_kernel<T>(ctx, op);
     if (!L.f) return JFM_OK;
     const int64_t np = (ctx->n_el + L.g.elems - 1) / L.g.elems;
     if (np > kPersistPatches) return JFM_OK;
@@ -637,15 +903,21 @@ template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, bool *yes) {
         (void)hipGetLastError();
         return JFM_OK;
     }
+    if (op == kOpHeat && !ctx->heat_resident) return JFM_OK;
     if (int rc = jfem_cells_setup(ctx, L.g)) return rc;
-    *yes = ctx->cells.usable;
+    if (!ctx->cells.usable) return JFM_OK;
+    int m = want;  // as many systems side by side as fit, a divisor of those asked for
+    while (m > 1 && (want % m || m * np > (int64_t)per_cu * cus)) --m;
+    if (int rc = jfem_cells_systems(ctx, m)) return rc;
+    *nsys = m;
     return JFM_OK;
 }
 
 template <typename T>
-hipError_t launch_pcg_persist(jfm_ctx *ctx, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit) {
+hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit,
+                              int nsys, int64_t ss) {
     const auto &C = ctx->cells;
-    const PersistLaunch L = persist_kernel<T>(ctx);
+    const PersistLaunch L = persist_kernel<T>(ctx, op);
     const bool fold = sizeof(T) == 4 && C.gfQ32;
     PersistArgs<T> A{};
     A.n_el = (int)ctx->n_el;
@@ -653,6 +925,16 @@ hipError_t launch_pcg_persist(jfm_ctx *ctx, const T *Minv, const T *b, const T *
     A.connL = C.connL;
     A.el = sizeof(T) == 8 ? (const T *)C.gf64 : (fold ? (const T *)C.gfQ32 : (const T *)C.gf32);
     A.rho = fold ? (T)C.rho32 : T(0);
+    A.ngf = ctx->ngf;
+    A.kc = ctx->heat_k;
+    A.eperm = C.eperm;
+    if (op == kOpHeat && ctx->hf_h && ctx->hf_n > 0) {
+        A.ef = ctx->hf_first;
+        A.enext = ctx->hf_next;
+        A.fmap = ctx->hf_map;
+        A.fk = ctx->hf_K;
+        A.nfn = ctx->hf_nfn;
+    }
     A.pn_ptr = C.pn_ptr;
     A.pn_node = C.pn_node;
     A.pn_slot = C.pn_slot;
@@ -660,7 +942,7 @@ hipError_t launch_pcg_persist(jfm_ctx *ctx, const T *Minv, const T *b, const T *
     A.pn_cnt = C.pn_cnt;
     A.pn_inc = C.pn_inc;
     A.lin = C.lin;
-    A.fixed = ctx->fixed;
+    A.fixed = op == kOpMass ? nullptr : ctx->fixed;
     A.Minv = Minv;
     A.b = b;
     A.r0 = r0;
@@ -670,16 +952,18 @@ hipError_t launch_pcg_persist(jfm_ctx *ctx, const T *Minv, const T *b, const T *
     A.words = C.words;
     A.rtol2 = rtol * rtol;
     A.maxit = maxit;
-    A.S = ctx->S;
-    const int nw = kPersistWords * (C.npatch + kGroup * kGroup);
-    k_persist_clear<<<(nw + 255) / 256, 256, 0, ctx->stream>>>(nw, C.words, ctx->S);
+    A.S = nsys > 1 ? C.S : ctx->S;
+    A.nsys = nsys;
+    A.ss = ss;
+    const int nw = nsys * kPersistWords * (C.npatch + kGroup * kGroup);
+    k_persist_clear<<<(nw + 255) / 256, 256, 0, ctx->stream>>>(nw, C.words, nsys, A.S);
     void *args[] = {&A};
-    return hipLaunchCooperativeKernel(L.f, dim3(C.npatch), dim3(L.g.threads), args, 0, ctx->stream);
+    return hipLaunchCooperativeKernel(L.f, dim3(nsys * C.npatch), dim3(kNT), args, 0, ctx->stream);
 }
 
-template int jfem_persist_ready<double>(jfm_ctx *, int, bool *);
-template int jfem_persist_ready<float>(jfm_ctx *, int, bool *);
-template hipError_t launch_pcg_persist<double>(jfm_ctx *, const double *, const double *, const double *, double *, double, int);
-template hipError_t launch_pcg_persist<float>(jfm_ctx *, const float *, const float *, const float *, float *, double, int);
+template int jfem_persist_ready<double>(jfm_ctx *, int, int *);
+template int jfem_persist_ready<float>(jfm_ctx *, int, int *);
+template hipError_t launch_pcg_persist<double>(jfm_ctx *, int, const double *, const double *, const double *, double *, double, int, int, int64_t);
+template hipError_t launch_pcg_persist<float>(jfm_ctx *, int, const float *, const float *, const float *, float *, double, int, int, int64_t);
 
 }  // namespace jfem

@@ -228,6 +228,19 @@ __global__ __launch_bounds__(256) void k_diag_blocks(int N, const double *__rest
     for (int c = 0; c < 3; ++c) M[4 * c] = 1.0 / d[3 * (size_t)a + c];
 }
 
+__global__ __launch_bounds__(256) void k_post_join(int N, const double *__restrict__ x0, const double *__restrict__ x1,
+                                                  double *__restrict__ out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;  // (node, component) of the six
+    if (i >= 6 * N) return;
+    const int a = i / 6, c = i - 6 * a;
+    out[i] = c < 3 ? x0[3 * (size_t)a + c] : x1[3 * (size_t)a + c - 3];
+}
+
+hipError_t launch_post_join(jfm_ctx *ctx, const double *x0, const double *x1, double *out) {
+    k_post_join<<<nblk(6 * ctx->N), kBlock, 0, ctx->stream>>>((int)ctx->N, x0, x1, out);
+    return hipGetLastError();
+}
+
 template <int MODE>
 static hipError_t lsq_dispatch(jfm_ctx *ctx, const double *u, int field, int comp0, const double *x, const int *done) {
     const int n = (int)ctx->n_el;

@@ -5,8 +5,9 @@ groups of 16 workgroups and of its range (256 workgroups), against the oracle's
 direct solve, and against the launched iterations (JFEM_PERSIST=0, a child
 process): the FP64 iteration counts differ only by the order of the reductions
 (3% + 2; the FP32 inner solves restart at FP32's attainable residual, where
-rounding decides the count), the answers are bit-reproducible.  The bars follow from the solves'
-own tolerance: the residual 1e-10 (1e-11 is below what the FP64
+rounding decides the count), the answers are bit-reproducible.  Heat conduction (convection faces
+on elements, and one that is on none) and the nodal fits run resident too.  The
+bars follow from the solves' own tolerance: the residual 1e-10 (1e-11 is below what the FP64
 residual of such a cantilever can show) bounds the error at 1e-8 for these meshes
 (the direct solve itself is good to 1e-10).
 """
@@ -113,4 +114,54 @@ def test_resident_edges(oracle):
     u, la, _ = ctx.solve(rtol=1e-10, want_la=True)
     ud, lad, _ = oracle.solve_direct_lapack(csr, m.fixed_mask(), g, oracle.load_vector(m))
     assert np.linalg.norm(u - ud) <= 1e-8 * np.linalg.norm(ud)
+    ctx.close()
+
+
+# elements per patch: Tet10 128, Hex8 256, Tet4 512
+OTHER = [("box_tet10", (7, 3, 1)), ("box_tet10", (19, 6, 3)), ("box_hex8", (17, 5, 3)), ("box_hex8", (37, 7, 1)),
+         ("box_tet4", (24, 9, 8))]
+
+
+@pytest.mark.parametrize("gen,g", OTHER)
+@pytest.mark.parametrize("attached", [True, False])
+def test_resident_heat(oracle, gen, g, attached):
+    """Bar: rtol 1e-12 on the residual, 1e-8 on the temperatures, as the heat
+    tests of one patch ask."""
+    import jfem
+    m = getattr(M, gen)(*g, seed=6, jitter=0.1)
+    rng = np.random.default_rng(3)
+    k, q = np.exp(0.5 * rng.standard_normal(m.n_el)) * 3.0, rng.uniform(0.5, 2.0, m.n_el)
+    faces = m.faces.copy()
+    if not attached:   # a face whose nodes no element holds together
+        faces[0] = np.linspace(0, m.n_nodes - 1, faces.shape[1]).astype(np.int64)
+    nf = faces.shape[0]
+    flux, h, te = rng.uniform(0, 1, nf), rng.uniform(0.5, 1.0, nf), rng.uniform(10, 20, nf)
+    fixed = np.isclose(m.X[:, 0], 0.0)
+    Tf = np.full(m.n_nodes, 5.0)
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    say(f"resident heat {gen} {g} attached={attached}")
+    T, st = ctx.heat_solve(k, q, faces, flux=flux, h=h, T_ext=te, fixed=fixed, T_fixed=Tf, rtol=1e-12)
+    Kh, f = oracle.heat_system(m, k, q=q, faces=faces, ftype=m.ftype, flux=flux, h=h, T_ext=te)
+    To = oracle.heat_solve_direct(Kh, f, fixed, Tf)
+    assert st["converged"] == 1
+    assert np.abs(T - To).max() <= 1e-8 * np.abs(To).max()
+    ctx.close()
+
+
+@pytest.mark.parametrize("gen,g", OTHER)
+def test_resident_fit(oracle, gen, g):
+    """Bar: 1e-9 of the largest value, as the fit tests of one patch ask."""
+    import jfem
+    m = getattr(M, gen)(*g, seed=6, jitter=0.1)
+    u = np.random.default_rng(4).standard_normal(m.n_dofs) * 1e-3
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    say(f"resident fit {gen} {g}")
+    out = ctx.postprocess(u)
+    one = ctx.postprocess(u, gauss=False)
+    for field in ("strain", "stress"):
+        ref = oracle.lsq_fit(m, u, field)
+        assert np.abs(out[field + "_nodal"] - ref).max() <= 1e-9 * np.abs(ref).max()
+        assert np.array_equal(out[field + "_nodal"], one[field + "_nodal"])
     ctx.close()
