@@ -201,6 +201,7 @@ static void release_mesh(jfm_ctx *ctx) {
     jfem_coarse_release(ctx);
     jfem_patch_release(ctx);
     jfem_cells_release(ctx);
+    jfem_train_release(ctx);
     release_heat(ctx);
     ctx->h_X.clear();
     ctx->has_user = false;
@@ -1012,7 +1013,7 @@ static int true_residual(jfm_ctx *ctx, int op, const double *b, const double *u,
 static int learned_select(jfm_ctx *ctx, int op, int probe, int check, bool *use, int *iters, double *setup_ms,
                           bool coarse) {
     double lms = 0.0;
-    if (int rc = jfem_learned_prepare(ctx, &lms)) return rc;
+    if (int rc = jfem_learned_prepare(ctx, setup_ms ? &lms : nullptr)) return rc;
     if (setup_ms) *setup_ms += lms;
     *use = true;
     if (probe <= 0) return JFM_OK;

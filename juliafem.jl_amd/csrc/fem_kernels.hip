@@ -14,7 +14,8 @@
 // (g = grad N), which is what the kernels evaluate instead of the 6x30
 // products; the oracle keeps the reference's BL form and the tests compare.
 //
-// Every nodal sum runs over the node's incidences in ascending element id;
+// Every nodal sum of the operators runs over the node's incidences in ascending
+// element id, the diagonal blocks' over its lanes in a fixed order;
 // there are no floating-point atomics.
 #include <algorithm>
 
@@ -513,8 +514,8 @@ __global__ __launch_bounds__(256) void k_face(int nf, int nfn, const int32_t *__
 }
 
 // ----------------------------------------------------------- block Jacobi --
-// Diagonal 3x3 blocks sum_e K_e(i,i) over the node's incidences (ascending
-// element id), fixed rows/columns replaced by identity before inversion and
+// Diagonal 3x3 blocks sum_e K_e(i,i) over the node's incidences
+// (kNodeLanes lanes per node), fixed rows/columns replaced by identity before inversion and
 // zeroed after, so the preconditioner never touches fixed DOFs.
 template <int NPE>
 __global__ __launch_bounds__(256) void k_block_jacobi(int N, const int32_t *__restrict__ ptr,
@@ -523,11 +524,11 @@ __global__ __launch_bounds__(256) void k_block_jacobi(int N, const int32_t *__re
                                                      const uint8_t *__restrict__ fixed,
                                                      double *__restrict__ M64, float *__restrict__ M32) {
     using EL = Elem<NPE>;
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= N) return;
+    const int a = (blockIdx.x * blockDim.x + threadIdx.x) / kNodeLanes, lane = threadIdx.x % kNodeLanes;
+    if (a >= N) return;  // the node's lanes together
     double B[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     const int k1 = ptr[a + 1];
-    for (int k = ptr[a]; k < k1; ++k) {
+    for (int k = ptr[a] + lane; k < k1; k += kNodeLanes) {
         const int idx = inc[k];
         const int e = idx / NPE, i = idx - e * NPE;
         for (int q = 0; q < EL::NGP; ++q) {
@@ -543,6 +544,8 @@ __global__ __launch_bounds__(256) void k_block_jacobi(int N, const int32_t *__re
                 for (int c = 0; c < 3; ++c) B[r * 3 + c] += cl * g[r] * g[c] + cm * (g[c] * g[r] + (r == c ? dot : 0.0));
         }
     }
+    for (int m = 0; m < 9; ++m) B[m] = node_sum(B[m]);
+    if (lane != 0) return;
     const uint8_t f0 = fixed ? fixed[3 * (size_t)a] : 0, f1 = fixed ? fixed[3 * (size_t)a + 1] : 0,
                   f2 = fixed ? fixed[3 * (size_t)a + 2] : 0;
     const uint8_t fx[3] = {f0, f1, f2};
@@ -660,9 +663,9 @@ hipError_t launch_face_gather(jfm_ctx *ctx) {
 hipError_t launch_block_jacobi(jfm_ctx *ctx, double *Minv64, float *Minv32) {
     const int N = (int)ctx->N;
     switch (ctx->npe) {
-    case 10: k_block_jacobi<10><<<nblk(N), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, (int)ctx->n_el, ctx->ngf, ctx->gf64, ctx->fixed, Minv64, Minv32); break;
-    case 4: k_block_jacobi<4><<<nblk(N), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, (int)ctx->n_el, ctx->ngf, ctx->gf64, ctx->fixed, Minv64, Minv32); break;
-    case 8: k_block_jacobi<8><<<nblk(N), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, (int)ctx->n_el, ctx->ngf, ctx->gf64, ctx->fixed, Minv64, Minv32); break;
+    case 10: k_block_jacobi<10><<<nblk(N, kBlock / kNodeLanes), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, (int)ctx->n_el, ctx->ngf, ctx->gf64, ctx->fixed, Minv64, Minv32); break;
+    case 4: k_block_jacobi<4><<<nblk(N, kBlock / kNodeLanes), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, (int)ctx->n_el, ctx->ngf, ctx->gf64, ctx->fixed, Minv64, Minv32); break;
+    case 8: k_block_jacobi<8><<<nblk(N, kBlock / kNodeLanes), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, (int)ctx->n_el, ctx->ngf, ctx->gf64, ctx->fixed, Minv64, Minv32); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -236,6 +236,13 @@ struct jfm_ctx {
     float *feat = nullptr;         // N x 24 node features
     double *efeat = nullptr;       // 3 x n_el per-element feature inputs
     float *lout = nullptr;         // N x 6 network outputs
+    // training step (jfm_learned_grad): pairs, z, w = K z, dLoss/dM, gradient
+    // partials, the pairs' products
+    struct Train {
+        double *r = nullptr, *e = nullptr, *z = nullptr, *w = nullptr, *G = nullptr, *dots = nullptr;
+        float *gpart = nullptr, *grad = nullptr;
+        int pairs = 0, ndots = 0;
+    } train;
     // nonlinear state (tangent operator)
     double *ustate64 = nullptr;    // displacement the tangent is taken at
     float *ustate32 = nullptr;

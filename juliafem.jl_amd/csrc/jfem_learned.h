@@ -43,7 +43,8 @@ hipError_t launch_mblocks(jfm_ctx *ctx, const float *out, const double *Minv, fl
 }  // namespace jfem
 
 // Builds features, runs the network and forms Mlearn64/Mlearn32 for the
-// current mesh and boundary conditions.  *ms receives the device time.  If
+// current mesh and boundary conditions.  *ms (may be null) receives the device
+// time, for which the host then waits.  If
 // jfem_learned_launch started that work, joins it instead (the main stream
 // waits for it).
 int jfem_learned_prepare(jfm_ctx *ctx, double *ms);
@@ -52,5 +53,7 @@ int jfem_learned_prepare(jfm_ctx *ctx, double *ms);
 // (the coarse setup); jfem_learned_prepare joins it.  No-op when the blocks
 // are current or no weights are loaded.
 int jfem_learned_launch(jfm_ctx *ctx);
+// Frees the training step's buffers.
+void jfem_train_release(jfm_ctx *ctx);
 // Waits for a started, not yet joined, learned launch and drops it.
 void jfem_learned_drop(jfm_ctx *ctx);

@@ -82,8 +82,8 @@ __global__ __launch_bounds__(256) void k_features(int N, int n_el, int ngf, cons
                                                  const uint8_t *__restrict__ fixed, const int32_t *__restrict__ fptr,
                                                  const double *__restrict__ Dover, float *__restrict__ feat) {
     using EL = Elem<NPE>;
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= N) return;
+    const int a = (blockIdx.x * blockDim.x + threadIdx.x) / kNodeLanes, lane = threadIdx.x % kNodeLanes;
+    if (a >= N) return;  // the node's lanes together
     double D[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     double tmin = 1e300, tmax = 0, tsum = 0, tsq = 0;
     double emin = 1e300, emax = 0, esum = 0, lesum = 0, tle = 0;
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void k_features(int N, int n_el, int ngf, cons
     int ncorner = 0, nfixel = 0;
     const int k0 = ptr[a], k1 = ptr[a + 1];
     const int n = k1 - k0;
-    for (int k = k0; k < k1; ++k) {
+    for (int k = k0 + lane; k < k1; k += kNodeLanes) {
         const int idx = inc[k];
         const int e = idx / NPE, i = idx - e * NPE;
         double te = 0.0;
@@ -118,11 +118,19 @@ __global__ __launch_bounds__(256) void k_features(int N, int n_el, int ngf, cons
         if (i < corners<NPE>()) ++ncorner;
         if (ef[2 * (size_t)n_el + e] != 0.0) ++nfixel;
     }
+    for (int m = 0; m < 9; ++m) D[m] = node_sum(D[m]);
+    tmin = node_min(tmin); tmax = node_max(tmax); tsum = node_sum(tsum); tsq = node_sum(tsq);
+    emin = node_min(emin); emax = node_max(emax); esum = node_sum(esum); lesum = node_sum(lesum); tle = node_sum(tle);
+    qsum = node_sum(qsum); qmin = node_min(qmin); qmax = node_max(qmax);
+    ncorner = (int)node_sum((double)ncorner);
+    nfixel = (int)node_sum((double)nfixel);
     if (Dover)  // diagonal block of the tangent in place of the linear one
         for (int m = 0; m < 9; ++m) D[m] = Dover[9 * (size_t)a + m];
     const double emean = esum / n;
     int nabove = 0;
-    for (int k = k0; k < k1; ++k) nabove += (E[inc[k] / NPE] > emean) ? 1 : 0;
+    for (int k = k0 + lane; k < k1; k += kNodeLanes) nabove += (E[inc[k] / NPE] > emean) ? 1 : 0;
+    nabove = (int)node_sum((double)nabove);
+    if (lane != 0) return;
     const double T = D[0] + D[4] + D[8];
     const double s = 3.0 / T;
     const double d00 = D[0] * s, d11 = D[4] * s, d22 = D[8] * s, d01 = D[1] * s, d12 = D[5] * s, d02 = D[2] * s;
@@ -487,9 +495,31 @@ __global__ __launch_bounds__(256) void k_block_apply(int N, const double *__rest
     for (int i = 0; i < 3; ++i) z[o + i] = Ma[i * 3] * r[o] + Ma[i * 3 + 1] * r[o + 1] + Ma[i * 3 + 2] * r[o + 2];
 }
 
-// G_a += coef (r - c w)_a r_a'
-__global__ __launch_bounds__(256) void k_accum_dm(int N, double coef, double c, const double *__restrict__ r,
-                                                 const double *__restrict__ w, double *__restrict__ G) {
+// The three products of a training pair (z.r, z.w, e.r) in one pass: one
+// partial of each per block (part[k kMaxPart + block]).
+__global__ __launch_bounds__(256) void k_pair_dots(int n, const double *__restrict__ z, const double *__restrict__ r,
+                                                  const double *__restrict__ w, const double *__restrict__ e,
+                                                  double *__restrict__ part) {
+    double v[3] = {0.0, 0.0, 0.0};
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const double zi = z[i], ri = r[i];
+        v[0] += zi * ri;
+        v[1] += zi * w[i];
+        v[2] += e[i] * ri;
+    }
+    write_partials<3>(v, part);
+}
+
+// G_a += coef (r - c w)_a r_a' with c = z.r / z.w, coef = -2 c / (e.r n_pairs),
+// from the partials of k_pair_dots; block 0 leaves the three products in `dots`
+// for the host, which reads them once for all pairs.
+__global__ __launch_bounds__(256) void k_accum_dm(int N, int n_pairs, int npart, const double *__restrict__ part,
+                                                 const double *__restrict__ r, const double *__restrict__ w,
+                                                 double *__restrict__ G, double *__restrict__ dots) {
+    double t[3];
+    sum_partials<3>(part, npart, t);
+    const double c = t[0] / t[1], coef = -2.0 * c / (t[2] * n_pairs);
+    if (blockIdx.x == 0 && threadIdx.x < 3) dots[threadIdx.x] = t[threadIdx.x];
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= N) return;
     const size_t o = 3 * (size_t)a;
@@ -499,17 +529,29 @@ __global__ __launch_bounds__(256) void k_accum_dm(int N, double coef, double c, 
     }
 }
 
-// grad[p] = sum over wave partials, fixed order
-__global__ __launch_bounds__(256) void k_grad_reduce(int nparts, const float *__restrict__ gpart, float *__restrict__ grad) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kNParam) return;
+// grad[p] = sum over wave partials, fixed order: a block takes 64 parameters,
+// each of its 16 waves every 16th partial (one thread per parameter walking
+// all partials took 122 us for 512 of them, one dependent load after another).
+__global__ __launch_bounds__(1024) void k_grad_reduce(int nparts, const float *__restrict__ gpart, float *__restrict__ grad) {
+    __shared__ double sh[16][64];
+    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, p = blockIdx.x * 64 + l;
     double s = 0.0;
-    for (int w = 0; w < nparts; ++w) s += gpart[(size_t)w * kNParam + p];
-    grad[p] = (float)s;
+    if (p < kNParam)
+#pragma unroll 8
+        for (int w = wv; w < nparts; w += 16) s += gpart[(size_t)w * kNParam + p];
+    sh[wv][l] = s;
+    __syncthreads();
+    if (wv == 0 && p < kNParam) {
+#pragma unroll
+        for (int w = 1; w < 16; ++w) s += sh[w][l];
+        grad[p] = (float)s;
+    }
 }
 
 static inline unsigned nblk(int64_t n, int b = kBlock) { return (unsigned)((n + b - 1) / b); }
-constexpr int kTrainBlocks = 256;
+// two blocks per CU by their LDS (at 20,449 nodes, 640 pairs of tiles: the
+// training pass 60 us with 256 blocks)
+constexpr int kTrainBlocks = 512;
 
 // ef: 3 n_el doubles of per-element inputs (k_elem_features)
 hipError_t launch_features(jfm_ctx *ctx, double *ef, float *feat, hipStream_t s) {
@@ -518,15 +560,15 @@ hipError_t launch_features(jfm_ctx *ctx, double *ef, float *feat, hipStream_t s)
     switch (ctx->npe) {
     case 10:
         if (ne) k_elem_features<10><<<nblk(ne), kBlock, 0, s>>>(ne, ctx->conn, ctx->gf64, ctx->E, ctx->nu, ctx->fixed, ef);
-        k_features<10><<<nblk(N), kBlock, 0, s>>>(N, ne, ctx->ngf, ctx->inc_ptr, ctx->inc, ef, ctx->gf64, ctx->E, ctx->fixed, ctx->finc_ptr, Dover, feat);
+        k_features<10><<<nblk(N, kBlock / kNodeLanes), kBlock, 0, s>>>(N, ne, ctx->ngf, ctx->inc_ptr, ctx->inc, ef, ctx->gf64, ctx->E, ctx->fixed, ctx->finc_ptr, Dover, feat);
         break;
     case 4:
         if (ne) k_elem_features<4><<<nblk(ne), kBlock, 0, s>>>(ne, ctx->conn, ctx->gf64, ctx->E, ctx->nu, ctx->fixed, ef);
-        k_features<4><<<nblk(N), kBlock, 0, s>>>(N, ne, ctx->ngf, ctx->inc_ptr, ctx->inc, ef, ctx->gf64, ctx->E, ctx->fixed, ctx->finc_ptr, Dover, feat);
+        k_features<4><<<nblk(N, kBlock / kNodeLanes), kBlock, 0, s>>>(N, ne, ctx->ngf, ctx->inc_ptr, ctx->inc, ef, ctx->gf64, ctx->E, ctx->fixed, ctx->finc_ptr, Dover, feat);
         break;
     case 8:
         if (ne) k_elem_features<8><<<nblk(ne), kBlock, 0, s>>>(ne, ctx->conn, ctx->gf64, ctx->E, ctx->nu, ctx->fixed, ef);
-        k_features<8><<<nblk(N), kBlock, 0, s>>>(N, ne, ctx->ngf, ctx->inc_ptr, ctx->inc, ef, ctx->gf64, ctx->E, ctx->fixed, ctx->finc_ptr, Dover, feat);
+        k_features<8><<<nblk(N, kBlock / kNodeLanes), kBlock, 0, s>>>(N, ne, ctx->ngf, ctx->inc_ptr, ctx->inc, ef, ctx->gf64, ctx->E, ctx->fixed, ctx->finc_ptr, Dover, feat);
         break;
     default: return hipErrorInvalidValue;
     }
@@ -778,10 +820,12 @@ int jfem_learned_prepare(jfm_ctx *ctx, double *ms) {
     if (ms) *ms = 0.0;
     if (ctx->learned_pending) {  // started beside earlier work: join it
         JFM_HIP(ctx, hipStreamWaitEvent(ctx->stream, ctx->ev_l1, 0));
-        JFM_HIP(ctx, hipEventSynchronize(ctx->ev_l1));
-        float t = 0.f;
-        JFM_HIP(ctx, hipEventElapsedTime(&t, ctx->ev_l0, ctx->ev_l1));
-        if (ms) *ms = t;
+        if (ms) {  // the host waits only for a time that is asked for
+            JFM_HIP(ctx, hipEventSynchronize(ctx->ev_l1));
+            float t = 0.f;
+            JFM_HIP(ctx, hipEventElapsedTime(&t, ctx->ev_l0, ctx->ev_l1));
+            *ms = t;
+        }
         ctx->learned_pending = false;
         ctx->learned_ready = true;
         return JFM_OK;
@@ -791,10 +835,12 @@ int jfem_learned_prepare(jfm_ctx *ctx, double *ms) {
     JFM_HIP(ctx, hipEventRecord(ctx->ev_l0, ctx->stream));
     if (int rc = learned_enqueue(ctx, ctx->stream)) return rc;
     JFM_HIP(ctx, hipEventRecord(ctx->ev_l1, ctx->stream));
-    JFM_HIP(ctx, hipEventSynchronize(ctx->ev_l1));
-    float t = 0.f;
-    JFM_HIP(ctx, hipEventElapsedTime(&t, ctx->ev_l0, ctx->ev_l1));
-    if (ms) *ms = t;
+    if (ms) {
+        JFM_HIP(ctx, hipEventSynchronize(ctx->ev_l1));
+        float t = 0.f;
+        JFM_HIP(ctx, hipEventElapsedTime(&t, ctx->ev_l0, ctx->ev_l1));
+        *ms = t;
+    }
     ctx->learned_ready = true;
     return JFM_OK;
 }
@@ -821,6 +867,16 @@ extern "C" int jfm_learned_outputs(jfm_ctx *ctx, float *out, double *M) {
     return JFM_OK;
 }
 
+// residual/error pairs held on the device at a time
+constexpr int kPairRun = 8;
+
+void jfem_train_release(jfm_ctx *ctx) {
+    auto &W = ctx->train;
+    for (void *p : {(void *)W.r, (void *)W.e, (void *)W.z, (void *)W.w, (void *)W.G, (void *)W.gpart, (void *)W.grad, (void *)W.dots})
+        jfm_free(ctx, p);
+    W = {};
+}
+
 extern "C" int jfm_learned_grad(jfm_ctx *ctx, int32_t n_pairs, const double *r, const double *e, int32_t coarse_nodes,
                                 double *loss, float *grad) {
     if (!ctx || n_pairs <= 0 || !r || !e || !grad || coarse_nodes < 0) return JFM_EINVAL;
@@ -834,57 +890,74 @@ extern "C" int jfm_learned_grad(jfm_ctx *ctx, int32_t n_pairs, const double *r, 
         if (int rc = jfem_coarse_setup(ctx, JFM_OP_MATFREE, coarse_nodes, nullptr)) return rc;
     const int64_t n = ctx->ndof, N = ctx->N;
     hipStream_t s = ctx->stream;
-    double *dr = jfm_alloc<double>(ctx, n), *de = jfm_alloc<double>(ctx, n), *dz = jfm_alloc<double>(ctx, n),
-           *dw = jfm_alloc<double>(ctx, n), *G = jfm_alloc<double>(ctx, 9 * N);
-    float *gpart = jfm_alloc<float>(ctx, (int64_t)kTrainBlocks * kWaves * kNParam), *dgrad = jfm_alloc<float>(ctx, kNParam);
-    auto cleanup = [&] {
-        for (void *p : {(void *)dr, (void *)de, (void *)dz, (void *)dw, (void *)G, (void *)gpart, (void *)dgrad}) jfm_free(ctx, p);
-    };
-    if (!dr || !de || !dz || !dw || !G || !gpart || !dgrad) {
-        cleanup();
-        return jfm_fail(ctx, JFM_ENOMEM, "device allocation failed in jfm_learned_grad");
+    // the pairs go to the device in runs of up to kPairRun; the buffers stay
+    // with the mesh (a training loop calls this once per step)
+    auto &W = ctx->train;
+    const int run = std::min(n_pairs, kPairRun);
+    if (W.pairs < run) {
+        jfem_train_release(ctx);
+        W.r = jfm_alloc<double>(ctx, run * n);
+        W.e = jfm_alloc<double>(ctx, run * n);
+        W.z = jfm_alloc<double>(ctx, n);
+        W.w = jfm_alloc<double>(ctx, n);
+        W.G = jfm_alloc<double>(ctx, 9 * N);
+        W.gpart = jfm_alloc<float>(ctx, (int64_t)kTrainBlocks * kWaves * kNParam);
+        W.grad = jfm_alloc<float>(ctx, kNParam);
+        if (!W.r || !W.e || !W.z || !W.w || !W.G || !W.gpart || !W.grad) {
+            jfem_train_release(ctx);
+            return jfm_fail(ctx, JFM_ENOMEM, "device allocation failed in jfm_learned_grad");
+        }
+        W.pairs = run;
     }
-    int rc = JFM_OK;
-    double lsum = 0.0;
-    JFM_HIP(ctx, hipMemsetAsync(G, 0, sizeof(double) * 9 * N, s));
-    for (int p = 0; p < n_pairs && rc == JFM_OK; ++p) {
-        JFM_HIP(ctx, hipMemcpyAsync(dr, r + (size_t)p * n, sizeof(double) * n, hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(de, e + (size_t)p * n, sizeof(double) * n, hipMemcpyHostToDevice, s));
-        k_block_apply<<<nblk(N), kBlock, 0, s>>>((int)N, ctx->Mlearn64, dr, dz);
+    if (W.ndots < n_pairs) {
+        jfm_free(ctx, W.dots);
+        W.ndots = 0;
+        W.dots = jfm_alloc<double>(ctx, 3 * (int64_t)n_pairs);
+        if (!W.dots) return jfm_fail(ctx, JFM_ENOMEM, "device allocation failed in jfm_learned_grad");
+        W.ndots = n_pairs;
+    }
+    JFM_HIP(ctx, hipMemsetAsync(W.G, 0, sizeof(double) * 9 * N, s));
+    double *part = ctx->partials + kPartMisc;   // three rows of kMaxPart
+    static_assert(kPartTotal - kPartMisc >= 3 * kMaxPart, "room for three partials per block");
+    for (int p = 0; p < n_pairs; ++p) {
+        if (p % run == 0) {
+            const size_t m = (size_t)std::min(run, n_pairs - p) * n * sizeof(double);
+            JFM_HIP(ctx, hipMemcpyAsync(W.r, r + (size_t)p * n, m, hipMemcpyHostToDevice, s));
+            JFM_HIP(ctx, hipMemcpyAsync(W.e, e + (size_t)p * n, m, hipMemcpyHostToDevice, s));
+        }
+        const double *dr = W.r + (size_t)(p % run) * n, *de = W.e + (size_t)(p % run) * n;
+        k_block_apply<<<nblk(N), kBlock, 0, s>>>((int)N, ctx->Mlearn64, dr, W.z);
         if (coarse) {
             int np = 0;
-            hipError_t err = launch_coarse_correct<double>(ctx, dr, dz, nullptr, ctx->partials + kPartMisc, nullptr, &np);
-            if (err != hipSuccess) { rc = jfm_hip_fail(ctx, err, "coarse correction"); break; }
+            hipError_t err = launch_coarse_correct<double>(ctx, dr, W.z, nullptr, ctx->partials + kPartMisc, nullptr, &np);
+            if (err != hipSuccess) return jfm_hip_fail(ctx, err, "coarse correction");
         }
-        if ((rc = jfem_apply(ctx, JFM_OP_MATFREE, dz, dw))) break;
-        double zr = 0, zw = 0, er = 0;
-        if ((rc = jfem_dot(ctx, dz, dr, n, &zr)) || (rc = jfem_dot(ctx, dz, dw, n, &zw)) || (rc = jfem_dot(ctx, de, dr, n, &er)))
-            break;
-        if (!(zw > 0.0) || !(er > 0.0)) {
-            rc = jfm_fail(ctx, JFM_EINVAL, "training pair with non-positive energy (is e = K^-1 r on the free DOFs?)");
-            break;
-        }
-        const double c = zr / zw;
-        lsum += 1.0 - zr * c / er;
-        k_accum_dm<<<nblk(N), kBlock, 0, s>>>((int)N, -2.0 * c / (er * n_pairs), c, dr, dw, G);
+        if (int rc = jfem_apply(ctx, JFM_OP_MATFREE, W.z, W.w)) return rc;
+        const unsigned g = capped_grid(n, kBlock);
+        k_pair_dots<<<g, kBlock, 0, s>>>((int)n, W.z, dr, W.w, de, part);
+        k_accum_dm<<<nblk(N), kBlock, 0, s>>>((int)N, n_pairs, (int)g, part, dr, W.w, W.G, W.dots + 3 * p);
+        JFM_HIP(ctx, hipGetLastError());
     }
-    if (rc == JFM_OK) {
-        int nw = 0;
-        hipError_t err = launch_mlp(ctx, ctx->feat, ctx->mlp_w, ctx->lout, G, (const double *)ctx->ws64.Minv, gpart, &nw,
-                                    ctx->stream);
-        if (err == hipSuccess) {
-            k_grad_reduce<<<nblk(kNParam), kBlock, 0, s>>>(nw, gpart, dgrad);
-            err = hipGetLastError();
-        }
-        if (err != hipSuccess) rc = jfm_hip_fail(ctx, err, "launch_mlp(train)");
+    int nw = 0;
+    hipError_t err = launch_mlp(ctx, ctx->feat, ctx->mlp_w, ctx->lout, W.G, (const double *)ctx->ws64.Minv, W.gpart, &nw, s);
+    if (err == hipSuccess) {
+        k_grad_reduce<<<nblk(kNParam, 64), 1024, 0, s>>>(nw, W.gpart, W.grad);
+        err = hipGetLastError();
     }
-    if (rc == JFM_OK) {
-        hipError_t err = hipMemcpyAsync(grad, dgrad, sizeof(float) * kNParam, hipMemcpyDeviceToHost, s);
-        if (err == hipSuccess) err = hipStreamSynchronize(s);
-        if (err != hipSuccess) rc = jfm_hip_fail(ctx, err, "gradient copy");
-        if (loss) *loss = lsum / n_pairs;
+    if (err != hipSuccess) return jfm_hip_fail(ctx, err, "launch_mlp(train)");
+    std::vector<double> dots(3 * (size_t)n_pairs);
+    std::vector<float> gh(kNParam);
+    JFM_HIP(ctx, hipMemcpyAsync(gh.data(), W.grad, sizeof(float) * kNParam, hipMemcpyDeviceToHost, s));
+    JFM_HIP(ctx, hipMemcpyAsync(dots.data(), W.dots, sizeof(double) * dots.size(), hipMemcpyDeviceToHost, s));
+    JFM_HIP(ctx, hipStreamSynchronize(s));
+    double lsum = 0.0;
+    for (int p = 0; p < n_pairs; ++p) {
+        const double zr = dots[3 * p], zw = dots[3 * p + 1], er = dots[3 * p + 2];
+        if (!(zw > 0.0) || !(er > 0.0))
+            return jfm_fail(ctx, JFM_EINVAL, "training pair with non-positive energy (is e = K^-1 r on the free DOFs?)");
+        lsum += 1.0 - zr * (zr / zw) / er;
     }
-    (void)hipStreamSynchronize(s);
-    cleanup();
-    return rc;
+    std::memcpy(grad, gh.data(), sizeof(float) * kNParam);
+    if (loss) *loss = lsum / n_pairs;
+    return JFM_OK;
 }

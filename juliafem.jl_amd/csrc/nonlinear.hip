@@ -38,7 +38,7 @@ __global__ __launch_bounds__(256) void k_nh_elem(int n_el, const int32_t *__rest
 }
 
 // Diagonal 3x3 blocks of the tangent K_T(u), summed over the node's
-// incidences in ascending element id, inverted like the linear block Jacobi;
+// incidences (kNodeLanes lanes per node), inverted like the linear block Jacobi;
 // the raw blocks go to D (N x 9) for the learned preconditioner's features.
 template <int NPE>
 __global__ __launch_bounds__(256) void k_nh_block_jacobi(int N, const int32_t *__restrict__ ptr,
@@ -48,10 +48,10 @@ __global__ __launch_bounds__(256) void k_nh_block_jacobi(int N, const int32_t *_
                                                         double *__restrict__ M64, float *__restrict__ M32,
                                                         double *__restrict__ D) {
     using EL = Elem<NPE>;
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= N) return;
+    const int a = (blockIdx.x * blockDim.x + threadIdx.x) / kNodeLanes, lane = threadIdx.x % kNodeLanes;
+    if (a >= N) return;  // the node's lanes together
     double B[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    for (int k = ptr[a]; k < ptr[a + 1]; ++k) {
+    for (int k = ptr[a] + lane; k < ptr[a + 1]; k += kNodeLanes) {
         const int idx = inc[k];
         const int e = idx / NPE, i = idx - e * NPE;
         const size_t n0 = 3 * (size_t)conn[e];
@@ -84,6 +84,8 @@ __global__ __launch_bounds__(256) void k_nh_block_jacobi(int N, const int32_t *_
             }
         }
     }
+    for (int m = 0; m < 9; ++m) B[m] = node_sum(B[m]);
+    if (lane != 0) return;
     for (int m = 0; m < 9; ++m) D[9 * (size_t)a + m] = B[m];
     const uint8_t fx[3] = {fixed[3 * (size_t)a], fixed[3 * (size_t)a + 1], fixed[3 * (size_t)a + 2]};
     double M[9];
@@ -153,9 +155,9 @@ hipError_t launch_nh_elem(jfm_ctx *ctx, bool tangent, const T *gf, const T *u, c
 hipError_t launch_nh_block_jacobi(jfm_ctx *ctx, const double *u, double *M64, float *M32, double *D) {
     const int N = (int)ctx->N;
     switch (ctx->npe) {
-    case 10: k_nh_block_jacobi<10><<<nblk(N), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, ctx->conn, (int)ctx->n_el, ctx->ngf, ctx->gf64, u, ctx->fixed, M64, M32, D); break;
-    case 4: k_nh_block_jacobi<4><<<nblk(N), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, ctx->conn, (int)ctx->n_el, ctx->ngf, ctx->gf64, u, ctx->fixed, M64, M32, D); break;
-    case 8: k_nh_block_jacobi<8><<<nblk(N), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, ctx->conn, (int)ctx->n_el, ctx->ngf, ctx->gf64, u, ctx->fixed, M64, M32, D); break;
+    case 10: k_nh_block_jacobi<10><<<nblk(N, kBlock / kNodeLanes), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, ctx->conn, (int)ctx->n_el, ctx->ngf, ctx->gf64, u, ctx->fixed, M64, M32, D); break;
+    case 4: k_nh_block_jacobi<4><<<nblk(N, kBlock / kNodeLanes), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, ctx->conn, (int)ctx->n_el, ctx->ngf, ctx->gf64, u, ctx->fixed, M64, M32, D); break;
+    case 8: k_nh_block_jacobi<8><<<nblk(N, kBlock / kNodeLanes), kBlock, 0, ctx->stream>>>(N, ctx->inc_ptr, ctx->inc, ctx->conn, (int)ctx->n_el, ctx->ngf, ctx->gf64, u, ctx->fixed, M64, M32, D); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
