@@ -4,9 +4,11 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <thread>
 
 #include "jfem_device.h"
@@ -99,6 +101,7 @@ extern "C" int jfm_create(int device, jfm_ctx **out) {
     if (hipSetDevice(device) != hipSuccess) return JFM_EHIP;
     jfm_ctx *ctx = new jfm_ctx();
     ctx->device = device;
+    if (hipDeviceGetAttribute(&ctx->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) ctx->cus = 0;
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
         delete ctx;
         return JFM_EHIP;
@@ -914,6 +917,42 @@ static int finalize_misc(jfm_ctx *ctx, int npart, int nv, int fin) {
     return JFM_OK;
 }
 
+// The workgroups of resident kernels that run at once on a device, over all
+// contexts and threads of the process, never exceed its CUs, each of which
+// holds at least one of them: so every such kernel is resident as a whole once
+// the finite kernels beside it have ended.  A hold lasts until the kernel has
+// been waited for.
+namespace {
+struct ResidentHold {
+    static constexpr int kDevices = 64;
+    struct Device {
+        std::mutex m;
+        std::condition_variable cv;
+        int used = 0;
+    };
+    static Device &of(int device) {
+        static Device d[kDevices];
+        return d[device % kDevices];
+    }
+    Device &dev;
+    int n;
+    ResidentHold(const jfm_ctx *ctx, int workgroups) : dev(of(ctx->device)), n(std::min(workgroups, ctx->cus)) {
+        std::unique_lock<std::mutex> lock(dev.m);
+        dev.cv.wait(lock, [&] { return dev.used + n <= ctx->cus; });
+        dev.used += n;
+    }
+    ~ResidentHold() {
+        {
+            std::lock_guard<std::mutex> lock(dev.m);
+            dev.used -= n;
+        }
+        dev.cv.notify_all();
+    }
+    ResidentHold(const ResidentHold &) = delete;
+    ResidentHold &operator=(const ResidentHold &) = delete;
+};
+}  // namespace
+
 // PCG on the workspace of precision T: solves K x = b (free DOFs) from x = 0,
 // or from the current x with its true residual (warm, FP64 only).  The host
 // reads the scalars once per batch of `check_every` iterations.
@@ -925,24 +964,25 @@ static int pcg_run(jfm_ctx *ctx, int op, const T *Minv, double rtol, int maxit, 
     const int64_t n = ctx->ndof;
     hipStream_t s = ctx->stream;
     int np = 0;
-    int resident = coarse ? 0 : 1;
-    if (resident)
-        if (int rc = jfem_persist_ready<T>(ctx, op, &resident)) return rc;
+    int resident = 1;
+    if (int rc = jfem_persist_ready<T>(ctx, op, &resident, coarse)) return rc;
     if (resident) {
         const bool from_x = warm && sizeof(T) == 8;
         if (from_x) {
             CHECK_LAUNCH(ctx, op_apply<T>(ctx, op, x, q, nullptr, nullptr, nullptr, nullptr));
             CHECK_LAUNCH(ctx, launch_residual(ctx, (const double *)b, (const double *)q, ctx->fixed, (double *)r, n, &np));
         }
-        CHECK_LAUNCH(ctx, launch_pcg_persist<T>(ctx, op, Minv, b, from_x ? r : nullptr, x, rtol, maxit));
+        const ResidentHold hold(ctx, ctx->cells.npatch);  // until the kernel has ended
+        CHECK_LAUNCH(ctx, launch_pcg_persist<T>(ctx, op, Minv, b, from_x ? r : nullptr, x, rtol, maxit, coarse));
         if (int rc = read_scalars(ctx)) return rc;
         if (!ctx->S_host->fail) {
             *iters = ctx->S_host->iter;
             *status = ctx->S_host->done[0];
             return JFM_OK;
         }
-        ctx->persist_off = true;  // launched below, and from now on
+        ctx->persist_off = true;  // a wait gave up: launched below, and from now on
     }
+    if (int rc = prepare_op(ctx, op)) return rc;
     std::memset(ctx->S_host, 0, sizeof(PcgScalars));
     ctx->S_host->rtol2 = rtol * rtol;
     ctx->S_host->maxit = maxit;
@@ -1053,8 +1093,16 @@ extern "C" int jfm_solve(jfm_ctx *ctx, const jfm_solve_opts *opts, const double 
     JFM_HIP(ctx, hipSetDevice(ctx->device));
     const int op = opts->op;
     const int op_outer = opts->method == JFM_SOLVE_MIXED_IR ? opts->op_outer : op;
-    if (int rc = prepare_op(ctx, op)) return rc;
-    if (int rc = prepare_op(ctx, op_outer)) return rc;
+    // A solve whose iterations run resident applies the operator itself only
+    // for its few FP64 residuals: these take the two-phase form then, and the
+    // 480-element patches (7 ms of host work at 12,810 Tet10 elements) are
+    // built by pcg_run if it has to launch after all.
+    const bool inner32 = opts->method == JFM_SOLVE_MIXED_IR;
+    const bool resident = inner32 ? op == op_outer && jfem_persist_maybe<float>(ctx, op) : jfem_persist_maybe<double>(ctx, op);
+    if (!(resident && op == JFM_OP_MATFREE)) {
+        if (int rc = prepare_op(ctx, op)) return rc;
+        if (int rc = prepare_op(ctx, op_outer)) return rc;
+    }
     if (int rc = ensure_workspaces(ctx)) return rc;
     const int64_t n = ctx->ndof;
     hipStream_t s = ctx->stream;
@@ -1520,9 +1568,10 @@ static int mass_solves(jfm_ctx *ctx, const double *Mm, int nsys, const double *b
     int beside = nsys;
     if (int rc = jfem_persist_ready<double>(ctx, kOpMass, &beside)) return rc;
     if (beside > 1) {
-        std::vector<PcgScalars> S(beside);
+        std::vector<PcgScalars> S(beside);  // (outlives the copy into it)
         for (int k = 0; k < nsys && beside > 1; k += beside) {
-            CHECK_LAUNCH(ctx, launch_pcg_persist<double>(ctx, kOpMass, Mm, b + k * n, nullptr, x + k * n, rtol, maxit, beside, n));
+            const ResidentHold hold(ctx, beside * ctx->cells.npatch);
+            CHECK_LAUNCH(ctx, launch_pcg_persist<double>(ctx, kOpMass, Mm, b + k * n, nullptr, x + k * n, rtol, maxit, false, beside, n));
             JFM_HIP(ctx, hipMemcpyAsync(S.data(), ctx->cells.S, sizeof(PcgScalars) * beside, hipMemcpyDeviceToHost, s));
             if (int rc = sync(ctx)) return rc;
             for (const PcgScalars &v : S)

@@ -149,6 +149,7 @@ struct Workspace {        // PCG vectors of one precision
 
 struct jfm_ctx {
     int device = 0;
+    int cus = 0;                  // compute units
     hipStream_t stream = nullptr;
     std::string err;
     int64_t bytes = 0;
@@ -254,6 +255,7 @@ struct jfm_ctx {
     std::vector<double> h_X;       // host copy of the coordinates (aggregation)
     int coarse_built_nodes = 0;    // coarse_nodes the aggregation was built for
     int coarse_gen = 0;            // bumped per aggregation (keys captured graphs)
+    std::vector<int32_t> h_node_agg;
     bool coarse_ready = false;     // Ahat holds a coarse level
     int coarse_tag = -1;           // operator it was built from: 0 K, 1 the tangent
     int64_t n_agg = 0, nc = 0;
@@ -342,6 +344,15 @@ struct jfm_ctx {
         jfem::PcgScalars *S = nullptr;       // scalars of the systems solved side by side
         int nslot = 0, systems = 0;          // systems that words, part and S hold
         std::vector<int32_t> epos;           // element -> position in the patch order
+        std::vector<int32_t> h_ptr, h_node;  // patch nodes, and whether the patch owns each
+        std::vector<uint8_t> h_own;
+        // two-level form for the aggregation coarse_gen
+        int coarse_gen = -1;
+        bool coarse_usable = false;
+        int32_t *pn_agg = nullptr, *ce_ptr = nullptr, *ce_slot = nullptr, *cn_ptr = nullptr, *as_ptr = nullptr;
+        uint16_t *cn_list = nullptr;
+        double *wpart = nullptr;
+        uint64_t *zw = nullptr;
     } cells;
     bool persist_off = false;      // a resident solve gave up waiting: this context launches its iterations
     double *Muser64 = nullptr;     // N x 9 user blocks (JFM_PREC_USER)
@@ -440,11 +451,15 @@ constexpr int kPersistWords = 6;  // exchange words per workgroup (and 256 more)
 struct PersistGeometry { int elems = 0, threads = 0, stride = 0; };
 int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g);
 void jfem_cells_release(jfm_ctx *ctx);
+// Whether the PCG on `op` may run resident on this mesh (builds nothing).
+template <typename T> bool jfem_persist_maybe(const jfm_ctx *ctx, int op);
 // Whether the PCG on `op` runs resident on this context (builds its patches
 // on first use); JFEM_PERSIST=0 turns it off.
 // *nsys: the systems (right-hand sides of one operator) asked for; returns how
 // many of them can be solved side by side, 0: none, use the launched form.
-template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys);
+// With coarse, of the two-level form on the current aggregation.
+template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys, bool coarse = false);
+int jfem_cells_coarse(jfm_ctx *ctx, int max_entries);
 // makes room for m systems
 int jfem_cells_systems(jfm_ctx *ctx, int m);
 // heat: maps the convection faces to elements (ctx->heat_resident)
@@ -454,7 +469,7 @@ int jfem_heat_faces(jfm_ctx *ctx);
 // ss) in ctx->cells.S (fail set when a wait gave up, x then untouched).
 template <typename T>
 hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit,
-                              int nsys = 1, int64_t ss = 0);
+                              bool coarse = false, int nsys = 1, int64_t ss = 0);
 // coarse.hip
 // With learned_beside, the learned blocks start on the second stream
 // (jfem_learned_launch) once A_c is formed, beside its inversion.

@@ -38,23 +38,28 @@
 // the next iteration, whose exchange C a workgroup passes only after every
 // other one has read this iteration's.
 //
-// Progress.  The kernel is launched cooperatively, so all its workgroups are
-// resident, and every wait is bounded: past the bound a workgroup raises the
-// failure flag and returns, the others run into their own bounds, and the
-// host repeats the solve with the launched form.
+// Progress.  A grid is never larger than the device holds at once, and the
+// resident kernels of a process that run together are not either (ResidentHold
+// in api.hip), so all workgroups come to run.  Every wait is bounded all the
+// same (another process may hold compute units): past the bound a workgroup
+// raises the failure flag and returns, the others run into their own bounds,
+// and the host repeats the solve with the launched form.  (A cooperative launch
+// would be refused while another process has one, and the launched form in its
+// place would give other bits.)
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
 #include "jfem_device.h"
 #include "mf_element.h"
+#include "nh_element.h"
 
 namespace jfem {
 
 // ---------------------------------------------------------------- exchange --
 // Polls of one word before a workgroup gives up (each takes at least the
-// latency of a load past the L2, about 0.7 us: some seconds in all).
-constexpr int kMaxPolls = 1 << 22;
+// latency of a load past the L2, about 0.7 us: a second or so in all).
+constexpr int kMaxPolls = 1 << 20;
 
 __device__ __forceinline__ void put_word(uint64_t *w, uint32_t epoch, uint32_t bits) {
     __hip_atomic_store(w, (uint64_t)epoch << 32 | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -125,6 +130,12 @@ template <typename T> struct Partials {
         }
     }
 };
+__device__ __forceinline__ void put_shared(double *p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double get_shared(const double *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 // this wave's stores have reached the point where all XCDs see them
 __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
@@ -249,6 +260,7 @@ template <typename T> struct PersistArgs {
     int n_el, npatch;
     const uint16_t *connL;    // npe x n_el (patch order): the node's position in its patch
     const T *el;              // geometric factors, patch order
+    const double *el64;       // the same in FP64
     T rho;                    // lambda / mu of the folded factors
     int ngf;
     const double *kc;         // heat: conductivities (element order) and the elements' order
@@ -272,6 +284,19 @@ template <typename T> struct PersistArgs {
     double rtol2;
     int maxit;
     PcgScalars *S;
+    const double *ustate;     // tangent: the displacement it is taken at
+    // two-level: per patch node its aggregate; offsets from the aggregates'
+    // centroids (per node); the patch's entries, one per aggregate that its
+    // owned nodes are in (slot in wpart, nodes cn_list[cn_ptr[e]..]); the
+    // aggregates' slots; the coarse operator; exchange words
+    const int32_t *pn_agg;
+    const T *cd;
+    const int32_t *ce_ptr, *ce_slot, *cn_ptr, *as_ptr;
+    const uint16_t *cn_list;
+    const float *Ahat;
+    int nc, ldc;
+    double *wpart;
+    uint64_t *zw;
     // nsys systems of one operator side by side: workgroups npatch s .. of the
     // grid solve system s, its b and x ss values further, scalars at S + s
     int nsys;
@@ -393,6 +418,156 @@ template <typename T_, bool FOLD> struct ElasticTet10 : OpShape<10, 3, 4, 7, 4, 
 #pragma unroll
             for (int c = 0; c < 3; ++c) f[c] = T(4) * ((r[c] + quad_xor<d>(r[c])) + (s0[c] + sd[c]));
             if (k < (k ^ d))  // one of the edge's two lanes
+#pragma unroll
+                for (int c = 0; c < 3; ++c) oc(d, c, f[c]);
+        };
+        edge(std::integral_constant<int, 1>{});
+        edge(std::integral_constant<int, 2>{});
+        edge(std::integral_constant<int, 3>{});
+        return has ? (double)en : 0.0;
+    }
+};
+
+// Neo-Hookean tangent K_T(u) v of an affine Tet10 (nh_element.h), lane k at the
+// Gauss point near vertex k (barycentric a there, b elsewhere).  The state (F,
+// A = C^-1, S, ln J) is formed once per solve, in FP64, and held in registers.
+// With v relative to vertex k, index 0 vertex k and d = 1..3 the vertices k ^ d:
+//     grad v = sum_d (c_d - c_0) (x) g_d,  c_0 = 4 b (e_1 + e_2 + e_3),
+//     c_d = (4 b - 1) v_d + 4 a e_d + 4 b (the two mid nodes at k ^ d away from k),
+// and with P the weighted directional derivative of the first Piola-Kirchhoff
+// stress, r_d = P g_d, s_d = (sum of the lanes' P) g_d:
+//     y_corner k = (4 b - 1) s_0 + 4 (a - b) r_0,
+//     y_edge kj  = 4 (b (s_0 + s_d) + (a - b) (r_d + r_d of lane j)).
+template <typename T_> struct TangentTet10 : OpShape<10, 3, 4, 10, 4, false, 2> {
+    using T = T_;
+    static constexpr double qa = 0.585410196624968, qb = 0.138196601125011;
+    // slots 7..9: the mid node of the edge opposite to (k, k ^ d)
+    __device__ static int in_node(int kv, int m) {
+        constexpr int OPP[10] = {0, 0, 0, 0, 9, 7, 8, 5, 6, 4};  // mid node of the opposite edge
+        return m < 7 ? tet10_lane_node(kv, m) : OPP[tet10_lane_node(kv, m - 6)];
+    }
+    struct Data { T g[9], F[9], A[6], S[6], c1, cl; };  // symmetric ones: 11, 22, 33, 12, 23, 13
+    // grad of a nodal field, relative to vertex k
+    template <typename U, typename X> __device__ static void gradient(const U (&g)[9], X &&xc, U (&G)[9]) {
+        U c[3][3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const U v0 = xc(0, i);
+            const U e1 = xc(1, i) - v0, e2 = xc(2, i) - v0, e3 = xc(3, i) - v0;
+            const U f1 = xc(7, i) - v0, f2 = xc(8, i) - v0, f3 = xc(9, i) - v0;
+            const U c0 = U(4 * qb) * (e1 + e2 + e3);
+            c[0][i] = U(4 * qb - 1) * (xc(4, i) - v0) + U(4 * qa) * e1 + U(4 * qb) * (f2 + f3) - c0;
+            c[1][i] = U(4 * qb - 1) * (xc(5, i) - v0) + U(4 * qa) * e2 + U(4 * qb) * (f1 + f3) - c0;
+            c[2][i] = U(4 * qb - 1) * (xc(6, i) - v0) + U(4 * qa) * e3 + U(4 * qb) * (f1 + f2) - c0;
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int b = 0; b < 3; ++b) G[i * 3 + b] = c[0][i] * g[b] + c[1][i] * g[3 + b] + c[2][i] * g[6 + b];
+    }
+    __device__ static void load(const PersistArgs<T> &A, int k, int kv, bool has, Data &d) {
+        double Ji[9], g[9], H[9];
+#pragma unroll
+        for (int m = 0; m < 9; ++m) Ji[m] = has ? A.el64[(size_t)m * A.n_el + k] : (m % 4 == 0 ? 1.0 : 0.0);
+        lane_gradients<double>(Ji, kv, g);
+        const double cl = has ? A.el64[(size_t)9 * A.n_el + k] : 0.0, cm = has ? A.el64[(size_t)10 * A.n_el + k] : 0.0;
+        const int lb = A.pn_ptr[k / kEl];
+        gradient<double>(g, [&](int m, int c) -> double {
+            return has ? A.ustate[3 * (size_t)A.pn_node[lb + A.connL[(size_t)in_node(kv, m) * A.n_el + k]] + c] : 0.0;
+        }, H);
+        const double I[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
+        double F[9], C[9], S[9], lnJ;
+        nh_state<double>(H, I, cl, cm, F, C, S, lnJ);  // H is the physical gradient already
+#pragma unroll
+        for (int m = 0; m < 9; ++m) {
+            d.g[m] = (T)g[m];
+            d.F[m] = (T)F[m];
+        }
+        constexpr int ix[6] = {0, 4, 8, 1, 5, 2};
+#pragma unroll
+        for (int m = 0; m < 6; ++m) {
+            d.A[m] = (T)C[ix[m]];
+            d.S[m] = (T)S[ix[m]];
+        }
+        d.c1 = (T)(2.0 * (cm - cl * lnJ));
+        d.cl = (T)cl;
+    }
+    // o = m v for the symmetric m
+    __device__ static void mul(const T (&m)[6], const T *v, int stride, T (&o)[3]) {
+        const T v0 = v[0], v1 = v[stride], v2 = v[2 * stride];
+        o[0] = m[0] * v0 + m[3] * v1 + m[5] * v2;
+        o[1] = m[3] * v0 + m[1] * v1 + m[4] * v2;
+        o[2] = m[5] * v0 + m[4] * v1 + m[2] * v2;
+    }
+    template <typename XC, typename OC>
+    __device__ static double product(const PersistArgs<T> &, const Data &D, int, int k, bool has, XC &&xc, OC &&oc) {
+        T G[9], P[9];
+        gradient<T>(D.g, xc, G);
+        // dE = sym(F' G), AdE = A dE, dS = c1 AdE A + cl tr(AdE) A, P = G S + F dS
+        T E[6];
+        auto fg = [&](int a, int b) -> T { return D.F[a] * G[b] + D.F[3 + a] * G[3 + b] + D.F[6 + a] * G[6 + b]; };
+        E[0] = fg(0, 0);
+        E[1] = fg(1, 1);
+        E[2] = fg(2, 2);
+        E[3] = T(0.5) * (fg(0, 1) + fg(1, 0));
+        E[4] = T(0.5) * (fg(1, 2) + fg(2, 1));
+        E[5] = T(0.5) * (fg(0, 2) + fg(2, 0));
+        const T Ec[9] = {E[0], E[3], E[5], E[3], E[1], E[4], E[5], E[4], E[2]};
+        T B[9];  // A dE, row-major
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            T o[3];
+            mul(D.A, Ec + b, 3, o);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) B[a * 3 + b] = o[a];
+        }
+        const T tr = D.cl * (B[0] + B[4] + B[8]);
+        T dS[6];
+        auto ba = [&](int a, int b) -> T {  // (A dE A)_ab
+            constexpr int ix[9] = {0, 3, 5, 3, 1, 4, 5, 4, 2};
+            return B[a * 3] * D.A[ix[b]] + B[a * 3 + 1] * D.A[ix[3 + b]] + B[a * 3 + 2] * D.A[ix[6 + b]];
+        };
+        dS[0] = D.c1 * ba(0, 0) + tr * D.A[0];
+        dS[1] = D.c1 * ba(1, 1) + tr * D.A[1];
+        dS[2] = D.c1 * ba(2, 2) + tr * D.A[2];
+        dS[3] = D.c1 * ba(0, 1) + tr * D.A[3];
+        dS[4] = D.c1 * ba(1, 2) + tr * D.A[4];
+        dS[5] = D.c1 * ba(0, 2) + tr * D.A[5];
+        T en = T(0);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            T u[3], w[3];
+            mul(D.S, G + 3 * a, 1, u);     // row a of G S
+            mul(dS, D.F + 3 * a, 1, w);    // row a of F dS
+#pragma unroll
+            for (int b = 0; b < 3; ++b) {
+                P[a * 3 + b] = u[b] + w[b];
+                en += G[a * 3 + b] * P[a * 3 + b];
+            }
+        }
+        T Q[9];
+#pragma unroll
+        for (int m = 0; m < 9; ++m) Q[m] = quad_sum(P[m]);
+        const T *g = D.g;
+        T g0[3], s0[3], r0[3];
+#pragma unroll
+        for (int b = 0; b < 3; ++b) g0[b] = -(g[b] + g[3 + b] + g[6 + b]);
+        auto app = [&](const T (&M)[9], const T *v, T (&o)[3]) {
+#pragma unroll
+            for (int a = 0; a < 3; ++a) o[a] = M[a * 3] * v[0] + M[a * 3 + 1] * v[1] + M[a * 3 + 2] * v[2];
+        };
+        app(Q, g0, s0);
+        app(P, g0, r0);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) oc(0, c, T(4 * qb - 1) * s0[c] + T(4 * (qa - qb)) * r0[c]);
+        auto edge = [&](auto dc) {
+            constexpr int d = decltype(dc)::value;
+            T r[3], sd[3], f[3];
+            app(P, g + 3 * (d - 1), r);
+            app(Q, g + 3 * (d - 1), sd);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) f[c] = T(4 * (qa - qb)) * (r[c] + quad_xor<d>(r[c])) + T(4 * qb) * (s0[c] + sd[c]);
+            if (k < (k ^ d))
 #pragma unroll
                 for (int c = 0; c < 3; ++c) oc(d, c, f[c]);
         };
@@ -629,7 +804,23 @@ template <int NPE_> struct MassElem : OpShape<NPE_, 3, 1, NPE_, NPE_, true, 2> {
     }
 };
 
-template <class Op>
+// Most coarse unknowns (kCoarseRows per thread) and aggregates per patch of the
+// two-level form.
+constexpr int kCoarseRows = 3, kMaxCoarse = kCoarseRows * kNT, kMaxEntries = 64;
+template <typename T, bool COARSE> struct CoarseLds {};
+template <typename T> struct CoarseLds<T, true> {
+    float w[kMaxCoarse], z[kMaxCoarse];  // w = Q' m r (the GEMV's operand, zero padded), zc
+    T d[3 * kNT];                        // the nodes' offsets
+    double wz[kNT / 64];
+    int start[kMaxEntries + 1], slot[kMaxEntries];
+    uint16_t list[kNT];
+};
+
+// COARSE: the two-level preconditioner z = M r + m o Q zc, zc = Ahat Q' m r
+// (coarse.hip).  The patches' sums of Q' m r go out with exchange C; every
+// workgroup then forms w from them, computes its share of the rows of Ahat w,
+// and the rows travel as words (16 copies, one per group of workgroups).
+template <class Op, bool COARSE>
 __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistArgs<typename Op::T> A0) {
     using T = typename Op::T;
     constexpr int NPE = Op::NPE, NC = Op::NC, NL = Op::kLanes, EL = Op::kEl, ST = Op::kStride, NT = kNT, CS = NPE * ST;
@@ -638,6 +829,7 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
     __shared__ GridSumLds<1> shB;
     __shared__ GridSumLds<2> shC;
     __shared__ int bad;
+    __shared__ CoarseLds<T, COARSE> co;
     const PersistArgs<T> &A = A0;
     const int nwg = A.npatch, sys = (int)blockIdx.x / nwg, p = (int)blockIdx.x - sys * nwg;
     const int t = (int)threadIdx.x;
@@ -696,6 +888,29 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
         x[c] = in && A.r0 ? xvec[d] : T(0);
         pv[c] = T(0);
     }
+    T dv[3];               // two-level: the node's offset and aggregate
+    int agg = 0, ca0[kCoarseRows], ca1[kCoarseRows], ne = 0;
+    if constexpr (COARSE) {
+        const int e0 = A.ce_ptr[p];
+        ne = A.ce_ptr[p + 1] - e0;
+        agg = in ? 6 * A.pn_agg[lb + t] : 0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            dv[c] = in ? A.cd[3 * (size_t)node + c] : T(0);
+            co.d[3 * t + c] = dv[c];
+        }
+        const int n0 = A.cn_ptr[e0];
+        if (t <= ne) co.start[t] = A.cn_ptr[e0 + t] - n0;
+        if (t < ne) co.slot[t] = A.ce_slot[e0 + t];
+        if (t < A.cn_ptr[e0 + ne] - n0) co.list[t] = A.cn_list[n0 + t];
+#pragma unroll
+        for (int j = 0; j < kCoarseRows; ++j) {
+            const int i = t + j * NT, g = i / 6;
+            ca0[j] = i < A.nc ? A.as_ptr[g] : 0;
+            ca1[j] = i < A.nc ? A.as_ptr[g + 1] : 0;
+            co.w[i] = 0.0f;
+        }
+    }
     __syncthreads();  // bad
     uint32_t epoch = 1;
     if (!grid_sum<1, NT>(bb, wordsB, p, nwg, epoch, shB, &bad)) {
@@ -721,20 +936,108 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
             }
         }
         ++epoch;
+        if constexpr (COARSE) {
+            // the patch's sums of Q' m r per aggregate: [y; d x y], y = m r
+            const int lane = t & 63, wv = t >> 6;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) ps[3 * t + c] = fx >> c & 1u ? T(0) : r[c];
+            __syncthreads();
+            for (int e = wv; e < ne; e += NT / 64) {
+                double w[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+                for (int i = co.start[e] + lane; i < co.start[e + 1]; i += 64) {
+                    const int l = 3 * (int)co.list[i];
+                    const double y0 = ps[l], y1 = ps[l + 1], y2 = ps[l + 2];
+                    const double d0 = co.d[l], d1 = co.d[l + 1], d2 = co.d[l + 2];
+                    w[0] += y0;
+                    w[1] += y1;
+                    w[2] += y2;
+                    w[3] += d1 * y2 - d2 * y1;
+                    w[4] += d2 * y0 - d0 * y2;
+                    w[5] += d0 * y1 - d1 * y0;
+                }
+                double mine = 0.0;
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    const double v = wave_total(w[c]);
+                    mine = lane == c ? v : mine;
+                }
+                if (lane < 6) put_shared(A.wpart + 6 * (size_t)co.slot[e] + lane, mine);
+            }
+            stores_done();  // before the block barrier in grid_sum, hence before its words
+        }
         if (!grid_sum<2, NT>(s2, wordsC, p, nwg, epoch, shC, &bad)) break;
         rr = s2[1];
-        if (epoch == 2) {  // the start
-            rr0 = rr;
-            if (rr <= tol2) done = DONE_CONVERGED;
-        } else {
-            ++it;
+        if (epoch == 2) rr0 = rr;  // the start
+        else ++it;
+        if (rr <= tol2) {  // the same in every workgroup
+            done = DONE_CONVERGED;
+            break;
+        }
+        if constexpr (COARSE) {
+            const int lane = t & 63, wv = t >> 6, nc = A.nc;
+            double w64[kCoarseRows];
+#pragma unroll
+            for (int j = 0; j < kCoarseRows; ++j) {
+                const int i = t + j * NT, c = i % 6;
+                w64[j] = 0.0;
+                if (i < nc) {
+                    for (int k0 = ca0[j]; k0 < ca1[j]; k0 += 4) {  // four in flight
+                        double v[4];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) v[u] = k0 + u < ca1[j] ? get_shared(A.wpart + 6 * (size_t)(k0 + u) + c) : 0.0;
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) w64[j] += v[u];
+                    }
+                    co.w[i] = (float)w64[j];
+                }
+            }
+            __syncthreads();
+            uint64_t *zw = A.zw + (size_t)(p / kGroup) * nc;
+            const int copies = (nwg + kGroup - 1) / kGroup, ld4 = A.ldc / 4;
+            const float4 *w4 = reinterpret_cast<const float4 *>(co.w);
+            for (int row = p + nwg * wv; row < nc; row += nwg * (NT / 64)) {
+                const float4 *Ar = reinterpret_cast<const float4 *>(A.Ahat) + (size_t)row * ld4;
+                double s = 0.0;
+#pragma unroll 4
+                for (int q = lane; q < ld4; q += 64) {
+                    const float4 a = Ar[q], b = w4[q];
+                    s += (double)a.x * b.x + (double)a.y * b.y + (double)a.z * b.z + (double)a.w * b.w;
+                }
+                const float zr = (float)wave_total(s);
+                if (lane < copies) put_word(A.zw + (size_t)lane * nc + row, epoch, __float_as_uint(zr));
+            }
+            double wz = 0.0;
+#pragma unroll
+            for (int j = 0; j < kCoarseRows; ++j) {
+                const int i = t + j * NT;
+                if (i < nc) {
+                    uint32_t bits[1];
+                    if (!poll_words<1>(zw + i, 1, epoch, bits)) bad = 1;
+                    const float zf = __uint_as_float(bits[0]);
+                    co.z[i] = zf;
+                    wz += w64[j] * (double)zf;
+                }
+            }
+            wz = wave_total(wz);
+            if (lane == 0) co.wz[wv] = wz;
+            __syncthreads();
+            if (bad) break;
+#pragma unroll
+            for (int q = 0; q < NT / 64; ++q) s2[0] += co.wz[q];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const int c1 = (c + 1) % 3, c2 = (c + 2) % 3;
+                const T corr = (T)co.z[agg + c] + (T)co.z[agg + 3 + c1] * dv[c2] - (T)co.z[agg + 3 + c2] * dv[c1];
+                z[c] += fx >> c & 1u ? T(0) : corr;
+            }
+        }
+        if (epoch > 2) {
             beta_d = s2[0] / rz;
-            if (rr <= tol2) done = DONE_CONVERGED;
-            else if (!(pq > 0.0) || !(s2[0] > 0.0) || !finite(s2[0])) done = DONE_BREAKDOWN;
+            if (!(pq > 0.0) || !(s2[0] > 0.0) || !finite(s2[0])) done = DONE_BREAKDOWN;
             else if (it >= A.maxit) done = DONE_MAXIT;
         }
         rz = s2[0];
-        if (done) break;  // the same in every workgroup
+        if (done) break;
         // p = z + beta p
         const T beta = (T)beta_d;
 #pragma unroll
@@ -847,67 +1150,86 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
 }
 
 // no word of an earlier solve is taken for one of this
-__global__ __launch_bounds__(256) void k_persist_clear(int n, uint64_t *__restrict__ words, int nsys, PcgScalars *S) {
+__global__ __launch_bounds__(256) void k_persist_clear(int n, uint64_t *__restrict__ words, int nz, uint64_t *__restrict__ zw,
+                                                      int nsys, PcgScalars *S) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) words[i] = 0;
+    if (i < nz) zw[i] = 0;
     if (i < nsys) S[i].fail = 0;
 }
 
 // --------------------------------------------------------------- launchers ---
 struct PersistLaunch { const void *f = nullptr; PersistGeometry g; };
-template <class Op> static PersistLaunch persist_of() {
-    return {(const void *)k_pcg_persist<Op>, {Op::kEl, kNT, Op::kStride}};
+template <class Op> static PersistLaunch persist_of(bool coarse) {
+    const void *f = (const void *)k_pcg_persist<Op, false>;
+    if constexpr (!Op::kDiag)
+        if (coarse) f = (const void *)k_pcg_persist<Op, true>;
+    return {f, {Op::kEl, kNT, Op::kStride}};
 }
 // the kernel of an operator on this mesh; none: the launched form
-template <typename T> static PersistLaunch persist_kernel(const jfm_ctx *ctx, int op) {
+template <typename T> static PersistLaunch persist_kernel(const jfm_ctx *ctx, int op, bool coarse) {
+    if (coarse && (ctx->nc > kMaxCoarse || ctx->ldc > kMaxCoarse)) return {};
     const bool tet10 = ctx->npe == 10 && ctx->affine;
     if (op == JFM_OP_MATFREE) {
         if constexpr (sizeof(T) == 4)
-            if (tet10 && ctx->nu_uniform) return persist_of<ElasticTet10<T, true>>();
-        if (tet10) return persist_of<ElasticTet10<T, false>>();
-        if (ctx->npe == 4) return persist_of<ElasticTet4<T>>();
+            if (tet10 && ctx->nu_uniform) return persist_of<ElasticTet10<T, true>>(coarse);
+        if (tet10) return persist_of<ElasticTet10<T, false>>(coarse);
+        if (ctx->npe == 4) return persist_of<ElasticTet4<T>>(coarse);
     }
+    if (op == JFM_OP_TANGENT && tet10) return persist_of<TangentTet10<T>>(coarse);
     if constexpr (sizeof(T) == 8) {
         if (op == kOpHeat) {
-            if (tet10) return persist_of<HeatTet10>();
-            if (ctx->npe == 4) return persist_of<HeatElem<4>>();
-            if (ctx->npe == 8) return persist_of<HeatElem<8>>();
+            if (tet10) return persist_of<HeatTet10>(coarse);
+            if (ctx->npe == 4) return persist_of<HeatElem<4>>(coarse);
+            if (ctx->npe == 8) return persist_of<HeatElem<8>>(coarse);
         }
         if (op == kOpMass) {
-            if (tet10) return persist_of<MassTet10>();
-            if (ctx->npe == 4) return persist_of<MassElem<4>>();
-            if (ctx->npe == 8) return persist_of<MassElem<8>>();
+            if (tet10) return persist_of<MassTet10>(coarse);
+            if (ctx->npe == 4) return persist_of<MassElem<4>>(coarse);
+            if (ctx->npe == 8) return persist_of<MassElem<8>>(coarse);
         }
     }
     return {};
 }
 
-template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys) {
-    const int want = *nsys;
-    *nsys = 0;
+static bool persist_on() {
     static const bool on = [] {
         const char *v = std::getenv("JFEM_PERSIST");
         return !(v && v[0] == '0');
     }();
-    if (!on || ctx->persist_off || !jfem_patch_enabled() || ctx->n_el < 1) return JFM_OK;
-    const PersistLaunch L = persist_kernel<T>(ctx, op);
+    return on;
+}
+
+template <typename T> bool jfem_persist_maybe(const jfm_ctx *ctx, int op) {
+    if (!persist_on() || ctx->persist_off || !jfem_patch_enabled() || ctx->n_el < 1) return false;
+    const PersistLaunch L = persist_kernel<T>(ctx, op, false);
+    if (!L.f) return false;
+    const int64_t np = (ctx->n_el + L.g.elems - 1) / L.g.elems;
+    return np <= kPersistPatches && np <= ctx->cus && (!ctx->cells.ready || ctx->cells.usable);
+}
+
+template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys, bool coarse) {
+    const int want = *nsys;
+    *nsys = 0;
+    if (!jfem_persist_maybe<T>(ctx, op)) return JFM_OK;
+    const PersistLaunch L = persist_kernel<T>(ctx, op, coarse);
     if (!L.f) return JFM_OK;
     const int64_t np = (ctx->n_el + L.g.elems - 1) / L.g.elems;
-    if (np > kPersistPatches) return JFM_OK;
     // every workgroup must be resident at once
-    int per_cu = 0, cus = 0, coop = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, L.f, L.g.threads, 0) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess ||
-        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device) != hipSuccess || !coop ||
-        np > (int64_t)per_cu * cus) {
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, L.f, L.g.threads, 0) != hipSuccess || per_cu < 1) {
         (void)hipGetLastError();
         return JFM_OK;
     }
     if (op == kOpHeat && !ctx->heat_resident) return JFM_OK;
     if (int rc = jfem_cells_setup(ctx, L.g)) return rc;
     if (!ctx->cells.usable) return JFM_OK;
+    if (coarse) {
+        if (int rc = jfem_cells_coarse(ctx, kMaxEntries)) return rc;
+        if (!ctx->cells.coarse_usable) return JFM_OK;
+    }
     int m = want;  // as many systems side by side as fit, a divisor of those asked for
-    while (m > 1 && (want % m || m * np > (int64_t)per_cu * cus)) --m;
+    while (m > 1 && (want % m || m * np > (int64_t)per_cu * ctx->cus)) --m;
     if (int rc = jfem_cells_systems(ctx, m)) return rc;
     *nsys = m;
     return JFM_OK;
@@ -915,16 +1237,34 @@ template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys) {
 
 template <typename T>
 hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit,
-                              int nsys, int64_t ss) {
+                              bool coarse, int nsys, int64_t ss) {
     const auto &C = ctx->cells;
-    const PersistLaunch L = persist_kernel<T>(ctx, op);
+    const PersistLaunch L = persist_kernel<T>(ctx, op, coarse);
     const bool fold = sizeof(T) == 4 && C.gfQ32;
     PersistArgs<T> A{};
     A.n_el = (int)ctx->n_el;
     A.npatch = C.npatch;
     A.connL = C.connL;
     A.el = sizeof(T) == 8 ? (const T *)C.gf64 : (fold ? (const T *)C.gfQ32 : (const T *)C.gf32);
+    A.el64 = C.gf64;
     A.rho = fold ? (T)C.rho32 : T(0);
+    A.ustate = ctx->ustate64;
+    int nz = 0;
+    if (coarse) {
+        A.pn_agg = C.pn_agg;
+        A.cd = sizeof(T) == 8 ? (const T *)ctx->cd64 : (const T *)ctx->cd32;
+        A.ce_ptr = C.ce_ptr;
+        A.ce_slot = C.ce_slot;
+        A.cn_ptr = C.cn_ptr;
+        A.as_ptr = C.as_ptr;
+        A.cn_list = C.cn_list;
+        A.Ahat = ctx->Ahat32;
+        A.nc = (int)ctx->nc;
+        A.ldc = (int)ctx->ldc;
+        A.wpart = C.wpart;
+        A.zw = C.zw;
+        nz = (C.npatch + kGroup - 1) / kGroup * A.nc;
+    }
     A.ngf = ctx->ngf;
     A.kc = ctx->heat_k;
     A.eperm = C.eperm;
@@ -956,14 +1296,16 @@ hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, c
     A.nsys = nsys;
     A.ss = ss;
     const int nw = nsys * kPersistWords * (C.npatch + kGroup * kGroup);
-    k_persist_clear<<<(nw + 255) / 256, 256, 0, ctx->stream>>>(nw, C.words, nsys, A.S);
+    k_persist_clear<<<(std::max(nw, nz) + 255) / 256, 256, 0, ctx->stream>>>(nw, C.words, nz, C.zw, nsys, A.S);
     void *args[] = {&A};
-    return hipLaunchCooperativeKernel(L.f, dim3(nsys * C.npatch), dim3(kNT), args, 0, ctx->stream);
+    return hipLaunchKernel(L.f, dim3(nsys * C.npatch), dim3(kNT), args, 0, ctx->stream);
 }
 
-template int jfem_persist_ready<double>(jfm_ctx *, int, int *);
-template int jfem_persist_ready<float>(jfm_ctx *, int, int *);
-template hipError_t launch_pcg_persist<double>(jfm_ctx *, int, const double *, const double *, const double *, double *, double, int, int, int64_t);
-template hipError_t launch_pcg_persist<float>(jfm_ctx *, int, const float *, const float *, const float *, float *, double, int, int, int64_t);
+template bool jfem_persist_maybe<double>(const jfm_ctx *, int);
+template bool jfem_persist_maybe<float>(const jfm_ctx *, int);
+template int jfem_persist_ready<double>(jfm_ctx *, int, int *, bool);
+template int jfem_persist_ready<float>(jfm_ctx *, int, int *, bool);
+template hipError_t launch_pcg_persist<double>(jfm_ctx *, int, const double *, const double *, const double *, double *, double, int, bool, int, int64_t);
+template hipError_t launch_pcg_persist<float>(jfm_ctx *, int, const float *, const float *, const float *, float *, double, int, bool, int, int64_t);
 
 }  // namespace jfem

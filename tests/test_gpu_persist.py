@@ -165,3 +165,46 @@ def test_resident_fit(oracle, gen, g):
         assert np.abs(out[field + "_nodal"] - ref).max() <= 1e-9 * np.abs(ref).max()
         assert np.array_equal(out[field + "_nodal"], one[field + "_nodal"])
     ctx.close()
+
+
+@pytest.mark.parametrize("name,coarse_nodes", [("tet10_6", 64), ("tet10_132", 1000000), ("tet10_2016", 40),
+                                               ("tet10_2052", 300), ("tet4_10368", 200)])
+def test_resident_two_level(oracle, name, coarse_nodes):
+    """The coarse correction in the resident PCG: one aggregate for the whole
+    mesh, many in one patch and aggregates over several patches, to the bars of
+    test_resident_pcg."""
+    import jfem
+    gen, g = CASES[name]
+    m = getattr(M, gen)(*g, seed=5, jitter=0.1, E_sigma=0.4)
+    csr = oracle.assemble_csr(m)
+    ud, _, _ = oracle.solve_direct_lapack(csr, m.fixed_mask(), np.zeros(m.n_dofs), oracle.load_vector(m))
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    for meth in (0, 1):
+        say(f"resident two-level {name} method={meth} coarse_nodes={coarse_nodes}")
+        kw = dict(method=meth, rtol=1e-10, inner_rtol=1e-2, coarse_nodes=coarse_nodes)
+        u, _, _ = ctx.solve(**kw)
+        assert np.linalg.norm(u - ud) <= 1e-8 * np.linalg.norm(ud)
+        assert np.array_equal(u, ctx.solve(**kw)[0])
+    ctx.close()
+
+
+@pytest.mark.parametrize("name", ["tet10_6", "tet10_132", "tet10_2052"])
+@pytest.mark.parametrize("coarse_nodes", [0, 100])
+def test_resident_tangent(oracle, name, coarse_nodes):
+    """The neo-Hookean tangent in the resident PCG against the oracle's Newton
+    with direct tangent solves: 1e-7, as the nonlinear tests ask."""
+    import jfem
+    gen, g = CASES[name]
+    m = getattr(M, gen)(*g, seed=5, jitter=0.1, E_sigma=0.4, traction=(0.0, 0.0, -2.0))
+    uo, _ = oracle.nh_newton(m, load_steps=1, rtol=1e-10)
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    for meth in (0, 1):
+        say(f"resident tangent {name} method={meth} coarse_nodes={coarse_nodes}")
+        kw = dict(load_steps=1, rtol=1e-10, method=meth, coarse_nodes=coarse_nodes)
+        u, st = ctx.solve_nonlinear(**kw)
+        assert st["converged"] == 1
+        assert np.linalg.norm(u - uo) <= 1e-7 * np.linalg.norm(uo)
+        assert np.array_equal(u, ctx.solve_nonlinear(**kw)[0])
+    ctx.close()
