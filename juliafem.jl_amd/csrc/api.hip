@@ -68,9 +68,12 @@ template <typename T> static void free_ptr(jfm_ctx *ctx, T *&p) {
         if (e_ != hipSuccess) return jfm_hip_fail(ctx, e_, #call); \
     } while (0)
 
-template <typename F> static void parallel_for(int64_t n, F f) {
+// On up to 16 threads with at least `grain` items each: a thread costs some 20 us
+// to start.
+template <typename F> static void parallel_for(int64_t n, int64_t grain, F f) {
     int nt = (int)std::min<unsigned>(16u, std::max(1u, std::thread::hardware_concurrency()));
-    if (n < 4096 || nt == 1) {
+    nt = (int)std::min<int64_t>(nt, n / grain);
+    if (nt <= 1) {
         f(0, n);
         return;
     }
@@ -213,38 +216,6 @@ static void release_mesh(jfm_ctx *ctx) {
     ctx->h_conn.clear(); ctx->h_brow.clear(); ctx->h_bcol.clear();
 }
 
-// Tet10 edge mid nodes at their edge midpoints (and Hex8 parallelepipeds) make
-// J constant over the element; one factor set per element then suffices.
-static bool detect_affine(const std::vector<int32_t> &conn, const double *X, int64_t n_el, int npe) {
-    if (npe == 4) return true;
-    std::atomic<bool> ok{true};
-    parallel_for(n_el, [&](int64_t a, int64_t b) {
-        for (int64_t e = a; e < b && ok.load(std::memory_order_relaxed); ++e) {
-            const int32_t *c = conn.data() + e * npe;
-            auto P = [&](int i, int k) { return X[3 * (int64_t)c[i] + k]; };
-            double h = 0;
-            for (int k = 0; k < 3; ++k) h = std::max(h, std::fabs(P(1, k) - P(0, k)));
-            const double tol = 1e-12 * std::max(h, 1e-300);
-            if (npe == 10) {
-                static const int ed[6][2] = {{0, 1}, {1, 2}, {2, 0}, {0, 3}, {1, 3}, {2, 3}};
-                for (int m = 0; m < 6; ++m)
-                    for (int k = 0; k < 3; ++k)
-                        if (std::fabs(P(4 + m, k) - 0.5 * (P(ed[m][0], k) + P(ed[m][1], k))) > tol) ok = false;
-            } else {  // Hex8: x_i = x0 + sum of the three edge vectors it spans
-                static const int s[8][3] = {{0, 0, 0}, {1, 0, 0}, {1, 1, 0}, {0, 1, 0},
-                                            {0, 0, 1}, {1, 0, 1}, {1, 1, 1}, {0, 1, 1}};
-                for (int i = 0; i < 8; ++i)
-                    for (int k = 0; k < 3; ++k) {
-                        const double v = P(0, k) + s[i][0] * (P(1, k) - P(0, k)) + s[i][1] * (P(3, k) - P(0, k)) +
-                                         s[i][2] * (P(4, k) - P(0, k));
-                        if (std::fabs(P(i, k) - v) > tol * 8) ok = false;
-                    }
-            }
-        }
-    });
-    return ok.load();
-}
-
 extern "C" int jfm_upload_mesh(jfm_ctx *ctx, int64_t n_nodes, const double *X, int64_t n_el, int32_t npe,
                                const int64_t *conn, const double *E, const double *nu, int32_t index_base) {
     if (!ctx) return JFM_EINVAL;
@@ -268,7 +239,7 @@ extern "C" int jfm_upload_mesh(jfm_ctx *ctx, int64_t n_nodes, const double *X, i
     // connectivity -> 0-based int32, range checked
     ctx->h_conn.resize((size_t)n_el * npe);
     std::atomic<bool> bad{false};
-    parallel_for(n_el * npe, [&](int64_t a, int64_t b) {
+    parallel_for(n_el * npe, 65536, [&](int64_t a, int64_t b) {
         for (int64_t k = a; k < b; ++k) {
             const int64_t v = conn[k] - index_base;
             if (v < 0 || v >= n_nodes) bad = true;
@@ -283,114 +254,47 @@ extern "C" int jfm_upload_mesh(jfm_ctx *ctx, int64_t n_nodes, const double *X, i
     for (int64_t e = 1; e < n_el && ctx->nu_uniform; ++e) ctx->nu_uniform = nu[e] == nu[0];
     ctx->nu0 = n_el > 0 ? nu[0] : 0.0;
 
-    const std::vector<int32_t> &hc = ctx->h_conn;
-    // node -> incidences (e*npe + i), ascending e  (ext/JuliaFEMCUDAExt.jl:179-193)
-    std::vector<int32_t> inc_ptr(n_nodes + 1, 0), inc((size_t)n_el * npe);
-    for (int64_t k = 0; k < n_el * npe; ++k) inc_ptr[hc[k] + 1]++;
-    for (int64_t a = 0; a < n_nodes; ++a) inc_ptr[a + 1] += inc_ptr[a];
-    {
-        std::vector<int32_t> pos(inc_ptr.begin(), inc_ptr.end() - 1);
-        for (int64_t e = 0; e < n_el; ++e)
-            for (int i = 0; i < npe; ++i) inc[pos[hc[e * npe + i]]++] = (int32_t)(e * npe + i);
-    }
-
-    // 3x3-block pattern = node adjacency, columns sorted (parallel over rows)
-    const int nt = (int)std::min<unsigned>(16u, std::max(1u, std::thread::hardware_concurrency()));
-    std::vector<int32_t> rowlen(n_nodes);
-    std::vector<std::vector<int32_t>> parts(nt);
-    {
-        const int64_t chunk = (n_nodes + nt - 1) / nt;
-        std::vector<std::thread> th;
-        for (int t = 0; t < nt; ++t) {
-            th.emplace_back([&, t] {
-                const int64_t a0 = t * chunk, a1 = std::min<int64_t>(n_nodes, a0 + chunk);
-                std::vector<int32_t> tmp;
-                auto &out = parts[t];
-                for (int64_t a = a0; a < a1; ++a) {
-                    tmp.clear();
-                    for (int k = inc_ptr[a]; k < inc_ptr[a + 1]; ++k) {
-                        const int e = inc[k] / npe;
-                        for (int j = 0; j < npe; ++j) tmp.push_back(hc[(int64_t)e * npe + j]);
-                    }
-                    std::sort(tmp.begin(), tmp.end());
-                    tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
-                    rowlen[a] = (int32_t)tmp.size();
-                    out.insert(out.end(), tmp.begin(), tmp.end());
-                }
-            });
-        }
-        for (auto &x : th) x.join();
-    }
-    ctx->h_brow.assign(n_nodes + 1, 0);
-    for (int64_t a = 0; a < n_nodes; ++a) {
-        if ((int64_t)ctx->h_brow[a] + rowlen[a] > INT32_MAX)
-            return jfm_fail(ctx, JFM_EINVAL, "too many nonzero blocks for 32-bit offsets");
-        ctx->h_brow[a + 1] = ctx->h_brow[a] + rowlen[a];
-    }
-    ctx->nnzb = ctx->h_brow[n_nodes];
-    ctx->h_bcol.resize(ctx->nnzb);
-    {
-        size_t off = 0;
-        for (int t = 0; t < nt; ++t) {
-            std::copy(parts[t].begin(), parts[t].end(), ctx->h_bcol.begin() + off);
-            off += parts[t].size();
-            std::vector<int32_t>().swap(parts[t]);
-        }
-    }
-    const std::vector<int32_t> &brow = ctx->h_brow, &bcol = ctx->h_bcol;
-    const int64_t nnzb = ctx->nnzb;
-
-    // per-block contribution lists (e, i, j), ascending e
-    std::vector<int32_t> cptr(nnzb + 1, 0);
-    auto block_of = [&](int64_t a, int32_t b) -> int64_t {
-        const int32_t *lo = bcol.data() + brow[a], *hi = bcol.data() + brow[a + 1];
-        return (std::lower_bound(lo, hi, b) - bcol.data());
-    };
-    parallel_for(n_nodes, [&](int64_t a0, int64_t a1) {
-        for (int64_t a = a0; a < a1; ++a)
-            for (int k = inc_ptr[a]; k < inc_ptr[a + 1]; ++k) {
-                const int e = inc[k] / npe;
-                for (int j = 0; j < npe; ++j) cptr[block_of(a, hc[(int64_t)e * npe + j]) + 1]++;
-            }
-    });
-    for (int64_t s = 0; s < nnzb; ++s) cptr[s + 1] += cptr[s];
-    std::vector<int32_t> contrib(cptr[nnzb]), blk_row(nnzb), bdiag(n_nodes);
-    parallel_for(n_nodes, [&](int64_t a0, int64_t a1) {
-        std::vector<int32_t> cur;
-        for (int64_t a = a0; a < a1; ++a) {
-            cur.assign(cptr.begin() + brow[a], cptr.begin() + brow[a + 1]);
-            for (int k = inc_ptr[a]; k < inc_ptr[a + 1]; ++k) {
-                const int e = inc[k] / npe, i = inc[k] - e * npe;
-                for (int j = 0; j < npe; ++j) {
-                    const int64_t s = block_of(a, hc[(int64_t)e * npe + j]);
-                    contrib[cur[s - brow[a]]++] = (int32_t)(((int64_t)e * npe + i) * npe + j);
-                }
-            }
-            for (int32_t s = brow[a]; s < brow[a + 1]; ++s) blk_row[s] = (int32_t)a;
-            bdiag[a] = (int32_t)block_of(a, (int32_t)a);
-        }
-    });
-
-    ctx->affine = detect_affine(hc, X, n_el, npe);
-    ctx->ngf = ctx->affine ? 1 : ctx->ngp;
-
-    // device copies
+    // device copies, incidences and the pattern's sizes (mesh_lists.hip)
+    const int64_t n_inc = n_el * npe;
     ALLOC(ctx, ctx->X, double, 3 * n_nodes);
-    ALLOC(ctx, ctx->conn, int32_t, n_el * npe);
+    ALLOC(ctx, ctx->conn, int32_t, n_inc);
     ALLOC(ctx, ctx->E, double, n_el);
     ALLOC(ctx, ctx->nu, double, n_el);
+    ALLOC(ctx, ctx->inc_ptr, int32_t, n_nodes + 1);
+    ALLOC(ctx, ctx->inc, int32_t, n_inc);
+    ALLOC(ctx, ctx->inc_slot, int32_t, n_inc);
+    ALLOC(ctx, ctx->brow, int32_t, n_nodes + 1);
+    ALLOC(ctx, ctx->bdiag, int32_t, n_nodes);
+    ALLOC(ctx, ctx->contrib, int32_t, n_inc * npe);
+    struct Scratch {
+        jfm_ctx *ctx;
+        int32_t *p;
+        ~Scratch() { jfm_free(ctx, p); }
+    } scratch{ctx, jfm_alloc<int32_t>(ctx, mesh_lists_scratch(n_nodes, n_el, npe))};
+    if (!scratch.p) return jfm_fail(ctx, JFM_ENOMEM, "device allocation failed: mesh lists");
+    hipStream_t s = ctx->stream;
+    JFM_HIP(ctx, hipMemcpyAsync(ctx->X, X, sizeof(double) * 3 * n_nodes, hipMemcpyHostToDevice, s));
+    if (n_el > 0) {
+        JFM_HIP(ctx, hipMemcpyAsync(ctx->E, E, sizeof(double) * n_el, hipMemcpyHostToDevice, s));
+        JFM_HIP(ctx, hipMemcpyAsync(ctx->nu, nu, sizeof(double) * n_el, hipMemcpyHostToDevice, s));
+    }
+    int32_t *d_flags = nullptr, flags = 0, nnzb = 0;
+    CHECK_LAUNCH(ctx, launch_mesh_lists(ctx, scratch.p, &d_flags));
+    JFM_HIP(ctx, hipMemcpyAsync(&flags, d_flags, sizeof flags, hipMemcpyDeviceToHost, s));
+    JFM_HIP(ctx, hipMemcpyAsync(&nnzb, ctx->brow + n_nodes, sizeof nnzb, hipMemcpyDeviceToHost, s));
+    if (int rc = sync(ctx)) return rc;
+    ctx->nnzb = nnzb;
+    ctx->affine = !(flags & kMeshCurved);
+    ctx->orphans = (flags & kMeshOrphans) != 0;
+    ctx->ngf = ctx->affine ? 1 : ctx->ngp;
     ALLOC(ctx, ctx->gf64, double, (int64_t)GF * ctx->ngf * n_el);
     ALLOC(ctx, ctx->gf32, float, (int64_t)GF * ctx->ngf * n_el);
-    ALLOC(ctx, ctx->inc_ptr, int32_t, n_nodes + 1);
-    ALLOC(ctx, ctx->inc, int32_t, n_el * npe);
-    ALLOC(ctx, ctx->brow, int32_t, n_nodes + 1);
     ALLOC(ctx, ctx->bcol, int32_t, nnzb);
-    ALLOC(ctx, ctx->bdiag, int32_t, n_nodes);
     ALLOC(ctx, ctx->blk_row, int32_t, nnzb);
-    ALLOC(ctx, ctx->cptr, int32_t, nnzb + 1);
-    ALLOC(ctx, ctx->contrib, int32_t, (int64_t)contrib.size());
-    ALLOC(ctx, ctx->ye64, double, n_el * npe * 3);
-    ALLOC(ctx, ctx->ye32, float, n_el * npe * 3);
+    ALLOC(ctx, ctx->cptr, int32_t, (int64_t)nnzb + 1);
+    CHECK_LAUNCH(ctx, launch_pattern_write(ctx, scratch.p));
+    ALLOC(ctx, ctx->ye64, double, n_inc * 3);
+    ALLOC(ctx, ctx->ye32, float, n_inc * 3);
     ALLOC(ctx, ctx->fixed, uint8_t, 3 * n_nodes);
     ALLOC(ctx, ctx->g, double, 3 * n_nodes);
     ALLOC(ctx, ctx->f_ext, double, 3 * n_nodes);
@@ -402,36 +306,6 @@ extern "C" int jfm_upload_mesh(jfm_ctx *ctx, int64_t n_nodes, const double *X, i
     ALLOC(ctx, ctx->vy32, float, 3 * n_nodes);
     ALLOC(ctx, ctx->partials, double, kPartTotal);
     ALLOC(ctx, ctx->counter, unsigned, 64);
-    ALLOC(ctx, ctx->inc_slot, int32_t, n_el * npe);
-    // slot of incidence (e, i) in the node-sorted list, SoA by local index
-    std::vector<int32_t> slot_soa((size_t)n_el * npe);
-    parallel_for(n_nodes, [&](int64_t a0, int64_t a1) {
-        for (int64_t a = a0; a < a1; ++a)
-            for (int k = inc_ptr[a]; k < inc_ptr[a + 1]; ++k) {
-                const int e = inc[k] / npe, i = inc[k] - e * npe;
-                slot_soa[(size_t)i * n_el + e] = k;
-            }
-    });
-
-    std::vector<int32_t> conn_soa((size_t)n_el * npe);
-    parallel_for(n_el, [&](int64_t a, int64_t b) {
-        for (int64_t e = a; e < b; ++e)
-            for (int i = 0; i < npe; ++i) conn_soa[(size_t)i * n_el + e] = hc[(size_t)e * npe + i];
-    });
-    hipStream_t s = ctx->stream;
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->X, X, sizeof(double) * 3 * n_nodes, hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->conn, conn_soa.data(), sizeof(int32_t) * n_el * npe, hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->E, E, sizeof(double) * n_el, hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->nu, nu, sizeof(double) * n_el, hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->inc_ptr, inc_ptr.data(), sizeof(int32_t) * (n_nodes + 1), hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->inc, inc.data(), sizeof(int32_t) * n_el * npe, hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->brow, brow.data(), sizeof(int32_t) * (n_nodes + 1), hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->bcol, bcol.data(), sizeof(int32_t) * nnzb, hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->bdiag, bdiag.data(), sizeof(int32_t) * n_nodes, hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->blk_row, blk_row.data(), sizeof(int32_t) * nnzb, hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->cptr, cptr.data(), sizeof(int32_t) * (nnzb + 1), hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->contrib, contrib.data(), sizeof(int32_t) * contrib.size(), hipMemcpyHostToDevice, s));
-    JFM_HIP(ctx, hipMemcpyAsync(ctx->inc_slot, slot_soa.data(), sizeof(int32_t) * slot_soa.size(), hipMemcpyHostToDevice, s));
     JFM_HIP(ctx, hipMemsetAsync(ctx->fixed, 0, 3 * n_nodes, s));
     JFM_HIP(ctx, hipMemsetAsync(ctx->g, 0, sizeof(double) * 3 * n_nodes, s));
     JFM_HIP(ctx, hipMemsetAsync(ctx->f_ext, 0, sizeof(double) * 3 * n_nodes, s));
@@ -443,7 +317,6 @@ extern "C" int jfm_upload_mesh(jfm_ctx *ctx, int64_t n_nodes, const double *X, i
     int h_bad = 0;
     JFM_HIP(ctx, hipMemcpyAsync(&h_bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, s));
     if (int rc = sync(ctx)) return rc;
-    // synchronous copies above read pageable host buffers that go out of scope here
     if (h_bad) return jfm_fail(ctx, JFM_ENOTSPD, "element with detJ <= 0 at a Gauss point (inverted or degenerate)");
     ctx->has_mesh = true;
     return JFM_OK;
@@ -527,8 +400,20 @@ extern "C" int jfm_csr_pattern(jfm_ctx *ctx, int64_t *nnz_out, int64_t *rowptr, 
     if (!ctx->has_mesh) return jfm_fail(ctx, JFM_ESTATE, "no mesh");
     if (nnz_out) *nnz_out = 9 * ctx->nnzb;
     if (!rowptr && !colind) return JFM_OK;
+    std::unique_lock<std::mutex> lock(ctx->pattern_mutex);
+    if (ctx->h_brow.empty()) {  // the first call on this mesh
+        JFM_HIP(ctx, hipSetDevice(ctx->device));
+        std::vector<int32_t> br(ctx->N + 1);
+        ctx->h_bcol.resize(ctx->nnzb);
+        JFM_HIP(ctx, hipMemcpyAsync(br.data(), ctx->brow, 4 * br.size(), hipMemcpyDeviceToHost, ctx->stream));
+        if (ctx->nnzb)
+            JFM_HIP(ctx, hipMemcpyAsync(ctx->h_bcol.data(), ctx->bcol, 4 * ctx->h_bcol.size(), hipMemcpyDeviceToHost, ctx->stream));
+        if (int rc = sync(ctx)) return rc;
+        ctx->h_brow.swap(br);
+    }
+    lock.unlock();
     const std::vector<int32_t> &br = ctx->h_brow, &bc = ctx->h_bcol;
-    parallel_for(ctx->N, [&](int64_t a0, int64_t a1) {
+    parallel_for(ctx->N, 1024, [&](int64_t a0, int64_t a1) {
         for (int64_t a = a0; a < a1; ++a) {
             const int64_t r0 = br[a], nb = br[a + 1] - r0;
             for (int c = 0; c < 3; ++c) {

@@ -1117,7 +1117,6 @@ void jfem_coarse_release(jfm_ctx *ctx) {
     ctx->coarse_ready = false;
     ctx->coarse_tag = -1;
     ctx->coarse_built_nodes = 0;
-    ctx->h_node_agg.clear();
     ctx->n_agg = ctx->nc = 0;
 }
 
@@ -1260,7 +1259,6 @@ static int coarse_prepare(jfm_ctx *ctx, int op, int coarse_nodes) {
         const int64_t nc = 6 * (int64_t)A.n_agg;
         if (nc > 20000) return jfm_fail(ctx, JFM_EINVAL, "coarse level too large: raise coarse_nodes");
         ctx->n_agg = A.n_agg;
-        ctx->h_node_agg = A.node_agg;
         ctx->nc = nc;
         ctx->ncolor = A.ncolor;
         std::vector<float> cd32(A.cd.begin(), A.cd.end());

@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -159,6 +160,7 @@ struct jfm_ctx {
     int64_t N = 0, n_el = 0, ndof = 0;
     int npe = 0, ngp = 0, npair = 0;
     bool affine = false, has_mesh = false;
+    bool orphans = false;         // a node of no element
     bool nu_uniform = false;      // every element has Poisson's ratio nu0
     double nu0 = 0.0;
     std::vector<int32_t> h_conn;  // n_el x npe (element-major), 0-based
@@ -173,7 +175,8 @@ struct jfm_ctx {
 
     // pattern and assembly
     int64_t nnzb = 0;
-    std::vector<int32_t> h_brow, h_bcol;
+    std::vector<int32_t> h_brow, h_bcol;  // host copy, from the first jfm_csr_pattern on
+    std::mutex pattern_mutex;             // and its making
     int32_t *brow = nullptr, *bcol = nullptr, *bdiag = nullptr, *blk_row = nullptr;
     int32_t *cptr = nullptr, *contrib = nullptr;
     double *vals64 = nullptr;
@@ -255,7 +258,6 @@ struct jfm_ctx {
     std::vector<double> h_X;       // host copy of the coordinates (aggregation)
     int coarse_built_nodes = 0;    // coarse_nodes the aggregation was built for
     int coarse_gen = 0;            // bumped per aggregation (keys captured graphs)
-    std::vector<int32_t> h_node_agg;
     bool coarse_ready = false;     // Ahat holds a coarse level
     int coarse_tag = -1;           // operator it was built from: 0 K, 1 the tangent
     int64_t n_agg = 0, nc = 0;
@@ -335,7 +337,7 @@ struct jfm_ctx {
         bool ready = false, usable = false;
         int npatch = 0;
         float rho32 = 0.0f;
-        int32_t *eperm = nullptr, *pn_ptr = nullptr, *pn_node = nullptr, *pn_slot = nullptr, *pn_sh = nullptr;
+        int32_t *eperm = nullptr, *pn_n = nullptr, *pn_node = nullptr, *pn_slot = nullptr, *pn_sh = nullptr;
         int32_t *pn_inc = nullptr;
         uint16_t *connL = nullptr, *pn_cnt = nullptr, *lin = nullptr;
         double *gf64 = nullptr, *part = nullptr;  // part: 4 values per slot (FP32 or FP64 view)
@@ -344,12 +346,10 @@ struct jfm_ctx {
         jfem::PcgScalars *S = nullptr;       // scalars of the systems solved side by side
         int nslot = 0, systems = 0;          // systems that words, part and S hold
         std::vector<int32_t> epos;           // element -> position in the patch order
-        std::vector<int32_t> h_ptr, h_node;  // patch nodes, and whether the patch owns each
-        std::vector<uint8_t> h_own;
         // two-level form for the aggregation coarse_gen
         int coarse_gen = -1;
         bool coarse_usable = false;
-        int32_t *pn_agg = nullptr, *ce_ptr = nullptr, *ce_slot = nullptr, *cn_ptr = nullptr, *as_ptr = nullptr;
+        int32_t *pn_agg = nullptr, *ce_n = nullptr, *ce_slot = nullptr, *cn_ptr = nullptr, *as_ptr = nullptr;
         uint16_t *cn_list = nullptr;
         double *wpart = nullptr;
         uint64_t *zw = nullptr;
@@ -383,6 +383,15 @@ void jfm_free(jfm_ctx *ctx, void *p);
 // fem_kernels.hip
 namespace jfem {
 hipError_t launch_geom_factors(jfm_ctx *ctx, int *d_bad);
+// Incidences, sorted pattern rows and contributions of the uploaded mesh
+// (mesh_lists.hip) into ctx->conn, inc*, brow and contrib; scratch of
+// mesh_lists_scratch() int32.  *flags: a device word of kMesh bits.  Then, with
+// bcol, blk_row and cptr allocated for brow[N] blocks, the pattern.
+constexpr int kMeshOrphans = 1;  // a node of no element
+constexpr int kMeshCurved = 2;   // an element whose J is not constant
+int64_t mesh_lists_scratch(int64_t N, int64_t n_el, int npe);
+hipError_t launch_mesh_lists(jfm_ctx *ctx, int32_t *scratch, int32_t **flags);
+hipError_t launch_pattern_write(jfm_ctx *ctx, const int32_t *scratch);
 hipError_t launch_element_matrices(jfm_ctx *ctx);
 hipError_t launch_assemble_values(jfm_ctx *ctx);
 // finite-strain element matrices (which: 0 Km, 1 Kg, 2 Km + Kg), element-major
@@ -448,6 +457,8 @@ constexpr int kPersistPatches = 256;
 constexpr int kPersistWords = 6;  // exchange words per workgroup (and 256 more)
 // elements of a patch, its workgroup's threads (and most nodes), the row
 // stride of its LDS image of the element terms
+// Geometric factors in the element order perm (gfQ32: folded ones too, or null).
+hipError_t launch_patch_factors(jfm_ctx *ctx, const int32_t *perm, double *gf64, float *gf32, float *gfQ32);
 struct PersistGeometry { int elems = 0, threads = 0, stride = 0; };
 int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g);
 void jfem_cells_release(jfm_ctx *ctx);

@@ -337,6 +337,15 @@ __global__ __launch_bounds__(256) void k_fold_gf(int n_el, const double *__restr
     }
 }
 
+hipError_t launch_patch_factors(jfm_ctx *ctx, const int32_t *perm, double *gf64, float *gf32, float *gfQ32) {
+    const int64_t rows = (int64_t)ctx->ngf * GF;
+    const int n = (int)ctx->n_el;
+    k_permute_gf<double><<<1024, 256, 0, ctx->stream>>>(rows, n, perm, ctx->gf64, gf64);
+    k_permute_gf<float><<<1024, 256, 0, ctx->stream>>>(rows, n, perm, ctx->gf32, gf32);
+    if (gfQ32) k_fold_gf<<<1024, 256, 0, ctx->stream>>>(n, gf64, gfQ32);
+    return hipGetLastError();
+}
+
 // ------------------------------------------------------------ host setup ---
 namespace {
 
@@ -386,24 +395,14 @@ void jfem_patch_release(jfm_ctx *ctx) {
 // not fit its type.
 struct PatchHost {
     int npatch = 0;
-    // with `cells`: patch nodes' ids, partial slots (-1: interior), first slot
-    // of the node << 5 | slots, local connectivity (position in the patch)
-    // and the incidences (i, e) of patch node l at lin[pn_inc[l]..]: i stride
-    // + local element, ascending
-    std::vector<int32_t> pn_node, pn_slot, pn_sh, pn_inc;
-    std::vector<uint16_t> connL, lin;
-    int pn_max = 0, slots_max = 0;
-    bool orphans = false;  // a node of no element
     std::vector<int32_t> perm, connP, pn_ptr, pn_out, rstart, rbase, bnode, bptr, pbase;
     std::vector<uint16_t> connP16;  // empty when a patch spans more than 65,536 node ids
     std::vector<uint16_t> pn_cnt, linT;
 };
 
-// ps: elements per patch (and nodes per round); stride > 0: the form of the
-// resident PCG (cells), whose LDS rows have this stride.
 static bool build_patches(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int64_t N,
-                          int npe, int ps, int stride, PatchHost &P) {
-    const bool cells = stride > 0;
+                          int npe, PatchHost &P) {
+    constexpr int ps = kPatch;
     // Morton order of the element centroids (stable in element id)
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
     for (int64_t a = 0; a < N; ++a)
@@ -411,10 +410,6 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
             lo[c] = std::min(lo[c], X[3 * a + c]);
             hi[c] = std::max(hi[c], X[3 * a + c]);
         }
-    // one scale for the three axes in the cells form: compact patches, with
-    // 35% fewer shared-node partials than cells scaled to the bounding box at
-    // 61 x 7 x 5 hexes (24,868 against 38,391) and at most 393 nodes instead of 535
-    const double side = std::max({hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]});
     std::vector<uint64_t> code(n_el);
     for (int64_t e = 0; e < n_el; ++e) {
         double cen[3] = {0.0, 0.0, 0.0};
@@ -422,7 +417,7 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
             for (int c = 0; c < 3; ++c) cen[c] += X[3 * (size_t)conn[e * npe + i] + c];
         uint64_t q[3];
         for (int c = 0; c < 3; ++c) {
-            const double ext = cells ? side : hi[c] - lo[c];
+            const double ext = hi[c] - lo[c];
             const double f = ext > 0.0 ? (cen[c] / npe - lo[c]) / ext : 0.0;
             q[c] = (uint64_t)std::min(std::max(f, 0.0) * 2097151.0, 2097151.0);
         }
@@ -445,7 +440,6 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
     P.pn_cnt.clear();
     P.rbase.clear();
     P.linT.clear();
-    if (cells) P.connL.assign((size_t)npe * n_el, 0);
     std::vector<std::vector<int32_t>> shared_l(N);  // per node: patch-node indices, ascending patch
     std::vector<std::pair<int64_t, int32_t>> pairs;  // (node * ps + local element, i)
     struct PNode { int32_t a, first, cnt; };
@@ -473,7 +467,7 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
         // most incidences first, so that a round's counts are close
         std::stable_sort(nodes.begin(), nodes.end(), [](const PNode &u, const PNode &v) { return u.cnt > v.cnt; });
         const int64_t l0 = (int64_t)P.pn_out.size();
-        for (size_t u = 0; u < nodes.size() && !cells; u += ps) {
+        for (size_t u = 0; u < nodes.size(); u += ps) {
             const int cntmax = nodes[u].cnt;
             const int64_t base = (int64_t)P.linT.size();
             if (base > INT32_MAX) return false;
@@ -488,20 +482,9 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
                 }
             }
         }
-        P.pn_max = std::max(P.pn_max, (int)nodes.size());
         for (size_t u = 0; u < nodes.size(); ++u) {
             const PNode &nd = nodes[u];
             if (nd.cnt > 65535) return false;
-            if (cells) {
-                P.pn_node.push_back(nd.a);
-                P.pn_inc.push_back((int32_t)P.lin.size());
-                for (int j = 0; j < nd.cnt; ++j) {
-                    const auto &pr = pairs[nd.first + j];
-                    const int kl = (int)(pr.first % ps);
-                    P.connL[(size_t)pr.second * n_el + k0 + kl] = (uint16_t)u;
-                    P.lin.push_back((uint16_t)(pr.second * stride + kl));
-                }
-            }
             P.pn_cnt.push_back((uint16_t)nd.cnt);
             if (nd.cnt == val[nd.a]) {
                 P.pn_out.push_back(nd.a);  // interior
@@ -520,10 +503,7 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
         if (!shared_l[a].empty()) order.push_back((int32_t)a);
     std::sort(order.begin(), order.end(), [&](int32_t u, int32_t v) { return shared_l[u][0] < shared_l[v][0]; });
     for (int64_t a = 0; a < N; ++a)
-        if (val[a] == 0) {
-            order.push_back((int32_t)a);
-            P.orphans = true;
-        }
+        if (val[a] == 0) order.push_back((int32_t)a);
     P.bnode.clear();
     P.bptr.assign(1, 0);
     for (int32_t a : order) {
@@ -531,20 +511,6 @@ static bool build_patches(const std::vector<int32_t> &conn, const std::vector<do
         // slots of node a: consecutive, in ascending patch order
         for (size_t j = 0; j < shared_l[a].size(); ++j) P.pn_out[shared_l[a][j]] = -(P.bptr.back() + (int32_t)j + 1);
         P.bptr.push_back(P.bptr.back() + (int32_t)shared_l[a].size());
-    }
-    if (cells) {
-        P.pn_slot.assign(P.pn_out.size(), -1);
-        P.pn_sh.assign(P.pn_out.size(), 0);
-        for (size_t b = 0; b < P.bnode.size(); ++b) {
-            const int32_t first = P.bptr[b], n = P.bptr[b + 1] - first;
-            P.slots_max = std::max(P.slots_max, (int)n);
-            for (int j = 0; j < n; ++j) {
-                const int32_t l = shared_l[P.bnode[b]][j];
-                P.pn_slot[l] = first + j;
-                P.pn_sh[l] = first << 5 | (n & 31);
-            }
-        }
-        return npe * stride <= 65536 && (int64_t)P.pn_out.size() < INT32_MAX / 3;
     }
     // 16-bit connectivity relative to each patch's lowest node id, when every
     // patch's ids span at most 65,536
@@ -579,7 +545,7 @@ int jfem_patch_setup(jfm_ctx *ctx) {
     if ((int64_t)ctx->h_conn.size() != n_el * npe || (int64_t)ctx->h_X.size() != 3 * N)
         return jfm_fail(ctx, JFM_ESTATE, "patch setup needs the host mesh");
     PatchHost P;
-    if (!build_patches(ctx->h_conn, ctx->h_X, n_el, N, npe, kPatch, 0, P))
+    if (!build_patches(ctx->h_conn, ctx->h_X, n_el, N, npe, P))
         return jfm_fail(ctx, JFM_EINVAL, "patch structure out of range");
     const int npatch = P.npatch;
     const int64_t npn = (int64_t)P.pn_out.size(), nb = (int64_t)P.bnode.size();
@@ -630,8 +596,6 @@ int jfem_patch_setup(jfm_ctx *ctx) {
         PUP(ctx->pbase, P.pbase);
     }
 #undef PUP
-    k_permute_gf<double><<<1024, 256, 0, s>>>(ngfr, (int)n_el, ctx->eperm, ctx->gf64, ctx->gfP64);
-    k_permute_gf<float><<<1024, 256, 0, s>>>(ngfr, (int)n_el, ctx->eperm, ctx->gf32, ctx->gfP32);
     if (ctx->affine && npe == 10 && ctx->nu_uniform) {
         // FP32 folded factors: sqrt(cm) invJ, cm = mu w detJ / 5, and lambda / mu
         ctx->gfQ32 = jfm_alloc<float>(ctx, 9 * n_el);
@@ -639,10 +603,9 @@ int jfem_patch_setup(jfm_ctx *ctx) {
             jfem_patch_release(ctx);
             return jfm_fail(ctx, JFM_ENOMEM, "patch operator allocation failed");
         }
-        k_fold_gf<<<1024, 256, 0, s>>>((int)n_el, ctx->gfP64, ctx->gfQ32);
         ctx->rho32 = (float)(2.0 * ctx->nu0 / (1.0 - 2.0 * ctx->nu0));
     }
-    JFM_HIP(ctx, hipGetLastError());
+    JFM_HIP(ctx, launch_patch_factors(ctx, ctx->eperm, ctx->gfP64, ctx->gfP32, ctx->gfQ32));
     JFM_HIP(ctx, hipStreamSynchronize(s));  // host vectors go out of scope
     ctx->npatch = npatch;
     ctx->npn = (int)npn;
@@ -652,138 +615,6 @@ int jfem_patch_setup(jfm_ctx *ctx) {
     for (int64_t i = 0; i < nb; ++i) ctx->bmaxcnt = std::max(ctx->bmaxcnt, P.bptr[i + 1] - P.bptr[i]);
     ctx->patch_ready = true;
     return JFM_OK;
-}
-
-// The resident PCG's patches (persist.hip), once per mesh: the same structure
-// in that kernel's patch size, with local connectivity and, per patch node,
-// its id, slots and incidences.  cells.usable tells whether the mesh fits.
-int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g) {
-    auto &C = ctx->cells;
-    if (C.ready) return JFM_OK;
-    C.ready = true;
-    C.usable = false;
-    const int64_t n_el = ctx->n_el, N = ctx->N;
-    const int npe = ctx->npe;
-    if ((int64_t)ctx->h_conn.size() != n_el * npe || (int64_t)ctx->h_X.size() != 3 * N) return JFM_OK;
-    PatchHost P;
-    if (!build_patches(ctx->h_conn, ctx->h_X, n_el, N, npe, g.elems, g.stride, P)) return JFM_OK;
-    // pn_sh holds 26 bits of slot and 5 of count; a node of no element is in no patch
-    if (P.orphans || P.slots_max > 31 || P.bptr.back() >= (1 << 25) || P.pn_max > g.threads) return JFM_OK;
-    hipStream_t s = ctx->stream;
-    auto put = [&](auto *&dst, const auto &v) -> bool {
-        using V = std::decay_t<decltype(v[0])>;
-        dst = jfm_alloc<V>(ctx, std::max<int64_t>(1, (int64_t)v.size()));
-        return dst && (v.empty() || hipMemcpyAsync(dst, v.data(), sizeof(V) * v.size(), hipMemcpyHostToDevice, s) == hipSuccess);
-    };
-    const int64_t rows = (int64_t)ctx->ngf * GF;
-    bool ok = put(C.eperm, P.perm) && put(C.connL, P.connL) && put(C.pn_ptr, P.pn_ptr) && put(C.pn_cnt, P.pn_cnt) &&
-              put(C.pn_node, P.pn_node) && put(C.pn_slot, P.pn_slot) && put(C.pn_sh, P.pn_sh) &&
-              put(C.pn_inc, P.pn_inc) && put(C.lin, P.lin);
-    ok = ok && (C.gf64 = jfm_alloc<double>(ctx, rows * n_el)) && (C.gf32 = jfm_alloc<float>(ctx, rows * n_el));
-    const bool fold = ctx->affine && npe == 10 && ctx->nu_uniform;
-    if (ok && fold) ok = (C.gfQ32 = jfm_alloc<float>(ctx, 9 * n_el)) != nullptr;
-    if (!ok) {
-        jfem_cells_release(ctx);
-        (void)hipStreamSynchronize(s);  // host vectors go out of scope
-        return jfm_fail(ctx, JFM_ENOMEM, "resident PCG allocation failed");
-    }
-    k_permute_gf<double><<<1024, 256, 0, s>>>(rows, (int)n_el, C.eperm, ctx->gf64, C.gf64);
-    k_permute_gf<float><<<1024, 256, 0, s>>>(rows, (int)n_el, C.eperm, ctx->gf32, C.gf32);
-    if (fold) k_fold_gf<<<1024, 256, 0, s>>>((int)n_el, C.gf64, C.gfQ32);
-    JFM_HIP(ctx, hipGetLastError());
-    JFM_HIP(ctx, hipStreamSynchronize(s));
-    C.npatch = P.npatch;
-    C.nslot = P.bptr.back();
-    C.epos.resize(n_el);
-    for (int64_t k = 0; k < n_el; ++k) C.epos[P.perm[k]] = (int32_t)k;
-    C.h_own.resize(P.pn_node.size());
-    for (size_t l = 0; l < P.pn_node.size(); ++l) C.h_own[l] = P.pn_slot[l] < 0 || P.pn_slot[l] == P.pn_sh[l] >> 5;
-    C.h_node = std::move(P.pn_node);
-    C.h_ptr = std::move(P.pn_ptr);
-    C.rho32 = (float)(2.0 * ctx->nu0 / (1.0 - 2.0 * ctx->nu0));
-    C.usable = true;
-    return JFM_OK;
-}
-
-// Per patch the aggregates of its owned nodes, with those nodes (ascending), and
-// per aggregate the patches' slots (ascending patch), for the current
-// aggregation.
-int jfem_cells_coarse(jfm_ctx *ctx, int max_entries) {
-    auto &C = ctx->cells;
-    if (C.coarse_gen == ctx->coarse_gen) return JFM_OK;
-    C.coarse_usable = false;
-    for (void **q : {(void **)&C.pn_agg, (void **)&C.ce_ptr, (void **)&C.ce_slot, (void **)&C.cn_ptr, (void **)&C.as_ptr,
-                     (void **)&C.cn_list, (void **)&C.wpart, (void **)&C.zw}) {
-        jfm_free(ctx, *q);
-        *q = nullptr;
-    }
-    const std::vector<int32_t> &agg = ctx->h_node_agg;
-    const int n_agg = (int)ctx->n_agg;
-    std::vector<int32_t> pn_agg(C.h_node.size()), ce_ptr(1, 0), ce_agg, cn_ptr(1, 0), as_ptr(n_agg + 1, 0);
-    std::vector<uint16_t> cn_list;
-    std::vector<std::pair<int32_t, int32_t>> own;  // (aggregate, position)
-    bool fits = (int64_t)agg.size() == ctx->N;
-    for (int p = 0; p < C.npatch && fits; ++p) {
-        own.clear();
-        for (int32_t l = C.h_ptr[p]; l < C.h_ptr[p + 1]; ++l) {
-            pn_agg[l] = agg[C.h_node[l]];
-            if (C.h_own[l]) own.emplace_back(pn_agg[l], l - C.h_ptr[p]);
-        }
-        std::sort(own.begin(), own.end());
-        for (size_t i = 0; i < own.size(); ++i) {
-            if (i == 0 || own[i].first != own[i - 1].first) {
-                if (i) cn_ptr.push_back((int32_t)cn_list.size());
-                ce_agg.push_back(own[i].first);
-                ++as_ptr[own[i].first + 1];
-            }
-            cn_list.push_back((uint16_t)own[i].second);
-        }
-        if (!own.empty()) cn_ptr.push_back((int32_t)cn_list.size());
-        ce_ptr.push_back((int32_t)ce_agg.size());
-        fits = ce_ptr[p + 1] - ce_ptr[p] <= max_entries;
-    }
-    C.coarse_gen = ctx->coarse_gen;
-    if (!fits) return JFM_OK;
-    for (int g = 0; g < n_agg; ++g) as_ptr[g + 1] += as_ptr[g];
-    std::vector<int32_t> pos(as_ptr.begin(), as_ptr.end() - 1), ce_slot(ce_agg.size());
-    for (size_t e = 0; e < ce_agg.size(); ++e) ce_slot[e] = pos[ce_agg[e]]++;
-    hipStream_t s = ctx->stream;
-    auto put = [&](auto *&dst, const auto &v) -> bool {
-        using V = std::decay_t<decltype(v[0])>;
-        dst = jfm_alloc<V>(ctx, std::max<int64_t>(1, (int64_t)v.size()));
-        return dst && (v.empty() || hipMemcpyAsync(dst, v.data(), sizeof(V) * v.size(), hipMemcpyHostToDevice, s) == hipSuccess);
-    };
-    const bool ok = put(C.pn_agg, pn_agg) && put(C.ce_ptr, ce_ptr) && put(C.ce_slot, ce_slot) && put(C.cn_ptr, cn_ptr) &&
-                    put(C.as_ptr, as_ptr) && put(C.cn_list, cn_list) &&
-                    (C.wpart = jfm_alloc<double>(ctx, 6 * std::max<int64_t>(1, (int64_t)ce_slot.size()))) &&
-                    (C.zw = jfm_alloc<uint64_t>(ctx, 16 * std::max<int64_t>(1, ctx->nc)));
-    JFM_HIP(ctx, hipStreamSynchronize(s));  // host vectors go out of scope
-    if (!ok) return jfm_fail(ctx, JFM_ENOMEM, "resident PCG allocation failed");
-    C.coarse_usable = true;
-    return JFM_OK;
-}
-
-int jfem_cells_systems(jfm_ctx *ctx, int m) {
-    auto &C = ctx->cells;
-    if (m <= C.systems) return JFM_OK;
-    for (void *q : {(void *)C.part, (void *)C.words, (void *)C.S}) jfm_free(ctx, q);
-    C.systems = 0;
-    C.part = jfm_alloc<double>(ctx, (int64_t)m * 4 * std::max(1, C.nslot));
-    C.words = jfm_alloc<uint64_t>(ctx, (int64_t)m * kPersistWords * (C.npatch + 256));
-    C.S = jfm_alloc<PcgScalars>(ctx, m);
-    if (!C.part || !C.words || !C.S) return jfm_fail(ctx, JFM_ENOMEM, "resident PCG allocation failed");
-    C.systems = m;
-    return JFM_OK;
-}
-
-void jfem_cells_release(jfm_ctx *ctx) {
-    auto &C = ctx->cells;
-    for (void *p : {(void *)C.eperm, (void *)C.connL, (void *)C.pn_ptr, (void *)C.pn_cnt, (void *)C.pn_node, (void *)C.pn_slot,
-                    (void *)C.pn_sh, (void *)C.pn_inc, (void *)C.lin, (void *)C.gf64, (void *)C.gf32,
-                    (void *)C.gfQ32, (void *)C.part, (void *)C.words, (void *)C.S, (void *)C.pn_agg, (void *)C.ce_ptr,
-                    (void *)C.ce_slot, (void *)C.cn_ptr, (void *)C.as_ptr, (void *)C.cn_list, (void *)C.wpart, (void *)C.zw})
-        jfm_free(ctx, p);
-    C = {};
 }
 
 // qsrc for the update kernel of the two-level PCG (nodes in aggregate order)

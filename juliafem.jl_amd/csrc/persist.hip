@@ -268,7 +268,7 @@ template <typename T> struct PersistArgs {
     const int32_t *ef, *enext, *fmap;  // heat: the element's first convection face (or -1), the next
     const double *fk;         // one, its element-local nodes (4 bits each) and its matrix
     int nfn;
-    const int32_t *pn_ptr;    // patch nodes: range per patch
+    const int32_t *pn_n;      // patch nodes: their number; patch p's at kNT p
     const int32_t *pn_node;   // patch node -> node
     const int32_t *pn_slot;   // its partial slot, or -1 (interior)
     const int32_t *pn_sh;     // shared: first slot of its node << 5 | slots
@@ -287,11 +287,12 @@ template <typename T> struct PersistArgs {
     const double *ustate;     // tangent: the displacement it is taken at
     // two-level: per patch node its aggregate; offsets from the aggregates'
     // centroids (per node); the patch's entries, one per aggregate that its
-    // owned nodes are in (slot in wpart, nodes cn_list[cn_ptr[e]..]); the
+    // owned nodes are in (ce_n[p] of them, at kMaxEntries p: slot in wpart; nodes
+    // cn_list[kNT p + cn_ptr[(kMaxEntries + 1) p + e]..]); the
     // aggregates' slots; the coarse operator; exchange words
     const int32_t *pn_agg;
     const T *cd;
-    const int32_t *ce_ptr, *ce_slot, *cn_ptr, *as_ptr;
+    const int32_t *ce_n, *ce_slot, *cn_ptr, *as_ptr;
     const uint16_t *cn_list;
     const float *Ahat;
     int nc, ldc;
@@ -471,7 +472,7 @@ template <typename T_> struct TangentTet10 : OpShape<10, 3, 4, 10, 4, false, 2> 
         for (int m = 0; m < 9; ++m) Ji[m] = has ? A.el64[(size_t)m * A.n_el + k] : (m % 4 == 0 ? 1.0 : 0.0);
         lane_gradients<double>(Ji, kv, g);
         const double cl = has ? A.el64[(size_t)9 * A.n_el + k] : 0.0, cm = has ? A.el64[(size_t)10 * A.n_el + k] : 0.0;
-        const int lb = A.pn_ptr[k / kEl];
+        const int lb = kNT * (k / kEl);
         gradient<double>(g, [&](int m, int c) -> double {
             return has ? A.ustate[3 * (size_t)A.pn_node[lb + A.connL[(size_t)in_node(kv, m) * A.n_el + k]] + c] : 0.0;
         }, H);
@@ -836,7 +837,7 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
     const int el = t / NL, kv = NL == 4 ? t & 3 : 0;   // its element (and vertex or component)
     const int k = p * EL + el;
     const bool has_el = el < EL && k < A.n_el;
-    const int lb = A.pn_ptr[p], nn = A.pn_ptr[p + 1] - lb;
+    const int lb = NT * p, nn = A.pn_n[p];
     const int rows = nwg + kGroup * kGroup;
     uint64_t *wordsB = A.words + (size_t)sys * kPersistWords * rows, *wordsC = wordsB + 2 * (size_t)rows;
     PcgScalars *S = A.S + sys;
@@ -891,18 +892,17 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
     T dv[3];               // two-level: the node's offset and aggregate
     int agg = 0, ca0[kCoarseRows], ca1[kCoarseRows], ne = 0;
     if constexpr (COARSE) {
-        const int e0 = A.ce_ptr[p];
-        ne = A.ce_ptr[p + 1] - e0;
+        ne = A.ce_n[p];
         agg = in ? 6 * A.pn_agg[lb + t] : 0;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             dv[c] = in ? A.cd[3 * (size_t)node + c] : T(0);
             co.d[3 * t + c] = dv[c];
         }
-        const int n0 = A.cn_ptr[e0];
-        if (t <= ne) co.start[t] = A.cn_ptr[e0 + t] - n0;
-        if (t < ne) co.slot[t] = A.ce_slot[e0 + t];
-        if (t < A.cn_ptr[e0 + ne] - n0) co.list[t] = A.cn_list[n0 + t];
+        const int32_t *start = A.cn_ptr + (kMaxEntries + 1) * p;
+        if (t <= ne) co.start[t] = start[t];
+        if (t < ne) co.slot[t] = A.ce_slot[kMaxEntries * p + t];
+        if (t < start[ne]) co.list[t] = A.cn_list[lb + t];
 #pragma unroll
         for (int j = 0; j < kCoarseRows; ++j) {
             const int i = t + j * NT, g = i / 6;
@@ -1253,7 +1253,7 @@ hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, c
     if (coarse) {
         A.pn_agg = C.pn_agg;
         A.cd = sizeof(T) == 8 ? (const T *)ctx->cd64 : (const T *)ctx->cd32;
-        A.ce_ptr = C.ce_ptr;
+        A.ce_n = C.ce_n;
         A.ce_slot = C.ce_slot;
         A.cn_ptr = C.cn_ptr;
         A.as_ptr = C.as_ptr;
@@ -1275,7 +1275,7 @@ hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, c
         A.fk = ctx->hf_K;
         A.nfn = ctx->hf_nfn;
     }
-    A.pn_ptr = C.pn_ptr;
+    A.pn_n = C.pn_n;
     A.pn_node = C.pn_node;
     A.pn_slot = C.pn_slot;
     A.pn_sh = C.pn_sh;

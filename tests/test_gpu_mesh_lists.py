@@ -1,0 +1,110 @@
+"""The lists that an upload builds on the device (mesh_lists.hip), through the C ABI.
+
+A star of tetrahedra around one node: its row of the pattern has thousands of
+contributions (more than the LDS of the row kernel holds: 1,024), beside rows of
+a few.  One element, nodes in random order, and nodes of no element.  The
+pattern is compared exactly with the one of the elements, the values with the
+oracle's assembly (1e-13 of the largest: the same FP64 sums, in element order),
+and a solve on the star, one of whose nodes lies in every patch, with the
+oracle's direct solve (rtol 1e-10: 1e-8, as the resident PCG's tests ask).
+"""
+import numpy as np
+import pytest
+
+from jfem import mesh as M
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print(f"[gpu] {msg}", flush=True)
+
+
+def star(n, quadratic):
+    """The tetrahedra between the centre of a cube and its surface of 12 n^2 triangles."""
+    b = M.box_tet4(n, n, n, L=(1.0, 1.0, 1.0))
+    f = np.concatenate([b.conn[:, list(c)] for c in ((0, 2, 1), (0, 1, 3), (1, 2, 3), (0, 3, 2))])
+    _, first, count = np.unique(np.sort(f, 1), axis=0, return_index=True, return_counts=True)
+    tri = f[first[count == 1]]
+    used, tri = np.unique(tri, return_inverse=True)
+    tri = tri.reshape(-1, 3)
+    X = np.vstack([b.X[used], [[0.5, 0.5, 0.5]]])
+    conn = np.column_stack([tri[:, 0], tri[:, 2], tri[:, 1], np.full(len(tri), len(used))])
+    if quadratic:
+        e = np.sort(conn[:, [[0, 1], [1, 2], [2, 0], [0, 3], [1, 3], [2, 3]]], 2)
+        ed, mid = np.unique(e.reshape(-1, 2), axis=0, return_inverse=True)
+        X, conn = np.vstack([X, 0.5 * (X[ed[:, 0]] + X[ed[:, 1]])]), np.column_stack([conn, len(X) + mid.reshape(-1, 6)])
+    E = np.exp(np.random.default_rng(1).normal(0.0, 0.4, len(conn)))
+    return M.Mesh(X=X, conn=conn, etype="Tet10" if quadratic else "Tet4", E=E, nu=np.full(len(conn), 0.3),
+                  faces=np.zeros((0, 3), np.int64), ftype="Tri3", clamp_nodes=np.flatnonzero(X[:, 0] == 0.0))
+
+
+def shuffled(m, extra):
+    """Nodes in random order, `extra` of them in no element."""
+    rng = np.random.default_rng(2)
+    N = m.n_nodes + extra
+    new = rng.permutation(N)[:m.n_nodes]
+    X = rng.uniform(0.0, 1.0, (N, 3))
+    X[new] = m.X
+    return M.Mesh(X=X, conn=new[m.conn], etype=m.etype, E=m.E, nu=m.nu, faces=np.zeros((0, 3), np.int64), ftype="Tri3",
+                  clamp_nodes=new[m.clamp_nodes])
+
+
+def one_hex():
+    m = M.box_hex8(1, 1, 1)
+    return M.Mesh(X=m.X, conn=m.conn, etype="Hex8", E=m.E, nu=m.nu, faces=np.zeros((0, 4), np.int64), ftype="Quad4",
+                  clamp_nodes=m.clamp_nodes)
+
+
+CASES = {
+    "one_hex8": one_hex,
+    "star_tet4": lambda: star(9, False),      # 972 elements: 3,888 entries
+    "star_tet10": lambda: star(4, True),      # 192 elements: 1,920 entries
+    "star_tet10_at_the_limit": lambda: star(3, True),  # 108: 1,080
+    "shuffled_hex8": lambda: shuffled(M.box_hex8(5, 4, 3, jitter=0.1, seed=3), 0),
+    "shuffled_tet10_orphans": lambda: shuffled(M.box_tet10(5, 4, 3, jitter=0.1, seed=3), 7),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_pattern_and_values(oracle, name):
+    import jfem
+    m = CASES[name]()
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    say(f"mesh lists {name}: nodes={m.n_nodes} el={m.n_el}")
+    rp, ci = ctx.csr_pattern()
+    rows = [[] for _ in range(m.n_nodes)]
+    for c in m.conn:
+        for a in c:
+            rows[a].append(c)
+    ptr, col = [0], []
+    for r in rows:
+        dofs = (3 * np.unique(np.concatenate(r))[:, None] + np.arange(3)).ravel() if r else np.zeros(0, np.int64)
+        for _ in range(3):
+            col.append(dofs)
+            ptr.append(ptr[-1] + len(dofs))
+    assert np.array_equal(rp, ptr) and np.array_equal(ci, np.concatenate(col))
+    vals = ctx.assemble()
+    vals = vals[0] if isinstance(vals, tuple) else vals
+    import scipy.sparse as sp
+    ro, co, vo = oracle.assemble_csr(m)
+    Ko = sp.csr_matrix((vo, co, ro), shape=(m.n_dofs, m.n_dofs))
+    K = sp.csr_matrix((vals, ci, rp), shape=(m.n_dofs, m.n_dofs))
+    assert abs(K - Ko).max() <= 1e-13 * np.abs(vo).max()
+    ctx.close()
+
+
+@pytest.mark.parametrize("name", ["star_tet4", "star_tet10"])
+def test_solve_on_a_star(oracle, name):
+    import jfem
+    m = CASES[name]()
+    f = np.random.default_rng(4).normal(size=m.n_dofs)
+    ud, _, _ = oracle.solve_direct_lapack(oracle.assemble_csr(m), m.fixed_mask(), np.zeros(m.n_dofs), f)
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    for kw in (dict(method=0), dict(method=1, inner_rtol=1e-2), dict(method=1, inner_rtol=1e-2, coarse_nodes=60)):
+        say(f"solve {name} {kw}")
+        u, _, _ = ctx.solve(f=f, rtol=1e-10, **kw)
+        assert np.linalg.norm(u - ud) <= 1e-8 * np.linalg.norm(ud)
+    ctx.close()
