@@ -782,10 +782,19 @@ void bin_nodes(const std::vector<double> &X, int64_t N, int target, std::vector<
         }
         key[a] = ((int64_t)b[0] * nb[1] + b[1]) * nb[2] + b[2];
     }
+    agg.resize(N);
+    const double nbin = (double)nb[0] * nb[1] * nb[2];
+    if (nbin <= 4.0 * N + 1024.0) {  // number the occupied bins in ascending order
+        std::vector<int32_t> id((size_t)nbin, 0);
+        for (int64_t a = 0; a < N; ++a) id[key[a]] = 1;
+        n_agg = 0;
+        for (int32_t &v : id) v = v ? n_agg++ : -1;
+        for (int64_t a = 0; a < N; ++a) agg[a] = id[key[a]];
+        return;
+    }
     std::vector<int64_t> uk(key);
     std::sort(uk.begin(), uk.end());
     uk.erase(std::unique(uk.begin(), uk.end()), uk.end());
-    agg.resize(N);
     for (int64_t a = 0; a < N; ++a) agg[a] = (int32_t)(std::lower_bound(uk.begin(), uk.end(), key[a]) - uk.begin());
     n_agg = (int)uk.size();
 }
@@ -793,18 +802,29 @@ void bin_nodes(const std::vector<double> &X, int64_t N, int target, std::vector<
 std::vector<std::vector<int32_t>> agg_adjacency(const std::vector<int32_t> &conn, int64_t n_el, int npe,
                                                 const std::vector<int32_t> &agg, int n_agg) {
     std::vector<std::vector<int32_t>> adj(n_agg);
+    // pairs met before, while a flag for each is small
+    std::vector<uint8_t> met(n_agg <= 2048 ? (size_t)n_agg * n_agg : 0, 0);
     int32_t loc[32];
     for (int64_t e = 0; e < n_el; ++e) {
-        int m = 0;
-        for (int i = 0; i < npe; ++i) {
-            const int32_t g = agg[conn[e * npe + i]];
+        const int32_t *c = conn.data() + e * npe;
+        int m = 1;
+        loc[0] = agg[c[0]];
+        for (int i = 1; i < npe; ++i) {
+            const int32_t g = agg[c[i]];
             bool seen = false;
             for (int k = 0; k < m; ++k) seen = seen || loc[k] == g;
             if (!seen) loc[m++] = g;
         }
-        for (int k = 0; k < m; ++k)
-            for (int l = 0; l < m; ++l)
-                if (k != l) adj[loc[k]].push_back(loc[l]);
+        for (int k = 0; k < m && m > 1; ++k)
+            for (int l = 0; l < m; ++l) {
+                if (k == l) continue;
+                if (!met.empty()) {
+                    uint8_t &f = met[(size_t)loc[k] * n_agg + loc[l]];
+                    if (f) continue;
+                    f = 1;
+                }
+                adj[loc[k]].push_back(loc[l]);
+            }
     }
     for (auto &v : adj) {
         std::sort(v.begin(), v.end());
@@ -884,20 +904,19 @@ void galerkin_lists(const jfm_ctx *ctx, const std::vector<int32_t> &agg, int n_a
 
 }  // namespace
 
-// Host-side aggregation, colouring and per-aggregate mode bases.
-static int coarse_host_setup(jfm_ctx *ctx, int coarse_nodes, const std::vector<uint8_t> &fixed,
-                             const std::vector<int32_t> &slot, Aggregation &A) {
+// Host-side aggregation and per-aggregate mode bases.
+static void coarse_host_setup(jfm_ctx *ctx, int coarse_nodes, const std::vector<uint8_t> &fixed, Aggregation &A) {
     const int64_t N = ctx->N;
     const std::vector<double> &X = ctx->h_X;
     int n_agg = 0;
     std::vector<int32_t> agg;
     bin_nodes(X, N, coarse_nodes, agg, n_agg);
     // merge aggregates far below the target size into their largest neighbour
-    {
+    std::vector<int64_t> cnt(n_agg, 0);
+    for (int64_t a = 0; a < N; ++a) cnt[agg[a]]++;
+    const int64_t small = std::max<int64_t>(8, coarse_nodes / 8);
+    if (n_agg > 0 && *std::min_element(cnt.begin(), cnt.end()) < small) {
         auto adj = agg_adjacency(ctx->h_conn, ctx->n_el, ctx->npe, agg, n_agg);
-        std::vector<int64_t> cnt(n_agg, 0);
-        for (int64_t a = 0; a < N; ++a) cnt[agg[a]]++;
-        const int64_t small = std::max<int64_t>(8, coarse_nodes / 8);
         std::vector<int32_t> into(n_agg);
         std::iota(into.begin(), into.end(), 0);
         for (int g = 0; g < n_agg; ++g) {
@@ -943,12 +962,14 @@ static int coarse_host_setup(jfm_ctx *ctx, int coarse_nodes, const std::vector<u
         for (int k = A.agg_ptr[g]; k < A.agg_ptr[g + 1]; ++k) {
             const int64_t a = A.agg_nodes[k];
             const double *d = &A.cd[3 * a];
-            // rows of the mode matrix for the three DOFs of node a
-            double Bm[3][6] = {{1, 0, 0, 0, d[2], -d[1]}, {0, 1, 0, -d[2], 0, d[0]}, {0, 0, 1, d[1], -d[0], 0}};
+            // rows of the mode matrix for the three DOFs of node a: three
+            // nonzeros each, at these modes
+            static const int at[3][3] = {{0, 4, 5}, {1, 3, 5}, {2, 3, 4}};
+            const double Bm[3][3] = {{1, d[2], -d[1]}, {1, -d[2], d[0]}, {1, d[1], -d[0]}};
             for (int c = 0; c < 3; ++c) {
                 if (fixed[3 * a + c]) continue;
-                for (int i = 0; i < 6; ++i)
-                    for (int j = 0; j < 6; ++j) G[i * 6 + j] += Bm[c][i] * Bm[c][j];
+                for (int i = 0; i < 3; ++i)
+                    for (int j = 0; j < 3; ++j) G[at[c][i] * 6 + at[c][j]] += Bm[c][i] * Bm[c][j];
             }
         }
         // Cholesky G = R'R with column dropping
@@ -982,6 +1003,14 @@ static int coarse_host_setup(jfm_ctx *ctx, int coarse_nodes, const std::vector<u
         }
         for (int i = 0; i < 6; ++i) A.dropped[6 * g + i] = keep[i] ? 0 : 1;
     }
+}
+
+// The lists of the probed setup: a colouring of the aggregates and, per colour,
+// the elements and nodes that its probe touches.  slot[i * n_el + e]: the
+// incidence (e, i).
+static int probe_lists(const jfm_ctx *ctx, const std::vector<int32_t> &agg, int n_agg, const std::vector<int32_t> &slot,
+                       Aggregation &A) {
+    const int64_t N = ctx->N;
     // distance-2 greedy colouring of the aggregate graph
     auto adj = agg_adjacency(ctx->h_conn, ctx->n_el, ctx->npe, agg, n_agg);
     A.color.assign(n_agg, -1);
@@ -1003,13 +1032,12 @@ static int coarse_host_setup(jfm_ctx *ctx, int coarse_nodes, const std::vector<u
         ncolor = std::max(ncolor, c + 1);
     }
     A.ncolor = ncolor;
-    galerkin_lists(ctx, agg, n_agg, adj, fixed, A);
     A.partner.assign((size_t)ncolor * n_agg, -1);
     for (int g = 0; g < n_agg; ++g) {
         A.partner[(size_t)A.color[g] * n_agg + g] = g;
         for (int32_t h : adj[g]) {
             int32_t &slot = A.partner[(size_t)A.color[h] * n_agg + g];
-            if (slot >= 0 && slot != h) return jfm_fail(ctx, JFM_EINVAL, "aggregate colouring is not distance-2");
+            if (slot >= 0 && slot != h) return JFM_EINVAL;
             slot = h;
         }
     }
@@ -1103,6 +1131,7 @@ void jfem_coarse_release(jfm_ctx *ctx) {
     free_dev(ctx, ctx->gal_pptr); free_dev(ctx, ctx->gal_upair); free_dev(ctx, ctx->gal_C);
     ctx->gal_nitems = ctx->gal_nupair = 0;
     free_dev(ctx, ctx->dropped); free_dev(ctx, ctx->ecol); free_dev(ctx, ctx->ncol);
+    ctx->h_node_agg.clear();
     ctx->h_ecol_ptr.clear(); ctx->h_ncol_ptr.clear(); ctx->h_cseg.clear();
     free_dev(ctx, ctx->segb); free_dev(ctx, ctx->sega); free_dev(ctx, ctx->csub_ptr); free_dev(ctx, ctx->csub);
     for (int k = 0; k < 2; ++k)
@@ -1117,6 +1146,8 @@ void jfem_coarse_release(jfm_ctx *ctx) {
     ctx->coarse_ready = false;
     ctx->coarse_tag = -1;
     ctx->coarse_built_nodes = 0;
+    ctx->coarse_built = 0;
+    ctx->gal_lists = ctx->probe_lists = false;
     ctx->n_agg = ctx->nc = 0;
 }
 
@@ -1241,75 +1272,69 @@ static hipError_t setup_inverse_sequence(jfm_ctx *ctx) {
     return hipGetLastError();
 }
 
+// Offsets in FP32 and, with the nodes' positions, in the aggregates' node order.
+__global__ __launch_bounds__(256) void k_agg_order(int N, const int32_t *__restrict__ agg_nodes, const double *__restrict__ cd,
+                                                  float *__restrict__ cd32, double *__restrict__ cdA, float *__restrict__ cdA32,
+                                                  int32_t *__restrict__ apos) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= N) return;
+    const int a = agg_nodes[k];
+    apos[a] = k;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const double v = cd[3 * (size_t)a + c];
+        cd32[3 * (size_t)a + c] = (float)v;
+        cdA[3 * (size_t)k + c] = v;
+        cdA32[3 * (size_t)k + c] = (float)v;
+    }
+}
+
 // The aggregation for coarse_nodes (kept while the mesh, the fixed set and
 // coarse_nodes stay the same) and, for a probed operator, the probe vectors.
 static int coarse_prepare(jfm_ctx *ctx, int op, int coarse_nodes) {
     hipStream_t s = ctx->stream;
     const int64_t N = ctx->N, n = ctx->ndof;
-    if (ctx->coarse_built_nodes != coarse_nodes || !ctx->node_agg) {
-        jfem_coarse_release(ctx);
-        std::vector<uint8_t> fx(n);
+    // the lists that the operator's setup needs, in the current aggregation
+    const bool probe = coarse_probe(op == JFM_OP_TANGENT);
+    const bool fresh = ctx->coarse_built_nodes != coarse_nodes || !ctx->node_agg;
+    if (fresh) jfem_coarse_release(ctx);
+    const bool need_probe = probe && !ctx->probe_lists, need_gal = !probe && !ctx->gal_lists;
+#define CALLOC(ptr, T, cnt)                                   \
+    do {                                                      \
+        ptr = jfm_alloc<T>(ctx, std::max<int64_t>(1, (int64_t)(cnt))); \
+        if (!ptr) {                                           \
+            jfem_coarse_release(ctx);                         \
+            (void)hipStreamSynchronize(s);                    \
+            return jfm_fail(ctx, JFM_ENOMEM, "coarse level allocation failed"); \
+        }                                                     \
+    } while (0)
+    auto up = [&](auto *d, const auto &v) -> hipError_t {
+        return v.empty() ? hipSuccess : hipMemcpyAsync(d, v.data(), sizeof(v[0]) * v.size(), hipMemcpyHostToDevice, s);
+    };
+    std::vector<uint8_t> fx;
+    if (fresh || need_gal) {
+        fx.resize(n);
         JFM_HIP(ctx, hipMemcpyAsync(fx.data(), ctx->fixed, n, hipMemcpyDeviceToHost, s));
         JFM_HIP(ctx, hipStreamSynchronize(s));
-        std::vector<int32_t> slot((size_t)ctx->npe * ctx->n_el);
-        JFM_HIP(ctx, hipMemcpyAsync(slot.data(), ctx->inc_slot, 4 * slot.size(), hipMemcpyDeviceToHost, s));
-        JFM_HIP(ctx, hipStreamSynchronize(s));
-        Aggregation A;
-        if (int rc = coarse_host_setup(ctx, coarse_nodes, fx, slot, A)) return rc;
+    }
+    Aggregation A;
+    if (fresh) {
+        coarse_host_setup(ctx, coarse_nodes, fx, A);
         const int64_t nc = 6 * (int64_t)A.n_agg;
         if (nc > 20000) return jfm_fail(ctx, JFM_EINVAL, "coarse level too large: raise coarse_nodes");
         ctx->n_agg = A.n_agg;
+        ctx->h_node_agg = A.node_agg;
         ctx->nc = nc;
-        ctx->ncolor = A.ncolor;
-        std::vector<float> cd32(A.cd.begin(), A.cd.end());
-#define CALLOC(ptr, T, cnt)                                   \
-    do {                                                      \
-        ptr = jfm_alloc<T>(ctx, cnt);                         \
-        if (!ptr) return jfm_fail(ctx, JFM_ENOMEM, "coarse level allocation failed"); \
-    } while (0)
         CALLOC(ctx->node_agg, int32_t, N);
         CALLOC(ctx->agg_ptr, int32_t, A.n_agg + 1);
         CALLOC(ctx->agg_nodes, int32_t, N);
-        CALLOC(ctx->agg_color, int32_t, A.n_agg);
-        CALLOC(ctx->partner, int32_t, (int64_t)A.ncolor * A.n_agg);
         CALLOC(ctx->cd64, double, 3 * N);
         CALLOC(ctx->cd32, float, 3 * N);
         CALLOC(ctx->Rinv, double, 36 * (int64_t)A.n_agg);
         CALLOC(ctx->dropped, int32_t, nc);
-        CALLOC(ctx->ecol, int32_t, std::max<int64_t>(1, (int64_t)A.ecol.size()));
-        CALLOC(ctx->ncol, int32_t, std::max<int64_t>(1, (int64_t)A.ncol.size()));
-        CALLOC(ctx->segb, int32_t, (int64_t)A.segb.size());
-        CALLOC(ctx->csub_ptr, int32_t, (int64_t)A.csub_ptr.size());
-        CALLOC(ctx->csub, int32_t, std::max<int64_t>(1, (int64_t)A.csub.size()));
-        CALLOC(ctx->sega, int32_t, std::max<int64_t>(1, (int64_t)A.sega.size()));
         CALLOC(ctx->Ac, double, nc * nc);
         CALLOC(ctx->Ac2, double, nc * nc);
         CALLOC(ctx->gjP, double, 2 * kGJ * kGJ);
-        if ((int64_t)A.gal_el.size() >= (int64_t(1) << 27))
-            return jfm_fail(ctx, JFM_EINVAL, "too many elements for the coarse level");
-        ctx->gal_nitems = (int)A.gal_item.size();
-        ctx->gal_nupair = (int)(A.gal_upair.size() / 4);
-        const int64_t n_entries = A.gal_pptr.back();
-        CALLOC(ctx->gal_el, int32_t, std::max<int64_t>(1, (int64_t)A.gal_el.size()));
-        CALLOC(ctx->gal_gptr, int32_t, (int64_t)A.gal_gptr.size());
-        CALLOC(ctx->gal_glist, int32_t, std::max<int64_t>(1, (int64_t)A.gal_glist.size()));
-        CALLOC(ctx->gal_gq, int32_t, std::max<int64_t>(1, (int64_t)A.gal_gq.size()));
-        CALLOC(ctx->gal_gpos, int32_t, std::max<int64_t>(1, (int64_t)A.gal_gpos.size()));
-        CALLOC(ctx->gal_item, int32_t, std::max<int64_t>(1, (int64_t)A.gal_item.size()));
-        CALLOC(ctx->gal_pptr, int32_t, (int64_t)A.gal_pptr.size());
-        CALLOC(ctx->gal_upair, int32_t, std::max<int64_t>(4, (int64_t)A.gal_upair.size()));
-        CALLOC(ctx->gal_C, double, std::max<int64_t>(36, 36 * n_entries));
-        auto up = [&](int32_t *d, const std::vector<int32_t> &v) -> hipError_t {
-            return v.empty() ? hipSuccess : hipMemcpyAsync(d, v.data(), 4 * v.size(), hipMemcpyHostToDevice, s);
-        };
-        JFM_HIP(ctx, up(ctx->gal_el, A.gal_el));
-        JFM_HIP(ctx, up(ctx->gal_gptr, A.gal_gptr));
-        JFM_HIP(ctx, up(ctx->gal_glist, A.gal_glist));
-        JFM_HIP(ctx, up(ctx->gal_gq, A.gal_gq));
-        JFM_HIP(ctx, up(ctx->gal_gpos, A.gal_gpos));
-        JFM_HIP(ctx, up(ctx->gal_item, A.gal_item));
-        JFM_HIP(ctx, up(ctx->gal_pptr, A.gal_pptr));
-        JFM_HIP(ctx, up(ctx->gal_upair, A.gal_upair));
         const int64_t ldc = (nc + 255) / 256 * 256;
         ctx->ldc = ldc;
         CALLOC(ctx->Ahat32, float, nc * ldc);
@@ -1320,47 +1345,85 @@ static int coarse_prepare(jfm_ctx *ctx, int op, int coarse_nodes) {
         CALLOC(ctx->apos, int32_t, N);
         CALLOC(ctx->rA, double, 3 * N);
         CALLOC(ctx->cdA32, float, 3 * N);
-#undef CALLOC
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->node_agg, A.node_agg.data(), 4 * N, hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->agg_ptr, A.agg_ptr.data(), 4 * (A.n_agg + 1), hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->agg_nodes, A.agg_nodes.data(), 4 * N, hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->agg_color, A.color.data(), 4 * A.n_agg, hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->partner, A.partner.data(), 4 * A.partner.size(), hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->cd64, A.cd.data(), 8 * 3 * N, hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->cd32, cd32.data(), 4 * 3 * N, hipMemcpyHostToDevice, s));
-        std::vector<double> cdA(3 * N);
-        for (int64_t k = 0; k < N; ++k)
-            for (int c = 0; c < 3; ++c) cdA[3 * k + c] = A.cd[3 * (size_t)A.agg_nodes[k] + c];
-        std::vector<float> cdA32(cdA.begin(), cdA.end());
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->cdA64, cdA.data(), 8 * 3 * N, hipMemcpyHostToDevice, s));
-        {
-            std::vector<int32_t> apos(N);
-            for (int64_t k = 0; k < N; ++k) apos[A.agg_nodes[k]] = (int32_t)k;
-            JFM_HIP(ctx, hipMemcpyAsync(ctx->apos, apos.data(), 4 * N, hipMemcpyHostToDevice, s));
-            JFM_HIP(ctx, hipStreamSynchronize(s));  // apos goes out of scope
-        }
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->cdA32, cdA32.data(), 4 * 3 * N, hipMemcpyHostToDevice, s));
+        JFM_HIP(ctx, up(ctx->node_agg, A.node_agg));
+        JFM_HIP(ctx, up(ctx->agg_ptr, A.agg_ptr));
+        JFM_HIP(ctx, up(ctx->agg_nodes, A.agg_nodes));
+        JFM_HIP(ctx, up(ctx->cd64, A.cd));
+        JFM_HIP(ctx, up(ctx->Rinv, A.Rinv));
+        JFM_HIP(ctx, up(ctx->dropped, A.dropped));
         JFM_HIP(ctx, hipMemsetAsync(ctx->wc32, 0, 4 * ldc, s));  // padding stays zero
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->Rinv, A.Rinv.data(), 8 * A.Rinv.size(), hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->dropped, A.dropped.data(), 4 * nc, hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->ecol, A.ecol.data(), 4 * A.ecol.size(), hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->ncol, A.ncol.data(), 4 * A.ncol.size(), hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->segb, A.segb.data(), 4 * A.segb.size(), hipMemcpyHostToDevice, s));
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->csub_ptr, A.csub_ptr.data(), 4 * A.csub_ptr.size(), hipMemcpyHostToDevice, s));
-        if (!A.csub.empty())
-            JFM_HIP(ctx, hipMemcpyAsync(ctx->csub, A.csub.data(), 4 * A.csub.size(), hipMemcpyHostToDevice, s));
-        if (!A.sega.empty())
-            JFM_HIP(ctx, hipMemcpyAsync(ctx->sega, A.sega.data(), 4 * A.sega.size(), hipMemcpyHostToDevice, s));
+        k_agg_order<<<nblk(N), kBlock, 0, s>>>((int)N, ctx->agg_nodes, ctx->cd64, ctx->cd32, ctx->cdA64, ctx->cdA32, ctx->apos);
+        JFM_HIP(ctx, hipGetLastError());
+    }
+    if (need_gal) {
+        galerkin_lists(ctx, ctx->h_node_agg, (int)ctx->n_agg,
+                       agg_adjacency(ctx->h_conn, ctx->n_el, ctx->npe, ctx->h_node_agg, (int)ctx->n_agg), fx, A);
+        if ((int64_t)A.gal_el.size() >= (int64_t(1) << 27)) {
+            (void)hipStreamSynchronize(s);  // before the host vectors go
+            jfem_coarse_release(ctx);
+            return jfm_fail(ctx, JFM_EINVAL, "too many elements for the coarse level");
+        }
+        ctx->gal_nitems = (int)A.gal_item.size();
+        ctx->gal_nupair = (int)(A.gal_upair.size() / 4);
+        const int64_t n_entries = A.gal_pptr.back();
+        CALLOC(ctx->gal_el, int32_t, A.gal_el.size());
+        CALLOC(ctx->gal_gptr, int32_t, A.gal_gptr.size());
+        CALLOC(ctx->gal_glist, int32_t, A.gal_glist.size());
+        CALLOC(ctx->gal_gq, int32_t, A.gal_gq.size());
+        CALLOC(ctx->gal_gpos, int32_t, A.gal_gpos.size());
+        CALLOC(ctx->gal_item, int32_t, A.gal_item.size());
+        CALLOC(ctx->gal_pptr, int32_t, A.gal_pptr.size());
+        CALLOC(ctx->gal_upair, int32_t, A.gal_upair.size());
+        CALLOC(ctx->gal_C, double, std::max<int64_t>(36, 36 * n_entries));
+        JFM_HIP(ctx, up(ctx->gal_el, A.gal_el));
+        JFM_HIP(ctx, up(ctx->gal_gptr, A.gal_gptr));
+        JFM_HIP(ctx, up(ctx->gal_glist, A.gal_glist));
+        JFM_HIP(ctx, up(ctx->gal_gq, A.gal_gq));
+        JFM_HIP(ctx, up(ctx->gal_gpos, A.gal_gpos));
+        JFM_HIP(ctx, up(ctx->gal_item, A.gal_item));
+        JFM_HIP(ctx, up(ctx->gal_pptr, A.gal_pptr));
+        JFM_HIP(ctx, up(ctx->gal_upair, A.gal_upair));
+    }
+    if (need_probe) {
+        std::vector<int32_t> slot((size_t)ctx->npe * ctx->n_el);
+        JFM_HIP(ctx, hipMemcpyAsync(slot.data(), ctx->inc_slot, 4 * slot.size(), hipMemcpyDeviceToHost, s));
+        JFM_HIP(ctx, hipStreamSynchronize(s));
+        if (int rc = probe_lists(ctx, ctx->h_node_agg, (int)ctx->n_agg, slot, A)) {
+            jfem_coarse_release(ctx);
+            return jfm_fail(ctx, rc, "aggregate colouring is not distance-2");
+        }
+        ctx->ncolor = A.ncolor;
+        CALLOC(ctx->agg_color, int32_t, A.color.size());
+        CALLOC(ctx->partner, int32_t, A.partner.size());
+        CALLOC(ctx->ecol, int32_t, A.ecol.size());
+        CALLOC(ctx->ncol, int32_t, A.ncol.size());
+        CALLOC(ctx->segb, int32_t, A.segb.size());
+        CALLOC(ctx->csub_ptr, int32_t, A.csub_ptr.size());
+        CALLOC(ctx->csub, int32_t, A.csub.size());
+        CALLOC(ctx->sega, int32_t, A.sega.size());
+        JFM_HIP(ctx, up(ctx->agg_color, A.color));
+        JFM_HIP(ctx, up(ctx->partner, A.partner));
+        JFM_HIP(ctx, up(ctx->ecol, A.ecol));
+        JFM_HIP(ctx, up(ctx->ncol, A.ncol));
+        JFM_HIP(ctx, up(ctx->segb, A.segb));
+        JFM_HIP(ctx, up(ctx->csub_ptr, A.csub_ptr));
+        JFM_HIP(ctx, up(ctx->csub, A.csub));
+        JFM_HIP(ctx, up(ctx->sega, A.sega));
         ctx->h_ecol_ptr = A.ecol_ptr;
         ctx->h_ncol_ptr = A.ncol_ptr;
         ctx->h_cseg = A.cseg;
-        JFM_HIP(ctx, hipStreamSynchronize(s));
+    }
+#undef CALLOC
+    if (fresh || need_gal || need_probe) JFM_HIP(ctx, hipStreamSynchronize(s));  // the host vectors go out of scope
+    ctx->gal_lists = ctx->gal_lists || need_gal;
+    ctx->probe_lists = ctx->probe_lists || need_probe;
+    if (fresh) {
         ctx->coarse_built_nodes = coarse_nodes;
         ++ctx->coarse_gen;
     }
     const bool tangent = op == JFM_OP_TANGENT;
     if (tangent && !ctx->has_state) return jfm_fail(ctx, JFM_ESTATE, "tangent coarse level needs a state");
-    if (coarse_probe(tangent) && !ctx->pv6) {
+    if (probe && !ctx->pv6) {
         // probe vectors: zero outside the rows and slots each colour writes
         const int64_t nslots = 3 * (int64_t)ctx->npe * ctx->n_el;
         ctx->pv6 = jfm_alloc<double>(ctx, 6 * 3 * N);
@@ -1391,10 +1454,12 @@ int jfem_coarse_setup(jfm_ctx *ctx, int op, int coarse_nodes, double *ms, bool l
         return rc;
     }
     // each part is the same launch sequence every time for a given
-    // aggregation and operator, so it is captured once as a HIP graph
+    // aggregation and operator, so the second build captures it as a HIP graph
     const bool tangent = op == JFM_OP_TANGENT;
+    ++ctx->coarse_built;
     auto run = [&](hipGraphExec_t &ex, int &gen, auto &&seq) -> hipError_t {
-        if (!jfem_use_graphs()) return seq();
+        // (capture and instantiation cost more than the launches they save once)
+        if (!jfem_use_graphs() || ctx->coarse_built < 2) return seq();
         if (ex && gen != ctx->coarse_gen) {
             (void)hipGraphExecDestroy(ex);
             ex = nullptr;

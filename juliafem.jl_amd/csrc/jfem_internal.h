@@ -258,6 +258,9 @@ struct jfm_ctx {
     std::vector<double> h_X;       // host copy of the coordinates (aggregation)
     int coarse_built_nodes = 0;    // coarse_nodes the aggregation was built for
     int coarse_gen = 0;            // bumped per aggregation (keys captured graphs)
+    std::vector<int32_t> h_node_agg;  // the aggregation's host copy
+    bool gal_lists = false, probe_lists = false;  // the lists of the two setups, made when first needed
+    int coarse_built = 0;          // coarse levels built on this aggregation
     bool coarse_ready = false;     // Ahat holds a coarse level
     int coarse_tag = -1;           // operator it was built from: 0 K, 1 the tangent
     int64_t n_agg = 0, nc = 0;
