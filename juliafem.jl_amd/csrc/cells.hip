@@ -408,13 +408,13 @@ int jfem_cells_coarse(jfm_ctx *ctx, int max_entries) {
     return JFM_OK;
 }
 
-int jfem_cells_systems(jfm_ctx *ctx, int m) {
+int jfem_cells_systems(jfm_ctx *ctx, int m, int words) {
     auto &C = ctx->cells;
     if (m <= C.systems) return JFM_OK;
     for (void *q : {(void *)C.part, (void *)C.words, (void *)C.S}) jfm_free(ctx, q);
     C.systems = 0;
     C.part = jfm_alloc<double>(ctx, (int64_t)m * 4 * std::max(1, C.nslot));
-    C.words = jfm_alloc<uint64_t>(ctx, (int64_t)m * kPersistWords * (C.npatch + 256));
+    C.words = jfm_alloc<uint64_t>(ctx, (int64_t)m * words);
     C.S = jfm_alloc<PcgScalars>(ctx, m);
     if (!C.part || !C.words || !C.S) return jfm_fail(ctx, JFM_ENOMEM, "resident PCG allocation failed");
     C.systems = m;

@@ -457,7 +457,6 @@ bool jfem_patch_defer_shared(const jfm_ctx *ctx, int op);
 // persist.hip: the whole PCG in one resident kernel, one workgroup per patch
 // (meshes of up to kPersistPatches patches).
 constexpr int kPersistPatches = 256;
-constexpr int kPersistWords = 6;  // exchange words per workgroup (and 256 more)
 // elements of a patch, its workgroup's threads (and most nodes), the row
 // stride of its LDS image of the element terms
 // Geometric factors in the element order perm (gfQ32: folded ones too, or null).
@@ -474,8 +473,8 @@ template <typename T> bool jfem_persist_maybe(const jfm_ctx *ctx, int op);
 // With coarse, of the two-level form on the current aggregation.
 template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys, bool coarse = false);
 int jfem_cells_coarse(jfm_ctx *ctx, int max_entries);
-// makes room for m systems
-int jfem_cells_systems(jfm_ctx *ctx, int m);
+// makes room for m systems of `words` exchange words
+int jfem_cells_systems(jfm_ctx *ctx, int m, int words);
 // heat: maps the convection faces to elements (ctx->heat_resident)
 int jfem_heat_faces(jfm_ctx *ctx);
 // Solves K x = b (r0 null) or continues from x with its residual r0; the

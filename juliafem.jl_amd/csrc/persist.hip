@@ -3,8 +3,10 @@
 // On meshes of up to a few hundred patches an iteration launched kernel by
 // kernel is bound by its launches and dependent loads, not by its work: 24 us
 // per iteration at 139,587 DOFs (FP64, patch operator, shared nodes, update,
-// direction), 11.4 us at 1,575 DOFs; resident they take 13.2 and 3.8 us
-// (solves 73.9 -> 39.4 ms and 6.9 -> 2.3 ms).  Here one workgroup per patch stays
+// direction), 11.4 us at 1,575 DOFs; resident they take 11.1 and 3.5 us
+// (solves 73.9 -> 33.2 ms and 6.9 -> 2.1 ms).  What is left is latency: at
+// 139,587 DOFs 29,000 cycles, of which the element products and nodal sums take
+// 5,000, the exchanges 18,000.  Here one workgroup per patch stays
 // on its CU for the whole solve.  A patch's node vectors (r, x, z in
 // registers, p in LDS), its connectivity and its geometric factors never
 // leave the CU; what crosses workgroups in an iteration is the partial sums
@@ -28,8 +30,7 @@
 // one workgroup, so no cache is flushed or invalidated.  A scalar travels as
 // 64-bit words of 32 payload bits and a 32-bit epoch (the iteration): a word
 // proves itself current, so one store and one polling load are barrier,
-// transfer and reduction in one.  Words of one kind are contiguous over the
-// workgroups: a wave's poll is eight 64-byte requests.  The shared nodes'
+// transfer and reduction in one.  The shared nodes'
 // partials are stored first, waited for (vmcnt 0 in every wave, then the block
 // barrier), and only then is the scalar published that their readers wait
 // for; they move as one or two wide accesses per node, since such accesses
@@ -172,41 +173,56 @@ __device__ __forceinline__ double wave_total(double v) {
 
 // All-reduce of NV doubles over the workgroups: v in: the thread's share, out:
 // the grid's sums, the same bits in every thread of every workgroup; false
-// when a wait gave up.  Up to 16 workgroups read each other's words; more form
+// when a wait gave up.  Up to 16 workgroups read each other's entries; more form
 // groups of 16 (workgroup >> 4) whose first workgroup sums the group's values
-// and publishes the sum once per group, and every workgroup reads its group's
+// and publishes the sum once per 8 workgroups, and every workgroup reads its
 // copy of the groups' sums: uncached requests to one line are served one after
 // the other, so no line may have more than a few readers.  (240 workgroups
-// reading one set of words, or all of them, took 4-6 us per exchange.)  One
-// wave polls: lane 16 k + m reads value k of member m, so a sum over members
-// is a row sum.  `words` holds 2 NV rows of nwg words, then 16 copies of 2 NV
-// rows of 16.  Calls
-// that follow each other without a block barrier use different `sh` (a wave
-// may still read it when the next one starts).
+// reading one set of words, or all of them, took 4-6 us per exchange.)  A value
+// is an entry of two words, and the NV entries of a workgroup lie side by side,
+// one request to store and, with the neighbours', one to read (as rows of single
+// words, which is four requests for two values, an iteration of 240 workgroups
+// took 0.9 us longer; one hop with 16 copies of all entries, 0.4 us longer than
+// that).  One wave polls:
+// lane 16 k + m reads value k of member m, so a sum over members is a row sum.
+// Calls that follow each other without a block barrier use different `sh` (a
+// wave may still read it when the next one starts).
+constexpr int kGroup = 16, kCopy = 8;
 template <int NV> struct GridSumLds { double a[NV][16], b[NV]; };
-constexpr int kGroup = 16;
-static_assert(kPersistPatches <= kGroup * kGroup, "two levels");
+static_assert(kPersistPatches <= kGroup * kGroup && kPersistPatches / kCopy <= 32, "two levels, copies x values in a wave");
 
-// the sum over n <= 16 members' words, in every lane of row k (value k)
-template <int NV>
-__device__ __forceinline__ double sum_members(const uint64_t *words, int stride, int n, uint32_t epoch, int *bad) {
-    const int lane = (int)threadIdx.x & 63, k = lane >> 4, m = lane & 15;
-    double v = 0.0;
-    if (k < NV && m < n) {
-        uint32_t bits[2];
-        if (!poll_words<2>(words + (size_t)(2 * k) * stride + m, stride, epoch, bits)) *bad = 1;
-        v = __longlong_as_double((long long)((uint64_t)bits[1] << 32 | bits[0]));
-    }
-    return row_sum(v);
+// words of n workgroups: their entries, then the copies of the groups' sums
+__host__ __device__ constexpr int grid_words(int nv, int n) {
+    return 2 * nv * (n + (n > kGroup ? (n + kCopy - 1) / kCopy * kGroup : 0));
 }
-// lanes 0 and 1 of row k publish its value
-template <int NV>
-__device__ __forceinline__ void put_rows(uint64_t *words, int stride, int at, uint32_t epoch, double v) {
-    const int lane = (int)threadIdx.x & 63, k = lane >> 4, h = lane & 15;
-    if (k < NV && h < 2) {
+
+struct Entries {  // past the L2, as the partials
+    __amdgpu_buffer_rsrc_t rs;
+    __device__ __forceinline__ Entries(uint64_t *p, int words)
+        : rs(__builtin_amdgcn_make_buffer_rsrc(p, 0, 8 * words, 0x00027000)) {}
+    __device__ __forceinline__ void put(int i, uint32_t epoch, double v) const {
         const uint64_t b = (uint64_t)__double_as_longlong(v);
-        put_word(words + (size_t)(2 * k + h) * stride + at, epoch, (uint32_t)(h ? b >> 32 : b));
+        const u32x4 a = {(uint32_t)b, epoch, (uint32_t)(b >> 32), epoch};
+        __builtin_amdgcn_raw_buffer_store_b128(a, rs, 16 * i, 0, kSc1);
     }
+    // polls until both words of entry i are of this epoch
+    __device__ __forceinline__ double get(int i, uint32_t epoch, int *bad) const {
+        for (int k = 0; k < kMaxPolls; ++k) {
+            const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * i, 0, kSc1);
+            if (a.y == epoch && a.w == epoch) return __longlong_as_double((long long)((uint64_t)a.z << 32 | a.x));
+            __builtin_amdgcn_s_sleep(1);
+            asm volatile("" ::: "memory");  // the load is not to leave the loop
+        }
+        *bad = 1;
+        return 0.0;
+    }
+};
+
+// the sum over n <= 16 members' entries from `first` on, in every lane of row k (value k)
+template <int NV>
+__device__ __forceinline__ double sum_members(const Entries &en, int first, int n, uint32_t epoch, int *bad) {
+    const int lane = (int)threadIdx.x & 63, k = lane >> 4, m = lane & 15;
+    return row_sum(k < NV && m < n ? en.get((first + m) * NV + k, epoch, bad) : 0.0);
 }
 
 template <int NV, int NT>
@@ -225,26 +241,20 @@ __device__ __forceinline__ bool grid_sum(double (&v)[NV], uint64_t *words, int w
         const int k = lane >> 4, m = lane & 15;
         double s = row_sum(k < NV && m < kW ? sh.a[k < NV ? k : 0][m] : 0.0);  // row k: the block's value k
         if (nwg > 1) {
-            put_rows<NV>(words, nwg, wg, epoch, s);
+            const Entries en(words, grid_words(NV, nwg));
+            if (k < NV && m == 0) en.put(wg * NV + k, epoch, s);
             if (nwg > kGroup) {
-                uint64_t *top = words + (size_t)(2 * NV) * nwg;
+                const int g = wg / kGroup, copies = (nwg + kCopy - 1) / kCopy;
                 if (wg % kGroup == 0) {
-                    s = sum_members<NV>(words + wg, nwg, min(kGroup, nwg - wg), epoch, bad);
-                    // lane 16 r + c: word row r of copy c
-                    double mine = 0.0;
-#pragma unroll
-                    for (int q = 0; q < NV; ++q) {
-                        const double vq = lane_of(s, 16 * q);
-                        mine = k >> 1 == q ? vq : mine;
-                    }
-                    const uint64_t b = (uint64_t)__double_as_longlong(mine);
-                    if (k < 2 * NV)
-                        put_word(top + (size_t)m * (2 * NV * kGroup) + k * kGroup + wg / kGroup, epoch,
-                                 (uint32_t)(k & 1 ? b >> 32 : b));
+                    s = sum_members<NV>(en, wg, min(kGroup, nwg - wg), epoch, bad);
+                    double mine = lane_of(s, 0);
+                    if constexpr (NV == 2) mine = lane & 1 ? lane_of(s, 16) : mine;
+                    const int c = lane / NV;  // copy, value lane % NV
+                    if (c < copies) en.put((nwg + c * kGroup + g) * NV + lane % NV, epoch, mine);
                 }
-                s = sum_members<NV>(top + (size_t)(wg / kGroup) * (2 * NV * kGroup), kGroup, (nwg + kGroup - 1) / kGroup, epoch, bad);
+                s = sum_members<NV>(en, nwg + wg / kCopy * kGroup, (nwg + kGroup - 1) / kGroup, epoch, bad);
             } else {
-                s = sum_members<NV>(words, nwg, nwg, epoch, bad);
+                s = sum_members<NV>(en, 0, nwg, epoch, bad);
             }
         }
         if (k < NV && m == 0) sh.b[k] = s;
@@ -280,7 +290,7 @@ template <typename T> struct PersistArgs {
     T *x;
     T *part;                  // the shared nodes' partials, 4 values per slot
     int nslot;
-    uint64_t *words;          // the scalars': 2 rows (B), then 4 (C), of npatch + 256
+    uint64_t *words;          // the scalars' entries, B and then C
     double rtol2;
     int maxit;
     PcgScalars *S;
@@ -838,8 +848,7 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
     const int k = p * EL + el;
     const bool has_el = el < EL && k < A.n_el;
     const int lb = NT * p, nn = A.pn_n[p];
-    const int rows = nwg + kGroup * kGroup;
-    uint64_t *wordsB = A.words + (size_t)sys * kPersistWords * rows, *wordsC = wordsB + 2 * (size_t)rows;
+    uint64_t *wordsB = A.words + (size_t)sys * (grid_words(1, nwg) + grid_words(2, nwg)), *wordsC = wordsB + grid_words(1, nwg);
     PcgScalars *S = A.S + sys;
     const Partials<T> part(A.part + (size_t)sys * 4 * A.nslot, A.nslot);
     const T *bvec = A.b + sys * A.ss;
@@ -942,26 +951,31 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
 #pragma unroll
             for (int c = 0; c < 3; ++c) ps[3 * t + c] = fx >> c & 1u ? T(0) : r[c];
             __syncthreads();
-            for (int e = wv; e < ne; e += NT / 64) {
-                double w[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+            // a wave per aggregate and half (a patch has owned nodes in three or four)
+            for (int u = wv; u < 2 * ne; u += NT / 64) {
+                const int e = u >> 1, h = u & 1;
+                double w[3] = {0.0, 0.0, 0.0};
                 for (int i = co.start[e] + lane; i < co.start[e + 1]; i += 64) {
                     const int l = 3 * (int)co.list[i];
                     const double y0 = ps[l], y1 = ps[l + 1], y2 = ps[l + 2];
-                    const double d0 = co.d[l], d1 = co.d[l + 1], d2 = co.d[l + 2];
-                    w[0] += y0;
-                    w[1] += y1;
-                    w[2] += y2;
-                    w[3] += d1 * y2 - d2 * y1;
-                    w[4] += d2 * y0 - d0 * y2;
-                    w[5] += d0 * y1 - d1 * y0;
+                    if (h == 0) {
+                        w[0] += y0;
+                        w[1] += y1;
+                        w[2] += y2;
+                    } else {
+                        const double d0 = co.d[l], d1 = co.d[l + 1], d2 = co.d[l + 2];
+                        w[0] += d1 * y2 - d2 * y1;
+                        w[1] += d2 * y0 - d0 * y2;
+                        w[2] += d0 * y1 - d1 * y0;
+                    }
                 }
                 double mine = 0.0;
 #pragma unroll
-                for (int c = 0; c < 6; ++c) {
+                for (int c = 0; c < 3; ++c) {
                     const double v = wave_total(w[c]);
                     mine = lane == c ? v : mine;
                 }
-                if (lane < 6) put_shared(A.wpart + 6 * (size_t)co.slot[e] + lane, mine);
+                if (lane < 3) put_shared(A.wpart + 6 * (size_t)co.slot[e] + 3 * h + lane, mine);
             }
             stores_done();  // before the block barrier in grid_sum, hence before its words
         }
@@ -1230,7 +1244,7 @@ template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys, bo
     }
     int m = want;  // as many systems side by side as fit, a divisor of those asked for
     while (m > 1 && (want % m || m * np > (int64_t)per_cu * ctx->cus)) --m;
-    if (int rc = jfem_cells_systems(ctx, m)) return rc;
+    if (int rc = jfem_cells_systems(ctx, m, grid_words(1, (int)np) + grid_words(2, (int)np))) return rc;
     *nsys = m;
     return JFM_OK;
 }
@@ -1295,7 +1309,7 @@ hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, c
     A.S = nsys > 1 ? C.S : ctx->S;
     A.nsys = nsys;
     A.ss = ss;
-    const int nw = nsys * kPersistWords * (C.npatch + kGroup * kGroup);
+    const int nw = nsys * (grid_words(1, C.npatch) + grid_words(2, C.npatch));
     k_persist_clear<<<(std::max(nw, nz) + 255) / 256, 256, 0, ctx->stream>>>(nw, C.words, nz, C.zw, nsys, A.S);
     void *args[] = {&A};
     return hipLaunchKernel(L.f, dim3(nsys * C.npatch), dim3(kNT), args, 0, ctx->stream);
