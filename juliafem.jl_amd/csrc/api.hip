@@ -278,14 +278,14 @@ extern "C" int jfm_upload_mesh(jfm_ctx *ctx, int64_t n_nodes, const double *X, i
         JFM_HIP(ctx, hipMemcpyAsync(ctx->E, E, sizeof(double) * n_el, hipMemcpyHostToDevice, s));
         JFM_HIP(ctx, hipMemcpyAsync(ctx->nu, nu, sizeof(double) * n_el, hipMemcpyHostToDevice, s));
     }
-    int32_t *d_flags = nullptr, flags = 0, nnzb = 0;
+    int32_t *d_flags = nullptr, flags[2] = {0, 0}, nnzb = 0;
     CHECK_LAUNCH(ctx, launch_mesh_lists(ctx, scratch.p, &d_flags));
-    JFM_HIP(ctx, hipMemcpyAsync(&flags, d_flags, sizeof flags, hipMemcpyDeviceToHost, s));
+    JFM_HIP(ctx, hipMemcpyAsync(flags, d_flags, sizeof flags, hipMemcpyDeviceToHost, s));
     JFM_HIP(ctx, hipMemcpyAsync(&nnzb, ctx->brow + n_nodes, sizeof nnzb, hipMemcpyDeviceToHost, s));
     if (int rc = sync(ctx)) return rc;
     ctx->nnzb = nnzb;
-    ctx->affine = !(flags & kMeshCurved);
-    ctx->orphans = (flags & kMeshOrphans) != 0;
+    ctx->affine = flags[0] == 0;
+    ctx->orphans = flags[1];
     ctx->ngf = ctx->affine ? 1 : ctx->ngp;
     ALLOC(ctx, ctx->gf64, double, (int64_t)GF * ctx->ngf * n_el);
     ALLOC(ctx, ctx->gf32, float, (int64_t)GF * ctx->ngf * n_el);
@@ -319,6 +319,22 @@ extern "C" int jfm_upload_mesh(jfm_ctx *ctx, int64_t n_nodes, const double *X, i
     if (int rc = sync(ctx)) return rc;
     if (h_bad) return jfm_fail(ctx, JFM_ENOTSPD, "element with detJ <= 0 at a Gauss point (inverted or degenerate)");
     ctx->has_mesh = true;
+    // Meshes whose iterations are launched get the patch operator with the upload,
+    // so that the products of jfm_apply_noalloc, which may not allocate, take it
+    // too.  It needs patches for a good part of the CUs: FP64 Tet10 13.5 against
+    // 15.1 us of the two-phase form with 64 of them, 28.1 against 49.6 with 512;
+    // Hex8 (eight points: more per workgroup) 18.5 against 16.2 with 86, 19.1
+    // against 19.9 with 128, 26.1 against 33.0 with 254.  Without room for it the
+    // mesh is still good for the CSR operator.
+    const int64_t patches = (n_el + kPatchElems - 1) / kPatchElems;
+    if (jfem_patch_enabled() && !jfem_persist_maybe<double>(ctx, JFM_OP_MATFREE) && patches >= (npe == 8 ? 192 : 64)) {
+        if (jfem_patch_setup(ctx) == JFM_OK) {
+            ctx->na_part = jfm_alloc<double>(ctx, 3 * (int64_t)std::max(1, ctx->nslot));
+            ctx->patch_upload = ctx->patch_ready && ctx->na_part;
+        } else {
+            ctx->err.clear();
+        }
+    }
     return JFM_OK;
 }
 

@@ -11,52 +11,13 @@
 #include <algorithm>
 #include <vector>
 
-#include "jfem_device.h"
+#include "sort_scan.h"
 
 namespace jfem {
 
 constexpr int kCT = 512;    // threads, and the most nodes of a patch
 constexpr int kCK = 2048;   // most incidences of a patch
 enum { kCellNodes = 1, kCellShared = 2, kCellEntries = 4 };  // why a mesh does not fit
-
-// Ascending order of the n (a power of two) keys in LDS.
-template <typename K> __device__ __forceinline__ void sort_keys(K *key, int n) {
-    for (int size = 2; size <= n; size <<= 1)
-        for (int s = size >> 1; s > 0; s >>= 1) {
-            __syncthreads();
-            for (int q = (int)threadIdx.x; q < n / 2; q += kCT) {
-                const int i = 2 * q - (q & (s - 1)), j = i + s;
-                const K u = key[i], v = key[j];
-                if ((u > v) == ((i & size) == 0)) {
-                    key[i] = v;
-                    key[j] = u;
-                }
-            }
-        }
-    __syncthreads();
-}
-
-// exclusive scan over the workgroup; *total: the sum, to every thread
-__device__ __forceinline__ int scan_threads(int v, int *ws, int *total) {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    int s = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int u = __shfl_up(s, off, 64);
-        if (lane >= off) s += u;
-    }
-    if (lane == 63) ws[wid] = s;
-    __syncthreads();
-    int before = 0, all = 0;
-#pragma unroll
-    for (int w = 0; w < kCT / 64; ++w) {
-        if (w < wid) before += ws[w];
-        all += ws[w];
-    }
-    __syncthreads();
-    *total = all;
-    return before + s - v;
-}
 
 // One workgroup per patch.  Its incidences sorted by (node, element, local
 // node) give the patch's nodes and their incidences; the nodes are then ranked
@@ -72,7 +33,7 @@ __global__ __launch_bounds__(kCT) void k_cell_nodes(int n_el, int npe, int ps, i
                                                    uint16_t *__restrict__ connL, uint16_t *__restrict__ lin,
                                                    int32_t *__restrict__ psum, int32_t *__restrict__ flags) {
     __shared__ uint64_t key[kCK];
-    __shared__ int head[kCT + 1], cnt[kCT], ranked[kCT], ws[kCT / 64];
+    __shared__ int head[kCT + 1], cnt[kCT], ranked[kCT];
     const int p = blockIdx.x, t = threadIdx.x;
     const int k0 = p * ps, ne = min(ps, n_el - k0), m = ne * npe;
     int n2 = 2;
@@ -85,7 +46,7 @@ __global__ __launch_bounds__(kCT) void k_cell_nodes(int n_el, int npe, int ps, i
         }
         key[idx] = v;
     }
-    sort_keys(key, n2);
+    sort_keys<kCT>(key, n2);
     // the nodes, in ascending order: where each one's incidences start
     int first[4], heads = 0, nn;
 #pragma unroll
@@ -94,7 +55,7 @@ __global__ __launch_bounds__(kCT) void k_cell_nodes(int n_el, int npe, int ps, i
         first[j] = idx < m && (idx == 0 || key[idx] >> 32 != key[idx - 1] >> 32);
         heads += first[j];
     }
-    int h = scan_threads(heads, ws, &nn);
+    int h = block_scan<kCT>(heads, &nn);
     if (nn > kCT) {  // uniform
         if (t == 0) {
             pn_n[p] = 0;
@@ -118,7 +79,7 @@ __global__ __launch_bounds__(kCT) void k_cell_nodes(int n_el, int npe, int ps, i
     // thread t takes the node of rank t
     const int q = t < nn ? ranked[t] : 0, n = t < nn ? cnt[q] : 0, r0 = head[q];
     int all, total = 0, rank = -1;
-    const int off = scan_threads(n, ws, &all);
+    const int off = block_scan<kCT>(n, &all);
     const size_t l = (size_t)p * kCT + t;
     if (t < nn) {
         const int a = (int)(key[r0] >> 32);
@@ -152,7 +113,7 @@ __global__ __launch_bounds__(kCT) void k_cell_nodes(int n_el, int npe, int ps, i
         pn_sh[l] = total;
     }
     int owned;
-    (void)scan_threads(rank == 0 ? total : 0, ws, &owned);
+    (void)block_scan<kCT>(rank == 0 ? total : 0, &owned);
     if (t == 0) {
         pn_n[p] = nn;
         psum[p] = owned;
@@ -164,16 +125,15 @@ __global__ __launch_bounds__(kCT) void k_cell_slots(int npatch, const int32_t *_
                                                    const int32_t *__restrict__ pn_node, const int32_t *__restrict__ pn_slot,
                                                    const int32_t *__restrict__ pn_sh, const int32_t *__restrict__ psum,
                                                    int32_t *__restrict__ first, int32_t *__restrict__ nslot) {
-    __shared__ int ws[kCT / 64];
     const int p = blockIdx.x, t = threadIdx.x;
     int before = 0, part;
     for (int q0 = 0; q0 < p; q0 += kCT) {
-        (void)scan_threads(q0 + t < p ? psum[q0 + t] : 0, ws, &part);
+        (void)block_scan<kCT>(q0 + t < p ? psum[q0 + t] : 0, &part);
         before += part;
     }
     const size_t l = (size_t)p * kCT + t;
     const int n = t < pn_n[p] && pn_slot[l] == 0 ? pn_sh[l] : 0;
-    const int o = before + scan_threads(n, ws, &part);
+    const int o = before + block_scan<kCT>(n, &part);
     if (n) first[pn_node[l]] = o;
     if (p == npatch - 1 && t == 0) *nslot = before + part;
 }
@@ -197,7 +157,6 @@ __global__ __launch_bounds__(kCT) void k_cell_entries(int n_agg, int max_entries
                                                      int32_t *__restrict__ cn_ptr, uint16_t *__restrict__ cn_list,
                                                      int16_t *__restrict__ table, int32_t *__restrict__ flags) {
     __shared__ uint32_t key[kCT];
-    __shared__ int ws[kCT / 64];
     const int p = blockIdx.x, t = threadIdx.x;
     const size_t l = (size_t)p * kCT + t;
     uint32_t v = ~0u;
@@ -207,12 +166,12 @@ __global__ __launch_bounds__(kCT) void k_cell_entries(int n_agg, int max_entries
         if (slot < 0 || slot == pn_sh[l] >> 5) v = (uint32_t)g << 16 | (uint32_t)t;
     }
     key[t] = v;
-    sort_keys(key, kCT);
+    sort_keys<kCT>(key, kCT);
     const uint32_t k = key[t];
     const bool head = k != ~0u && (t == 0 || key[t - 1] >> 16 != k >> 16);
     int ne, nown;
-    const int e = scan_threads(head, ws, &ne);
-    (void)scan_threads(k != ~0u, ws, &nown);
+    const int e = block_scan<kCT>(head, &ne);
+    (void)block_scan<kCT>(k != ~0u, &nown);
     if (ne > max_entries) {  // uniform
         if (t == 0) {
             ce_n[p] = 0;
@@ -235,13 +194,12 @@ __global__ __launch_bounds__(kCT) void k_cell_entries(int n_agg, int max_entries
 // One workgroup, thread g for aggregate g: its entries' slots, ascending patch.
 __global__ __launch_bounds__(kCT) void k_cell_agg_slots(int npatch, int n_agg, int max_entries, const int16_t *__restrict__ table,
                                                        int32_t *__restrict__ as_ptr, int32_t *__restrict__ ce_slot) {
-    __shared__ int ws[kCT / 64];
     const int g = threadIdx.x;
     int n = 0, total;
     if (g < n_agg)
 #pragma unroll 8
         for (int p = 0; p < npatch; ++p) n += table[(size_t)p * n_agg + g] >= 0;
-    int s = scan_threads(n, ws, &total);
+    int s = block_scan<kCT>(n, &total);
     if (g < n_agg) {
         as_ptr[g] = s;
 #pragma unroll 8
@@ -254,10 +212,8 @@ __global__ __launch_bounds__(kCT) void k_cell_agg_slots(int npatch, int n_agg, i
 }
 
 // ------------------------------------------------------------------- host ---
-namespace {
-
 // the bits of v at every third position
-uint64_t spread16(uint64_t v) {
+static uint64_t spread16(uint64_t v) {
     v &= 0xffff;
     v = (v | v << 16) & 0x0000ff0000ffULL;
     v = (v | v << 8) & 0x00f00f00f00fULL;
@@ -299,8 +255,6 @@ std::vector<int32_t> morton_order(const std::vector<int32_t> &conn, const std::v
     }
     return perm;
 }
-
-}  // namespace
 
 // The resident PCG's patches, once per mesh; cells.usable tells whether the
 // mesh fits.

@@ -160,7 +160,7 @@ struct jfm_ctx {
     int64_t N = 0, n_el = 0, ndof = 0;
     int npe = 0, ngp = 0, npair = 0;
     bool affine = false, has_mesh = false;
-    bool orphans = false;         // a node of no element
+    int orphans = 0;              // nodes of no element
     bool nu_uniform = false;      // every element has Poisson's ratio nu0
     double nu0 = 0.0;
     std::vector<int32_t> h_conn;  // n_el x npe (element-major), 0-based
@@ -299,6 +299,8 @@ struct jfm_ctx {
     int gal_nitems = 0, gal_nupair = 0;
     // patch operator (patch.hip): elements in Morton order, 480 per patch
     bool patch_ready = false;
+    bool patch_upload = false;  // made with the upload
+    double *na_part = nullptr;  // partial sums of jfm_apply_noalloc, which may overlap other calls
     int npatch = 0, npn = 0, nbnode = 0, nslot = 0;
     int32_t *eperm = nullptr;                 // patch order -> element id
     int32_t *connP = nullptr;                 // npe x n_el, patch order
@@ -388,10 +390,9 @@ namespace jfem {
 hipError_t launch_geom_factors(jfm_ctx *ctx, int *d_bad);
 // Incidences, sorted pattern rows and contributions of the uploaded mesh
 // (mesh_lists.hip) into ctx->conn, inc*, brow and contrib; scratch of
-// mesh_lists_scratch() int32.  *flags: a device word of kMesh bits.  Then, with
+// mesh_lists_scratch() int32.  *flags: two device words, whether an element's J
+// is not constant and the number of nodes of no element.  Then, with
 // bcol, blk_row and cptr allocated for brow[N] blocks, the pattern.
-constexpr int kMeshOrphans = 1;  // a node of no element
-constexpr int kMeshCurved = 2;   // an element whose J is not constant
 int64_t mesh_lists_scratch(int64_t N, int64_t n_el, int npe);
 hipError_t launch_mesh_lists(jfm_ctx *ctx, int32_t *scratch, int32_t **flags);
 hipError_t launch_pattern_write(jfm_ctx *ctx, const int32_t *scratch);
@@ -433,6 +434,7 @@ hipError_t launch_nh_block_jacobi(jfm_ctx *ctx, const double *u, double *M64, fl
 // patch.hip: fused K.u over element patches (JFM_OP_MATFREE, and JFM_OP_EBE
 // when the element matrices are stored in the patch order)
 bool jfem_patch_enabled();  // false when JFEM_PATCH=0 (two-phase operator)
+constexpr int kPatchElems = 480;  // elements of a patch
 int jfem_patch_setup(jfm_ctx *ctx);
 void jfem_patch_release(jfm_ctx *ctx);
 // whether `op` runs in the patch form on this context
@@ -460,6 +462,8 @@ constexpr int kPersistPatches = 256;
 // elements of a patch, its workgroup's threads (and most nodes), the row
 // stride of its LDS image of the element terms
 // Geometric factors in the element order perm (gfQ32: folded ones too, or null).
+// Elements along a Morton curve of their centroids (cells.hip).
+std::vector<int32_t> morton_order(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int npe);
 hipError_t launch_patch_factors(jfm_ctx *ctx, const int32_t *perm, double *gf64, float *gf32, float *gfQ32);
 struct PersistGeometry { int elems = 0, threads = 0, stride = 0; };
 int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g);

@@ -12,7 +12,7 @@
 // Reference: the node -> element map of ext/JuliaFEMCUDAExt.jl:179-193.
 #include <algorithm>
 
-#include "jfem_device.h"
+#include "sort_scan.h"
 
 namespace jfem {
 
@@ -20,29 +20,6 @@ namespace jfem {
 // Exclusive prefix sums of int32: per-block sums of kScan values, their scan by
 // one workgroup, and the blocks again with their offsets.
 constexpr int kScan = 4 * kBlock;
-
-// exclusive scan over the block's threads; *total: the sum, to every thread
-template <int NT> __device__ __forceinline__ int block_scan(int v, int *total) {
-    __shared__ int ws[NT / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    int s = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int u = __shfl_up(s, off, 64);
-        if (lane >= off) s += u;
-    }
-    if (lane == 63) ws[wid] = s;
-    __syncthreads();
-    int before = 0, all = 0;
-#pragma unroll
-    for (int w = 0; w < NT / 64; ++w) {
-        if (w < wid) before += ws[w];
-        all += ws[w];
-    }
-    __syncthreads();
-    *total = all;
-    return before + s - v;
-}
 
 __global__ __launch_bounds__(kBlock) void k_scan_sums(int n, const int32_t *__restrict__ in, int32_t *__restrict__ bsum) {
     const int64_t i0 = (int64_t)blockIdx.x * kScan + 4 * threadIdx.x;
@@ -222,7 +199,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_row_sort(int N, const int32_
     for (int off = 32; off > 0; off >>= 1) distinct += __shfl_xor(distinct, off, 64);
     if (lane == 0 && a < N) {
         rowlen[a] = distinct;
-        if (m == 0) atomicOr(flags, kMeshOrphans);
+        if (m == 0) atomicAdd(flags + 1, 1);  // a node of no element
     }
 }
 
@@ -291,7 +268,7 @@ __global__ __launch_bounds__(kBlock) void k_not_affine(int n_el, const int32_t *
                 bad = bad || fabs(P[i][k] - v) > tol * 8;
             }
     }
-    if (bad) atomicOr(flags, kMeshCurved);
+    if (bad) flags[0] = 1;
 }
 
 // ----------------------------------------------------------------- launches ---

@@ -2,8 +2,8 @@
 // device allocation, for callers that cannot allocate (code under HIP graph
 // capture, fixed-memory serving loops).
 //
-// The two-phase operator's element results (3 npe n_el values per K.u) and,
-// in FP32, the converted input and output vectors live in `scratch`, one
+// The two-phase operator's element results (3 npe n_el values per K.u) and, in
+// FP32, the converted input and output vectors live in `scratch`, one
 // file-scope device array per GPU of kScratchBytes.  Host code never passes
 // the array's name to a kernel: jfem_noalloc_init() looks up its device
 // address once per device (with that device current) and every launch uses
@@ -28,6 +28,22 @@ std::mutex g_mu;
 unsigned char *g_scratch[kMaxDevices] = {};  // device address of `scratch`, per device
 
 size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
+
+// y = K x with the element results in ye, or by the patch operator with the
+// context's buffer of partial sums for these calls.  The patches are taken where
+// the upload made them and not where an earlier call did, so that a mesh always
+// gives the same bits.
+template <typename T> hipError_t product(jfm_ctx *ctx, int op, const T *x, T *y, T *ye) {
+    if (ctx->patch_upload && jfem_patch_form(ctx, op)) {
+        double *const part = ctx->bpart;
+        ctx->bpart = ctx->na_part;
+        const hipError_t e = launch_patch_apply<T>(ctx, op, x, y, nullptr, nullptr, nullptr, nullptr);
+        ctx->bpart = part;
+        return e;
+    }
+    const hipError_t e = launch_elem_into<T>(ctx, op, x, ye);
+    return e == hipSuccess ? launch_gather<T>(ctx, ye, ctx->fixed, y, nullptr, nullptr, nullptr, nullptr) : e;
+}
 }  // namespace
 
 // Called by jfm_create with ctx->device current.
@@ -71,16 +87,13 @@ extern "C" int jfm_apply_noalloc(jfm_ctx *ctx, int32_t op, int32_t precision, co
     if (stream) ctx->stream = (hipStream_t)stream;
     hipError_t e = hipSuccess;
     if (precision == JFM_FP64) {
-        double *ye = (double *)base;
-        e = launch_elem_into<double>(ctx, op, x, ye);
-        if (e == hipSuccess) e = launch_gather<double>(ctx, ye, ctx->fixed, y, nullptr, nullptr, nullptr, nullptr);
+        e = product<double>(ctx, op, x, y, (double *)base);
     } else {
         float *x32 = (float *)base;
         float *y32 = (float *)(base + align256(sizeof(float) * n));
         float *ye = (float *)(base + 2 * align256(sizeof(float) * n));
         e = launch_convert<double, float>(ctx, x, x32, n, 1.0);
-        if (e == hipSuccess) e = launch_elem_into<float>(ctx, op, x32, ye);
-        if (e == hipSuccess) e = launch_gather<float>(ctx, ye, ctx->fixed, y32, nullptr, nullptr, nullptr, nullptr);
+        if (e == hipSuccess) e = product<float>(ctx, op, x32, y32, ye);
         if (e == hipSuccess) e = launch_convert<float, double>(ctx, y32, y, n, 1.0);
     }
     ctx->stream = saved;

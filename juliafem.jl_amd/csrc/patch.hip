@@ -25,8 +25,8 @@
 #include <vector>
 
 #include "ebe_element.h"
-#include "jfem_device.h"
 #include "mf_element.h"
+#include "sort_scan.h"
 
 namespace jfem {
 
@@ -35,10 +35,7 @@ namespace jfem {
 // best a multiple of 2 x 256: 480 gives exactly 512 patches for 245,760
 // elements and 4,096 for 1,966,080 (512 elements: 480 patches, 32 CUs with
 // one, and 4% slower).
-#ifndef JFEM_PATCH_ELEMS
-#define JFEM_PATCH_ELEMS 480
-#endif
-constexpr int kPatch = JFEM_PATCH_ELEMS;
+constexpr int kPatch = kPatchElems;
 
 // Fused element product and patch-local nodal sums.  LDS holds the patch's
 // element terms as ys[(3 i + c) * kPatch + local element].  The patch's nodes
@@ -346,21 +343,7 @@ hipError_t launch_patch_factors(jfm_ctx *ctx, const int32_t *perm, double *gf64,
     return hipGetLastError();
 }
 
-// ------------------------------------------------------------ host setup ---
-namespace {
-
-uint64_t spread3(uint64_t v) {  // 21 bits -> every third bit
-    v &= 0x1fffff;
-    v = (v | v << 32) & 0x1f00000000ffffULL;
-    v = (v | v << 16) & 0x1f0000ff0000ffULL;
-    v = (v | v << 8) & 0x100f00f00f00f00fULL;
-    v = (v | v << 4) & 0x10c30c30c30c30c3ULL;
-    v = (v | v << 2) & 0x1249249249249249ULL;
-    return v;
-}
-
-}  // namespace
-
+// ------------------------------------------------------------------- setup ---
 bool jfem_patch_enabled() {
     static const bool use = [] {
         const char *v = std::getenv("JFEM_PATCH");
@@ -374,11 +357,11 @@ void jfem_patch_release(jfm_ctx *ctx) {
                      (void **)&ctx->pn_cnt, (void **)&ctx->pn_out, (void **)&ctx->rstart, (void **)&ctx->rbase,
                      (void **)&ctx->linT, (void **)&ctx->bptr, (void **)&ctx->bnode,
                      (void **)&ctx->bpart, (void **)&ctx->ppart, (void **)&ctx->eperm, (void **)&ctx->qsrc,
-                     (void **)&ctx->connP16, (void **)&ctx->pbase}) {
+                     (void **)&ctx->connP16, (void **)&ctx->pbase, (void **)&ctx->na_part}) {
         jfm_free(ctx, *p);
         *p = nullptr;
     }
-    ctx->patch_ready = false;
+    ctx->patch_ready = ctx->patch_upload = false;
     ctx->npatch = ctx->npn = ctx->nbnode = ctx->nslot = ctx->bmaxcnt = 0;
     ctx->qsrc_gen = -1;
     if (ctx->ke_perm) {  // element matrices stored in the released patch order
@@ -390,150 +373,188 @@ void jfem_patch_release(jfm_ctx *ctx) {
     }
 }
 
-// The patch structure on the host: element order, patch-local incidences in
-// rounds and the shared-node partial lists.  Returns false if an index does
-// not fit its type.
-struct PatchHost {
-    int npatch = 0;
-    std::vector<int32_t> perm, connP, pn_ptr, pn_out, rstart, rbase, bnode, bptr, pbase;
-    std::vector<uint16_t> connP16;  // empty when a patch spans more than 65,536 node ids
-    std::vector<uint16_t> pn_cnt, linT;
-};
+// The structure is built by one workgroup per patch from the element order
+// (morton_order): it sorts the patch's incidences by (node, element, local node)
+// in LDS, ranks the nodes by count, and finds the shared ones and their patches
+// from their elements' positions.  The patches' lists lie side by side, so the
+// kernel runs twice: sizes, their sums, lists.  (On the host this took 7 ms at
+// 12,810 Tet10 elements and 118 ms at 245,760; the upload with it takes less
+// than without it before.)
+constexpr int kPT = 512;                                   // threads
+constexpr int kPerThread = (10 * kPatch + kPT - 1) / kPT;  // incidences at most
+constexpr int kPKeys = 8192;
+static_assert(10 * kPatch <= kPKeys && 3 * 9 * kPatch + kPatch <= 65536, "keys in LDS, 16-bit incidences");
 
-static bool build_patches(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int64_t N,
-                          int npe, PatchHost &P) {
-    constexpr int ps = kPatch;
-    // Morton order of the element centroids (stable in element id)
-    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    for (int64_t a = 0; a < N; ++a)
-        for (int c = 0; c < 3; ++c) {
-            lo[c] = std::min(lo[c], X[3 * a + c]);
-            hi[c] = std::max(hi[c], X[3 * a + c]);
+// Per patch its nodes, rounds, incidence entries, slots and shared nodes that it
+// holds first; then their exclusive sums.  Rows of npatch + 1.
+enum { kNodes, kRounds, kLin, kSlots, kShared, kSizes };
+
+// WRITE = false: the sizes, the patch's lowest node id, in out[0] whether a
+// patch's ids span 65,536 or more, in out[1] the most patches of a node, and in
+// total the incidence entries of all patches.  WRITE = true: the lists;
+// pn_out of a shared node is -(its rank among the node's patches + 1) here.
+template <bool WRITE>
+__global__ __launch_bounds__(kPT) void k_patch_build(int n_el, int npe, int npatch, const int32_t *__restrict__ conn,
+                                                    const int32_t *__restrict__ perm, const int32_t *__restrict__ epos,
+                                                    const int32_t *__restrict__ inc_ptr, const int32_t *__restrict__ inc,
+                                                    int32_t *__restrict__ sizes, int32_t *__restrict__ pbase,
+                                                    int32_t *__restrict__ out, unsigned long long *__restrict__ total_lin,
+                                                    uint16_t *__restrict__ pn_cnt, int32_t *__restrict__ pn_out,
+                                                    int32_t *__restrict__ pn_node, int32_t *__restrict__ rbase,
+                                                    uint16_t *__restrict__ linT, int32_t *__restrict__ first,
+                                                    int32_t *__restrict__ bnode, int32_t *__restrict__ bptr) {
+    __shared__ uint64_t key[kPKeys];
+    __shared__ uint16_t head[10 * kPatch + 1], cnt[10 * kPatch], ranked[10 * kPatch];
+    const int p = blockIdx.x, t = threadIdx.x;
+    const int k0 = p * kPatch, ne = min(kPatch, n_el - k0), m = ne * npe;
+    auto size_of = [&](int what) -> int32_t & { return sizes[(size_t)what * (npatch + 1) + p]; };
+    int n2 = 2;
+    while (n2 < m) n2 <<= 1;
+    for (int idx = t; idx < n2; idx += kPT) {
+        uint64_t v = ~0ull;
+        if (idx < m) {
+            const int i = idx / ne, kl = idx - i * ne;
+            v = (uint64_t)(uint32_t)conn[(size_t)i * n_el + perm[k0 + kl]] << 32 | (uint32_t)(kl << 8 | i);
         }
-    std::vector<uint64_t> code(n_el);
-    for (int64_t e = 0; e < n_el; ++e) {
-        double cen[3] = {0.0, 0.0, 0.0};
-        for (int i = 0; i < npe; ++i)
-            for (int c = 0; c < 3; ++c) cen[c] += X[3 * (size_t)conn[e * npe + i] + c];
-        uint64_t q[3];
-        for (int c = 0; c < 3; ++c) {
-            const double ext = hi[c] - lo[c];
-            const double f = ext > 0.0 ? (cen[c] / npe - lo[c]) / ext : 0.0;
-            q[c] = (uint64_t)std::min(std::max(f, 0.0) * 2097151.0, 2097151.0);
-        }
-        code[e] = spread3(q[0]) << 2 | spread3(q[1]) << 1 | spread3(q[2]);
+        key[idx] = v;
     }
-    std::vector<int32_t> &perm = P.perm;
-    perm.resize(n_el);
-    std::iota(perm.begin(), perm.end(), 0);
-    std::stable_sort(perm.begin(), perm.end(), [&](int32_t a, int32_t b) { return code[a] < code[b]; });
-    code.clear();
-    code.shrink_to_fit();
-    std::vector<int32_t> val(N, 0);  // node valences
-    for (int32_t v : conn) ++val[v];
-    const int npatch = (int)((n_el + ps - 1) / ps);
-    P.npatch = npatch;
-    P.connP.assign((size_t)npe * n_el, 0);
-    P.pn_ptr.assign(npatch + 1, 0);
-    P.rstart.assign(npatch + 1, 0);
-    P.pn_out.clear();
-    P.pn_cnt.clear();
-    P.rbase.clear();
-    P.linT.clear();
-    std::vector<std::vector<int32_t>> shared_l(N);  // per node: patch-node indices, ascending patch
-    std::vector<std::pair<int64_t, int32_t>> pairs;  // (node * ps + local element, i)
-    struct PNode { int32_t a, first, cnt; };
-    std::vector<PNode> nodes;
-    for (int p = 0; p < npatch; ++p) {
-        const int64_t k0 = (int64_t)p * ps, k1 = std::min<int64_t>(k0 + ps, n_el);
-        pairs.clear();
-        for (int64_t k = k0; k < k1; ++k) {
-            const int32_t e = perm[k];
-            for (int i = 0; i < npe; ++i) {
-                const int32_t a = conn[(size_t)e * npe + i];
-                P.connP[(size_t)i * n_el + k] = a;
-                pairs.emplace_back((int64_t)a * ps + (k - k0), i);
+    sort_keys<kPT>(key, n2);
+    // the nodes, ascending: where each one's incidences start
+    auto is_head = [&](int idx) { return idx < m && (idx == 0 || key[idx] >> 32 != key[idx - 1] >> 32); };
+    int heads = 0, nn;
+    for (int j = 0; j < kPerThread; ++j) heads += is_head(kPerThread * t + j);
+    int h = block_scan<kPT>(heads, &nn);
+    for (int j = 0; j < kPerThread; ++j)
+        if (is_head(kPerThread * t + j)) head[h++] = (uint16_t)(kPerThread * t + j);
+    if (t == 0) head[nn] = (uint16_t)m;
+    __syncthreads();
+    for (int q = t; q < nn; q += kPT) cnt[q] = head[q + 1] - head[q];
+    __syncthreads();
+    // most incidences first, so that a round's counts are close
+    for (int q = t; q < nn; q += kPT) {
+        const int c = cnt[q];
+        int u = 0;
+        for (int o = 0; o < nn; ++o) u += cnt[o] > c || (cnt[o] == c && o < q);
+        ranked[u] = (uint16_t)q;
+    }
+    __syncthreads();
+    const int rounds = (nn + kPatch - 1) / kPatch;
+    int lin = 0;  // the rounds' largest counts
+    for (int r = 0; r < rounds; ++r) {
+        if (WRITE && t == 0) rbase[size_of(kRounds) + r] = size_of(kLin) + lin * kPatch;
+        lin += cnt[ranked[kPatch * r]];
+    }
+    if (!WRITE && t == 0) {
+        const int lo = (int)(key[0] >> 32), hi = (int)(key[m - 1] >> 32);
+        size_of(kNodes) = nn;
+        size_of(kRounds) = rounds;
+        size_of(kLin) = lin * kPatch;
+        pbase[p] = lo;
+        if (hi - lo >= 65536) out[0] = 1;
+        atomicAdd(total_lin, (unsigned long long)lin * kPatch);
+    }
+    int slots = WRITE ? size_of(kSlots) : 0, shared = WRITE ? size_of(kShared) : 0;
+    for (int u0 = 0; u0 < nn; u0 += kPT) {
+        const int u = u0 + t, q = u < nn ? ranked[u] : 0;
+        const int n = u < nn ? cnt[q] : 0, a = u < nn ? (int)(key[head[q]] >> 32) : 0;
+        int total = 0, rank = -1;
+        const int b0 = u < nn ? inc_ptr[a] : 0, b1 = u < nn ? inc_ptr[a + 1] : 0;
+        if (n < b1 - b0) {  // shared: its patches, in ascending order
+            rank = 0;
+            for (int last = -1;;) {
+                int next = INT32_MAX;
+                for (int k = b0; k < b1; ++k) {
+                    const int o = epos[inc[k] / npe] / kPatch;
+                    if (o > last && o < next) next = o;
+                }
+                if (next == INT32_MAX) break;
+                ++total;
+                rank += next < p;
+                last = next;
             }
         }
-        std::sort(pairs.begin(), pairs.end());  // by node, then local element
-        nodes.clear();
-        for (size_t r = 0; r < pairs.size();) {
-            const int32_t a = (int32_t)(pairs[r].first / ps);
-            size_t r2 = r;
-            while (r2 < pairs.size() && pairs[r2].first / ps == a) ++r2;
-            nodes.push_back({a, (int32_t)r, (int32_t)(r2 - r)});
-            r = r2;
-        }
-        // most incidences first, so that a round's counts are close
-        std::stable_sort(nodes.begin(), nodes.end(), [](const PNode &u, const PNode &v) { return u.cnt > v.cnt; });
-        const int64_t l0 = (int64_t)P.pn_out.size();
-        for (size_t u = 0; u < nodes.size(); u += ps) {
-            const int cntmax = nodes[u].cnt;
-            const int64_t base = (int64_t)P.linT.size();
-            if (base > INT32_MAX) return false;
-            P.rbase.push_back((int32_t)base);
-            P.linT.resize(base + (size_t)cntmax * ps, 0);
-            for (size_t t = 0; t < (size_t)ps && u + t < nodes.size(); ++t) {
-                const PNode &nd = nodes[u + t];
-                for (int j = 0; j < nd.cnt; ++j) {
-                    const auto &pr = pairs[nd.first + j];
-                    const int kl = (int)(pr.first % ps), i = pr.second;
-                    P.linT[base + (size_t)j * ps + t] = (uint16_t)(3 * i * ps + kl);
+        int sum, num;
+        const int so = slots + block_scan<kPT>(rank == 0 ? total : 0, &sum);
+        const int bo = shared + block_scan<kPT>(rank == 0, &num);
+        slots += sum;
+        shared += num;
+        if constexpr (WRITE) {
+            if (rank == 0) {
+                first[a] = so;
+                bnode[bo] = a;
+                bptr[bo] = so;
+            }
+            if (u < nn) {
+                const int l = size_of(kNodes) + u, r = u / kPatch, at = u - r * kPatch;
+                pn_cnt[l] = (uint16_t)n;
+                pn_out[l] = rank < 0 ? a : -(rank + 1);
+                pn_node[l] = a;
+                int base = size_of(kLin);
+                for (int o = 0; o < r; ++o) base += cnt[ranked[kPatch * o]] * kPatch;
+                for (int j = 0; j < n; ++j) {
+                    const uint32_t w = (uint32_t)key[head[q] + j];
+                    linT[base + (size_t)j * kPatch + at] = (uint16_t)(3 * (w & 255) * kPatch + (w >> 8));
                 }
             }
+        } else if (total > 0) {
+            atomicMax(out + 1, total);
         }
-        for (size_t u = 0; u < nodes.size(); ++u) {
-            const PNode &nd = nodes[u];
-            if (nd.cnt > 65535) return false;
-            P.pn_cnt.push_back((uint16_t)nd.cnt);
-            if (nd.cnt == val[nd.a]) {
-                P.pn_out.push_back(nd.a);  // interior
-            } else {
-                P.pn_out.push_back(-1);  // shared
-                shared_l[nd.a].push_back((int32_t)(l0 + (int64_t)u));
-            }
+    }
+    if (!WRITE && t == 0) {
+        size_of(kSlots) = slots;
+        size_of(kShared) = shared;
+    }
+}
+
+// the exclusive sums of each row of sizes, the total at its end
+__global__ __launch_bounds__(1024) void k_patch_sums(int npatch, int32_t *__restrict__ sizes) {
+    int32_t *row = sizes + (size_t)blockIdx.x * (npatch + 1);
+    int carry = 0;
+    for (int b0 = 0; b0 < npatch; b0 += 1024) {
+        const int b = b0 + (int)threadIdx.x;
+        int total;
+        const int ex = block_scan<1024>(b < npatch ? row[b] : 0, &total);
+        if (b < npatch) row[b] = carry + ex;
+        carry += total;
+    }
+    if (threadIdx.x == 0) row[npatch] = carry;
+}
+
+// pn_out of the shared nodes: -(the slot of the patch's own partial + 1)
+__global__ __launch_bounds__(256) void k_patch_slots(int npn, const int32_t *__restrict__ pn_node,
+                                                    const int32_t *__restrict__ first, int32_t *__restrict__ pn_out) {
+    const int l = blockIdx.x * blockDim.x + threadIdx.x;
+    if (l < npn && pn_out[l] < 0) pn_out[l] -= first[pn_node[l]];
+}
+
+// the nodes of no element, ascending, after the shared ones; one workgroup
+__global__ __launch_bounds__(1024) void k_patch_orphans(int N, const int32_t *__restrict__ inc_ptr, int nslot,
+                                                       int32_t *__restrict__ bnode, int32_t *__restrict__ bptr) {
+    int carry = 0;
+    for (int a0 = 0; a0 < N; a0 += 1024) {
+        const int a = a0 + (int)threadIdx.x;
+        const bool o = a < N && inc_ptr[a] == inc_ptr[a + 1];
+        int total;
+        const int at = carry + block_scan<1024>(o, &total);
+        if (o) {
+            bnode[at] = a;
+            bptr[at] = nslot;
         }
-        P.pn_ptr[p + 1] = (int32_t)P.pn_out.size();
-        P.rstart[p + 1] = (int32_t)P.rbase.size();
+        carry += total;
     }
-    // shared nodes in the order of their first patch entry, then the nodes
-    // of no element
-    std::vector<int32_t> order;
-    for (int64_t a = 0; a < N; ++a)
-        if (!shared_l[a].empty()) order.push_back((int32_t)a);
-    std::sort(order.begin(), order.end(), [&](int32_t u, int32_t v) { return shared_l[u][0] < shared_l[v][0]; });
-    for (int64_t a = 0; a < N; ++a)
-        if (val[a] == 0) order.push_back((int32_t)a);
-    P.bnode.clear();
-    P.bptr.assign(1, 0);
-    for (int32_t a : order) {
-        P.bnode.push_back(a);
-        // slots of node a: consecutive, in ascending patch order
-        for (size_t j = 0; j < shared_l[a].size(); ++j) P.pn_out[shared_l[a][j]] = -(P.bptr.back() + (int32_t)j + 1);
-        P.bptr.push_back(P.bptr.back() + (int32_t)shared_l[a].size());
-    }
-    // 16-bit connectivity relative to each patch's lowest node id, when every
-    // patch's ids span at most 65,536
-    P.pbase.assign(npatch, 0);
-    bool fits16 = true;
-    for (int p = 0; p < npatch && fits16; ++p) {
-        const int64_t k0 = (int64_t)p * ps, k1 = std::min<int64_t>(k0 + ps, n_el);
-        int32_t lo = INT32_MAX, hi = -1;
-        for (int i = 0; i < npe; ++i)
-            for (int64_t k = k0; k < k1; ++k) {
-                lo = std::min(lo, P.connP[(size_t)i * n_el + k]);
-                hi = std::max(hi, P.connP[(size_t)i * n_el + k]);
-            }
-        P.pbase[p] = lo;
-        fits16 = hi - lo < 65536;
-    }
-    if (fits16) {
-        P.connP16.assign((size_t)npe * n_el, 0);
-        for (int i = 0; i < npe; ++i)
-            for (int64_t k = 0; k < n_el; ++k)
-                P.connP16[(size_t)i * n_el + k] = (uint16_t)(P.connP[(size_t)i * n_el + k] - P.pbase[k / ps]);
-    }
-    return 3 * (npe - 1) * ps + ps <= 65536 && (int64_t)P.pn_out.size() < INT32_MAX / 3;
+    if (threadIdx.x == 0) bptr[carry] = nslot;
+}
+
+// connectivity in the patch order, with 16-bit ids from each patch's lowest
+__global__ __launch_bounds__(256) void k_patch_conn(int n_el, int npe, const int32_t *__restrict__ perm,
+                                                   const int32_t *__restrict__ conn, const int32_t *__restrict__ pbase,
+                                                   int32_t *__restrict__ connP, uint16_t *__restrict__ connP16) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= (int64_t)n_el * npe) return;
+    const int i = (int)(q / n_el), k = (int)(q - (int64_t)i * n_el);
+    const int a = conn[(size_t)i * n_el + perm[k]];
+    connP[q] = a;
+    if (connP16) connP16[q] = (uint16_t)(a - pbase[k / kPatch]);
 }
 
 // Builds the patch structure for the uploaded mesh (once per mesh).
@@ -544,76 +565,97 @@ int jfem_patch_setup(jfm_ctx *ctx) {
     if (n_el == 0) return JFM_OK;
     if ((int64_t)ctx->h_conn.size() != n_el * npe || (int64_t)ctx->h_X.size() != 3 * N)
         return jfm_fail(ctx, JFM_ESTATE, "patch setup needs the host mesh");
-    PatchHost P;
-    if (!build_patches(ctx->h_conn, ctx->h_X, n_el, N, npe, P))
-        return jfm_fail(ctx, JFM_EINVAL, "patch structure out of range");
-    const int npatch = P.npatch;
-    const int64_t npn = (int64_t)P.pn_out.size(), nb = (int64_t)P.bnode.size();
+    const int npatch = (int)((n_el + kPatch - 1) / kPatch);
+    const std::vector<int32_t> perm = morton_order(ctx->h_conn, ctx->h_X, n_el, npe);
+    std::vector<int32_t> epos(n_el);
+    for (int64_t k = 0; k < n_el; ++k) epos[perm[k]] = (int32_t)k;
     hipStream_t s = ctx->stream;
-    const int64_t ngfr = (int64_t)ctx->ngf * GF;  // rows of the geometric factors
+    const int64_t ngfr = (int64_t)ctx->ngf * GF, rows = npatch + 1;  // rows of the geometric factors
+    struct Scratch {  // element positions, first slots, sizes, results; waits before the host vectors go
+        jfm_ctx *ctx;
+        int32_t *p = nullptr, *node = nullptr;
+        ~Scratch() {
+            (void)hipStreamSynchronize(ctx->stream);
+            jfm_free(ctx, p);
+            jfm_free(ctx, node);
+        }
+    } tmp{ctx};
+    bool done = false;
+    struct Release {  // a setup that did not end leaves nothing
+        jfm_ctx *ctx;
+        bool *done;
+        ~Release() {
+            if (!*done) jfem_patch_release(ctx);
+        }
+    } release{ctx, &done};
 #define PALLOC(ptr, T, cnt)                                                                 \
     do {                                                                                    \
         ptr = jfm_alloc<T>(ctx, std::max<int64_t>(1, (cnt)));                               \
-        if (!ptr) {                                                                         \
-            jfem_patch_release(ctx);                                                        \
-            return jfm_fail(ctx, JFM_ENOMEM, "patch operator allocation failed");            \
-        }                                                                                   \
+        if (!ptr) return jfm_fail(ctx, JFM_ENOMEM, "patch operator allocation failed");     \
     } while (0)
-#define PUP(ptr, vec)                                                                       \
-    if (!(vec).empty())                                                                     \
-        JFM_HIP(ctx, hipMemcpyAsync(ptr, (vec).data(), sizeof((vec)[0]) * (vec).size(), hipMemcpyHostToDevice, s))
-    PALLOC(ctx->connP, int32_t, npe * n_el);
+    PALLOC(tmp.p, int32_t, n_el + N + kSizes * rows + 8);
+    int32_t *d_epos = tmp.p, *first = d_epos + n_el, *sizes = first + N;
+    int32_t *out = sizes + kSizes * rows;  // two words, then (aligned) a 64-bit one
+    unsigned long long *total = (unsigned long long *)(((uintptr_t)(out + 2) + 7) & ~(uintptr_t)7);
     PALLOC(ctx->eperm, int32_t, n_el);
+    PALLOC(ctx->pbase, int32_t, npatch);
+    JFM_HIP(ctx, hipMemcpyAsync(ctx->eperm, perm.data(), 4 * n_el, hipMemcpyHostToDevice, s));
+    JFM_HIP(ctx, hipMemcpyAsync(d_epos, epos.data(), 4 * n_el, hipMemcpyHostToDevice, s));
+    JFM_HIP(ctx, hipMemsetAsync(out, 0, 24, s));
+    k_patch_build<false><<<npatch, kPT, 0, s>>>((int)n_el, npe, npatch, ctx->conn, ctx->eperm, d_epos, ctx->inc_ptr, ctx->inc,
+                                                sizes, ctx->pbase, out, total, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                                nullptr, nullptr, nullptr);
+    k_patch_sums<<<kSizes, 1024, 0, s>>>(npatch, sizes);
+    int32_t got[2], sum[kSizes];
+    unsigned long long lin = 0;
+    JFM_HIP(ctx, hipMemcpyAsync(got, out, sizeof got, hipMemcpyDeviceToHost, s));
+    JFM_HIP(ctx, hipMemcpyAsync(&lin, total, sizeof lin, hipMemcpyDeviceToHost, s));
+    JFM_HIP(ctx, hipMemcpy2DAsync(sum, 4, sizes + npatch, 4 * rows, 4, kSizes, hipMemcpyDeviceToHost, s));
+    JFM_HIP(ctx, hipStreamSynchronize(s));
+    if (lin > (unsigned long long)INT32_MAX || sum[kNodes] >= INT32_MAX / 3)
+        return jfm_fail(ctx, JFM_EINVAL, "patch structure out of range");
+    const int64_t npn = sum[kNodes], nb = (int64_t)sum[kShared] + ctx->orphans;
+    PALLOC(tmp.node, int32_t, npn);
+    PALLOC(ctx->connP, int32_t, npe * n_el);
     PALLOC(ctx->gfP64, double, ngfr * n_el);
     PALLOC(ctx->gfP32, float, ngfr * n_el);
-    PALLOC(ctx->pn_ptr, int32_t, npatch + 1);
+    PALLOC(ctx->pn_ptr, int32_t, rows);
     PALLOC(ctx->pn_cnt, uint16_t, npn);
     PALLOC(ctx->pn_out, int32_t, npn);
-    PALLOC(ctx->rstart, int32_t, npatch + 1);
-    PALLOC(ctx->rbase, int32_t, (int64_t)P.rbase.size());
-    PALLOC(ctx->linT, uint16_t, (int64_t)P.linT.size());
+    PALLOC(ctx->rstart, int32_t, rows);
+    PALLOC(ctx->rbase, int32_t, sum[kRounds]);
+    PALLOC(ctx->linT, uint16_t, (int64_t)lin);
     PALLOC(ctx->bptr, int32_t, nb + 1);
     PALLOC(ctx->bnode, int32_t, nb);
-    PALLOC(ctx->bpart, double, 3 * (int64_t)P.bptr.back());
+    PALLOC(ctx->bpart, double, 3 * (int64_t)sum[kSlots]);
     PALLOC(ctx->ppart, double, npatch);
-    if (!P.connP16.empty()) {
-        PALLOC(ctx->connP16, uint16_t, npe * n_el);
-        PALLOC(ctx->pbase, int32_t, npatch);
-    }
+    // 16-bit connectivity when every patch's ids span at most 65,536
+    if (!got[0]) PALLOC(ctx->connP16, uint16_t, npe * n_el);
+    // FP32 folded factors: sqrt(cm) invJ, cm = mu w detJ / 5, and lambda / mu
+    if (ctx->affine && npe == 10 && ctx->nu_uniform) PALLOC(ctx->gfQ32, float, 9 * n_el);
 #undef PALLOC
-    PUP(ctx->connP, P.connP);
-    PUP(ctx->eperm, P.perm);
-    PUP(ctx->pn_ptr, P.pn_ptr);
-    PUP(ctx->pn_cnt, P.pn_cnt);
-    PUP(ctx->pn_out, P.pn_out);
-    PUP(ctx->rstart, P.rstart);
-    PUP(ctx->rbase, P.rbase);
-    PUP(ctx->linT, P.linT);
-    PUP(ctx->bptr, P.bptr);
-    PUP(ctx->bnode, P.bnode);
-    if (!P.connP16.empty()) {
-        PUP(ctx->connP16, P.connP16);
-        PUP(ctx->pbase, P.pbase);
-    }
-#undef PUP
-    if (ctx->affine && npe == 10 && ctx->nu_uniform) {
-        // FP32 folded factors: sqrt(cm) invJ, cm = mu w detJ / 5, and lambda / mu
-        ctx->gfQ32 = jfm_alloc<float>(ctx, 9 * n_el);
-        if (!ctx->gfQ32) {
-            jfem_patch_release(ctx);
-            return jfm_fail(ctx, JFM_ENOMEM, "patch operator allocation failed");
-        }
-        ctx->rho32 = (float)(2.0 * ctx->nu0 / (1.0 - 2.0 * ctx->nu0));
-    }
+    ctx->rho32 = (float)(2.0 * ctx->nu0 / (1.0 - 2.0 * ctx->nu0));
+    k_patch_build<true><<<npatch, kPT, 0, s>>>((int)n_el, npe, npatch, ctx->conn, ctx->eperm, d_epos, ctx->inc_ptr, ctx->inc,
+                                               sizes, ctx->pbase, out, total, ctx->pn_cnt, ctx->pn_out, tmp.node, ctx->rbase,
+                                               ctx->linT, first, ctx->bnode, ctx->bptr);
+    k_patch_slots<<<(unsigned)((npn + 255) / 256), 256, 0, s>>>((int)npn, tmp.node, first, ctx->pn_out);
+    if (ctx->orphans)
+        k_patch_orphans<<<1, 1024, 0, s>>>((int)N, ctx->inc_ptr, sum[kSlots], ctx->bnode + sum[kShared], ctx->bptr + sum[kShared]);
+    else
+        JFM_HIP(ctx, hipMemcpyAsync(ctx->bptr + nb, sizes + kSlots * rows + npatch, 4, hipMemcpyDeviceToDevice, s));
+    k_patch_conn<<<(unsigned)((npe * n_el + 255) / 256), 256, 0, s>>>((int)n_el, npe, ctx->eperm, ctx->conn, ctx->pbase, ctx->connP,
+                                                                      ctx->connP16);
+    JFM_HIP(ctx, hipMemcpyAsync(ctx->pn_ptr, sizes + kNodes * rows, 4 * rows, hipMemcpyDeviceToDevice, s));
+    JFM_HIP(ctx, hipMemcpyAsync(ctx->rstart, sizes + kRounds * rows, 4 * rows, hipMemcpyDeviceToDevice, s));
     JFM_HIP(ctx, launch_patch_factors(ctx, ctx->eperm, ctx->gfP64, ctx->gfP32, ctx->gfQ32));
-    JFM_HIP(ctx, hipStreamSynchronize(s));  // host vectors go out of scope
+    JFM_HIP(ctx, hipStreamSynchronize(s));
     ctx->npatch = npatch;
     ctx->npn = (int)npn;
     ctx->nbnode = (int)nb;
-    ctx->nslot = P.bptr.back();
-    ctx->bmaxcnt = 0;
-    for (int64_t i = 0; i < nb; ++i) ctx->bmaxcnt = std::max(ctx->bmaxcnt, P.bptr[i + 1] - P.bptr[i]);
+    ctx->nslot = sum[kSlots];
+    ctx->bmaxcnt = got[1];
     ctx->patch_ready = true;
+    done = true;
     return JFM_OK;
 }
 

@@ -124,3 +124,39 @@ def test_noalloc_rejects_what_it_cannot_hold(env):
     rc, y = noalloc(env, ctx, "matfree", 1, np.zeros(big.n_dofs))
     assert rc == 0 and not np.any(y)
     ctx.close()
+
+
+@pytest.mark.parametrize("gen,g", [("box_tet10", (91, 9, 7)), ("box_tet4", (40, 30, 28)), ("box_hex8", (48, 44, 44))])
+def test_patches_of_the_upload(env, gen, g):
+    """Meshes beyond the resident PCG's range: the call runs the patch operator,
+    made with the upload, and gives the bits of jfm_apply; also where the calls of
+    two contexts overlap."""
+    from jfem import mesh as M
+    jfem, lib, hip = env
+    ms = [getattr(M, gen)(*g, seed=s, jitter=0.1, E_sigma=0.3) for s in (1, 2)]
+    cs = [jfem.Context(0) for _ in ms]
+    for c, m in zip(cs, ms):
+        c.upload(m)
+        assert c.info()["n_patches"] == (m.n_el + 479) // 480
+    rng = np.random.default_rng(3)
+    xs = [rng.standard_normal(m.n_dofs) for m in ms]
+    say(f"noalloc on the upload's patches {gen} {g}")
+    for prec in (0, 1):
+        ref = [c.apply(x, op="matfree", precision=prec) for c, x in zip(cs, xs)]
+        dx, dy = ([DeviceVec(hip, m.n_dofs) for m in ms] for _ in range(2))
+        for k in (0, 1):
+            dx[k].put(xs[k])
+            dy[k].put(np.full(xs[k].size, np.nan))
+        assert hip.hipDeviceSynchronize() == 0
+        for _ in range(3):
+            for k in (0, 1):
+                assert lib.jfm_apply_noalloc(cs[k]._h, _lib.OPS["matfree"], prec, dx[k].p, dy[k].p, None) == 0
+                if prec:   # the FP32 vectors of all contexts share an array
+                    assert hip.hipDeviceSynchronize() == 0
+        assert hip.hipDeviceSynchronize() == 0
+        for k in (0, 1):
+            assert np.array_equal(dy[k].get(), ref[k])
+        for v in dx + dy:
+            v.free()
+    for c in cs:
+        c.close()
