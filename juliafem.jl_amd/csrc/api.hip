@@ -207,6 +207,7 @@ static void release_mesh(jfm_ctx *ctx) {
     jfem_coarse_release(ctx);
     jfem_patch_release(ctx);
     jfem_cells_release(ctx);
+    jfem_rows_release(ctx);
     jfem_train_release(ctx);
     release_heat(ctx);
     ctx->h_X.clear();
@@ -873,7 +874,7 @@ static int pcg_run(jfm_ctx *ctx, int op, const T *Minv, double rtol, int maxit, 
             CHECK_LAUNCH(ctx, op_apply<T>(ctx, op, x, q, nullptr, nullptr, nullptr, nullptr));
             CHECK_LAUNCH(ctx, launch_residual(ctx, (const double *)b, (const double *)q, ctx->fixed, (double *)r, n, &np));
         }
-        const ResidentHold hold(ctx, ctx->cells.npatch);  // until the kernel has ended
+        const ResidentHold hold(ctx, jfem_persist_workgroups(ctx, op));  // until the kernel has ended
         CHECK_LAUNCH(ctx, launch_pcg_persist<T>(ctx, op, Minv, b, from_x ? r : nullptr, x, rtol, maxit, coarse));
         if (int rc = read_scalars(ctx)) return rc;
         if (!ctx->S_host->fail) {

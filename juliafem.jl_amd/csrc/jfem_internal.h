@@ -359,6 +359,16 @@ struct jfm_ctx {
         double *wpart = nullptr;
         uint64_t *zw = nullptr;
     } cells;
+    // resident PCG on the CSR matrix (persist_csr.hip): the nodes each workgroup
+    // holds, and the blocks' columns as positions among them
+    struct Rows {
+        bool ready = false, usable = false;
+        int nwg = 0, per = 0;                // workgroups, nodes of each
+        int32_t *nloc = nullptr, *loc = nullptr;
+        uint16_t *lcol = nullptr;
+        double *z = nullptr;                 // exchanged vector, 4 values per node (FP32 or FP64 view)
+        uint64_t *words = nullptr;
+    } rows;
     bool persist_off = false;      // a resident solve gave up waiting: this context launches its iterations
     double *Muser64 = nullptr;     // N x 9 user blocks (JFM_PREC_USER)
     float *Muser32 = nullptr;
@@ -477,6 +487,15 @@ template <typename T> bool jfem_persist_maybe(const jfm_ctx *ctx, int op);
 // With coarse, of the two-level form on the current aggregation.
 template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys, bool coarse = false);
 int jfem_cells_coarse(jfm_ctx *ctx, int max_entries);
+// the same for the assembled matrix (persist_csr.hip)
+bool jfem_rows_maybe(const jfm_ctx *ctx);
+int jfem_rows_setup(jfm_ctx *ctx);
+void jfem_rows_release(jfm_ctx *ctx);
+template <typename T>
+hipError_t launch_pcg_rows(jfm_ctx *ctx, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit);
+void launch_persist_clear(jfm_ctx *ctx, int n, uint64_t *words, int nz, uint64_t *zw, int nsys, PcgScalars *S);
+// workgroups of a resident solve on `op`
+int jfem_persist_workgroups(const jfm_ctx *ctx, int op);
 // makes room for m systems of `words` exchange words
 int jfem_cells_systems(jfm_ctx *ctx, int m, int words);
 // heat: maps the convection faces to elements (ctx->heat_resident)

@@ -208,3 +208,36 @@ def test_resident_tangent(oracle, name, coarse_nodes):
         assert np.linalg.norm(u - uo) <= 1e-7 * np.linalg.norm(uo)
         assert np.array_equal(u, ctx.solve_nonlinear(**kw)[0])
     ctx.close()
+
+
+# nodes: 27 (one workgroup), 2,016 (63, four groups), 3,451, 2,250; 10,496 nodes: 41 of each
+# of 256 workgroups, also in random order (long lists of other workgroups' nodes)
+CSR = {"tet10_6": CASES["tet10_6"], "hex8_1435": ("box_hex8", (41, 5, 7)), "tet10_2052": CASES["tet10_2052"],
+       "tet4_10368": CASES["tet4_10368"], "hex8_9000": ("box_hex8", (40, 15, 15)), "hex8_9000_shuffled": ("box_hex8", (40, 15, 15))}
+
+
+@pytest.mark.parametrize("name", list(CSR))
+def test_resident_csr(oracle, name):
+    """The assembled matrix in the resident PCG against the oracle's direct solve,
+    or against the matrix-free solve where that is too large: a hundred times the
+    solve's tolerance, as above.  That is 1e-9 here: the FP64 residual with this
+    matrix ends at 1.0e-10 to 2.2e-10, launched or resident."""
+    import jfem
+    gen, g = CSR[name]
+    m = getattr(M, gen)(*g, seed=5, jitter=0.1, E_sigma=0.4)
+    if "shuffled" in name:
+        m = M.renumber(m, np.random.default_rng(1).permutation(m.n_nodes))
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    if m.n_dofs < 12000:
+        ud, lad, _ = oracle.solve_direct_lapack(oracle.assemble_csr(m), m.fixed_mask(), np.zeros(m.n_dofs), oracle.load_vector(m))
+    else:
+        ud, lad, _ = ctx.solve(op="matfree", rtol=1e-10, want_la=True)
+    for meth in (0, 1):
+        say(f"resident csr {name} method={meth} nodes={m.n_nodes}")
+        kw = dict(op="csr", method=meth, rtol=1e-9, inner_rtol=1e-2, want_la=True)
+        u, la, _ = ctx.solve(**kw)
+        assert np.linalg.norm(u - ud) <= 1e-7 * np.linalg.norm(ud)
+        u2, la2, _ = ctx.solve(**kw)
+        assert np.array_equal(u, u2) and np.array_equal(la, la2)
+    ctx.close()
