@@ -243,7 +243,8 @@ struct jfm_ctx {
     // training step (jfm_learned_grad): pairs, z, w = K z, dLoss/dM, gradient
     // partials, the pairs' products
     struct Train {
-        double *r = nullptr, *e = nullptr, *z = nullptr, *w = nullptr, *G = nullptr, *dots = nullptr;
+        double *r = nullptr, *e = nullptr, *z = nullptr, *w = nullptr, *G = nullptr, *dots = nullptr, *part = nullptr,
+               *bpart = nullptr;
         float *gpart = nullptr, *grad = nullptr;
         int pairs = 0, ndots = 0;
     } train;
@@ -454,6 +455,7 @@ hipError_t launch_patch_phase(jfm_ctx *ctx, int op, const T *x, T *y, const T *d
                               double *pout = nullptr);
 template <typename T>
 hipError_t launch_patch_combine(jfm_ctx *ctx, T *y, const T *dotv, double *part, const int *done, int *npart);
+hipError_t launch_patch_batch(jfm_ctx *ctx, const double *x, double *y, double *bpart, int batch);
 template <typename T>
 hipError_t launch_patch_apply(jfm_ctx *ctx, int op, const T *x, T *y, const T *dotv, double *part, const int *done,
                               int *npart);

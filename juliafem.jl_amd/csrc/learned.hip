@@ -491,42 +491,55 @@ __global__ __launch_bounds__(256) void k_block_apply(int N, const double *__rest
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= N) return;
     const double *Ma = M + 9 * (size_t)a;
-    const size_t o = 3 * (size_t)a;
+    const size_t o = 3 * ((size_t)blockIdx.y * N + a);  // blockIdx.y: the pair
     for (int i = 0; i < 3; ++i) z[o + i] = Ma[i * 3] * r[o] + Ma[i * 3 + 1] * r[o + 1] + Ma[i * 3 + 2] * r[o + 2];
 }
 
 // The three products of a training pair (z.r, z.w, e.r) in one pass: one
-// partial of each per block (part[k kMaxPart + block]).
+// partial of each per block (part[k kMaxPart + block]).  blockIdx.y: the pair.
 __global__ __launch_bounds__(256) void k_pair_dots(int n, const double *__restrict__ z, const double *__restrict__ r,
                                                   const double *__restrict__ w, const double *__restrict__ e,
                                                   double *__restrict__ part) {
     double v[3] = {0.0, 0.0, 0.0};
+    const size_t o = (size_t)blockIdx.y * n;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const double zi = z[i], ri = r[i];
+        const double zi = z[o + i], ri = r[o + i];
         v[0] += zi * ri;
-        v[1] += zi * w[i];
-        v[2] += e[i] * ri;
+        v[1] += zi * w[o + i];
+        v[2] += e[o + i] * ri;
     }
-    write_partials<3>(v, part);
+    write_partials<3>(v, part + (size_t)blockIdx.y * 3 * kMaxPart);
 }
 
-// G_a += coef (r - c w)_a r_a' with c = z.r / z.w, coef = -2 c / (e.r n_pairs),
-// from the partials of k_pair_dots; block 0 leaves the three products in `dots`
-// for the host, which reads them once for all pairs.
-__global__ __launch_bounds__(256) void k_accum_dm(int N, int n_pairs, int npart, const double *__restrict__ part,
-                                                 const double *__restrict__ r, const double *__restrict__ w,
-                                                 double *__restrict__ G, double *__restrict__ dots) {
-    double t[3];
-    sum_partials<3>(part, npart, t);
-    const double c = t[0] / t[1], coef = -2.0 * c / (t[2] * n_pairs);
-    if (blockIdx.x == 0 && threadIdx.x < 3) dots[threadIdx.x] = t[threadIdx.x];
+// G_a (+)= sum over the m pairs of coef (r - c w)_a r_a' with c = z.r / z.w, coef =
+// -2 c / (e.r n_pairs), from the partials of k_pair_dots; block 0 leaves the
+// pairs' three products in `dots` for the host, which reads them once.
+__global__ __launch_bounds__(256) void k_accum_dm(int N, int n_pairs, int m, int npart, bool first,
+                                                 const double *__restrict__ part, const double *__restrict__ r,
+                                                 const double *__restrict__ w, double *__restrict__ G,
+                                                 double *__restrict__ dots) {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= N) return;
-    const size_t o = 3 * (size_t)a;
-    for (int i = 0; i < 3; ++i) {
-        const double gi = coef * (r[o + i] - c * w[o + i]);
-        for (int j = 0; j < 3; ++j) G[9 * (size_t)a + i * 3 + j] += gi * r[o + j];
+    double g[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) g[i] = a < N && !first ? G[9 * (size_t)a + i] : 0.0;
+    for (int p = 0; p < m; ++p) {
+        double t[3];
+        sum_partials<3>(part + (size_t)p * 3 * kMaxPart, npart, t);
+        const double c = t[0] / t[1], coef = -2.0 * c / (t[2] * n_pairs);
+        if (blockIdx.x == 0 && threadIdx.x < 3) dots[3 * p + threadIdx.x] = t[threadIdx.x];
+        if (a >= N) continue;
+        const size_t o = 3 * ((size_t)p * N + a);
+        const double rv[3] = {r[o], r[o + 1], r[o + 2]};
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const double gi = coef * (rv[i] - c * w[o + i]);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) g[3 * i + j] += gi * rv[j];
+        }
     }
+    if (a >= N) return;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) G[9 * (size_t)a + i] = g[i];
 }
 
 // grad[p] = sum over wave partials, fixed order: a block takes 64 parameters,
@@ -872,7 +885,8 @@ constexpr int kPairRun = 8;
 
 void jfem_train_release(jfm_ctx *ctx) {
     auto &W = ctx->train;
-    for (void *p : {(void *)W.r, (void *)W.e, (void *)W.z, (void *)W.w, (void *)W.G, (void *)W.gpart, (void *)W.grad, (void *)W.dots})
+    for (void *p : {(void *)W.r, (void *)W.e, (void *)W.z, (void *)W.w, (void *)W.G, (void *)W.gpart, (void *)W.grad, (void *)W.dots,
+                    (void *)W.part, (void *)W.bpart})
         jfm_free(ctx, p);
     W = {};
 }
@@ -888,6 +902,8 @@ extern "C" int jfm_learned_grad(jfm_ctx *ctx, int32_t n_pairs, const double *r, 
     const bool coarse = coarse_nodes > 0;
     if (coarse && !(ctx->coarse_ready && ctx->coarse_built_nodes == coarse_nodes && ctx->coarse_tag == 0))
         if (int rc = jfem_coarse_setup(ctx, JFM_OP_MATFREE, coarse_nodes, nullptr)) return rc;
+    if (jfem_patch_enabled())
+        if (int rc = jfem_patch_setup(ctx)) return rc;
     const int64_t n = ctx->ndof, N = ctx->N;
     hipStream_t s = ctx->stream;
     // the pairs go to the device in runs of up to kPairRun; the buffers stay
@@ -898,12 +914,14 @@ extern "C" int jfm_learned_grad(jfm_ctx *ctx, int32_t n_pairs, const double *r, 
         jfem_train_release(ctx);
         W.r = jfm_alloc<double>(ctx, run * n);
         W.e = jfm_alloc<double>(ctx, run * n);
-        W.z = jfm_alloc<double>(ctx, n);
-        W.w = jfm_alloc<double>(ctx, n);
+        W.z = jfm_alloc<double>(ctx, run * n);
+        W.w = jfm_alloc<double>(ctx, run * n);
+        W.part = jfm_alloc<double>(ctx, (int64_t)run * 3 * kMaxPart);
+        W.bpart = jfm_alloc<double>(ctx, (int64_t)run * 3 * ctx->nslot);
         W.G = jfm_alloc<double>(ctx, 9 * N);
         W.gpart = jfm_alloc<float>(ctx, (int64_t)kTrainBlocks * kWaves * kNParam);
         W.grad = jfm_alloc<float>(ctx, kNParam);
-        if (!W.r || !W.e || !W.z || !W.w || !W.G || !W.gpart || !W.grad) {
+        if (!W.r || !W.e || !W.z || !W.w || !W.part || !W.bpart || !W.G || !W.gpart || !W.grad) {
             jfem_train_release(ctx);
             return jfm_fail(ctx, JFM_ENOMEM, "device allocation failed in jfm_learned_grad");
         }
@@ -916,26 +934,40 @@ extern "C" int jfm_learned_grad(jfm_ctx *ctx, int32_t n_pairs, const double *r, 
         if (!W.dots) return jfm_fail(ctx, JFM_ENOMEM, "device allocation failed in jfm_learned_grad");
         W.ndots = n_pairs;
     }
-    JFM_HIP(ctx, hipMemsetAsync(W.G, 0, sizeof(double) * 9 * N, s));
-    double *part = ctx->partials + kPartMisc;   // three rows of kMaxPart
-    static_assert(kPartTotal - kPartMisc >= 3 * kMaxPart, "room for three partials per block");
-    for (int p = 0; p < n_pairs; ++p) {
-        if (p % run == 0) {
-            const size_t m = (size_t)std::min(run, n_pairs - p) * n * sizeof(double);
-            JFM_HIP(ctx, hipMemcpyAsync(W.r, r + (size_t)p * n, m, hipMemcpyHostToDevice, s));
-            JFM_HIP(ctx, hipMemcpyAsync(W.e, e + (size_t)p * n, m, hipMemcpyHostToDevice, s));
-        }
-        const double *dr = W.r + (size_t)(p % run) * n, *de = W.e + (size_t)(p % run) * n;
-        k_block_apply<<<nblk(N), kBlock, 0, s>>>((int)N, ctx->Mlearn64, dr, W.z);
-        if (coarse) {
+    // The pairs of a run side by side: one launch each for z = M r, w = K z, the
+    // products and dLoss/dM.  (Pair by pair, with copies and a host wait around each
+    // product, a gradient of four pairs took 416 us at 20,449 nodes instead of 333.)
+    // They are copied on the second stream while the blocks are formed.
+    if (!ctx->stream2) JFM_HIP(ctx, hipStreamCreateWithFlags(&ctx->stream2, hipStreamNonBlocking));
+    if (int rc = learned_events(ctx)) return rc;
+    struct Copies {  // no copy from the caller's arrays outlives the call
+        hipStream_t s;
+        ~Copies() { (void)hipStreamSynchronize(s); }
+    } copies{ctx->stream2};
+    for (int p = 0; p < n_pairs; p += run) {
+        const int m = std::min(run, n_pairs - p);
+        if (p > 0) JFM_HIP(ctx, hipStreamSynchronize(s));  // the run before has read the pairs
+        JFM_HIP(ctx, hipMemcpyAsync(W.r, r + (size_t)p * n, sizeof(double) * m * n, hipMemcpyHostToDevice, ctx->stream2));
+        JFM_HIP(ctx, hipMemcpyAsync(W.e, e + (size_t)p * n, sizeof(double) * m * n, hipMemcpyHostToDevice, ctx->stream2));
+        JFM_HIP(ctx, hipEventRecord(ctx->ev_fork, ctx->stream2));
+        JFM_HIP(ctx, hipStreamWaitEvent(s, ctx->ev_fork, 0));
+        k_block_apply<<<dim3(nblk(N), m), kBlock, 0, s>>>((int)N, ctx->Mlearn64, W.r, W.z);
+        for (int q = 0; q < m && coarse; ++q) {
             int np = 0;
-            hipError_t err = launch_coarse_correct<double>(ctx, dr, W.z, nullptr, ctx->partials + kPartMisc, nullptr, &np);
+            hipError_t err = launch_coarse_correct<double>(ctx, W.r + q * n, W.z + q * n, nullptr, ctx->partials + kPartMisc,
+                                                           nullptr, &np);
             if (err != hipSuccess) return jfm_hip_fail(ctx, err, "coarse correction");
         }
-        if (int rc = jfem_apply(ctx, JFM_OP_MATFREE, W.z, W.w)) return rc;
+        hipError_t err = hipSuccess;
+        if (jfem_patch_form(ctx, JFM_OP_MATFREE))
+            err = launch_patch_batch(ctx, W.z, W.w, W.bpart, m);
+        else
+            for (int q = 0; q < m && err == hipSuccess; ++q)
+                err = launch_two_phase<double>(ctx, JFM_OP_MATFREE, W.z + q * n, W.w + q * n, nullptr, nullptr, nullptr, nullptr);
+        if (err != hipSuccess) return jfm_hip_fail(ctx, err, "training product");
         const unsigned g = capped_grid(n, kBlock);
-        k_pair_dots<<<g, kBlock, 0, s>>>((int)n, W.z, dr, W.w, de, part);
-        k_accum_dm<<<nblk(N), kBlock, 0, s>>>((int)N, n_pairs, (int)g, part, dr, W.w, W.G, W.dots + 3 * p);
+        k_pair_dots<<<dim3(g, m), kBlock, 0, s>>>((int)n, W.z, W.r, W.w, W.e, W.part);
+        k_accum_dm<<<nblk(N), kBlock, 0, s>>>((int)N, n_pairs, m, (int)g, p == 0, W.part, W.r, W.w, W.G, W.dots + 3 * p);
         JFM_HIP(ctx, hipGetLastError());
     }
     int nw = 0;

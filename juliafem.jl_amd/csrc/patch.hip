@@ -62,7 +62,11 @@ __global__ __launch_bounds__(kPatch) void k_ku_patch(int n_el, int npatch, int n
                                                     const uint8_t *__restrict__ fixed, T *__restrict__ y,
                                                     T *__restrict__ bpart, const T *__restrict__ dotv,
                                                     double *__restrict__ ppart, const int *__restrict__ done,
-                                                    T rho) {
+                                                    T rho, int xs, int bs) {
+    // blockIdx.y: product of vector y of a batch, xs values further (no dotv then)
+    x += (size_t)blockIdx.y * xs;
+    y += (size_t)blockIdx.y * xs;
+    bpart += (size_t)blockIdx.y * bs;
     __shared__ T ys[3 * NPE * kPatch];
     const int p = xcd_block();
     if (p >= npatch) return;  // whole workgroup (grid padded to a multiple of 8)
@@ -256,7 +260,10 @@ __global__ __launch_bounds__(256) void k_ku_combine(int nb, int chunk, const int
                                                    const int32_t *__restrict__ bnode, const T *__restrict__ bpart,
                                                    const uint8_t *__restrict__ fixed, T *__restrict__ y,
                                                    const T *__restrict__ dotv, const double *__restrict__ ppart,
-                                                   int npatch, double *__restrict__ part, const int *__restrict__ done) {
+                                                   int npatch, double *__restrict__ part, const int *__restrict__ done,
+                                                   int xs, int bs) {
+    y += (size_t)blockIdx.y * xs;
+    bpart += (size_t)blockIdx.y * bs;
     // the first node's slot range, its first kPre partials, its mask and its
     // dotv values are all in flight before the convergence flag is tested
     // (the grid gives most threads exactly one node)
@@ -733,8 +740,10 @@ template <typename T> static bool energy_dot(const jfm_ctx *ctx, int op, const T
 
 // The block partials of the dot go to pout (ctx->ppart when null).
 template <int NPE, typename T>
-static void patch_kernel(jfm_ctx *ctx, int op, const T *x, T *y, const T *dotv, const int *done, double *pout) {
-    const dim3 grid(xcd_grid(ctx->npatch));
+static void patch_kernel(jfm_ctx *ctx, int op, const T *x, T *y, const T *dotv, const int *done, double *pout,
+                         T *bpart, int batch) {
+    const dim3 grid(xcd_grid(ctx->npatch), batch);
+    const int xs = 3 * (int)ctx->N, bs = 3 * ctx->nslot;
     const int n = (int)ctx->n_el;
     double *pp = dotv ? (pout ? pout : ctx->ppart) : nullptr;
     if (energy_dot<T>(ctx, op, x, dotv)) dotv = nullptr;
@@ -742,7 +751,7 @@ static void patch_kernel(jfm_ctx *ctx, int op, const T *x, T *y, const T *dotv, 
         kernel<<<grid, kPatch, 0, ctx->stream>>>(n, ctx->npatch, ctx->npn, ctx->connP, ctx->connP16, ctx->pbase, el, x,
                                                  ctx->pn_ptr, ctx->pn_cnt,
                                                  ctx->pn_out, ctx->rstart, ctx->rbase, ctx->linT, ctx->fixed, y,
-                                                 (T *)ctx->bpart, dotv, pp, done, rho);
+                                                 bpart, dotv, pp, done, rho, xs, bs);
     };
     const bool c16 = ctx->connP16 != nullptr;
     if (op == JFM_OP_EBE) {
@@ -764,17 +773,22 @@ static void patch_kernel(jfm_ctx *ctx, int op, const T *x, T *y, const T *dotv, 
 }
 
 template <typename T>
-hipError_t launch_patch_phase(jfm_ctx *ctx, int op, const T *x, T *y, const T *dotv, const int *done,
-                              double *pout) {
+static hipError_t patch_phase(jfm_ctx *ctx, int op, const T *x, T *y, const T *dotv, const int *done, double *pout, T *bpart,
+                              int batch) {
     if (ctx->n_el == 0) return hipSuccess;
     if (!jfem_patch_form(ctx, op)) return hipErrorInvalidValue;
     switch (ctx->npe) {
-    case 10: patch_kernel<10, T>(ctx, op, x, y, dotv, done, pout); break;
-    case 4: patch_kernel<4, T>(ctx, op, x, y, dotv, done, pout); break;
-    case 8: patch_kernel<8, T>(ctx, op, x, y, dotv, done, pout); break;
+    case 10: patch_kernel<10, T>(ctx, op, x, y, dotv, done, pout, bpart, batch); break;
+    case 4: patch_kernel<4, T>(ctx, op, x, y, dotv, done, pout, bpart, batch); break;
+    case 8: patch_kernel<8, T>(ctx, op, x, y, dotv, done, pout, bpart, batch); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+template <typename T>
+hipError_t launch_patch_phase(jfm_ctx *ctx, int op, const T *x, T *y, const T *dotv, const int *done,
+                              double *pout) {
+    return patch_phase<T>(ctx, op, x, y, dotv, done, pout, (T *)ctx->bpart, 1);
 }
 
 template <typename T>
@@ -788,7 +802,21 @@ hipError_t launch_patch_combine(jfm_ctx *ctx, T *y, const T *dotv, double *part,
     if (npart) *npart = (int)g;
     k_ku_combine<T><<<g, kBlock, 0, ctx->stream>>>(nb, chunk, ctx->bptr, ctx->bnode, (const T *)ctx->bpart,
                                                    ctx->fixed, y, dotv, (ctx->n_el && part) ? ctx->ppart : nullptr,
-                                                   ctx->n_el ? ctx->npatch : 0, part, done);
+                                                   ctx->n_el ? ctx->npatch : 0, part, done, 0, 0);
+    return hipGetLastError();
+}
+
+// y_i = K x_i for `batch` vectors, 3 N values apart, partial sums in bpart
+// (3 nslot values each).  A small mesh has fewer patches than the chip has CUs: at
+// 27 patches four products in turn took 60 us.
+hipError_t launch_patch_batch(jfm_ctx *ctx, const double *x, double *y, double *bpart, int batch) {
+    hipError_t e = patch_phase<double>(ctx, JFM_OP_MATFREE, x, y, nullptr, nullptr, nullptr, bpart, batch);
+    if (e != hipSuccess || ctx->nbnode == 0) return e;
+    const unsigned g = std::min<unsigned>(xcd_grid((unsigned)((ctx->nbnode + kBlock - 1) / kBlock)), kMaxPart);
+    const int chunk = (int)((ctx->nbnode + g - 1) / g);
+    k_ku_combine<double><<<dim3(g, batch), kBlock, 0, ctx->stream>>>(ctx->nbnode, chunk, ctx->bptr, ctx->bnode, bpart, ctx->fixed, y,
+                                                                     nullptr, nullptr, 0, nullptr, nullptr, 3 * (int)ctx->N,
+                                                                     3 * ctx->nslot);
     return hipGetLastError();
 }
 
