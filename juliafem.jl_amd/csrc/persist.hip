@@ -381,6 +381,91 @@ template <typename T_> struct TangentTet10 : OpShape<10, 3, 4, 10, 4, false, 2> 
     }
 };
 
+// Hex8 elasticity (2 x 2 x 2 Gauss points) on two lanes per element, lane k with
+// the four nodes and the four points of one face zeta = -+1.  Lane 1 works in the
+// frame mirrored in zeta: its node m is node m ^ 4, its derivatives along zeta
+// change sign, and both lanes run the same code.  Gradients are formed from the
+// edges' differences, so translations drop out exactly; in the end the lanes swap
+// their terms of the other's nodes.  (One lane per element would hold 72 values
+// of gradients, or idle half of the threads.)
+template <typename T_> struct ElasticHex8 : OpShape<8, 3, 2, 8, 4, false, 2> {
+    using T = T_;
+    struct Data {};
+    __device__ static int in_node(int kv, int m) { return m ^ (4 * kv); }
+    __device__ static void load(const PersistArgs<T> &, int, int, bool, Data &) {}
+    template <typename XC, typename OC>
+    __device__ static double product(const PersistArgs<T> &A, const Data &, int k, int kv, bool has, XC &&xc, OC &&oc) {
+        if (!has) return 0.0;  // both lanes of the element
+        constexpr T a0 = T(0.57735026918962576451), dm = T(0.125 * 1.57735026918962576451), dp = T(0.125 * 0.42264973081037423549);
+        // the edges' nodes along xi, eta and zeta, ordered by the other two coordinates' signs
+        constexpr int E[3][4][2] = {{{0, 1}, {3, 2}, {4, 5}, {7, 6}}, {{0, 3}, {1, 2}, {4, 7}, {5, 6}}, {{0, 4}, {1, 5}, {3, 7}, {2, 6}}};
+        const T sg = kv ? T(-1) : T(1);
+        T x[8][3], y[8][3];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                x[i][c] = xc(i, c);
+                y[i][c] = T(0);
+            }
+#pragma unroll 1  // (unrolled, the points' factors would take 88 registers)
+        for (int q = 0; q < 4; ++q) {
+            const T xi = q & 1 ? a0 : -a0, eta = q & 2 ? a0 : -a0;
+            const T am = T(1) - xi, ap = T(1) + xi, bm = T(1) - eta, bp = T(1) + eta;
+            const T w[3][4] = {{bm * dm, bp * dm, bm * dp, bp * dp},
+                               {am * dm, ap * dm, am * dp, ap * dp},
+                               {sg * T(0.125) * am * bm, sg * T(0.125) * ap * bm, sg * T(0.125) * am * bp, sg * T(0.125) * ap * bp}};
+            const T *el = A.el + (size_t)((A.ngf > 1 ? q + 4 * kv : 0) * GF) * A.n_el + k;
+            T H[9], Ji[9];
+#pragma unroll
+            for (int m = 0; m < 9; ++m) Ji[m] = el[(size_t)m * A.n_el];
+            const T cl = el[(size_t)9 * A.n_el], cm = el[(size_t)10 * A.n_el];
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    T h = T(0);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) h += w[c][e] * (x[E[c][e][1]][a] - x[E[c][e][0]][a]);
+                    H[3 * a + c] = h;
+                }
+            T G[9];
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+#pragma unroll
+                for (int b = 0; b < 3; ++b)
+                    G[a * 3 + b] = H[a * 3] * Ji[b * 3] + H[a * 3 + 1] * Ji[b * 3 + 1] + H[a * 3 + 2] * Ji[b * 3 + 2];
+            const T tr = cl * (G[0] + G[4] + G[8]);
+            const T s01 = cm * (G[1] + G[3]), s02 = cm * (G[2] + G[6]), s12 = cm * (G[5] + G[7]);
+            const T s[9] = {tr + T(2) * cm * G[0], s01, s02, s01, tr + T(2) * cm * G[4], s12, s02, s12, tr + T(2) * cm * G[8]};
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const T P = s[a * 3] * Ji[c] + s[a * 3 + 1] * Ji[3 + c] + s[a * 3 + 2] * Ji[6 + c];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const T f = P * w[c][e];
+                        y[E[c][e][1]][a] += f;
+                        y[E[c][e][0]][a] -= f;
+                    }
+                }
+        }
+        double en = 0.0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const T x0 = kv ? x[4][c] : x[0][c];  // node 0 in both lanes
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const T f = y[m][c] + quad_xor<1>(y[m + 4][c]);
+                oc(m, c, f);
+                en += (double)(x[m][c] - x0) * (double)f;
+            }
+        }
+        return en;
+    }
+};
+
 template <typename T_> struct ElasticTet4 : OpShape<4, 3, 1, 4, 4, false, 2> {
     using T = T_;
     struct Data { T f[GF]; };
@@ -636,7 +721,7 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
     const PersistArgs<T> &A = A0;
     const int nwg = A.npatch, sys = (int)blockIdx.x / nwg, p = (int)blockIdx.x - sys * nwg;
     const int t = (int)threadIdx.x;
-    const int el = t / NL, kv = NL == 4 ? t & 3 : 0;   // its element (and vertex or component)
+    const int el = t / NL, kv = NL > 1 ? t & (NL - 1) : 0;   // its element (and vertex or component)
     const int k = p * EL + el;
     const bool has_el = el < EL && k < A.n_el;
     const int lb = NT * p, nn = A.pn_n[p];
@@ -987,6 +1072,7 @@ template <typename T> static PersistLaunch persist_kernel(const jfm_ctx *ctx, in
             if (tet10 && ctx->nu_uniform) return persist_of<ElasticTet10<T, true>>(coarse);
         if (tet10) return persist_of<ElasticTet10<T, false>>(coarse);
         if (ctx->npe == 4) return persist_of<ElasticTet4<T>>(coarse);
+        if (ctx->npe == 8) return persist_of<ElasticHex8<T>>(coarse);
     }
     if (op == JFM_OP_TANGENT && tet10) return persist_of<TangentTet10<T>>(coarse);
     if constexpr (sizeof(T) == 8) {

@@ -241,3 +241,27 @@ def test_resident_csr(oracle, name):
         u2, la2, _ = ctx.solve(**kw)
         assert np.array_equal(u, u2) and np.array_equal(la, la2)
     ctx.close()
+
+
+# 256 elements per patch: one element, one short of a patch, a full one, two, 18
+@pytest.mark.parametrize("g", [(1, 1, 1), (17, 5, 3), (16, 4, 4), (13, 5, 4), (40, 11, 10)])
+@pytest.mark.parametrize("jitter", [0.0, 0.15])
+def test_resident_hex8(oracle, g, jitter):
+    """Hex8 elasticity, parallelepipeds and general hexahedra, one-level and
+    two-level, to the bars of test_resident_pcg (the larger mesh, whose residual
+    ends above 1e-10, at ten times both)."""
+    import jfem
+    m = M.box_hex8(*g, L=(4.0, 4.0 * g[1] / g[0], 4.0 * g[2] / g[0]), seed=5, jitter=jitter, E_sigma=0.4)
+    k = 10.0 if m.n_el > 4000 else 1.0
+    csr = oracle.assemble_csr(m)
+    ud, _, _ = oracle.solve_direct_lapack(csr, m.fixed_mask(), np.zeros(m.n_dofs), oracle.load_vector(m))
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    for meth in (0, 1):
+        for coarse_nodes in (0, 100):
+            say(f"resident hex8 {g} jitter={jitter} method={meth} coarse_nodes={coarse_nodes}")
+            kw = dict(method=meth, rtol=k * 1e-10, inner_rtol=1e-2, coarse_nodes=coarse_nodes)
+            u, _, _ = ctx.solve(**kw)
+            assert np.linalg.norm(u - ud) <= k * 1e-8 * np.linalg.norm(ud)
+            assert np.array_equal(u, ctx.solve(**kw)[0])
+    ctx.close()
