@@ -185,6 +185,8 @@ static void release_mesh(jfm_ctx *ctx) {
     jfem_learned_drop(ctx);  // no stream2 work may still use the buffers freed here
     free_ptr(ctx, ctx->X); free_ptr(ctx, ctx->conn); free_ptr(ctx, ctx->E); free_ptr(ctx, ctx->nu);
     free_ptr(ctx, ctx->gf64); free_ptr(ctx, ctx->gf32); free_ptr(ctx, ctx->inc_ptr); free_ptr(ctx, ctx->inc);
+    free_ptr(ctx, ctx->tl_ws);
+    ctx->tl_ws_n = 0;
     free_ptr(ctx, ctx->brow); free_ptr(ctx, ctx->bcol); free_ptr(ctx, ctx->bdiag); free_ptr(ctx, ctx->blk_row);
     free_ptr(ctx, ctx->cptr); free_ptr(ctx, ctx->contrib); free_ptr(ctx, ctx->vals64); free_ptr(ctx, ctx->vals32);
     free_ptr(ctx, ctx->Ke); free_ptr(ctx, ctx->Ke32); free_ptr(ctx, ctx->ye64); free_ptr(ctx, ctx->ye32);
@@ -631,32 +633,44 @@ extern "C" int jfm_assemble_tl(jfm_ctx *ctx, int32_t geometric, const double *u,
     hipStream_t s = ctx->stream;
     const int64_t n = ctx->ndof;
     const size_t vbytes = sizeof(double) * 9 * (size_t)ctx->nnzb;
-    double *Ke = nullptr;   // finite-strain element blocks, element-major, freed below
-    ALLOC(ctx, Ke, double, ctx->n_el * ctx->npair * 9);
+    // finite-strain element blocks, the factors of Kg's, and the values of Km and
+    // Kg that are asked for beside those of Km + Kg: a workspace that stays with the
+    // mesh up to 512 MB (its allocation and release took 0.1 ms a call)
+    const int64_t pairs = ctx->n_el * ctx->npair, nv = 9 * ctx->nnzb;
+    const int64_t want = 9 * pairs + (geometric ? pairs + (vals ? nv : 0) + (vals_kg ? nv : 0) : 0);
+    if (ctx->tl_ws_n < want) {
+        free_ptr(ctx, ctx->tl_ws);
+        ctx->tl_ws_n = 0;
+        ALLOC(ctx, ctx->tl_ws, double, want);
+        ctx->tl_ws_n = want;
+    }
+    struct Keep {
+        jfm_ctx *ctx;
+        ~Keep() {
+            if (ctx->tl_ws_n <= int64_t(64) << 20) return;
+            (void)hipStreamSynchronize(ctx->stream);
+            free_ptr(ctx, ctx->tl_ws);
+            ctx->tl_ws_n = 0;
+        }
+    } keep{ctx};
+    double *Ke = ctx->tl_ws, *Kg = geometric ? Ke + 9 * pairs : nullptr;
+    double *vm = geometric && vals ? Kg + pairs : nullptr;
+    double *vg = geometric && vals_kg ? Kg + pairs + (vals ? nv : 0) : nullptr;
     if (!ctx->vals64) ALLOC(ctx, ctx->vals64, double, 9 * ctx->nnzb);
     if (!ctx->vals32) ALLOC(ctx, ctx->vals32, float, 9 * ctx->nnzb);
     ctx->assembled = false;
     if (u) JFM_HIP(ctx, hipMemcpyAsync(ctx->vx64, u, sizeof(double) * n, hipMemcpyHostToDevice, s));
     else JFM_HIP(ctx, hipMemsetAsync(ctx->vx64, 0, sizeof(double) * n, s));
-    if (geometric && vals_kg) {
-        CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, 1, Ke, nullptr));
-        CHECK_LAUNCH(ctx, launch_assemble_values_ke(ctx, Ke));
-        JFM_HIP(ctx, hipMemcpyAsync(vals_kg, ctx->vals64, vbytes, hipMemcpyDeviceToHost, s));
-    }
-    // Km and the element forces; f = f_ext - f_int (src/problems_elasticity.jl:432-433)
-    CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, 0, Ke, ctx->ye64));
-    CHECK_LAUNCH(ctx, launch_assemble_values_ke(ctx, Ke));
-    if (vals) JFM_HIP(ctx, hipMemcpyAsync(vals, ctx->vals64, vbytes, hipMemcpyDeviceToHost, s));
+    // Km, Kg and the element forces; f = f_ext - f_int (src/problems_elasticity.jl:432-433)
+    CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, Ke, Kg, ctx->ye64));
+    CHECK_LAUNCH(ctx, launch_assemble_values_ke(ctx, Ke, Kg, vm, vg));
     CHECK_LAUNCH(ctx, launch_gather<double>(ctx, ctx->ye64, nullptr, ctx->vy64, nullptr, nullptr, nullptr, nullptr));
     CHECK_LAUNCH(ctx, (launch_convert<double, double>(ctx, ctx->vy64, ctx->vy64, n, -1.0)));
     CHECK_LAUNCH(ctx, launch_add(ctx, ctx->f_ext, ctx->vy64, ctx->load, n));
-    if (geometric) {
-        CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, 2, Ke, nullptr));
-        CHECK_LAUNCH(ctx, launch_assemble_values_ke(ctx, Ke));
-    }
+    if (vals_kg) JFM_HIP(ctx, hipMemcpyAsync(vals_kg, vg, vbytes, hipMemcpyDeviceToHost, s));
+    if (vals) JFM_HIP(ctx, hipMemcpyAsync(vals, vm ? vm : ctx->vals64, vbytes, hipMemcpyDeviceToHost, s));
     if (f) JFM_HIP(ctx, hipMemcpyAsync(f, ctx->load, sizeof(double) * n, hipMemcpyDeviceToHost, s));
     if (int rc = sync(ctx)) return rc;
-    free_ptr(ctx, Ke);
     ctx->assembled = true;
     ctx->has_load = true;
     return JFM_OK;

@@ -264,14 +264,15 @@ __global__ __launch_bounds__(256) void k_elem_mat(int n_el, int ngf, const doubl
 // D the 3x3 block (i,j) of BL(F)' D BL(F) is
 //     lambda a_i (x) a_j + mu ((g_i . g_j) F F' + a_j (x) a_i),   a = F g,
 // the block of BNL' S3 BNL is (g_i' S g_j) I, and BL' S at node i is F S g_i
-// (all times w detJ in the reference configuration).  which = 0: Km, 1: Kg,
-// 2: Km + Kg, into the packed pair blocks `Ke`; f_int (when ye != null) goes
-// to the incidence slots for the nodal gather.  One 64-lane block per element.
+// (all times w detJ in the reference configuration).  Km goes to the packed pair
+// blocks `Ke`, the factors of I of Kg's blocks to `Kg` (when not null), f_int
+// (when ye != null) to the incidence slots for the nodal gather.  One 64-lane
+// block per element.
 template <int NPE>
 __global__ __launch_bounds__(64) void k_tl_elem(int n_el, int ngf, const double *__restrict__ gf,
                                                const int32_t *__restrict__ conn, const int32_t *__restrict__ slot,
-                                               const double *__restrict__ u, int which, double *__restrict__ Ke,
-                                               double *__restrict__ ye) {
+                                               const double *__restrict__ u, double *__restrict__ Ke,
+                                               double *__restrict__ Kg, double *__restrict__ ye) {
     using EL = Elem<NPE>;
     constexpr int NG = EL::NGP, NP = EL::NPAIR;
     constexpr PairTable<NPE> PT = make_pairs<NPE>();
@@ -337,38 +338,35 @@ __global__ __launch_bounds__(64) void k_tl_elem(int n_el, int ngf, const double 
     __syncthreads();
     if (Ke && t < NP) {
         const int i = PT.i[t], j = PT.j[t];
-        double K[9];
+        double K[9], kg = 0.0;
 #pragma unroll
         for (int m = 0; m < 9; ++m) K[m] = 0.0;
 #pragma unroll
         for (int q = 0; q < NG; ++q) {
             const double gi[3] = {g[q][i][0], g[q][i][1], g[q][i][2]};
             const double gj[3] = {g[q][j][0], g[q][j][1], g[q][j][2]};
-            if (which != 1) {
-                const double cl = scl[q], cm = scm[q];
-                const double dot = gi[0] * gj[0] + gi[1] * gj[1] + gi[2] * gj[2];
-                double ai[3], aj[3];
+            const double cl = scl[q], cm = scm[q];
+            const double dot = gi[0] * gj[0] + gi[1] * gj[1] + gi[2] * gj[2];
+            double ai[3], aj[3];
 #pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    ai[c] = Fq[q][c * 3] * gi[0] + Fq[q][c * 3 + 1] * gi[1] + Fq[q][c * 3 + 2] * gi[2];
-                    aj[c] = Fq[q][c * 3] * gj[0] + Fq[q][c * 3 + 1] * gj[1] + Fq[q][c * 3 + 2] * gj[2];
-                }
-#pragma unroll
-                for (int c = 0; c < 3; ++c)
-#pragma unroll
-                    for (int d = 0; d < 3; ++d)
-                        K[c * 3 + d] += cl * ai[c] * aj[d] + cm * (dot * FFq[q][c * 3 + d] + aj[c] * ai[d]);
+            for (int c = 0; c < 3; ++c) {
+                ai[c] = Fq[q][c * 3] * gi[0] + Fq[q][c * 3 + 1] * gi[1] + Fq[q][c * 3 + 2] * gi[2];
+                aj[c] = Fq[q][c * 3] * gj[0] + Fq[q][c * 3 + 1] * gj[1] + Fq[q][c * 3 + 2] * gj[2];
             }
-            if (which != 0) {
-                double kg = 0.0;
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    K[c * 3 + d] += cl * ai[c] * aj[d] + cm * (dot * FFq[q][c * 3 + d] + aj[c] * ai[d]);
+            if (Kg) {
+                double v = 0.0;
 #pragma unroll
                 for (int A = 0; A < 3; ++A)
-                    kg += gi[A] * (Sq[q][A * 3] * gj[0] + Sq[q][A * 3 + 1] * gj[1] + Sq[q][A * 3 + 2] * gj[2]);
-                K[0] += kg;
-                K[4] += kg;
-                K[8] += kg;
+                    v += gi[A] * (Sq[q][A * 3] * gj[0] + Sq[q][A * 3 + 1] * gj[1] + Sq[q][A * 3 + 2] * gj[2]);
+                kg += v;
             }
         }
+        if (Kg) Kg[(size_t)e * NP + t] = kg;
         double *out = Ke + ((size_t)e * NP + t) * 9;
 #pragma unroll
         for (int m = 0; m < 9; ++m) out[m] = K[m];
@@ -430,17 +428,23 @@ __global__ __launch_bounds__(256) void k_asm_vals(int nnzb, int n_el, int ngf, c
 }
 
 // The same from stored element matrices, element-major packed pairs
-// Ke[(e * NPAIR + p) * 9 + m] (the finite-strain blocks of k_tl_elem).
-template <int NPE>
+// Ke[(e * NPAIR + p) * 9 + m] (the finite-strain blocks of k_tl_elem).  With Kg
+// (GEO) the values are those of Km + Kg, and Km's and Kg's alone go to vm and vg
+// where asked for: one pass over the contributions instead of one each for Km, Kg
+// and their sum, and one of the elements (37 x 3 x 5 hexes: 133 us for the three
+// of each).
+template <int NPE, bool GEO>
 __global__ __launch_bounds__(256) void k_asm_vals_ke(int nnzb, const int32_t *__restrict__ cptr,
                                                  const int32_t *__restrict__ contrib,
                                                  const int32_t *__restrict__ blk_row,
                                                  const int32_t *__restrict__ brow, const double *__restrict__ Ke,
-                                                 double *__restrict__ vals, float *__restrict__ vals32) {
+                                                 const double *__restrict__ Kg, double *__restrict__ vals,
+                                                 float *__restrict__ vals32, double *__restrict__ vm,
+                                                 double *__restrict__ vg) {
     using EL = Elem<NPE>;
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nnzb) return;
-    double acc[9];
+    double acc[9], kg = 0.0;
 #pragma unroll
     for (int m = 0; m < 9; ++m) acc[m] = 0.0;
     const int k1 = cptr[s + 1];
@@ -448,12 +452,13 @@ __global__ __launch_bounds__(256) void k_asm_vals_ke(int nnzb, const int32_t *__
         const int c = contrib[k];
         const int e = c / (NPE * NPE), rem = c - e * NPE * NPE;
         const int i = rem / NPE, j = rem - i * NPE;
+        const size_t pair = (size_t)e * EL::NPAIR + (i <= j ? pair_index<NPE>(i, j) : pair_index<NPE>(j, i));
+        const double *B = Ke + 9 * pair;
+        if (GEO) kg += Kg[pair];
         if (i <= j) {
-            const double *B = Ke + ((size_t)e * EL::NPAIR + pair_index<NPE>(i, j)) * 9;
 #pragma unroll
             for (int m = 0; m < 9; ++m) acc[m] += B[m];
         } else {
-            const double *B = Ke + ((size_t)e * EL::NPAIR + pair_index<NPE>(j, i)) * 9;
 #pragma unroll
             for (int a = 0; a < 3; ++a)
 #pragma unroll
@@ -468,8 +473,11 @@ __global__ __launch_bounds__(256) void k_asm_vals_ke(int nnzb, const int32_t *__
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             const size_t o = base + (size_t)c * 3 * nb + d;
-            vals[o] = acc[c * 3 + d];
-            vals32[o] = (float)acc[c * 3 + d];
+            const double g = GEO && c == d ? kg : 0.0, v = acc[c * 3 + d] + g;
+            vals[o] = v;
+            vals32[o] = (float)v;
+            if (GEO && vm) vm[o] = acc[c * 3 + d];
+            if (GEO && vg) vg[o] = g;
         }
 }
 
@@ -606,13 +614,13 @@ hipError_t launch_element_matrices(jfm_ctx *ctx) {
     return hipGetLastError();
 }
 
-hipError_t launch_tl_element_matrices(jfm_ctx *ctx, const double *u, int which, double *Ke, double *ye) {
+hipError_t launch_tl_element_matrices(jfm_ctx *ctx, const double *u, double *Ke, double *Kg, double *ye) {
     const int n = (int)ctx->n_el;
     if (n == 0) return hipSuccess;
     switch (ctx->npe) {
-    case 10: k_tl_elem<10><<<n, 64, 0, ctx->stream>>>(n, ctx->ngf, ctx->gf64, ctx->conn, ctx->inc_slot, u, which, Ke, ye); break;
-    case 4: k_tl_elem<4><<<n, 64, 0, ctx->stream>>>(n, ctx->ngf, ctx->gf64, ctx->conn, ctx->inc_slot, u, which, Ke, ye); break;
-    case 8: k_tl_elem<8><<<n, 64, 0, ctx->stream>>>(n, ctx->ngf, ctx->gf64, ctx->conn, ctx->inc_slot, u, which, Ke, ye); break;
+    case 10: k_tl_elem<10><<<n, 64, 0, ctx->stream>>>(n, ctx->ngf, ctx->gf64, ctx->conn, ctx->inc_slot, u, Ke, Kg, ye); break;
+    case 4: k_tl_elem<4><<<n, 64, 0, ctx->stream>>>(n, ctx->ngf, ctx->gf64, ctx->conn, ctx->inc_slot, u, Ke, Kg, ye); break;
+    case 8: k_tl_elem<8><<<n, 64, 0, ctx->stream>>>(n, ctx->ngf, ctx->gf64, ctx->conn, ctx->inc_slot, u, Ke, Kg, ye); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -632,13 +640,17 @@ hipError_t launch_assemble_values(jfm_ctx *ctx) {
     return hipGetLastError();
 }
 
-hipError_t launch_assemble_values_ke(jfm_ctx *ctx, const double *Ke) {
+hipError_t launch_assemble_values_ke(jfm_ctx *ctx, const double *Ke, const double *Kg, double *vm, double *vg) {
     const int n = (int)ctx->nnzb;
     if (n == 0) return hipSuccess;
+    auto launch = [&](auto kernel) {
+        kernel<<<nblk(n), kBlock, 0, ctx->stream>>>(n, ctx->cptr, ctx->contrib, ctx->blk_row, ctx->brow, Ke, Kg, ctx->vals64,
+                                                    ctx->vals32, vm, vg);
+    };
     switch (ctx->npe) {
-    case 10: k_asm_vals_ke<10><<<nblk(n), kBlock, 0, ctx->stream>>>(n, ctx->cptr, ctx->contrib, ctx->blk_row, ctx->brow, Ke, ctx->vals64, ctx->vals32); break;
-    case 4: k_asm_vals_ke<4><<<nblk(n), kBlock, 0, ctx->stream>>>(n, ctx->cptr, ctx->contrib, ctx->blk_row, ctx->brow, Ke, ctx->vals64, ctx->vals32); break;
-    case 8: k_asm_vals_ke<8><<<nblk(n), kBlock, 0, ctx->stream>>>(n, ctx->cptr, ctx->contrib, ctx->blk_row, ctx->brow, Ke, ctx->vals64, ctx->vals32); break;
+    case 10: launch(Kg ? k_asm_vals_ke<10, true> : k_asm_vals_ke<10, false>); break;
+    case 4: launch(Kg ? k_asm_vals_ke<4, true> : k_asm_vals_ke<4, false>); break;
+    case 8: launch(Kg ? k_asm_vals_ke<8, true> : k_asm_vals_ke<8, false>); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -179,6 +179,8 @@ struct jfm_ctx {
     std::mutex pattern_mutex;             // and its making
     int32_t *brow = nullptr, *bcol = nullptr, *bdiag = nullptr, *blk_row = nullptr;
     int32_t *cptr = nullptr, *contrib = nullptr;
+    double *tl_ws = nullptr;      // finite-strain assembly: element blocks, Km's and Kg's values (kept up to 512 MB)
+    int64_t tl_ws_n = 0;
     double *vals64 = nullptr;
     float *vals32 = nullptr;
     double *Ke = nullptr;      // EBE element matrices: entry q = 9 p + m at [((q / 2) n_el + e) 2 + q % 2]
@@ -409,14 +411,16 @@ hipError_t launch_mesh_lists(jfm_ctx *ctx, int32_t *scratch, int32_t **flags);
 hipError_t launch_pattern_write(jfm_ctx *ctx, const int32_t *scratch);
 hipError_t launch_element_matrices(jfm_ctx *ctx);
 hipError_t launch_assemble_values(jfm_ctx *ctx);
-// finite-strain element matrices (which: 0 Km, 1 Kg, 2 Km + Kg), element-major
-// into Ke and, when ye != null, f_int(u) into the incidence slots
-hipError_t launch_tl_element_matrices(jfm_ctx *ctx, const double *u, int which, double *Ke, double *ye);
+// finite-strain element matrices Km, element-major into Ke, the factors of I of
+// Kg's blocks into Kg (when not null) and, when ye != null, f_int(u) into the
+// incidence slots
+hipError_t launch_tl_element_matrices(jfm_ctx *ctx, const double *u, double *Ke, double *Kg, double *ye);
 // Values per element of the EBE matrices: 9 NPAIR rounded up to a multiple
 // of the chunk width V (2 doubles or 4 floats).
 inline int64_t ke_stride(int npair, int V) { return (9 * (int64_t)npair + V - 1) / V * V; }
-// CSR values from element-major packed blocks Ke[(e * NPAIR + p) * 9 + m]
-hipError_t launch_assemble_values_ke(jfm_ctx *ctx, const double *Ke);
+// CSR values from element-major packed blocks Ke[(e * NPAIR + p) * 9 + m] (and Kg's
+// factors: then of the sum, and Km's and Kg's alone to vm and vg when not null)
+hipError_t launch_assemble_values_ke(jfm_ctx *ctx, const double *Ke, const double *Kg, double *vm, double *vg);
 hipError_t launch_face_loads(jfm_ctx *ctx);
 hipError_t launch_block_jacobi(jfm_ctx *ctx, double *Minv64, float *Minv32);
 // Two-phase operators; `part` (may be null) receives one partial of
