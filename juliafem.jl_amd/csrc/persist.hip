@@ -699,6 +699,7 @@ template <typename T, bool COARSE> struct CoarseLds {};
 template <typename T> struct CoarseLds<T, true> {
     float w[kMaxCoarse], z[kMaxCoarse];  // w = Q' m r (the GEMV's operand, zero padded), zc
     T d[3 * kNT];                        // the nodes' offsets
+    float zr[kMaxCoarse];                // the workgroup's rows of zc
     double wz[kNT / 64];
     int start[kMaxEntries + 1], slot[kMaxEntries];
     uint16_t list[kNT];
@@ -886,7 +887,11 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
             uint64_t *zw = A.zw + (size_t)(p / kGroup) * nc;
             const int copies = (nwg + kGroup - 1) / kGroup, ld4 = A.ldc / 4;
             const float4 *w4 = reinterpret_cast<const float4 *>(co.w);
-            for (int row = p + nwg * wv; row < nc; row += nwg * (NT / 64)) {
+            // this workgroup's rows, stored together: a row at a time from any
+            // wave, each line of a copy took eight stores
+            const int per = (nc + nwg - 1) / nwg, row0 = p * per, nrow = min(per, nc - row0);
+            for (int i = wv; i < nrow; i += NT / 64) {
+                const int row = row0 + i;
                 const float4 *Ar = reinterpret_cast<const float4 *>(A.Ahat) + (size_t)row * ld4;
                 double s = 0.0;
 #pragma unroll 4
@@ -895,7 +900,12 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
                     s += (double)a.x * b.x + (double)a.y * b.y + (double)a.z * b.z + (double)a.w * b.w;
                 }
                 const float zr = (float)wave_total(s);
-                if (lane < copies) put_word(A.zw + (size_t)lane * nc + row, epoch, __float_as_uint(zr));
+                if (lane == 0) co.zr[i] = zr;
+            }
+            __syncthreads();
+            for (int i = t; i < nrow * copies; i += NT) {
+                const int c = i / nrow, k = i - c * nrow;
+                put_word(A.zw + (size_t)c * nc + row0 + k, epoch, __float_as_uint(co.zr[k]));
             }
             double wz = 0.0;
 #pragma unroll
