@@ -106,7 +106,7 @@ __global__ __launch_bounds__(kRT, 2) void k_pcg_rows(const RowsArgs<T> A0) {
     const int g = (int)blockIdx.x, t = (int)threadIdx.x, nwg = A.nwg;
     const int n0 = min(g * A.per, A.N), nown = min(n0 + A.per, A.N) - n0, nloc = A.nloc[g];
     const int32_t *loc = A.loc + (size_t)g * kLocal;
-    uint64_t *wordsB = A.words, *wordsC = wordsB + grid_words(1, nwg);
+    uint64_t *wordsB = A.words, *wordsC = wordsB + grid_words(1, nwg, true);
     const Partials<T> zb(A.z, A.N);
     if (t == 0) bad = 0;
     const bool own = t < nown;
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(kRT, 2) void k_pcg_rows(const RowsArgs<T> A0) {
     __syncthreads();  // bad, own0, ps
     const int me = 3 * (own0 + t);
     uint32_t epoch = 1;
-    if (!grid_sum<1, kRT>(bb, wordsB, g, nwg, epoch, shB, &bad)) {
+    if (!grid_sum<1, kRT, true>(bb, wordsB, g, nwg, epoch, shB, &bad)) {
         if (t == 0) A.S->fail = 1;
         return;
     }
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kRT, 2) void k_pcg_rows(const RowsArgs<T> A0) {
         ++epoch;
         if (own) zb.template put<3>(node, z);
         stores_done();  // before the block barrier in grid_sum, hence before its words
-        if (!grid_sum<2, kRT>(s2, wordsC, g, nwg, epoch, shC, &bad)) break;
+        if (!grid_sum<2, kRT, true>(s2, wordsC, g, nwg, epoch, shC, &bad)) break;
         rr = s2[1];
         if (epoch == 2) rr0 = rr;  // the start
         else ++it;
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(kRT, 2) void k_pcg_rows(const RowsArgs<T> A0) {
             q[c] = own && !(fx >> c & 1u) ? qs[3 * t + c] : T(0);
             e1[0] += (double)pv[c] * (double)q[c];
         }
-        if (!grid_sum<1, kRT>(e1, wordsB, g, nwg, epoch, shB, &bad)) break;
+        if (!grid_sum<1, kRT, true>(e1, wordsB, g, nwg, epoch, shB, &bad)) break;
         pq = e1[0];
         alpha_d = (pq > 0.0 && finite(pq)) ? rz / pq : 0.0;
         const T alpha = (T)alpha_d;
@@ -296,7 +296,7 @@ int jfem_rows_setup(jfm_ctx *ctx) {
     const bool ok = d_bad && (R.nloc = jfm_alloc<int32_t>(ctx, R.nwg)) &&
                     (R.loc = jfm_alloc<int32_t>(ctx, (int64_t)R.nwg * kLocal)) &&
                     (R.lcol = jfm_alloc<uint16_t>(ctx, ctx->nnzb)) && (R.z = jfm_alloc<double>(ctx, 4 * (int64_t)N)) &&
-                    (R.words = jfm_alloc<uint64_t>(ctx, grid_words(1, R.nwg) + grid_words(2, R.nwg)));
+                    (R.words = jfm_alloc<uint64_t>(ctx, grid_words(1, R.nwg, true) + grid_words(2, R.nwg, true)));
     if (!ok) {
         jfm_free(ctx, d_bad);
         jfem_rows_release(ctx);
@@ -350,7 +350,7 @@ hipError_t launch_pcg_rows(jfm_ctx *ctx, const T *Minv, const T *b, const T *r0,
     A.rtol2 = rtol * rtol;
     A.maxit = maxit;
     A.S = ctx->S;
-    launch_persist_clear(ctx, grid_words(1, R.nwg) + grid_words(2, R.nwg), R.words, 0, nullptr, 1, A.S);
+    launch_persist_clear(ctx, grid_words(1, R.nwg, true) + grid_words(2, R.nwg, true), R.words, 0, nullptr, 1, A.S);
     k_pcg_rows<T><<<R.nwg, kRT, 0, ctx->stream>>>(A);
     return hipGetLastError();
 }

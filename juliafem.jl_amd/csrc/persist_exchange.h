@@ -133,17 +133,22 @@ __device__ __forceinline__ double wave_total(double v) {
 // one request to store and, with the neighbours', one to read (as rows of single
 // words, which is four requests for two values, an iteration of 240 workgroups
 // took 0.9 us longer; one hop with 16 copies of all entries, 0.4 us longer than
-// that).  One wave polls:
-// lane 16 k + m reads value k of member m, so a sum over members is a row sum.
+// that).  One wave polls: lane 16 k + m reads value k of member m, so a sum over
+// members is a row sum.
+// FLAT: 17 to 64 workgroups store their entries once per 8 workgroups, and each
+// reads its copy of all of them, one hop (63 workgroups on the CSR matrix: 0.4 us
+// an iteration less; nothing gained with 102, and the element kernels, which have
+// no registers for it, lose 2-5%).
 // Calls that follow each other without a block barrier use different `sh` (a
 // wave may still read it when the next one starts).
-constexpr int kGroup = 16, kCopy = 8;
-template <int NV> struct GridSumLds { double a[NV][16], b[NV]; };
+constexpr int kGroup = 16, kCopy = 8, kFlat = 64;
+template <int NV> struct GridSumLds { double a[NV][16], b[NV], f[NV][2]; };
 static_assert(kPersistPatches <= kGroup * kGroup && kPersistPatches / kCopy <= 32, "two levels, copies x values in a wave");
 
 // words of n workgroups: their entries, then the copies of the groups' sums
-__host__ __device__ constexpr int grid_words(int nv, int n) {
-    return 2 * nv * (n + (n > kGroup ? (n + kCopy - 1) / kCopy * kGroup : 0));
+__host__ __device__ constexpr int grid_words(int nv, int n, bool flat = false) {
+    const int copies = (n + kCopy - 1) / kCopy;
+    return 2 * nv * (flat && n > kGroup && n <= kFlat ? copies * n : n + (n > kGroup ? copies * kGroup : 0));
 }
 
 struct Entries {  // past the L2, as the partials
@@ -175,7 +180,7 @@ __device__ __forceinline__ double sum_members(const Entries &en, int first, int 
     return row_sum(k < NV && m < n ? en.get((first + m) * NV + k, epoch, bad) : 0.0);
 }
 
-template <int NV, int NT>
+template <int NV, int NT, bool FLAT = false>
 __device__ __forceinline__ bool grid_sum(double (&v)[NV], uint64_t *words, int wg, int nwg, uint32_t epoch,
                                          GridSumLds<NV> &sh, int *bad) {
     static_assert(NV <= 2 && NT / 64 <= 16, "one row of 16 lanes per value");
@@ -187,6 +192,30 @@ __device__ __forceinline__ bool grid_sum(double (&v)[NV], uint64_t *words, int w
         if (lane == 0) sh.a[k][wv] = w;
     }
     __syncthreads();
+    if (FLAT && nwg > kGroup && nwg <= kFlat) {
+        const Entries en(words, grid_words(NV, nwg, true));
+        if (wv == 0) {
+            const int k = lane >> 4, m = lane & 15;
+            const double s = row_sum(k < NV && m < kW ? sh.a[k < NV ? k : 0][m] : 0.0);
+            double mine = lane_of(s, 0);
+            if constexpr (NV == 2) mine = lane & 1 ? lane_of(s, 16) : mine;
+            const int c = lane / NV;
+            if (c < (nwg + kCopy - 1) / kCopy) en.put((c * nwg + wg) * NV + lane % NV, epoch, mine);
+        }
+        if (wv < NV) {
+            const int i = (int)threadIdx.x;  // member i / NV, value i % NV
+            const double e = i < nwg * NV ? en.get(wg / kCopy * nwg * NV + i, epoch, bad) : 0.0;
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                const double w = wave_total(i % NV == k ? e : 0.0);
+                if (lane == 0) sh.f[k][wv] = w;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NV; ++k) v[k] = NV == 2 ? sh.f[k][0] + sh.f[k][NV - 1] : sh.f[k][0];
+        return *bad == 0;
+    }
     if (wv == 0) {
         const int k = lane >> 4, m = lane & 15;
         double s = row_sum(k < NV && m < kW ? sh.a[k < NV ? k : 0][m] : 0.0);  // row k: the block's value k
