@@ -23,9 +23,12 @@
  *   - Results are deterministic: no floating-point atomics anywhere; every
  *     sum has a fixed order (ascending element id for nodal sums, fixed
  *     reduction trees for dot products), so repeated calls give identical bits.
- *   - PCG iterations run in batches captured as HIP graphs; setting the
- *     environment variable JFEM_GRAPHS=0 launches the same kernels one by
- *     one instead (for tools that do not follow graph launches).
+ *   - On small and medium meshes a whole PCG runs in one kernel that stays
+ *     resident (persist.hip, persist_csr.hip); JFEM_PERSIST=0 launches its
+ *     iterations instead (same answers up to the order of the reductions).
+ *     Launched iterations run in batches captured as HIP graphs; JFEM_GRAPHS=0
+ *     launches the same kernels one by one (for tools that do not follow graph
+ *     launches).
  */
 #ifndef JFEM_H
 #define JFEM_H
@@ -108,7 +111,8 @@ typedef struct {
     int64_t n_nodes, n_el, n_dofs, nnz, nnzb, n_faces;
     int32_t npe, affine;
     int64_t device_bytes;  /* bytes currently allocated by the context */
-    /* patch form of the matrix-free operator (0 until it is first used):
+    /* patch form of the matrix-free operator (0 until it is made: with the
+     * upload where iterations will be launched, else on its first use):
      * patches of 480 elements, their (patch, node) entries, the nodes shared
      * between patches and their partial sums; the bytes per connectivity
      * entry the patch kernel reads (2: offsets from each patch's lowest node
@@ -179,13 +183,16 @@ int jfm_apply(jfm_ctx *ctx, int32_t op, int32_t precision, const double *x, doub
  * loops with fixed memory).  x and y are DEVICE pointers (n_dofs doubles);
  * the work is enqueued on `stream` (a hipStream_t; NULL = the context's
  * stream) and the call returns without synchronising.  op is
- * JFM_OP_MATFREE (two-phase form) or JFM_OP_EBE (after the element matrices
- * exist, i.e. after one jfm_apply or jfm_assemble with it).  The element
- * results (3 npe n_el values) and, in FP32, the converted vectors live in
+ * JFM_OP_MATFREE or JFM_OP_EBE (after the element matrices exist, i.e. after one
+ * jfm_apply or jfm_assemble with it).  The patch form runs where the upload made
+ * the patches (meshes beyond the resident PCG's range of at least 64 patches of
+ * 480 elements, Hex8 192), the two-phase form elsewhere.  The two-phase form's
+ * element results (3 npe n_el values) and, in FP32, the converted vectors live in
  * one 64 MiB device array per GPU held until the process ends: meshes that
- * need more (e.g. more than 279,620 Tet10 elements in FP64) get JFM_EINVAL.
- * Every call on a GPU shares that array, so calls that overlap on one GPU
- * race.  Same result as jfm_apply up to the order of the nodal sums. */
+ * would need more (e.g. more than 279,620 Tet10 elements in FP64) get JFM_EINVAL
+ * in either form.  Calls that overlap on one GPU race on that array, or, in the
+ * patch form in FP64, only where they are of one context.  Same result as
+ * jfm_apply up to the order of the nodal sums. */
 int jfm_apply_noalloc(jfm_ctx *ctx, int32_t op, int32_t precision, const double *x, double *y, void *stream);
 
 /* Average device times (ms) over `reps` back-to-back applications on
