@@ -913,10 +913,15 @@ static int pcg_run(jfm_ctx *ctx, int op, const T *Minv, double rtol, int maxit, 
     }
     CHECK_LAUNCH(ctx, launch_dot<T>(ctx, b, b, n, &np));
     if (int rc = finalize_misc(ctx, np, 1, FIN_BB)) return rc;
-    CHECK_LAUNCH(ctx, launch_pcg_init<T>(ctx, r, z, p, Minv, &np));
+    const bool ordered = coarse && jfem_coarse_fused_restriction(ctx);
+    if (ordered)
+        if (int rc = jfem_coarse_order(ctx)) return rc;
+    CHECK_LAUNCH(ctx, launch_pcg_init<T>(ctx, r, z, p, Minv, &np, ordered));
     if (coarse) CHECK_LAUNCH(ctx, launch_coarse_correct<T>(ctx, r, z, p, ctx->partials + kPartMisc, nullptr, &np));
-    if (coarse && jfem_coarse_fused_restriction(ctx))
+    if (ordered) {
         if (int rc = jfem_patch_qsrc(ctx)) return rc;
+        Minv = (const T *)ctx->MA;  // what the iterations read (one captured graph for all blocks)
+    }
     if (int rc = finalize_misc(ctx, np, 2, FIN_INIT)) return rc;
     // Batches of up to check_every iterations; once the residual falls, the
     // next batch is the power of two that covers the iterations its rate

@@ -1124,6 +1124,7 @@ void jfem_coarse_release(jfm_ctx *ctx) {
     free_dev(ctx, ctx->Rinv); free_dev(ctx, ctx->Ac); free_dev(ctx, ctx->Ac2); free_dev(ctx, ctx->Ahat32);
     free_dev(ctx, ctx->wc32); free_dev(ctx, ctx->zc32); free_dev(ctx, ctx->wc64);
     free_dev(ctx, ctx->cdA64); free_dev(ctx, ctx->cdA32); free_dev(ctx, ctx->apos); free_dev(ctx, ctx->rA);
+    free_dev(ctx, ctx->MA); free_dev(ctx, ctx->fixedA);
     free_dev(ctx, ctx->gjP);
     free_dev(ctx, ctx->pv6); free_dev(ctx, ctx->qv6); free_dev(ctx, ctx->ye6);
     free_dev(ctx, ctx->gal_el); free_dev(ctx, ctx->gal_gptr); free_dev(ctx, ctx->gal_glist);
@@ -1597,6 +1598,13 @@ hipError_t launch_coarse_gemv_fused(jfm_ctx *ctx, int slot, int *npart_wz) {
 
 template <> double *coarse_rA<double>(jfm_ctx *ctx) { return ctx->rA; }
 template <> float *coarse_rA<float>(jfm_ctx *ctx) { return (float *)ctx->rA; }
+
+int jfem_coarse_order(jfm_ctx *ctx) {
+    if (!ctx->MA) ctx->MA = jfm_alloc<double>(ctx, 9 * ctx->N);
+    if (!ctx->fixedA) ctx->fixedA = jfm_alloc<uint8_t>(ctx, ctx->N);
+    if (!ctx->MA || !ctx->fixedA) return jfm_fail(ctx, JFM_ENOMEM, "ordered preconditioner blocks: allocation failed");
+    return JFM_OK;
+}
 
 // coarse correction outside the iteration (PCG start, training):
 // z += Q A_c^-1 Q' r, optionally p = z; partials (r.z, r.r) to `part`

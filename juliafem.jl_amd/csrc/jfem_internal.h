@@ -286,6 +286,8 @@ struct jfm_ctx {
     double *Ac2 = nullptr;
     int32_t *apos = nullptr;       // node -> its position in agg_nodes
     double *rA = nullptr;          // 3 x N: the masked residual in aggregate order (FP64 or FP32 view)
+    double *MA = nullptr;          // 9 x N: the PCG's blocks in aggregate order (FP64 or FP32 view)
+    uint8_t *fixedA = nullptr;     // N: the fixed mask in aggregate order, a bit per component
     double *cdA64 = nullptr;       // cd in aggregate order (agg_nodes), for the restriction
     float *cdA32 = nullptr;
     int64_t ldc = 0;               // row stride of Ahat32: nc rounded up to 256, zero padded
@@ -530,6 +532,9 @@ hipError_t launch_coarse_product(jfm_ctx *ctx, const T *r, const int *done, int 
 template <typename T>
 hipError_t launch_coarse_product_agg(jfm_ctx *ctx, const T *rA, const int *done, int *npart_wz);
 template <typename T> T *coarse_rA(jfm_ctx *ctx);
+// Room for the blocks and the fixed mask in aggregate order (MA, fixedA), which
+// the update with the fused restriction reads.
+int jfem_coarse_order(jfm_ctx *ctx);
 // The iteration's coarse right-hand side w = Q' m r of the new residual,
 // formed inside the update kernel, one block per aggregate
 // (launch_pcg_update(..., restrict_q = true)), in FP64 at wc64 + (slot ^ 1)
@@ -561,8 +566,10 @@ hipError_t launch_post_join(jfm_ctx *ctx, const double *x0, const double *x1, do
 template <typename T>
 hipError_t launch_bsr_spmv(jfm_ctx *ctx, const T *vals, const T *x, T *y, const T *dotv, double *part,
                            const int *done, int *npart);
+// order: r (to coarse_rA<T>(ctx)), the blocks and the fixed mask also in
+// aggregate order; the update with the fused restriction keeps r there
 template <typename T>
-hipError_t launch_pcg_init(jfm_ctx *ctx, T *r, T *z, T *p, const T *Minv, int *npart);
+hipError_t launch_pcg_init(jfm_ctx *ctx, T *r, T *z, T *p, const T *Minv, int *npart, bool order = false);
 // With shared_q (and restrict_q), q holds only what the patch kernel writes
 // and the update sums the shared nodes' partial slots itself (qsrc).
 template <typename T>

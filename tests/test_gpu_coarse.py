@@ -269,3 +269,50 @@ def test_coarse_matrix_element_products(oracle, tmp_path, gen, dims, seed, sig, 
     db = np.abs(_block_norms(A, nag) - _block_norms(Ao, nag)).max() / s
     say(f"  eigenvalues {evo.min():.3e}..{evo.max():.3e}: rel diff {de:.2e}; block norms rel diff {db:.2e}")
     assert de <= 1e-11 and db <= 1e-11
+
+
+_CHILD_ORDER = r"""
+import sys
+import numpy as np
+sys.path[:0] = [{root!r}, {pkg!r}]
+import jfem
+from jfem import mesh as M
+m = M.{gen}(*{dims}, seed=5, jitter=0.1, E_sigma=0.4)
+c = jfem.Context(0)
+c.upload_mesh(m.X, m.conn, m.etype, m.E, m.nu)
+c.upload_bcs(np.load({fixed!r}), None, m.faces, m.ftype, m.face_traction())
+out = {{}}
+for meth in (0, 1):
+    for rep in (0, 1):
+        print("launched two-level, method", meth, flush=True)
+        out["u%d%d" % (meth, rep)] = c.solve(method=meth, rtol=1e-10, inner_rtol=1e-2, coarse_nodes={cn})[0]
+np.savez({out!r}, **out)
+"""
+
+
+@pytest.mark.parametrize("gen,dims,cn", [("box_tet10", (1, 1, 1), 64), ("box_tet10", (19, 6, 3), 1000000),
+                                         ("box_tet10", (14, 6, 4), 40), ("box_tet4", (24, 9, 8), 200),
+                                         ("box_hex8", (17, 5, 3), 100)])
+def test_launched_update_in_aggregate_order(oracle, tmp_path, gen, dims, cn):
+    """The launched two-level iterations (JFEM_PERSIST=0, a child process) keep
+    r, the blocks and the fixed mask in aggregate order: one aggregate of the
+    whole mesh (more nodes than a block's first loads hold), many small ones,
+    and nodes with one or two fixed components (the mask's bits).  To the bar
+    of the FP64 solves, and the second solve bit for bit the first."""
+    m = getattr(M, gen)(*dims, seed=5, jitter=0.1, E_sigma=0.4)
+    fixed = m.fixed_mask().copy()
+    far = np.flatnonzero(m.X[:, 1] == m.X[:, 1].max())
+    fixed[3 * far + 1] = 1
+    fixed[3 * far[::3] + 2] = 1
+    np.save(str(tmp_path / "fixed.npy"), fixed)
+    csr = oracle.assemble_csr(m)
+    ud, _, _ = oracle.solve_direct_lapack(csr, fixed, np.zeros(m.n_dofs), oracle.load_vector(m))
+    out = str(tmp_path / "u.npz")
+    say(f"{gen} {dims} coarse_nodes={cn}")
+    code = _CHILD_ORDER.format(root=ROOT, pkg=os.path.join(ROOT, "juliafem.jl_amd"), gen=gen, dims=dims, cn=cn,
+                               fixed=str(tmp_path / "fixed.npy"), out=out)
+    subprocess.run([sys.executable, "-c", code], env=dict(os.environ, JFEM_PERSIST="0"), check=True, timeout=60)
+    r = np.load(out)
+    for meth in (0, 1):
+        assert np.linalg.norm(r[f"u{meth}0"] - ud) <= 1e-8 * np.linalg.norm(ud)
+        assert np.array_equal(r[f"u{meth}0"], r[f"u{meth}1"])
