@@ -503,11 +503,21 @@ static hipError_t op_apply(jfm_ctx *ctx, int op, const T *x, T *y, const T *dotv
     return launch_two_phase<T>(ctx, op, x, y, dotv, part, done, npart);
 }
 
+// y = K x in FP64 outside of an iteration (residuals, reactions, internal
+// forces).  The matrix-free product takes the patch form where the upload made the
+// patches and not where an earlier call did: the two forms sum in different orders,
+// and a mesh always gives the same bits.
+static hipError_t op_product(jfm_ctx *ctx, int op, const double *x, double *y) {
+    if (op != JFM_OP_MATFREE || ctx->patch_upload) return op_apply<double>(ctx, op, x, y, nullptr, nullptr, nullptr, nullptr);
+    const hipError_t e = launch_elem_only<double>(ctx, op, x, nullptr);
+    return e == hipSuccess ? launch_gather<double>(ctx, ctx->ye64, ctx->fixed, y, nullptr, nullptr, nullptr, nullptr) : e;
+}
+
 // Same without the row mask (all rows), for f_int and reactions.
-static hipError_t op_apply_all_rows(jfm_ctx *ctx, int op, const double *x, double *y) {
+static hipError_t op_product_all_rows(jfm_ctx *ctx, int op, const double *x, double *y) {
     uint8_t *saved = ctx->fixed;
     ctx->fixed = nullptr;
-    hipError_t e = op_apply<double>(ctx, op, x, y, nullptr, nullptr, nullptr, nullptr);
+    hipError_t e = op_product(ctx, op, x, y);
     ctx->fixed = saved;
     return e;
 }
@@ -602,7 +612,7 @@ extern "C" int jfm_assemble(jfm_ctx *ctx, const double *u, double *vals, double 
     // f = f_ext - f_int(u)  (src/problems_elasticity.jl:432-433)
     if (u) {
         JFM_HIP(ctx, hipMemcpyAsync(ctx->vx64, u, sizeof(double) * n, hipMemcpyHostToDevice, s));
-        CHECK_LAUNCH(ctx, op_apply_all_rows(ctx, JFM_OP_MATFREE, ctx->vx64, ctx->vy64));
+        CHECK_LAUNCH(ctx, op_product_all_rows(ctx, JFM_OP_MATFREE, ctx->vx64, ctx->vy64));
         CHECK_LAUNCH(ctx, (launch_convert<double, double>(ctx, ctx->vy64, ctx->vy64, n, -1.0)));
         std::vector<double> fi(n), fe(n);
         JFM_HIP(ctx, hipMemcpyAsync(fi.data(), ctx->vy64, sizeof(double) * n, hipMemcpyDeviceToHost, s));
@@ -869,6 +879,15 @@ struct ResidentHold {
 };
 }  // namespace
 
+// r = b - K x on the FP64 workspace, for a PCG that continues from x
+static int warm_residual(jfm_ctx *ctx, int op) {
+    const Workspace &w = ctx->ws64;
+    int np = 0;
+    CHECK_LAUNCH(ctx, op_product(ctx, op, (const double *)w.x, (double *)w.q));
+    CHECK_LAUNCH(ctx, launch_residual(ctx, (const double *)w.b, (const double *)w.q, ctx->fixed, (double *)w.r, ctx->ndof, &np));
+    return JFM_OK;
+}
+
 // PCG on the workspace of precision T: solves K x = b (free DOFs) from x = 0,
 // or from the current x with its true residual (warm, FP64 only).  The host
 // reads the scalars once per batch of `check_every` iterations.
@@ -876,18 +895,16 @@ template <typename T>
 static int pcg_run(jfm_ctx *ctx, int op, const T *Minv, double rtol, int maxit, int check_every, int *iters,
                    int *status, bool warm = false, bool coarse = false) {
     Workspace &w = ws_of<T>(ctx);
-    T *x = (T *)w.x, *r = (T *)w.r, *z = (T *)w.z, *p = (T *)w.p, *q = (T *)w.q, *b = (T *)w.b;
+    T *x = (T *)w.x, *r = (T *)w.r, *z = (T *)w.z, *p = (T *)w.p, *b = (T *)w.b;
     const int64_t n = ctx->ndof;
     hipStream_t s = ctx->stream;
+    const bool from_x = warm && sizeof(T) == 8;
     int np = 0;
     int resident = 1;
     if (int rc = jfem_persist_ready<T>(ctx, op, &resident, coarse)) return rc;
     if (resident) {
-        const bool from_x = warm && sizeof(T) == 8;
-        if (from_x) {
-            CHECK_LAUNCH(ctx, op_apply<T>(ctx, op, x, q, nullptr, nullptr, nullptr, nullptr));
-            CHECK_LAUNCH(ctx, launch_residual(ctx, (const double *)b, (const double *)q, ctx->fixed, (double *)r, n, &np));
-        }
+        if (from_x)
+            if (int rc = warm_residual(ctx, op)) return rc;
         const ResidentHold hold(ctx, jfem_persist_workgroups(ctx, op));  // until the kernel has ended
         CHECK_LAUNCH(ctx, launch_pcg_persist<T>(ctx, op, Minv, b, from_x ? r : nullptr, x, rtol, maxit, coarse));
         if (int rc = read_scalars(ctx)) return rc;
@@ -903,10 +920,9 @@ static int pcg_run(jfm_ctx *ctx, int op, const T *Minv, double rtol, int maxit, 
     ctx->S_host->rtol2 = rtol * rtol;
     ctx->S_host->maxit = maxit;
     if (int rc = write_scalars(ctx)) return rc;
-    if (warm && sizeof(T) == 8) {
+    if (from_x) {
         // restart from the current x with the true residual r = b - K x
-        CHECK_LAUNCH(ctx, op_apply<T>(ctx, op, x, q, nullptr, nullptr, nullptr, nullptr));
-        CHECK_LAUNCH(ctx, launch_residual(ctx, (const double *)b, (const double *)q, ctx->fixed, (double *)r, n, &np));
+        if (int rc = warm_residual(ctx, op)) return rc;
     } else {
         JFM_HIP(ctx, hipMemsetAsync(x, 0, sizeof(T) * n, s));
         JFM_HIP(ctx, hipMemcpyAsync(r, b, sizeof(T) * n, hipMemcpyDeviceToDevice, s));
@@ -957,7 +973,7 @@ static int pcg_run(jfm_ctx *ctx, int op, const T *Minv, double rtol, int maxit, 
 // FP64 true residual r = b - K u over free DOFs; *rnorm = |r|.
 static int true_residual(jfm_ctx *ctx, int op, const double *b, const double *u, double *r, double *rnorm) {
     int np = 0;
-    CHECK_LAUNCH(ctx, op_apply<double>(ctx, op, u, ctx->vy64, nullptr, nullptr, nullptr, nullptr));
+    CHECK_LAUNCH(ctx, op_product(ctx, op, u, ctx->vy64));
     CHECK_LAUNCH(ctx, launch_residual(ctx, b, ctx->vy64, ctx->fixed, r, ctx->ndof, &np));
     if (int rc = finalize_misc(ctx, np, 1, FIN_DOT)) return rc;
     if (int rc = read_scalars(ctx)) return rc;
@@ -1014,16 +1030,15 @@ extern "C" int jfm_solve(jfm_ctx *ctx, const jfm_solve_opts *opts, const double 
     JFM_HIP(ctx, hipSetDevice(ctx->device));
     const int op = opts->op;
     const int op_outer = opts->method == JFM_SOLVE_MIXED_IR ? opts->op_outer : op;
-    // A solve whose iterations run resident applies the operator itself only
-    // for its few FP64 residuals: these take the two-phase form then, and the
-    // 480-element patches (7 ms of host work at 12,810 Tet10 elements) are
-    // built by pcg_run if it has to launch after all.
+    // The 480-element patches of the matrix-free operator serve launched
+    // iterations (and, made with the upload, op_product): where the iterations may
+    // run resident, pcg_run makes them if it has to launch after all.
     const bool inner32 = opts->method == JFM_SOLVE_MIXED_IR;
-    const bool resident = inner32 ? op == op_outer && jfem_persist_maybe<float>(ctx, op) : jfem_persist_maybe<double>(ctx, op);
-    if (!(resident && op == JFM_OP_MATFREE)) {
+    const bool resident = inner32 ? jfem_persist_maybe<float>(ctx, op) : jfem_persist_maybe<double>(ctx, op);
+    if (op != JFM_OP_MATFREE || !resident)
         if (int rc = prepare_op(ctx, op)) return rc;
+    if (op_outer != JFM_OP_MATFREE)
         if (int rc = prepare_op(ctx, op_outer)) return rc;
-    }
     if (int rc = ensure_workspaces(ctx)) return rc;
     const int64_t n = ctx->ndof;
     hipStream_t s = ctx->stream;
@@ -1164,7 +1179,7 @@ extern "C" int jfm_solve(jfm_ctx *ctx, const jfm_solve_opts *opts, const double 
     JFM_HIP(ctx, hipMemcpyAsync(u, ctx->u64, sizeof(double) * n, hipMemcpyDeviceToHost, s));
     if (la) {
         // la = f - K u on fixed DOFs (src/solvers.jl:212-213), 0 elsewhere
-        CHECK_LAUNCH(ctx, op_apply_all_rows(ctx, op_outer, ctx->u64, ctx->vy64));
+        CHECK_LAUNCH(ctx, op_product_all_rows(ctx, op_outer, ctx->u64, ctx->vy64));
         std::vector<double> ku(n), ff(n);
         std::vector<uint8_t> fxd(n);
         JFM_HIP(ctx, hipMemcpyAsync(ku.data(), ctx->vy64, sizeof(double) * n, hipMemcpyDeviceToHost, s));
