@@ -180,9 +180,10 @@ int jfm_apply(jfm_ctx *ctx, int32_t op, int32_t precision, const double *x, doub
 
 /* K.u that allocates nothing: no counterpart in the reference.  For callers
  * that cannot allocate device memory (code under HIP graph capture, serving
- * loops with fixed memory).  x and y are DEVICE pointers (n_dofs doubles);
- * the work is enqueued on `stream` (a hipStream_t; NULL = the context's
- * stream) and the call returns without synchronising.  op is
+ * loops with fixed memory).  x and y are DEVICE pointers (n_dofs doubles), which
+ * may be the same or overlap (the two-phase form then); the work is enqueued on
+ * `stream` (a hipStream_t; NULL = the context's stream) and the call returns
+ * without synchronising.  op is
  * JFM_OP_MATFREE or JFM_OP_EBE (after the element matrices exist, i.e. after one
  * jfm_apply or jfm_assemble with it).  The patch form runs where the upload made
  * the patches (meshes beyond the resident PCG's range of at least 64 patches of

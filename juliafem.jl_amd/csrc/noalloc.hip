@@ -32,9 +32,12 @@ size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 // y = K x with the element results in ye, or by the patch operator with the
 // context's buffer of partial sums for these calls.  The patches are taken where
 // the upload made them and not where an earlier call did, so that a mesh always
-// gives the same bits.
+// gives the same bits, and where x and y are apart: the patch kernel writes y
+// while other workgroups still read x, the two-phase form only once x is read.
 template <typename T> hipError_t product(jfm_ctx *ctx, int op, const T *x, T *y, T *ye) {
-    if (ctx->patch_upload && jfem_patch_form(ctx, op)) {
+    const uintptr_t bytes = sizeof(T) * (uintptr_t)ctx->ndof, x0 = (uintptr_t)x, y0 = (uintptr_t)y;
+    const bool apart = x0 + bytes <= y0 || y0 + bytes <= x0;
+    if (apart && ctx->patch_upload && jfem_patch_form(ctx, op)) {
         double *const part = ctx->bpart;
         ctx->bpart = ctx->na_part;
         const hipError_t e = launch_patch_apply<T>(ctx, op, x, y, nullptr, nullptr, nullptr, nullptr);

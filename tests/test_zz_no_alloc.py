@@ -160,3 +160,27 @@ def test_patches_of_the_upload(env, gen, g):
             v.free()
     for c in cs:
         c.close()
+
+
+@pytest.mark.parametrize("op,prec", [("matfree", 0), ("matfree", 1), ("ebe", 0)])
+@pytest.mark.parametrize("shift", [0, 300])
+def test_noalloc_in_place(env, op, prec, shift):
+    """y = x, and y beginning inside x, on a mesh with the upload's patches: the
+    product of the values that x held, to the bars of jfm_apply (above)."""
+    jfem, lib, hip = env
+    m = box_tet10(91, 9, 7, seed=1, jitter=0.1, E_sigma=0.3)
+    c = jfem.Context(0)
+    c.upload(m)
+    assert c.info()["n_patches"] > 0
+    x = np.random.default_rng(3).standard_normal(m.n_dofs)
+    ref = c.apply(x, op=op)
+    say(f"noalloc in place {op} precision={prec} shift={shift}")
+    v = DeviceVec(hip, m.n_dofs + shift)
+    for _ in range(2):
+        v.put(np.concatenate([x, np.full(shift, np.nan)]))
+        assert hip.hipDeviceSynchronize() == 0
+        assert lib.jfm_apply_noalloc(c._h, _lib.OPS[op], prec, v.p, C.c_void_p(v.p.value + 8 * shift), None) == 0
+        assert hip.hipDeviceSynchronize() == 0
+        assert np.abs(v.get()[shift:] - ref).max() <= (1e-12 if prec == 0 else 2e-6) * np.abs(ref).max()
+    v.free()
+    c.close()
