@@ -142,7 +142,8 @@ __global__ __launch_bounds__(256) void k_heat_face(int nf, int nfn, const int32_
 
 // For the resident form: the element that holds all nodes of a face (the first
 // in the incidence order of the face's first node), the face's nodes in that
-// element's numbering (4 bits each), and its convection matrix sum_q w detJ h
+// element's numbering (4 bits each; the first place of a node that the element
+// holds twice, as a collapsed hex does), and its convection matrix sum_q w detJ h
 // N N' (6 x 6, zero padded).
 __global__ __launch_bounds__(256) void k_heat_owner(int nf, int nfn, int npe, int n_el, const int32_t *__restrict__ fconn,
                                                    const int32_t *__restrict__ conn, const int32_t *__restrict__ ptr,
@@ -161,18 +162,18 @@ __global__ __launch_bounds__(256) void k_heat_owner(int nf, int nfn, int npe, in
     }
     for (int k = ptr[nd[0]]; k < ptr[nd[0] + 1] && found < 0; ++k) {
         const int e = inc[k] / npe;
-        int hit = 0;
+        unsigned met = 0;  // the face's nodes, a bit each
         m = 0;
         for (int i = 0; i < npe; ++i) {
             const int a = conn[(size_t)i * n_el + e];
 #pragma unroll
             for (int j = 0; j < 6; ++j)
-                if (j < nfn && nd[j] == a) {
+                if (j < nfn && nd[j] == a && !(met >> j & 1u)) {
                     m |= i << (4 * j);
-                    ++hit;
+                    met |= 1u << j;
                 }
         }
-        if (hit == nfn) found = e;
+        if (met == (1u << nfn) - 1u) found = e;
     }
     owner[f] = found;
     map[f] = m;

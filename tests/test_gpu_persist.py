@@ -265,3 +265,37 @@ def test_resident_hex8(oracle, g, jitter):
             assert np.linalg.norm(u - ud) <= k * 1e-8 * np.linalg.norm(ud)
             assert np.array_equal(u, ctx.solve(**kw)[0])
     ctx.close()
+
+
+@pytest.mark.parametrize("whose", ["none", "wedge"])
+def test_heat_face_at_a_collapsed_hex(oracle, whose):
+    """A wedge (a Hex8 with two of its nodes twice): a convection face of four nodes
+    of which it has three, one of them twice (no element's face), and one of its own
+    with both doubled nodes.  Bars as test_resident_heat."""
+    import jfem
+    b = M.box_hex8(4, 3, 2, seed=6, jitter=0.05)
+    conn = b.conn.copy()
+    w = conn[0].copy()          # its edges 2-6 onto 1-5: the wedge 0 1 3, 4 5 7
+    w[2], w[6] = w[1], w[5]
+    conn[0] = w
+    used, conn = np.unique(conn, return_inverse=True)
+    m = M.Mesh(X=b.X[used], conn=conn.reshape(-1, 8), etype="Hex8", E=b.E, nu=b.nu, faces=np.zeros((0, 4), np.int64),
+               ftype="Quad4", clamp_nodes=np.zeros(0, np.int64))
+    c = m.conn[0]
+    far = int(m.conn[-1].max())
+    assert len(set(c)) == 6 and far not in c
+    faces = np.array([[c[1], c[3], c[0], far] if whose == "none" else [c[0], c[1], c[5], c[4]], m.conn[-1][4:]], np.int64)
+    rng = np.random.default_rng(3)
+    k, q = np.exp(0.5 * rng.standard_normal(m.n_el)) * 3.0, rng.uniform(0.5, 2.0, m.n_el)
+    flux, h, te = rng.uniform(0, 1, 2), rng.uniform(0.5, 1.0, 2), rng.uniform(10, 20, 2)
+    fixed = np.isclose(m.X[:, 0], m.X[:, 0].max())
+    Tf = np.full(m.n_nodes, 5.0)
+    ctx = jfem.Context(0)
+    ctx.upload_mesh(m.X, m.conn, m.etype, m.E, m.nu)
+    say(f"heat, a face at a collapsed hex: {whose}")
+    T, st = ctx.heat_solve(k, q, faces, flux=flux, h=h, T_ext=te, fixed=fixed, T_fixed=Tf, rtol=1e-12)
+    Kh, f = oracle.heat_system(m, k, q=q, faces=faces, ftype="Quad4", flux=flux, h=h, T_ext=te)
+    To = oracle.heat_solve_direct(Kh, f, fixed, Tf)
+    assert st["converged"] == 1
+    assert np.abs(T - To).max() <= 1e-8 * np.abs(To).max()
+    ctx.close()
