@@ -26,6 +26,9 @@
  *   - On small and medium meshes a whole PCG runs in one kernel that stays
  *     resident (persist.hip, persist_csr.hip); JFEM_PERSIST=0 launches its
  *     iterations instead (same answers up to the order of the reductions).
+ *     Its workgroups wait for each other, a second or so at most
+ *     (JFEM_PERSIST_POLLS: that many looks); a solve that gives up is repeated
+ *     with launched iterations (jfm_resident_counts).
  *     Launched iterations run in batches captured as HIP graphs; JFEM_GRAPHS=0
  *     launches the same kernels one by one (for tools that do not follow graph
  *     launches).
@@ -127,6 +130,11 @@ int jfm_create(int device, jfm_ctx **out);
 void jfm_destroy(jfm_ctx *ctx);
 const char *jfm_last_error(const jfm_ctx *ctx);
 int jfm_get_info(jfm_ctx *ctx, jfm_info *info);
+
+/* Linear systems that this context has solved in a resident kernel, and those
+ * whose resident solve gave up waiting and was repeated with launched
+ * iterations (either pointer may be NULL). */
+int jfm_resident_counts(const jfm_ctx *ctx, int64_t *solves, int64_t *gave_up);
 
 /* ---- problem upload (ext/JuliaFEMCUDAExt.jl:86-217 initialize_gpu_data!) --
  * Replaces the host-side renumbering and CuArray uploads.  npe = 10 (Tet10),

@@ -95,6 +95,12 @@ static int sync(jfm_ctx *ctx) {
 }
 
 // ================================================================ context ==
+// where the calls that solve begin
+static void resident_begin(jfm_ctx *ctx) {
+    const char *v = std::getenv("JFEM_PERSIST_POLLS");
+    ctx->persist_polls = v ? std::min(std::max(std::atoi(v), 0), kMaxPolls) : kMaxPolls;
+}
+
 extern "C" int jfm_create(int device, jfm_ctx **out) {
     if (!out) return JFM_EINVAL;
     *out = nullptr;
@@ -104,6 +110,7 @@ extern "C" int jfm_create(int device, jfm_ctx **out) {
     if (hipSetDevice(device) != hipSuccess) return JFM_EHIP;
     jfm_ctx *ctx = new jfm_ctx();
     ctx->device = device;
+    resident_begin(ctx);
     if (hipDeviceGetAttribute(&ctx->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) ctx->cus = 0;
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
         delete ctx;
@@ -140,6 +147,13 @@ extern "C" void jfm_destroy(jfm_ctx *ctx) {
         if (ev) (void)hipEventDestroy(ev);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
+}
+
+extern "C" int jfm_resident_counts(const jfm_ctx *ctx, int64_t *solves, int64_t *gave_up) {
+    if (!ctx) return JFM_EINVAL;
+    if (solves) *solves = ctx->resident_solves;
+    if (gave_up) *gave_up = ctx->resident_gave_up;
+    return JFM_OK;
 }
 
 extern "C" const char *jfm_last_error(const jfm_ctx *ctx) { return ctx ? ctx->err.c_str() : "null context"; }
@@ -906,13 +920,17 @@ static int pcg_run(jfm_ctx *ctx, int op, const T *Minv, double rtol, int maxit, 
         if (from_x)
             if (int rc = warm_residual(ctx, op)) return rc;
         const ResidentHold hold(ctx, jfem_persist_workgroups(ctx, op));  // until the kernel has ended
-        CHECK_LAUNCH(ctx, launch_pcg_persist<T>(ctx, op, Minv, b, from_x ? r : nullptr, x, rtol, maxit, coarse));
+        T *out = from_x ? z : x;
+        CHECK_LAUNCH(ctx, launch_pcg_persist<T>(ctx, op, Minv, b, from_x ? x : nullptr, from_x ? r : nullptr, out, rtol, maxit, coarse));
         if (int rc = read_scalars(ctx)) return rc;
         if (!ctx->S_host->fail) {
+            if (from_x) JFM_HIP(ctx, hipMemcpyAsync(x, out, sizeof(T) * n, hipMemcpyDeviceToDevice, s));
+            ++ctx->resident_solves;
             *iters = ctx->S_host->iter;
             *status = ctx->S_host->done[0];
             return JFM_OK;
         }
+        ++ctx->resident_gave_up;
         ctx->persist_off = true;  // a wait gave up: launched below, and from now on
     }
     if (int rc = prepare_op(ctx, op)) return rc;
@@ -1028,6 +1046,7 @@ extern "C" int jfm_solve(jfm_ctx *ctx, const jfm_solve_opts *opts, const double 
     if (opts->precond == JFM_PREC_USER && !ctx->has_user)
         return jfm_fail(ctx, JFM_ESTATE, "no user preconditioner blocks set");
     JFM_HIP(ctx, hipSetDevice(ctx->device));
+    resident_begin(ctx);
     const int op = opts->op;
     const int op_outer = opts->method == JFM_SOLVE_MIXED_IR ? opts->op_outer : op;
     // The 480-element patches of the matrix-free operator serve launched
@@ -1338,6 +1357,7 @@ extern "C" int jfm_solve_nonlinear(jfm_ctx *ctx, const jfm_newton_opts *opts, do
     if (opts->precond == JFM_PREC_LEARNED && !ctx->has_mlp)
         return jfm_fail(ctx, JFM_ESTATE, "learned preconditioner requested but no weights are loaded");
     JFM_HIP(ctx, hipSetDevice(ctx->device));
+    resident_begin(ctx);
     if (int rc = ensure_workspaces(ctx)) return rc;
     if (int rc = nl_buffers(ctx)) return rc;
     const int64_t n = ctx->ndof;
@@ -1507,11 +1527,13 @@ static int mass_solves(jfm_ctx *ctx, const double *Mm, int nsys, const double *b
         std::vector<PcgScalars> S(beside);  // (outlives the copy into it)
         for (int k = 0; k < nsys && beside > 1; k += beside) {
             const ResidentHold hold(ctx, beside * ctx->cells.npatch);
-            CHECK_LAUNCH(ctx, launch_pcg_persist<double>(ctx, kOpMass, Mm, b + k * n, nullptr, x + k * n, rtol, maxit, false, beside, n));
+            CHECK_LAUNCH(ctx, launch_pcg_persist<double>(ctx, kOpMass, Mm, b + k * n, nullptr, nullptr, x + k * n, rtol, maxit, false, beside, n));
             JFM_HIP(ctx, hipMemcpyAsync(S.data(), ctx->cells.S, sizeof(PcgScalars) * beside, hipMemcpyDeviceToHost, s));
             if (int rc = sync(ctx)) return rc;
-            for (const PcgScalars &v : S)
+            for (const PcgScalars &v : S) {
+                ++(v.fail ? ctx->resident_gave_up : ctx->resident_solves);
                 if (v.fail) ctx->persist_off = true;
+            }
             if (ctx->persist_off) beside = 0;
         }
         if (beside) return JFM_OK;
@@ -1530,6 +1552,7 @@ extern "C" int jfm_postprocess(jfm_ctx *ctx, const double *u, double *strain_gp,
     if (!ctx || !u) return JFM_EINVAL;
     if (!ctx->has_mesh) return jfm_fail(ctx, JFM_ESTATE, "no mesh");
     JFM_HIP(ctx, hipSetDevice(ctx->device));
+    resident_begin(ctx);
     if (int rc = ensure_workspaces(ctx)) return rc;
     const int64_t n = ctx->ndof, N = ctx->N, nq = ctx->n_el * ctx->ngp * 6;
     hipStream_t s = ctx->stream;
@@ -1600,6 +1623,7 @@ extern "C" int jfm_heat_solve(jfm_ctx *ctx, const double *k, const double *q, in
         return jfm_fail(ctx, JFM_EUNSUPPORTED, "nodes_per_face must be 6 (Tri6), 3 (Tri3) or 4 (Quad4)");
     if ((h == nullptr) != (T_ext == nullptr)) return jfm_fail(ctx, JFM_EINVAL, "convection needs both h and T_ext");
     JFM_HIP(ctx, hipSetDevice(ctx->device));
+    resident_begin(ctx);
     if (int rc = ensure_workspaces(ctx)) return rc;
     const int64_t N = ctx->N, n = ctx->ndof, n_el = ctx->n_el;
     hipStream_t s = ctx->stream;

@@ -375,6 +375,8 @@ struct jfm_ctx {
         uint64_t *words = nullptr;
     } rows;
     bool persist_off = false;      // a resident solve gave up waiting: this context launches its iterations
+    int persist_polls = 0;         // looks at a word before a resident solve gives up
+    int64_t resident_solves = 0, resident_gave_up = 0;  // of this context
     double *Muser64 = nullptr;     // N x 9 user blocks (JFM_PREC_USER)
     float *Muser32 = nullptr;
     bool has_user = false;
@@ -477,6 +479,10 @@ bool jfem_patch_defer_shared(const jfm_ctx *ctx, int op);
 // persist.hip: the whole PCG in one resident kernel, one workgroup per patch
 // (meshes of up to kPersistPatches patches).
 constexpr int kPersistPatches = 256;
+// Looks at one word before a workgroup gives up (each takes at least the
+// latency of a load past the L2, about 0.7 us: a second or so in all);
+// JFEM_PERSIST_POLLS sets fewer.
+constexpr int kMaxPolls = 1 << 20;
 // elements of a patch, its workgroup's threads (and most nodes), the row
 // stride of its LDS image of the element terms
 // Geometric factors in the element order perm (gfQ32: folded ones too, or null).
@@ -500,7 +506,7 @@ bool jfem_rows_maybe(const jfm_ctx *ctx);
 int jfem_rows_setup(jfm_ctx *ctx);
 void jfem_rows_release(jfm_ctx *ctx);
 template <typename T>
-hipError_t launch_pcg_rows(jfm_ctx *ctx, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit);
+hipError_t launch_pcg_rows(jfm_ctx *ctx, const T *Minv, const T *b, const T *x0, const T *r0, T *x, double rtol, int maxit);
 void launch_persist_clear(jfm_ctx *ctx, int n, uint64_t *words, int nz, uint64_t *zw, int nsys, PcgScalars *S);
 // workgroups of a resident solve on `op`
 int jfem_persist_workgroups(const jfm_ctx *ctx, int op);
@@ -508,12 +514,14 @@ int jfem_persist_workgroups(const jfm_ctx *ctx, int op);
 int jfem_cells_systems(jfm_ctx *ctx, int m, int words);
 // heat: maps the convection faces to elements (ctx->heat_resident)
 int jfem_heat_faces(jfm_ctx *ctx);
-// Solves K x = b (r0 null) or continues from x with its residual r0; the
-// scalars are in ctx->S afterwards, for nsys > 1 (b and x of system s at + s
-// ss) in ctx->cells.S (fail set when a wait gave up, x then untouched).
+// Solves K x = b from 0 (r0 null) or from x0 (another vector than x) with its
+// residual r0; the scalars are in ctx->S afterwards, for nsys > 1 (b and x of
+// system s at + s ss) in ctx->cells.S.  fail set: a wait gave up after
+// ctx->persist_polls looks, and x holds nothing (workgroups that saw the last sums
+// in time have written theirs).
 template <typename T>
-hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit,
-                              bool coarse = false, int nsys = 1, int64_t ss = 0);
+hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, const T *x0, const T *r0, T *x, double rtol,
+                              int maxit, bool coarse = false, int nsys = 1, int64_t ss = 0);
 // coarse.hip
 // With learned_beside, the learned blocks start on the second stream
 // (jfem_learned_launch) once A_c is formed, beside its inversion.

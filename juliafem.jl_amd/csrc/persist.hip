@@ -78,13 +78,13 @@ template <typename T> struct PersistArgs {
     const int32_t *pn_inc;    // their start in lin
     const uint16_t *lin;      // incidences (i, e): i stride + e, ascending e
     const uint8_t *fixed;     // (null: no row mask)
-    const T *Minv, *b, *r0;   // r0: the true residual at the x that is given (null: x = 0)
-    T *x;
+    const T *Minv, *b, *x0, *r0;  // the start and its true residual (null: from 0)
+    T *x;                     // (not x0: a solve that gives up leaves the start as it was)
     T *part;                  // the shared nodes' partials, 4 values per slot
     int nslot;
     uint64_t *words;          // the scalars' entries, B and then C
     double rtol2;
-    int maxit;
+    int maxit, polls;
     PcgScalars *S;
     const double *ustate;     // tangent: the displacement it is taken at
     // two-level: per patch node its aggregate; offsets from the aggregates'
@@ -773,7 +773,7 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
         const T bv = in ? bvec[d] : T(0);
         if (own) bb[0] += (double)bv * (double)bv;
         r[c] = in && A.r0 ? A.r0[d] : bv;
-        x[c] = in && A.r0 ? xvec[d] : T(0);
+        x[c] = in && A.r0 ? A.x0[d] : T(0);
         pv[c] = T(0);
     }
     T dv[3];               // two-level: the node's offset and aggregate
@@ -800,7 +800,7 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
     }
     __syncthreads();  // bad
     uint32_t epoch = 1;
-    if (!grid_sum<1, NT>(bb, wordsB, p, nwg, epoch, shB, &bad)) {
+    if (!grid_sum<1, NT>(bb, wordsB, p, nwg, epoch, A.polls, shB, &bad)) {
         if (t == 0) S->fail = 1;
         return;
     }
@@ -857,7 +857,7 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
             }
             stores_done();  // before the block barrier in grid_sum, hence before its words
         }
-        if (!grid_sum<2, NT>(s2, wordsC, p, nwg, epoch, shC, &bad)) break;
+        if (!grid_sum<2, NT>(s2, wordsC, p, nwg, epoch, A.polls, shC, &bad)) break;
         rr = s2[1];
         if (epoch == 2) rr0 = rr;  // the start
         else ++it;
@@ -913,7 +913,7 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
                 const int i = t + j * NT;
                 if (i < nc) {
                     uint32_t bits[1];
-                    if (!poll_words<1>(zw + i, 1, epoch, bits)) bad = 1;
+                    if (!poll_words<1>(zw + i, 1, epoch, A.polls, bits)) bad = 1;
                     const float zf = __uint_as_float(bits[0]);
                     co.z[i] = zf;
                     wz += w64[j] * (double)zf;
@@ -989,7 +989,7 @@ __global__ __launch_bounds__(kNT, Op::kWaves) void k_pcg_persist(const PersistAr
         }
         if (slot >= 0) part.template put<NC>(slot, q);
         stores_done();  // before the block barrier in grid_sum, hence before its words
-        if (!grid_sum<1, NT>(en, wordsB, p, nwg, epoch, shB, &bad)) break;
+        if (!grid_sum<1, NT>(en, wordsB, p, nwg, epoch, A.polls, shB, &bad)) break;
         pq = en[0];
         alpha_d = (pq > 0.0 && finite(pq)) ? rz / pq : 0.0;
         const T alpha = (T)alpha_d;
@@ -1151,9 +1151,9 @@ template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys, bo
 }
 
 template <typename T>
-hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit,
-                              bool coarse, int nsys, int64_t ss) {
-    if (op == JFM_OP_CSR) return launch_pcg_rows<T>(ctx, Minv, b, r0, x, rtol, maxit);
+hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, const T *x0, const T *r0, T *x, double rtol,
+                              int maxit, bool coarse, int nsys, int64_t ss) {
+    if (op == JFM_OP_CSR) return launch_pcg_rows<T>(ctx, Minv, b, x0, r0, x, rtol, maxit);
     const auto &C = ctx->cells;
     const PersistLaunch L = persist_kernel<T>(ctx, op, coarse);
     const bool fold = sizeof(T) == 4 && C.gfQ32;
@@ -1201,6 +1201,7 @@ hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, c
     A.fixed = op == kOpMass ? nullptr : ctx->fixed;
     A.Minv = Minv;
     A.b = b;
+    A.x0 = x0;
     A.r0 = r0;
     A.x = x;
     A.part = (T *)C.part;
@@ -1208,6 +1209,7 @@ hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, c
     A.words = C.words;
     A.rtol2 = rtol * rtol;
     A.maxit = maxit;
+    A.polls = ctx->persist_polls;
     A.S = nsys > 1 ? C.S : ctx->S;
     A.nsys = nsys;
     A.ss = ss;
@@ -1221,7 +1223,7 @@ template bool jfem_persist_maybe<double>(const jfm_ctx *, int);
 template bool jfem_persist_maybe<float>(const jfm_ctx *, int);
 template int jfem_persist_ready<double>(jfm_ctx *, int, int *, bool);
 template int jfem_persist_ready<float>(jfm_ctx *, int, int *, bool);
-template hipError_t launch_pcg_persist<double>(jfm_ctx *, int, const double *, const double *, const double *, double *, double, int, bool, int, int64_t);
-template hipError_t launch_pcg_persist<float>(jfm_ctx *, int, const float *, const float *, const float *, float *, double, int, bool, int, int64_t);
+template hipError_t launch_pcg_persist<double>(jfm_ctx *, int, const double *, const double *, const double *, const double *, double *, double, int, bool, int, int64_t);
+template hipError_t launch_pcg_persist<float>(jfm_ctx *, int, const float *, const float *, const float *, const float *, float *, double, int, bool, int, int64_t);
 
 }  // namespace jfem

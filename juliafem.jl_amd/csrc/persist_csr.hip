@@ -86,12 +86,12 @@ template <typename T> struct RowsArgs {
     const uint16_t *lcol;
     const T *vals;
     const uint8_t *fixed;
-    const T *Minv, *b, *r0;   // r0: the true residual at the x that is given (null: x = 0)
-    T *x;
+    const T *Minv, *b, *x0, *r0;  // the start and its true residual (null: from 0)
+    T *x;                     // (not x0)
     void *z;                  // 4 values per node
     uint64_t *words;
     double rtol2;
-    int maxit;
+    int maxit, polls;
     PcgScalars *S;
 };
 
@@ -150,12 +150,12 @@ __global__ __launch_bounds__(kRT, 2) void k_pcg_rows(const RowsArgs<T> A0) {
         const T bv = own ? A.b[d] : T(0);
         bb[0] += (double)bv * (double)bv;
         r[c] = own && A.r0 ? A.r0[d] : bv;
-        x[c] = own && A.r0 ? A.x[d] : T(0);
+        x[c] = own && A.r0 ? A.x0[d] : T(0);
     }
     __syncthreads();  // bad, own0, ps
     const int me = 3 * (own0 + t);
     uint32_t epoch = 1;
-    if (!grid_sum<1, kRT, true>(bb, wordsB, g, nwg, epoch, shB, &bad)) {
+    if (!grid_sum<1, kRT, true>(bb, wordsB, g, nwg, epoch, A.polls, shB, &bad)) {
         if (t == 0) A.S->fail = 1;
         return;
     }
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kRT, 2) void k_pcg_rows(const RowsArgs<T> A0) {
         ++epoch;
         if (own) zb.template put<3>(node, z);
         stores_done();  // before the block barrier in grid_sum, hence before its words
-        if (!grid_sum<2, kRT, true>(s2, wordsC, g, nwg, epoch, shC, &bad)) break;
+        if (!grid_sum<2, kRT, true>(s2, wordsC, g, nwg, epoch, A.polls, shC, &bad)) break;
         rr = s2[1];
         if (epoch == 2) rr0 = rr;  // the start
         else ++it;
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(kRT, 2) void k_pcg_rows(const RowsArgs<T> A0) {
             q[c] = own && !(fx >> c & 1u) ? qs[3 * t + c] : T(0);
             e1[0] += (double)pv[c] * (double)q[c];
         }
-        if (!grid_sum<1, kRT, true>(e1, wordsB, g, nwg, epoch, shB, &bad)) break;
+        if (!grid_sum<1, kRT, true>(e1, wordsB, g, nwg, epoch, A.polls, shB, &bad)) break;
         pq = e1[0];
         alpha_d = (pq > 0.0 && finite(pq)) ? rz / pq : 0.0;
         const T alpha = (T)alpha_d;
@@ -326,7 +326,7 @@ void jfem_rows_release(jfm_ctx *ctx) {
 }
 
 template <typename T>
-hipError_t launch_pcg_rows(jfm_ctx *ctx, const T *Minv, const T *b, const T *r0, T *x, double rtol, int maxit) {
+hipError_t launch_pcg_rows(jfm_ctx *ctx, const T *Minv, const T *b, const T *x0, const T *r0, T *x, double rtol, int maxit) {
     const auto &R = ctx->rows;
     RowsArgs<T> A{};
     A.N = (int)ctx->N;
@@ -343,19 +343,21 @@ hipError_t launch_pcg_rows(jfm_ctx *ctx, const T *Minv, const T *b, const T *r0,
     A.fixed = ctx->fixed;
     A.Minv = Minv;
     A.b = b;
+    A.x0 = x0;
     A.r0 = r0;
     A.x = x;
     A.z = R.z;
     A.words = R.words;
     A.rtol2 = rtol * rtol;
     A.maxit = maxit;
+    A.polls = ctx->persist_polls;
     A.S = ctx->S;
     launch_persist_clear(ctx, grid_words(1, R.nwg, true) + grid_words(2, R.nwg, true), R.words, 0, nullptr, 1, A.S);
     k_pcg_rows<T><<<R.nwg, kRT, 0, ctx->stream>>>(A);
     return hipGetLastError();
 }
 
-template hipError_t launch_pcg_rows<double>(jfm_ctx *, const double *, const double *, const double *, double *, double, int);
-template hipError_t launch_pcg_rows<float>(jfm_ctx *, const float *, const float *, const float *, float *, double, int);
+template hipError_t launch_pcg_rows<double>(jfm_ctx *, const double *, const double *, const double *, const double *, double *, double, int);
+template hipError_t launch_pcg_rows<float>(jfm_ctx *, const float *, const float *, const float *, const float *, float *, double, int);
 
 }  // namespace jfem

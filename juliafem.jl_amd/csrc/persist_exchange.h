@@ -8,20 +8,17 @@
 namespace jfem {
 
 // ---------------------------------------------------------------- exchange --
-// Polls of one word before a workgroup gives up (each takes at least the
-// latency of a load past the L2, about 0.7 us: a second or so in all).
-constexpr int kMaxPolls = 1 << 20;
-
 __device__ __forceinline__ void put_word(uint64_t *w, uint32_t epoch, uint32_t bits) {
     __hip_atomic_store(w, (uint64_t)epoch << 32 | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ uint64_t get_word(const uint64_t *w) {
     return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// the payloads of the N words w[i stride] once all of them are of this epoch
+// the payloads of the N words w[i stride] once all of them are of this epoch;
+// false after `polls` looks
 template <int N>
-__device__ __forceinline__ bool poll_words(const uint64_t *w, int stride, uint32_t epoch, uint32_t (&bits)[N]) {
-    for (int k = 0; k < kMaxPolls; ++k) {
+__device__ __forceinline__ bool poll_words(const uint64_t *w, int stride, uint32_t epoch, int polls, uint32_t (&bits)[N]) {
+    for (int k = 0; k < polls; ++k) {
         bool ok = true;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
@@ -123,7 +120,8 @@ __device__ __forceinline__ double wave_total(double v) {
 
 // All-reduce of NV doubles over the workgroups: v in: the thread's share, out:
 // the grid's sums, the same bits in every thread of every workgroup; false
-// when a wait gave up.  Up to 16 workgroups read each other's entries; more form
+// when a wait gave up after `polls` looks (others may then get sums without this
+// workgroup's share: the host discards the solve).  Up to 16 workgroups read each other's entries; more form
 // groups of 16 (workgroup >> 4) whose first workgroup sums the group's values
 // and publishes the sum once per 8 workgroups, and every workgroup reads its
 // copy of the groups' sums: uncached requests to one line are served one after
@@ -153,8 +151,9 @@ __host__ __device__ constexpr int grid_words(int nv, int n, bool flat = false) {
 
 struct Entries {  // past the L2, as the partials
     __amdgpu_buffer_rsrc_t rs;
-    __device__ __forceinline__ Entries(uint64_t *p, int words)
-        : rs(__builtin_amdgcn_make_buffer_rsrc(p, 0, 8 * words, 0x00027000)) {}
+    int polls;
+    __device__ __forceinline__ Entries(uint64_t *p, int words, int polls_)
+        : rs(__builtin_amdgcn_make_buffer_rsrc(p, 0, 8 * words, 0x00027000)), polls(polls_) {}
     __device__ __forceinline__ void put(int i, uint32_t epoch, double v) const {
         const uint64_t b = (uint64_t)__double_as_longlong(v);
         const u32x4 a = {(uint32_t)b, epoch, (uint32_t)(b >> 32), epoch};
@@ -162,7 +161,7 @@ struct Entries {  // past the L2, as the partials
     }
     // polls until both words of entry i are of this epoch
     __device__ __forceinline__ double get(int i, uint32_t epoch, int *bad) const {
-        for (int k = 0; k < kMaxPolls; ++k) {
+        for (int k = 0; k < polls; ++k) {
             const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * i, 0, kSc1);
             if (a.y == epoch && a.w == epoch) return __longlong_as_double((long long)((uint64_t)a.z << 32 | a.x));
             __builtin_amdgcn_s_sleep(1);
@@ -181,7 +180,7 @@ __device__ __forceinline__ double sum_members(const Entries &en, int first, int 
 }
 
 template <int NV, int NT, bool FLAT = false>
-__device__ __forceinline__ bool grid_sum(double (&v)[NV], uint64_t *words, int wg, int nwg, uint32_t epoch,
+__device__ __forceinline__ bool grid_sum(double (&v)[NV], uint64_t *words, int wg, int nwg, uint32_t epoch, int polls,
                                          GridSumLds<NV> &sh, int *bad) {
     static_assert(NV <= 2 && NT / 64 <= 16, "one row of 16 lanes per value");
     constexpr int kW = NT / 64;
@@ -193,7 +192,7 @@ __device__ __forceinline__ bool grid_sum(double (&v)[NV], uint64_t *words, int w
     }
     __syncthreads();
     if (FLAT && nwg > kGroup && nwg <= kFlat) {
-        const Entries en(words, grid_words(NV, nwg, true));
+        const Entries en(words, grid_words(NV, nwg, true), polls);
         if (wv == 0) {
             const int k = lane >> 4, m = lane & 15;
             const double s = row_sum(k < NV && m < kW ? sh.a[k < NV ? k : 0][m] : 0.0);
@@ -220,7 +219,7 @@ __device__ __forceinline__ bool grid_sum(double (&v)[NV], uint64_t *words, int w
         const int k = lane >> 4, m = lane & 15;
         double s = row_sum(k < NV && m < kW ? sh.a[k < NV ? k : 0][m] : 0.0);  // row k: the block's value k
         if (nwg > 1) {
-            const Entries en(words, grid_words(NV, nwg));
+            const Entries en(words, grid_words(NV, nwg), polls);
             if (k < NV && m == 0) en.put(wg * NV + k, epoch, s);
             if (nwg > kGroup) {
                 const int g = wg / kGroup, copies = (nwg + kCopy - 1) / kCopy;

@@ -23,7 +23,7 @@ OPS = {"csr": OP_CSR, "ebe": OP_EBE, "matfree": OP_MATFREE, "tangent": OP_TANGEN
 ERRORS = {-1: "EINVAL", -2: "EHIP", -3: "ENOTSPD", -4: "ENOCONV", -5: "ESTATE", -6: "ENOMEM", -7: "EUNSUPPORTED"}
 
 # Exported symbols (must match include/jfem.h)
-SYMBOLS = ("jfm_create", "jfm_destroy", "jfm_last_error", "jfm_get_info", "jfm_upload_mesh",
+SYMBOLS = ("jfm_create", "jfm_destroy", "jfm_last_error", "jfm_get_info", "jfm_resident_counts", "jfm_upload_mesh",
            "jfm_upload_bcs", "jfm_csr_pattern", "jfm_assemble", "jfm_assemble_tl", "jfm_apply", "jfm_apply_noalloc", "jfm_time_apply", "jfm_coarse_matrix",
            "jfm_solve", "jfm_solve_history", "jfm_precond_set_blocks", "jfm_learned_blob_bytes", "jfm_learned_n_params",
            "jfm_learned_set_weights", "jfm_learned_get_weights", "jfm_learned_features", "jfm_learned_outputs",
@@ -94,6 +94,7 @@ def load():
     lib.jfm_last_error.argtypes = [_P]
     lib.jfm_last_error.restype = C.c_char_p
     lib.jfm_get_info.argtypes = [_P, C.POINTER(Info)]
+    lib.jfm_resident_counts.argtypes = [_P, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]
     lib.jfm_upload_mesh.argtypes = [_P, C.c_int64, _P, C.c_int64, C.c_int32, _P, _P, _P, C.c_int32]
     lib.jfm_upload_bcs.argtypes = [_P, _P, _P, C.c_int64, C.c_int32, _P, _P, C.c_int32]
     lib.jfm_csr_pattern.argtypes = [_P, C.POINTER(C.c_int64), _P, _P, C.c_int32]
@@ -190,6 +191,13 @@ class Context:
         inf = Info()
         self._check(self._lib.jfm_get_info(self._h, C.byref(inf)))
         return {k: getattr(inf, k) for k, _ in inf._fields_}
+
+    def resident_counts(self):
+        """(linear systems solved in a resident kernel, those that gave up waiting
+        and were repeated with launched iterations) of this context."""
+        solves, gave_up = C.c_int64(0), C.c_int64(0)
+        self._check(self._lib.jfm_resident_counts(self._h, C.byref(solves), C.byref(gave_up)))
+        return solves.value, gave_up.value
 
     def csr_pattern(self, base: int = 0):
         nnz = C.c_int64(0)
