@@ -28,7 +28,8 @@
  *     iterations instead (same answers up to the order of the reductions).
  *     Its workgroups wait for each other, a second or so at most
  *     (JFEM_PERSIST_POLLS: that many looks); a solve that gives up is repeated
- *     with launched iterations (jfm_resident_counts).
+ *     with launched iterations (jfm_resident_counts), as is what follows in that
+ *     call, and further calls while it happens again.
  *     Launched iterations run in batches captured as HIP graphs; JFEM_GRAPHS=0
  *     launches the same kernels one by one (for tools that do not follow graph
  *     launches).

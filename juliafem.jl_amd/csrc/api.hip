@@ -95,8 +95,18 @@ static int sync(jfm_ctx *ctx) {
 }
 
 // ================================================================ context ==
+// A resident solve that gave up has waited a second or so, and something else may
+// hold the device for longer: the call goes on with launched iterations, and so do
+// the next 2^k - 1 calls after k + 1 give-ups in a row.
+static void resident_gave_up(jfm_ctx *ctx, int systems) {
+    ctx->resident_gave_up += systems;
+    ctx->persist_off = true;
+    ctx->persist_wait = 1 << std::min(ctx->persist_fails++, 10);
+}
+
 // where the calls that solve begin
 static void resident_begin(jfm_ctx *ctx) {
+    if (ctx->persist_off && --ctx->persist_wait <= 0) ctx->persist_off = false;
     const char *v = std::getenv("JFEM_PERSIST_POLLS");
     ctx->persist_polls = v ? std::min(std::max(std::atoi(v), 0), kMaxPolls) : kMaxPolls;
 }
@@ -225,6 +235,8 @@ static void release_mesh(jfm_ctx *ctx) {
     jfem_cells_release(ctx);
     jfem_rows_release(ctx);
     jfem_train_release(ctx);
+    ctx->persist_off = false;
+    ctx->persist_wait = ctx->persist_fails = 0;
     release_heat(ctx);
     ctx->h_X.clear();
     ctx->has_user = false;
@@ -926,12 +938,12 @@ static int pcg_run(jfm_ctx *ctx, int op, const T *Minv, double rtol, int maxit, 
         if (!ctx->S_host->fail) {
             if (from_x) JFM_HIP(ctx, hipMemcpyAsync(x, out, sizeof(T) * n, hipMemcpyDeviceToDevice, s));
             ++ctx->resident_solves;
+            ctx->persist_fails = 0;
             *iters = ctx->S_host->iter;
             *status = ctx->S_host->done[0];
             return JFM_OK;
         }
-        ++ctx->resident_gave_up;
-        ctx->persist_off = true;  // a wait gave up: launched below, and from now on
+        resident_gave_up(ctx, 1);  // launched below
     }
     if (int rc = prepare_op(ctx, op)) return rc;
     std::memset(ctx->S_host, 0, sizeof(PcgScalars));
@@ -1530,13 +1542,18 @@ static int mass_solves(jfm_ctx *ctx, const double *Mm, int nsys, const double *b
             CHECK_LAUNCH(ctx, launch_pcg_persist<double>(ctx, kOpMass, Mm, b + k * n, nullptr, nullptr, x + k * n, rtol, maxit, false, beside, n));
             JFM_HIP(ctx, hipMemcpyAsync(S.data(), ctx->cells.S, sizeof(PcgScalars) * beside, hipMemcpyDeviceToHost, s));
             if (int rc = sync(ctx)) return rc;
-            for (const PcgScalars &v : S) {
-                ++(v.fail ? ctx->resident_gave_up : ctx->resident_solves);
-                if (v.fail) ctx->persist_off = true;
+            int failed = 0;
+            for (const PcgScalars &v : S) failed += v.fail != 0;
+            ctx->resident_solves += beside - failed;
+            if (failed) {
+                resident_gave_up(ctx, failed);
+                beside = 0;
             }
-            if (ctx->persist_off) beside = 0;
         }
-        if (beside) return JFM_OK;
+        if (beside) {
+            ctx->persist_fails = 0;
+            return JFM_OK;
+        }
     }
     for (int k = 0; k < nsys; ++k) {
         JFM_HIP(ctx, hipMemcpyAsync(ctx->ws64.b, b + k * n, sizeof(double) * n, hipMemcpyDeviceToDevice, s));

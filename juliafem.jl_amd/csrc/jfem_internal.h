@@ -374,7 +374,8 @@ struct jfm_ctx {
         double *z = nullptr;                 // exchanged vector, 4 values per node (FP32 or FP64 view)
         uint64_t *words = nullptr;
     } rows;
-    bool persist_off = false;      // a resident solve gave up waiting: this context launches its iterations
+    bool persist_off = false;      // a resident solve gave up waiting: iterations are launched
+    int persist_wait = 0, persist_fails = 0;  // until so many calls from now; give-ups in a row on this mesh
     int persist_polls = 0;         // looks at a word before a resident solve gives up
     int64_t resident_solves = 0, resident_gave_up = 0;  // of this context
     double *Muser64 = nullptr;     // N x 9 user blocks (JFM_PREC_USER)

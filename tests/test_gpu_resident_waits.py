@@ -161,3 +161,31 @@ def test_launched_forms(oracle, name, make, kw):
     assert np.linalg.norm(u - ud) <= 1e-7 * np.linalg.norm(ud)
     assert ctx.resident_counts() == (0, 0)
     ctx.close()
+
+
+def test_resident_again_after_a_give_up(monkeypatch):
+    """The call after a give-up, and every call on a new mesh, runs resident again,
+    to the bits of a context that never gave up; while it happens again, one call,
+    then one of two, then one of four tries."""
+    import jfem
+    m = box()
+    kw = dict(rtol=1e-10)
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    u = ctx.solve(**kw)[0]
+    n = ctx.resident_counts()[0]
+    monkeypatch.setenv("JFEM_PERSIST_POLLS", "0")
+    say("resident again after a give-up")
+    tried = []
+    for _ in range(8):
+        before = ctx.resident_counts()[1]
+        ctx.solve(**kw)
+        tried.append(ctx.resident_counts()[1] - before)
+    assert tried == [1, 1, 0, 1, 0, 0, 0, 1]
+    ctx.upload(m)
+    ctx.solve(**kw)
+    monkeypatch.delenv("JFEM_PERSIST_POLLS")
+    assert ctx.resident_counts() == (n, 5)
+    assert np.array_equal(ctx.solve(**kw)[0], u)
+    assert ctx.resident_counts() == (2 * n, 5)
+    ctx.close()
