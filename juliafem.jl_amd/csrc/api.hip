@@ -872,8 +872,10 @@ static int finalize_misc(jfm_ctx *ctx, int npart, int nv, int fin) {
 // The workgroups of resident kernels that run at once on a device, over all
 // contexts and threads of the process, never exceed its CUs, each of which
 // holds at least one of them: so every such kernel is resident as a whole once
-// the finite kernels beside it have ended.  A hold lasts until the kernel has
-// been waited for.
+// the finite kernels beside it have ended.  A kernel's workgroups go to the XCDs
+// in turn and stay there, so a hold counts whole rounds of them: 85 workgroups are
+// 11 on some XCD, and 85 + 85 + 86, 256 in all, would need 33 of its 32 CUs.  A hold
+// lasts until the kernel has been waited for.
 namespace {
 struct ResidentHold {
     static constexpr int kDevices = 64;
@@ -888,7 +890,8 @@ struct ResidentHold {
     }
     Device &dev;
     int n;
-    ResidentHold(const jfm_ctx *ctx, int workgroups) : dev(of(ctx->device)), n(std::min(workgroups, ctx->cus)) {
+    ResidentHold(const jfm_ctx *ctx, int workgroups)
+        : dev(of(ctx->device)), n(std::min((int)xcd_grid((unsigned)workgroups), ctx->cus)) {
         std::unique_lock<std::mutex> lock(dev.m);
         dev.cv.wait(lock, [&] { return dev.used + n <= ctx->cus; });
         dev.used += n;

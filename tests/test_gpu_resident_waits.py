@@ -7,6 +7,8 @@ by itself, and the solve is repeated with launched iterations.  Results keep the
 bars of the resident PCG's tests (1e-8 of the direct solve at rtol 1e-10, 1e-7
 for Newton, 1e-9 for the nodal fits).
 """
+import threading
+
 import numpy as np
 import pytest
 
@@ -189,3 +191,36 @@ def test_resident_again_after_a_give_up(monkeypatch):
     assert np.array_equal(ctx.solve(**kw)[0], u)
     assert ctx.resident_counts() == (2 * n, 5)
     ctx.close()
+
+
+@pytest.mark.parametrize("patches", [(85, 85, 86), (80, 80, 80), (128, 128), (41, 43, 45, 47, 9)])
+def test_solves_from_several_threads(patches):
+    """Resident kernels of several contexts at once, workgroups that fill the device
+    or more: none gives up, and each has the bits of its solves alone."""
+    import jfem
+    big = M.box_tet10(18, 18, 9, L=(2.0, 2.0, 1.0), seed=5, jitter=0.1, E_sigma=0.4)
+    ms = [cut(big, 128 * n) for n in patches]
+    f = [np.random.default_rng(4 + k).normal(size=m.n_dofs) for k, m in enumerate(ms)]
+    cs = [jfem.Context(0) for _ in ms]
+    kw = dict(rtol=1e-8, method=1, inner_rtol=1e-2)
+    for c, m in zip(cs, ms):
+        c.upload(m)
+    alone = [c.solve(f=f[k], **kw)[0] for k, c in enumerate(cs)]
+    say(f"resident solves side by side: {patches}")
+    same = [[] for _ in cs]
+
+    def work(k):
+        for _ in range(6):
+            same[k].append(np.array_equal(cs[k].solve(f=f[k], **kw)[0], alone[k]))
+
+    th = [threading.Thread(target=work, args=(k,)) for k in range(len(cs))]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    counts = [c.resident_counts() for c in cs]
+    say(f"solves, give-ups: {counts}")
+    assert all(n > 0 and g == 0 for n, g in counts)
+    assert all(s == [True] * 6 for s in same)
+    for c in cs:
+        c.close()
