@@ -307,14 +307,19 @@ extern "C" int jfm_upload_mesh(jfm_ctx *ctx, int64_t n_nodes, const double *X, i
         JFM_HIP(ctx, hipMemcpyAsync(ctx->E, E, sizeof(double) * n_el, hipMemcpyHostToDevice, s));
         JFM_HIP(ctx, hipMemcpyAsync(ctx->nu, nu, sizeof(double) * n_el, hipMemcpyHostToDevice, s));
     }
-    int32_t *d_flags = nullptr, flags[2] = {0, 0}, nnzb = 0;
-    CHECK_LAUNCH(ctx, launch_mesh_lists(ctx, scratch.p, &d_flags));
-    JFM_HIP(ctx, hipMemcpyAsync(flags, d_flags, sizeof flags, hipMemcpyDeviceToHost, s));
-    JFM_HIP(ctx, hipMemcpyAsync(&nnzb, ctx->brow + n_nodes, sizeof nnzb, hipMemcpyDeviceToHost, s));
-    if (int rc = sync(ctx)) return rc;
+    MeshFlags flags;
+    CHECK_LAUNCH(ctx, launch_mesh_lists(ctx, scratch.p, &flags));
+    if (flags.large_rows) {
+        uint64_t *keys = jfm_alloc<uint64_t>(ctx, 2 * (int64_t)flags.large_entries);
+        if (!keys) return jfm_fail(ctx, JFM_ENOMEM, "device allocation failed: mesh lists");
+        const hipError_t e = launch_large_rows(ctx, scratch.p, keys, &flags);
+        jfm_free(ctx, keys);
+        if (e != hipSuccess) return jfm_hip_fail(ctx, e, "large pattern rows");
+    }
+    const int32_t nnzb = flags.nnzb;
     ctx->nnzb = nnzb;
-    ctx->affine = flags[0] == 0;
-    ctx->orphans = flags[1];
+    ctx->affine = flags.affine;
+    ctx->orphans = flags.orphans;
     ctx->ngf = ctx->affine ? 1 : ctx->ngp;
     ALLOC(ctx, ctx->gf64, double, (int64_t)GF * ctx->ngf * n_el);
     ALLOC(ctx, ctx->gf32, float, (int64_t)GF * ctx->ngf * n_el);

@@ -408,12 +408,19 @@ namespace jfem {
 hipError_t launch_geom_factors(jfm_ctx *ctx, int *d_bad);
 // Incidences, sorted pattern rows and contributions of the uploaded mesh
 // (mesh_lists.hip) into ctx->conn, inc*, brow and contrib; scratch of
-// mesh_lists_scratch() int32.  *flags: two device words, whether an element's J
-// is not constant and the number of nodes of no element.  Then, with
-// bcol, blk_row and cptr allocated for brow[N] blocks, the pattern.
+// mesh_lists_scratch() int32.  Waits for the flags: whether J is constant in every
+// element, nodes of no element, blocks of the pattern and, where rows are too large
+// for the kernel of the others, how many and their entries.  These take 2
+// large_entries keys and set nnzb.  Then, with bcol, blk_row and cptr allocated for
+// the nnzb blocks, the pattern.
+struct MeshFlags {
+    bool affine = false;
+    int32_t orphans = 0, large_rows = 0, large_entries = 0, nnzb = 0;
+};
 int64_t mesh_lists_scratch(int64_t N, int64_t n_el, int npe);
-hipError_t launch_mesh_lists(jfm_ctx *ctx, int32_t *scratch, int32_t **flags);
-hipError_t launch_pattern_write(jfm_ctx *ctx, const int32_t *scratch);
+hipError_t launch_mesh_lists(jfm_ctx *ctx, int32_t *scratch, MeshFlags *flags);
+hipError_t launch_large_rows(jfm_ctx *ctx, int32_t *scratch, uint64_t *keys, MeshFlags *flags);
+hipError_t launch_pattern_write(jfm_ctx *ctx, int32_t *scratch);
 hipError_t launch_element_matrices(jfm_ctx *ctx);
 hipError_t launch_assemble_values(jfm_ctx *ctx);
 // finite-strain element matrices Km, element-major into Ke, the factors of I of

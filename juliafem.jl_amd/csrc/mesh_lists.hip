@@ -112,9 +112,11 @@ __global__ __launch_bounds__(kBlock) void k_inc_rank(int n_el, const int32_t *__
 // the entries before it: m^2 comparisons, 60^2 for an average mid node of a
 // Tet10 box and 240^2 for its vertices, NV entries per lane against broadcast
 // reads of four columns from LDS (one entry and one column at a time: 255 us at
-// 20,295 nodes instead of 66).  Rows of more than kRowCap entries read the
-// columns from memory instead.
+// 20,295 nodes instead of 66).  Rows of more than kRowCap entries (nodes of more
+// than 102 Tet10, 256 Tet4 or 128 Hex8 elements) are listed for k_row_sort_large.
 constexpr int kRowCap = 1024, kRowWaves = 4;
+// flags: an element's J is not constant; nodes of no element; large rows, their entries
+enum { kNotAffine, kOrphans, kLargeRows, kLargeEntries, kFlags = 8 };
 
 // where the entries t0 + lane + 64 j of the m in cols[] belong
 template <int NV> __device__ __forceinline__ void row_places(const int32_t *cols, int m, int t0, int (&at)[NV], int (&first)[NV]) {
@@ -151,16 +153,16 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_row_sort(int N, const int32_
                                                             const int32_t *__restrict__ inc,
                                                             const int32_t *__restrict__ connE, int32_t *__restrict__ sorted,
                                                             int32_t *__restrict__ contrib, int32_t *__restrict__ rowlen,
-                                                            int32_t *__restrict__ flags) {
+                                                            int32_t *__restrict__ flags, int2 *__restrict__ large) {
     __shared__ __attribute__((aligned(16))) int32_t rows[kRowWaves][kRowCap];
     const int lane = threadIdx.x & 63;
     const int a = blockIdx.x * kRowWaves + (threadIdx.x >> 6);
     int32_t *cols = rows[threadIdx.x >> 6];
     const int k0 = a < N ? inc_ptr[a] : 0, m = a < N ? (inc_ptr[a + 1] - k0) * NPE : 0;
-    auto col = [&](int t) -> int32_t { return connE[(int64_t)(inc[k0 + t / NPE] / NPE) * NPE + t % NPE]; };
     const bool lds = m <= kRowCap;
     if (lds)
-        for (int t = lane; t < ((m + 3) & ~3); t += 64) cols[t] = t < m ? col(t) : INT32_MAX;
+        for (int t = lane; t < ((m + 3) & ~3); t += 64)
+            cols[t] = t < m ? connE[(int64_t)(inc[k0 + t / NPE] / NPE) * NPE + t % NPE] : INT32_MAX;
     __syncthreads();
     int distinct = 0;
     const int64_t base = (int64_t)k0 * NPE;
@@ -170,16 +172,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_row_sort(int N, const int32_
         distinct += first;
     };
     if (!lds) {
-        for (int t = lane; t < m; t += 64) {
-            const int32_t v = col(t);
-            int less = 0, same = 0;
-            for (int u = 0; u < m; ++u) {
-                const int32_t x = col(u);
-                less += x < v;
-                same += x == v && u < t;
-            }
-            put(t, less + same, same == 0, v);
-        }
+        if (lane == 0) large[atomicAdd(flags + kLargeRows, 1)] = {a, atomicAdd(flags + kLargeEntries, m)};
     } else if (m <= 64) {
         int at[1], first[1];
         row_places<1>(cols, m, 0, at, first);
@@ -199,8 +192,67 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_row_sort(int N, const int32_
     for (int off = 32; off > 0; off >>= 1) distinct += __shfl_xor(distinct, off, 64);
     if (lane == 0 && a < N) {
         rowlen[a] = distinct;
-        if (m == 0) atomicAdd(flags + 1, 1);  // a node of no element
+        if (m == 0) atomicAdd(flags + kOrphans, 1);
     }
+}
+
+// One workgroup per listed row: its entries as keys (column, t), sorted in LDS in
+// runs of kRun and merged in memory, run by run with its neighbour, each key to its
+// own place plus the smaller keys of the other run (a binary search).  At 2,000
+// Tet4 around a node (8,000 entries) the upload takes 0.7 ms instead of 142 with
+// the comparison of all pairs in one wave, at 968 Tet10 0.64 instead of 299.
+// `keys`: two arrays of `entries`.
+constexpr int kRun = 4096, kLargeThreads = 1024;
+template <int NPE>
+__global__ __launch_bounds__(kLargeThreads) void k_row_sort_large(const int2 *__restrict__ large, int64_t entries,
+                                                                 const int32_t *__restrict__ inc_ptr,
+                                                                 const int32_t *__restrict__ inc,
+                                                                 const int32_t *__restrict__ connE, uint64_t *keys,
+                                                                 int32_t *__restrict__ sorted, int32_t *__restrict__ contrib,
+                                                                 int32_t *__restrict__ rowlen) {
+    __shared__ uint64_t run[kRun];
+    const int a = large[blockIdx.x].x, k0 = inc_ptr[a], m = (inc_ptr[a + 1] - k0) * NPE;
+    uint64_t *from = keys + large[blockIdx.x].y, *to = from + entries;
+    for (int r0 = 0; r0 < m; r0 += kRun) {
+        const int n = min(kRun, m - r0);
+        int n2 = 2;
+        while (n2 < n) n2 <<= 1;
+        for (int i = threadIdx.x; i < n2; i += kLargeThreads) {
+            const int t = r0 + i;
+            run[i] = i < n ? (uint64_t)(uint32_t)connE[(int64_t)(inc[k0 + t / NPE] / NPE) * NPE + t % NPE] << 32 | (uint32_t)t : ~0ull;
+        }
+        sort_keys<kLargeThreads>(run, n2);
+        for (int i = threadIdx.x; i < n; i += kLargeThreads) from[r0 + i] = run[i];
+        __syncthreads();
+    }
+    for (int64_t w = kRun; w < m; w *= 2) {
+        for (int i = threadIdx.x; i < m; i += kLargeThreads) {
+            const uint64_t v = from[i];
+            const int64_t r = i / w, o0 = min((r ^ 1) * w, (int64_t)m), o1 = min(((r ^ 1) + 1) * w, (int64_t)m);
+            int64_t lo = o0, hi = o1;  // the first key of the other run above v
+            while (lo < hi) {
+                const int64_t mid = (lo + hi) / 2;
+                if (from[mid] < v) lo = mid + 1;
+                else hi = mid;
+            }
+            to[(r & ~(int64_t)1) * w + (i - r * w) + (lo - o0)] = v;
+        }
+        __syncthreads();
+        uint64_t *const swap = from;
+        from = to;
+        to = swap;
+    }
+    const int64_t base = (int64_t)k0 * NPE;
+    int distinct = 0, total;
+    for (int i = threadIdx.x; i < m; i += kLargeThreads) {
+        const uint64_t v = from[i];
+        const int t = (int)(uint32_t)v;
+        sorted[base + i] = (int32_t)(v >> 32);
+        contrib[base + i] = inc[k0 + t / NPE] * NPE + t % NPE;
+        distinct += i == 0 || from[i - 1] >> 32 != v >> 32;
+    }
+    (void)block_scan<kLargeThreads>(distinct, &total);
+    if (threadIdx.x == 0) rowlen[a] = total;
 }
 
 // One wave per node: the row's columns and the blocks' ranges of contributions
@@ -268,58 +320,106 @@ __global__ __launch_bounds__(kBlock) void k_not_affine(int n_el, const int32_t *
                 bad = bad || fabs(P[i][k] - v) > tol * 8;
             }
     }
-    if (bad) flags[0] = 1;
+    if (bad) flags[kNotAffine] = 1;
 }
 
 // ----------------------------------------------------------------- launches ---
-int64_t mesh_lists_scratch(int64_t N, int64_t n_el, int npe) {
-    // connE, any, cnt, rowlen, block sums, flags, sorted columns
-    return 2 * n_el * npe + 2 * N + (N + kScan - 1) / kScan + 8 + n_el * npe * npe;
-}
+// the arrays in the scratch of an upload
+namespace {
+struct ListScratch {
+    int32_t *connE, *any, *cnt, *flags, *rowlen, *bsum, *sorted;  // by element, placed incidences, counts, flags, ...
+    int2 *large;                                                  // large rows: node, first key
+    int64_t total;
+    ListScratch(int32_t *p, int64_t N, int64_t n_el, int npe) {
+        const int64_t q = n_el * npe;
+        int64_t at = 0;
+        auto take = [&](int64_t n) {
+            int32_t *r = p ? p + at : nullptr;
+            at += n;
+            return r;
+        };
+        large = (int2 *)take(2 * (q * npe / kRowCap + 1));  // first: its alignment
+        connE = take(q);
+        any = take(q);
+        cnt = take(N);
+        flags = take(kFlags);
+        rowlen = take(N);
+        bsum = take((N + kScan - 1) / kScan);
+        sorted = take(q * npe);
+        total = at;
+    }
+    ListScratch(jfm_ctx *ctx, int32_t *p) : ListScratch(p, ctx->N, ctx->n_el, ctx->npe) {}
+};
+}  // namespace
 
-template <int NPE>
-static void incidences(jfm_ctx *ctx, const int32_t *connE, int32_t *any, int32_t *cnt, int32_t *rowlen, int32_t *bsum,
-                       int32_t *flags, int32_t *sorted) {
+int64_t mesh_lists_scratch(int64_t N, int64_t n_el, int npe) { return ListScratch(nullptr, N, n_el, npe).total; }
+
+template <int NPE> static void incidences(jfm_ctx *ctx, const ListScratch &L) {
     hipStream_t s = ctx->stream;
     const int N = (int)ctx->N, n_el = (int)ctx->n_el;
     const int64_t q = (int64_t)n_el * NPE;
     const unsigned gq = (unsigned)((q + kBlock - 1) / kBlock);
-    if (gq) k_conn_split<NPE><<<gq, kBlock, 0, s>>>(n_el, connE, ctx->conn, cnt);
-    scan(s, N, cnt, ctx->inc_ptr, bsum);
+    if (gq) k_conn_split<NPE><<<gq, kBlock, 0, s>>>(n_el, L.connE, ctx->conn, L.cnt);
+    scan(s, N, L.cnt, ctx->inc_ptr, L.bsum);
     if (gq) {
-        k_inc_place<<<gq, kBlock, 0, s>>>(q, connE, ctx->inc_ptr, cnt, any);
-        k_inc_rank<NPE><<<gq, kBlock, 0, s>>>(n_el, connE, ctx->inc_ptr, any, ctx->inc, ctx->inc_slot);
+        k_inc_place<<<gq, kBlock, 0, s>>>(q, L.connE, ctx->inc_ptr, L.cnt, L.any);
+        k_inc_rank<NPE><<<gq, kBlock, 0, s>>>(n_el, L.connE, ctx->inc_ptr, L.any, ctx->inc, ctx->inc_slot);
     }
-    k_row_sort<NPE><<<(N + kRowWaves - 1) / kRowWaves, 64 * kRowWaves, 0, s>>>(N, ctx->inc_ptr, ctx->inc, connE, sorted,
-                                                                             ctx->contrib, rowlen, flags);
-    scan(s, N, rowlen, ctx->brow, bsum);
+    k_row_sort<NPE><<<(N + kRowWaves - 1) / kRowWaves, 64 * kRowWaves, 0, s>>>(N, ctx->inc_ptr, ctx->inc, L.connE, L.sorted,
+                                                                             ctx->contrib, L.rowlen, L.flags, L.large);
+    scan(s, N, L.rowlen, ctx->brow, L.bsum);
     if constexpr (NPE != 4)
-        if (gq) k_not_affine<NPE><<<(n_el + kBlock - 1) / kBlock, kBlock, 0, s>>>(n_el, ctx->conn, ctx->X, flags);
+        if (gq) k_not_affine<NPE><<<(n_el + kBlock - 1) / kBlock, kBlock, 0, s>>>(n_el, ctx->conn, ctx->X, L.flags);
 }
 
-hipError_t launch_mesh_lists(jfm_ctx *ctx, int32_t *scratch, int32_t **flags_out) {
-    const int64_t N = ctx->N, n_el = ctx->n_el, q = n_el * ctx->npe;
-    int32_t *connE = scratch, *any = connE + q, *cnt = any + q, *flags = cnt + N, *rowlen = flags + 8, *bsum = rowlen + N,
-            *sorted = bsum + (N + kScan - 1) / kScan;
-    *flags_out = flags;
-    hipError_t e = hipMemsetAsync(cnt, 0, 4 * (size_t)(N + 8), ctx->stream);  // and the flags
-    if (e == hipSuccess && q)
-        e = hipMemcpyAsync(connE, ctx->h_conn.data(), 4 * (size_t)q, hipMemcpyHostToDevice, ctx->stream);
+hipError_t launch_mesh_lists(jfm_ctx *ctx, int32_t *scratch, MeshFlags *flags) {
+    const int64_t q = ctx->n_el * ctx->npe;
+    hipStream_t s = ctx->stream;
+    const ListScratch L(ctx, scratch);
+    hipError_t e = hipMemsetAsync(L.cnt, 0, 4 * (size_t)(ctx->N + kFlags), s);  // and the flags
+    if (e == hipSuccess && q) e = hipMemcpyAsync(L.connE, ctx->h_conn.data(), 4 * (size_t)q, hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return e;
     switch (ctx->npe) {
-    case 10: incidences<10>(ctx, connE, any, cnt, rowlen, bsum, flags, sorted); break;
-    case 4: incidences<4>(ctx, connE, any, cnt, rowlen, bsum, flags, sorted); break;
-    case 8: incidences<8>(ctx, connE, any, cnt, rowlen, bsum, flags, sorted); break;
+    case 10: incidences<10>(ctx, L); break;
+    case 4: incidences<4>(ctx, L); break;
+    case 8: incidences<8>(ctx, L); break;
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
+    int32_t got[4] = {0, 0, 0, 0};
+    if ((e = hipGetLastError()) == hipSuccess) e = hipMemcpyAsync(got, L.flags, sizeof got, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(&flags->nnzb, ctx->brow + ctx->N, 4, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    flags->affine = got[kNotAffine] == 0;
+    flags->orphans = got[kOrphans];
+    flags->large_rows = got[kLargeRows];
+    flags->large_entries = got[kLargeEntries];
+    return e;
 }
 
-hipError_t launch_pattern_write(jfm_ctx *ctx, const int32_t *scratch) {
-    const int64_t N = ctx->N, q = ctx->n_el * ctx->npe;
-    const int32_t *sorted = scratch + 2 * q + 2 * N + 8 + (N + kScan - 1) / kScan;
-    k_row_write<<<(unsigned)((N + 3) / 4), kBlock, 0, ctx->stream>>>((int)N, ctx->npe, ctx->inc_ptr, sorted, ctx->brow, ctx->bcol,
-                                                                     ctx->blk_row, ctx->cptr, ctx->bdiag);
+hipError_t launch_large_rows(jfm_ctx *ctx, int32_t *scratch, uint64_t *keys, MeshFlags *flags) {
+    hipStream_t s = ctx->stream;
+    const ListScratch L(ctx, scratch);
+    auto sort = [&](auto kernel) {
+        kernel<<<(unsigned)flags->large_rows, kLargeThreads, 0, s>>>(L.large, flags->large_entries, ctx->inc_ptr, ctx->inc, L.connE, keys,
+                                                                     L.sorted, ctx->contrib, L.rowlen);
+    };
+    switch (ctx->npe) {
+    case 10: sort(k_row_sort_large<10>); break;
+    case 4: sort(k_row_sort_large<4>); break;
+    case 8: sort(k_row_sort_large<8>); break;
+    default: return hipErrorInvalidValue;
+    }
+    scan(s, (int)ctx->N, L.rowlen, ctx->brow, L.bsum);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(&flags->nnzb, ctx->brow + ctx->N, 4, hipMemcpyDeviceToHost, s);
+    const hipError_t w = hipStreamSynchronize(s);  // also before the keys go
+    return e == hipSuccess ? w : e;
+}
+
+hipError_t launch_pattern_write(jfm_ctx *ctx, int32_t *scratch) {
+    const ListScratch L(ctx, scratch);
+    k_row_write<<<(unsigned)((ctx->N + 3) / 4), kBlock, 0, ctx->stream>>>((int)ctx->N, ctx->npe, ctx->inc_ptr, L.sorted, ctx->brow, ctx->bcol,
+                                                                          ctx->blk_row, ctx->cptr, ctx->bdiag);
     return hipGetLastError();
 }
 

@@ -108,3 +108,51 @@ def test_solve_on_a_star(oracle, name):
         u, _, _ = ctx.solve(f=f, rtol=1e-10, **kw)
         assert np.linalg.norm(u - ud) <= 1e-8 * np.linalg.norm(ud)
     ctx.close()
+
+
+def fan(n, quadratic):
+    """The tetrahedra between a point and 2 n^2 triangles of a square below it."""
+    x = np.linspace(-1.0, 1.0, n + 1)
+    X, Y = np.meshgrid(x, x, indexing="ij")
+    i, j = (a.ravel() for a in np.meshgrid(np.arange(n), np.arange(n), indexing="ij"))
+    at = lambda a, b: a * (n + 1) + b
+    tri = np.concatenate([np.column_stack([at(i, j), at(i + 1, j), at(i, j + 1)]),
+                          np.column_stack([at(i + 1, j), at(i + 1, j + 1), at(i, j + 1)])])
+    X = np.vstack([np.column_stack([X.ravel(), Y.ravel(), np.zeros(X.size)]), [[0.1, 0.2, 1.0]]])
+    conn = np.column_stack([tri, np.full(len(tri), len(X) - 1)])
+    conn = conn[np.random.default_rng(1).permutation(len(conn))]
+    if quadratic:
+        e = np.sort(conn[:, [[0, 1], [1, 2], [2, 0], [0, 3], [1, 3], [2, 3]]], 2)
+        ed, mid = np.unique(e.reshape(-1, 2), axis=0, return_inverse=True)
+        X, conn = np.vstack([X, 0.5 * (X[ed[:, 0]] + X[ed[:, 1]])]), np.column_stack([conn, len(X) + mid.reshape(-1, 6)])
+    return M.Mesh(X=X, conn=conn, etype="Tet10" if quadratic else "Tet4", E=np.full(len(conn), 1e3), nu=np.full(len(conn), 0.3),
+                  faces=np.zeros((0, 3), np.int64), ftype="Tri3", clamp_nodes=np.flatnonzero((X[:, 2] == 0.0) & (X[:, 0] == -1.0)))
+
+
+# entries of the largest row: 39,200 (ten sorted runs), 18,000, 8,192 (two full runs), 2,592
+@pytest.mark.parametrize("n,quadratic", [(70, False), (30, True), (32, False), (18, False)])
+def test_large_rows(oracle, n, quadratic):
+    """Rows of nodes with thousands of elements: the pattern and the values, and an
+    upload (once the device is warm) that takes less than 0.1 s (comparing all
+    pairs of entries took 0.14 s at 1,922 Tet4 around a node, 0.3 s at 968 Tet10,
+    sixteen times as long at four times as many)."""
+    import time
+
+    import scipy.sparse as sp
+    import jfem
+    m = fan(n, quadratic)
+    ctx = jfem.Context(0)
+    say(f"large rows: {m.n_el} {m.etype} around a node")
+    ctx.upload(M.box_tet10(2, 2, 2))
+    ctx.upload(fan(4, quadratic))
+    t = time.perf_counter()
+    ctx.upload(m)
+    t = time.perf_counter() - t
+    say(f"upload {1e3 * t:.1f} ms")
+    rp, ci = ctx.csr_pattern()
+    vals = ctx.assemble()[0]
+    ro, co, vo = oracle.assemble_csr(m)
+    assert np.array_equal(rp, ro) and np.array_equal(ci, co)
+    assert np.abs(vals - vo).max() <= 1e-13 * np.abs(vo).max()
+    assert t <= 0.1
+    ctx.close()
