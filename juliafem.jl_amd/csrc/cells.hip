@@ -78,33 +78,20 @@ __global__ __launch_bounds__(kCT) void k_cell_nodes(int n_el, int npe, int ps, i
     __syncthreads();
     // thread t takes the node of rank t
     const int q = t < nn ? ranked[t] : 0, n = t < nn ? cnt[q] : 0, r0 = head[q];
-    int all, total = 0, rank = -1;
+    int all, total, rank;
     const int off = block_scan<kCT>(n, &all);
     const size_t l = (size_t)p * kCT + t;
+    const int a = t < nn ? (int)(key[r0] >> 32) : 0;
+    const int b0 = t < nn ? inc_ptr[a] : 0, b1 = t < nn ? inc_ptr[a + 1] : 0;
+    patches_of_node<kCT>(n < b1 - b0, b0, b1, npe, ps, (n_el + ps - 1) / ps, p, inc, epos, &total, &rank);
+    if (total > 31) atomicOr(flags, kCellShared);  // 5 bits
     if (t < nn) {
-        const int a = (int)(key[r0] >> 32);
         const size_t base = (size_t)k0 * npe + off;
         for (int j = 0; j < n; ++j) {
             const uint32_t w = (uint32_t)key[r0 + j];
             const int i = w & 255, kl = (int)(w >> 8);
             lin[base + j] = (uint16_t)(i * stride + kl);
             connL[(size_t)i * n_el + k0 + kl] = (uint16_t)t;
-        }
-        const int b0 = inc_ptr[a], b1 = inc_ptr[a + 1];
-        if (n < b1 - b0) {  // its patches, in ascending order
-            rank = 0;
-            for (int last = -1;;) {
-                int next = INT32_MAX;
-                for (int k = b0; k < b1; ++k) {
-                    const int o = epos[inc[k] / npe] / ps;
-                    if (o > last && o < next) next = o;
-                }
-                if (next == INT32_MAX) break;
-                ++total;
-                rank += next < p;
-                last = next;
-            }
-            if (total > 31) atomicOr(flags, kCellShared);  // 5 bits
         }
         pn_node[l] = a;
         pn_cnt[l] = (uint16_t)n;

@@ -198,8 +198,8 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_row_sort(int N, const int32_
 
 // One workgroup per listed row: its entries as keys (column, t), sorted in LDS in
 // runs of kRun and merged in memory, run by run with its neighbour, each key to its
-// own place plus the smaller keys of the other run (a binary search).  At 2,000
-// Tet4 around a node (8,000 entries) the upload takes 0.7 ms instead of 142 with
+// own place plus the smaller keys of the other run (a binary search).  At 1,922
+// Tet4 around a node (7,688 entries) the upload takes 0.7 ms instead of 142 with
 // the comparison of all pairs in one wave, at 968 Tet10 0.64 instead of 299.
 // `keys`: two arrays of `entries`.
 constexpr int kRun = 4096, kLargeThreads = 1024;

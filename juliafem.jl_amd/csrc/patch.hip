@@ -464,22 +464,9 @@ __global__ __launch_bounds__(kPT) void k_patch_build(int n_el, int npe, int npat
     for (int u0 = 0; u0 < nn; u0 += kPT) {
         const int u = u0 + t, q = u < nn ? ranked[u] : 0;
         const int n = u < nn ? cnt[q] : 0, a = u < nn ? (int)(key[head[q]] >> 32) : 0;
-        int total = 0, rank = -1;
+        int total, rank;
         const int b0 = u < nn ? inc_ptr[a] : 0, b1 = u < nn ? inc_ptr[a + 1] : 0;
-        if (n < b1 - b0) {  // shared: its patches, in ascending order
-            rank = 0;
-            for (int last = -1;;) {
-                int next = INT32_MAX;
-                for (int k = b0; k < b1; ++k) {
-                    const int o = epos[inc[k] / npe] / kPatch;
-                    if (o > last && o < next) next = o;
-                }
-                if (next == INT32_MAX) break;
-                ++total;
-                rank += next < p;
-                last = next;
-            }
-        }
+        patches_of_node<kPT>(n < b1 - b0, b0, b1, npe, kPatch, npatch, p, inc, epos, &total, &rank);
         int sum, num;
         const int so = slots + block_scan<kPT>(rank == 0 ? total : 0, &sum);
         const int bo = shared + block_scan<kPT>(rank == 0, &num);

@@ -126,7 +126,7 @@ def fan(n, quadratic):
         ed, mid = np.unique(e.reshape(-1, 2), axis=0, return_inverse=True)
         X, conn = np.vstack([X, 0.5 * (X[ed[:, 0]] + X[ed[:, 1]])]), np.column_stack([conn, len(X) + mid.reshape(-1, 6)])
     return M.Mesh(X=X, conn=conn, etype="Tet10" if quadratic else "Tet4", E=np.full(len(conn), 1e3), nu=np.full(len(conn), 0.3),
-                  faces=np.zeros((0, 3), np.int64), ftype="Tri3", clamp_nodes=np.flatnonzero((X[:, 2] == 0.0) & (X[:, 0] == -1.0)))
+                  faces=np.zeros((0, 3), np.int64), ftype="Tri3", clamp_nodes=np.flatnonzero((X[:, 2] == 0.0) & (X[:, :2].min(1) == -1.0)))
 
 
 # entries of the largest row: 39,200 (ten sorted runs), 18,000, 8,192 (two full runs), 2,592
@@ -155,4 +155,42 @@ def test_large_rows(oracle, n, quadratic):
     assert np.array_equal(rp, ro) and np.array_equal(ci, co)
     assert np.abs(vals - vo).max() <= 1e-13 * np.abs(vo).max()
     assert t <= 0.1
+    ctx.close()
+
+
+# patches of the launched and of the resident form: 21 and 20; 4 and 15; 34 and 32 (one more
+# than the resident form's lists hold)
+@pytest.mark.parametrize("n,quadratic,resident", [(70, False, True), (30, True, True), (90, False, False)])
+def test_patches_around_a_node(oracle, n, quadratic, resident):
+    """A node that lies in every patch: products of the patch operator against the
+    oracle's matrix (1e-12, the bar of jfm_apply), a resident solve against the
+    launched assembled one (100 times rtol), and the time to make the patches (below
+    the 40 ms that a quarter of these elements took one thread)."""
+    import time
+
+    import jfem
+    m = fan(n, quadratic)
+    x = np.random.default_rng(4).normal(size=m.n_dofs)
+    csr = oracle.assemble_csr(m)
+    ref = oracle.spmv(csr, x) * (1 - m.fixed_mask().ravel())
+    ctx = jfem.Context(0)
+    ctx.upload(fan(4, quadratic))
+    ctx.apply(np.ones(3 * fan(4, quadratic).n_nodes))
+    ctx.upload(m)
+    say(f"patches around a node: {m.n_el} {m.etype}")
+    t = time.perf_counter()
+    y = ctx.apply(x)
+    t = time.perf_counter() - t
+    say(f"first product {1e3 * t:.1f} ms, {ctx.info()['n_patches']} patches")
+    assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max()
+    assert np.array_equal(y, ctx.apply(x))
+    assert t <= 0.03
+    f = np.random.default_rng(5).normal(size=m.n_dofs)
+    ud = ctx.solve(f=f, op="csr", op_outer="csr", coarse_nodes=100, rtol=1e-9)[0]
+    assert ctx.resident_counts() == (0, 0)
+    t = time.perf_counter()
+    u = ctx.solve(f=f, rtol=1e-9)[0]
+    say(f"first solve {1e3 * (time.perf_counter() - t):.1f} ms, resident: {ctx.resident_counts()[0]}")
+    assert (ctx.resident_counts()[0] > 0) == resident
+    assert np.linalg.norm(u - ud) <= 1e-7 * np.linalg.norm(ud)
     ctx.close()
