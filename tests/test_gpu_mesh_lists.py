@@ -194,3 +194,28 @@ def test_patches_around_a_node(oracle, n, quadratic, resident):
     assert (ctx.resident_counts()[0] > 0) == resident
     assert np.linalg.norm(u - ud) <= 1e-7 * np.linalg.norm(ud)
     ctx.close()
+
+
+@pytest.mark.parametrize("n,quadratic", [(4, False), (6, False), (15, False), (6, True), (22, True)])
+def test_iterations_around_a_node(n, quadratic):
+    """A node of 32 to 968 elements in the resident form, whose sums the wave then
+    forms together: the launched assembled solve's answer (100 times rtol), the same
+    bits again, and below 15 us an iteration (the node's lane alone: 50 with 450 Tet4
+    in a patch; launched 33)."""
+    import jfem
+    m = fan(n, quadratic)
+    f = np.random.default_rng(5).normal(size=m.n_dofs)
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    say(f"iterations around a node: {m.n_el} {m.etype}")
+    ud = ctx.solve(f=f, op="csr", op_outer="csr", coarse_nodes=100, rtol=1e-10)[0]
+    for kw in (dict(), dict(method=1, inner_rtol=1e-2), dict(coarse_nodes=60)):
+        u = ctx.solve(f=f, rtol=1e-10, **kw)[0]
+        u2, _, st = ctx.solve(f=f, rtol=1e-10, **kw)
+        assert np.linalg.norm(u - ud) <= 1e-8 * np.linalg.norm(ud)
+        assert np.array_equal(u, u2)
+        if not kw:
+            say(f"{1e3 * st['solve_ms'] / st['iterations']:.1f} us an iteration")
+            assert st["solve_ms"] <= 0.2 + 0.015 * st["iterations"]
+    assert ctx.resident_counts()[0] > 0
+    ctx.close()
