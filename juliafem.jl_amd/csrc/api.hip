@@ -674,16 +674,23 @@ extern "C" int jfm_assemble_tl(jfm_ctx *ctx, int32_t geometric, const double *u,
     hipStream_t s = ctx->stream;
     const int64_t n = ctx->ndof;
     const size_t vbytes = sizeof(double) * 9 * (size_t)ctx->nnzb;
+    if (!ctx->vals64) ALLOC(ctx, ctx->vals64, double, 9 * ctx->nnzb);
+    if (!ctx->vals32) ALLOC(ctx, ctx->vals32, float, 9 * ctx->nnzb);
     // finite-strain element blocks, the factors of Kg's, and the values of Km and
     // Kg that are asked for beside those of Km + Kg: a workspace that stays with the
-    // mesh up to 512 MB (its allocation and release took 0.1 ms a call)
-    const int64_t pairs = ctx->n_el * ctx->npair, nv = 9 * ctx->nnzb;
-    const int64_t want = 9 * pairs + (geometric ? pairs + (vals ? nv : 0) + (vals_kg ? nv : 0) : 0);
+    // mesh up to 512 MB (its allocation and release took 0.1 ms a call).  Where all
+    // that does not fit, the element blocks alone, and Kg, Km and their sum one
+    // after the other (three passes over elements and blocks instead of one).
+    const int64_t pairs = ctx->n_el * ctx->npair, nv = 9 * ctx->nnzb, least = 9 * pairs;
+    const int64_t want = least + (geometric ? pairs + (vals ? nv : 0) + (vals_kg ? nv : 0) : 0);
+    bool one_pass = true;
     if (ctx->tl_ws_n < want) {
         free_ptr(ctx, ctx->tl_ws);
         ctx->tl_ws_n = 0;
-        ALLOC(ctx, ctx->tl_ws, double, want);
-        ctx->tl_ws_n = want;
+        ctx->tl_ws = jfm_alloc<double>(ctx, want);
+        one_pass = ctx->tl_ws != nullptr;
+        if (!one_pass) ALLOC(ctx, ctx->tl_ws, double, least);
+        ctx->tl_ws_n = one_pass ? want : least;
     }
     struct Keep {
         jfm_ctx *ctx;
@@ -694,22 +701,35 @@ extern "C" int jfm_assemble_tl(jfm_ctx *ctx, int32_t geometric, const double *u,
             ctx->tl_ws_n = 0;
         }
     } keep{ctx};
-    double *Ke = ctx->tl_ws, *Kg = geometric ? Ke + 9 * pairs : nullptr;
-    double *vm = geometric && vals ? Kg + pairs : nullptr;
-    double *vg = geometric && vals_kg ? Kg + pairs + (vals ? nv : 0) : nullptr;
-    if (!ctx->vals64) ALLOC(ctx, ctx->vals64, double, 9 * ctx->nnzb);
-    if (!ctx->vals32) ALLOC(ctx, ctx->vals32, float, 9 * ctx->nnzb);
     ctx->assembled = false;
     if (u) JFM_HIP(ctx, hipMemcpyAsync(ctx->vx64, u, sizeof(double) * n, hipMemcpyHostToDevice, s));
     else JFM_HIP(ctx, hipMemsetAsync(ctx->vx64, 0, sizeof(double) * n, s));
     // Km, Kg and the element forces; f = f_ext - f_int (src/problems_elasticity.jl:432-433)
-    CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, Ke, Kg, ctx->ye64));
-    CHECK_LAUNCH(ctx, launch_assemble_values_ke(ctx, Ke, Kg, vm, vg));
+    double *const ws = ctx->tl_ws;
+    if (one_pass) {
+        double *Kg = geometric ? ws + least : nullptr, *vm = geometric && vals ? Kg + pairs : nullptr;
+        double *vg = geometric && vals_kg ? Kg + pairs + (vals ? nv : 0) : nullptr;
+        CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, ws, Kg, ctx->ye64));
+        CHECK_LAUNCH(ctx, launch_assemble_values_ke(ctx, ws, Kg, vm, vg));
+        if (vals_kg) JFM_HIP(ctx, hipMemcpyAsync(vals_kg, vg, vbytes, hipMemcpyDeviceToHost, s));
+        if (vals) JFM_HIP(ctx, hipMemcpyAsync(vals, vm ? vm : ctx->vals64, vbytes, hipMemcpyDeviceToHost, s));
+    } else {
+        if (vals_kg) {
+            CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, nullptr, ws, nullptr));
+            CHECK_LAUNCH(ctx, launch_assemble_values_kg(ctx, ws, false));
+            JFM_HIP(ctx, hipMemcpyAsync(vals_kg, ctx->vals64, vbytes, hipMemcpyDeviceToHost, s));
+        }
+        CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, ws, nullptr, ctx->ye64));
+        CHECK_LAUNCH(ctx, launch_assemble_values_ke(ctx, ws, nullptr, nullptr, nullptr));
+        if (vals) JFM_HIP(ctx, hipMemcpyAsync(vals, ctx->vals64, vbytes, hipMemcpyDeviceToHost, s));
+        if (geometric) {
+            CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, nullptr, ws, nullptr));
+            CHECK_LAUNCH(ctx, launch_assemble_values_kg(ctx, ws, true));
+        }
+    }
     CHECK_LAUNCH(ctx, launch_gather<double>(ctx, ctx->ye64, nullptr, ctx->vy64, nullptr, nullptr, nullptr, nullptr));
     CHECK_LAUNCH(ctx, (launch_convert<double, double>(ctx, ctx->vy64, ctx->vy64, n, -1.0)));
     CHECK_LAUNCH(ctx, launch_add(ctx, ctx->f_ext, ctx->vy64, ctx->load, n));
-    if (vals_kg) JFM_HIP(ctx, hipMemcpyAsync(vals_kg, vg, vbytes, hipMemcpyDeviceToHost, s));
-    if (vals) JFM_HIP(ctx, hipMemcpyAsync(vals, vm ? vm : ctx->vals64, vbytes, hipMemcpyDeviceToHost, s));
     if (f) JFM_HIP(ctx, hipMemcpyAsync(f, ctx->load, sizeof(double) * n, hipMemcpyDeviceToHost, s));
     if (int rc = sync(ctx)) return rc;
     ctx->assembled = true;

@@ -265,9 +265,9 @@ __global__ __launch_bounds__(256) void k_elem_mat(int n_el, int ngf, const doubl
 //     lambda a_i (x) a_j + mu ((g_i . g_j) F F' + a_j (x) a_i),   a = F g,
 // the block of BNL' S3 BNL is (g_i' S g_j) I, and BL' S at node i is F S g_i
 // (all times w detJ in the reference configuration).  Km goes to the packed pair
-// blocks `Ke`, the factors of I of Kg's blocks to `Kg` (when not null), f_int
-// (when ye != null) to the incidence slots for the nodal gather.  One 64-lane
-// block per element.
+// blocks `Ke`, the factors of I of Kg's blocks to `Kg`, f_int to the incidence
+// slots `ye` for the nodal gather (each where not null).  One 64-lane block per
+// element.
 template <int NPE>
 __global__ __launch_bounds__(64) void k_tl_elem(int n_el, int ngf, const double *__restrict__ gf,
                                                const int32_t *__restrict__ conn, const int32_t *__restrict__ slot,
@@ -336,7 +336,7 @@ __global__ __launch_bounds__(64) void k_tl_elem(int n_el, int ngf, const double 
                 FFq[q][c * 3 + d] = F[c * 3] * F[d * 3] + F[c * 3 + 1] * F[d * 3 + 1] + F[c * 3 + 2] * F[d * 3 + 2];
     }
     __syncthreads();
-    if (Ke && t < NP) {
+    if ((Ke || Kg) && t < NP) {
         const int i = PT.i[t], j = PT.j[t];
         double K[9], kg = 0.0;
 #pragma unroll
@@ -367,9 +367,11 @@ __global__ __launch_bounds__(64) void k_tl_elem(int n_el, int ngf, const double 
             }
         }
         if (Kg) Kg[(size_t)e * NP + t] = kg;
-        double *out = Ke + ((size_t)e * NP + t) * 9;
+        if (Ke) {
+            double *out = Ke + ((size_t)e * NP + t) * 9;
 #pragma unroll
-        for (int m = 0; m < 9; ++m) out[m] = K[m];
+            for (int m = 0; m < 9; ++m) out[m] = K[m];
+        }
     }
     if (ye && t < NPE) {
         double fi[3] = {0.0, 0.0, 0.0};
@@ -521,6 +523,37 @@ __global__ __launch_bounds__(256) void k_face(int nf, int nfn, const int32_t *__
         for (int c = 0; c < 3; ++c) fe[((size_t)f * nfn + i) * 3 + c] = out[i][c];
 }
 
+// The values of Kg from the factors of its blocks: alone (add = false), or added to
+// those of Km, as k_asm_vals_ke with GEO forms them.
+template <int NPE>
+__global__ __launch_bounds__(256) void k_asm_vals_kg(int nnzb, const int32_t *__restrict__ cptr,
+                                                    const int32_t *__restrict__ contrib,
+                                                    const int32_t *__restrict__ blk_row, const int32_t *__restrict__ brow,
+                                                    const double *__restrict__ Kg, bool add, double *__restrict__ vals,
+                                                    float *__restrict__ vals32) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nnzb) return;
+    double kg = 0.0;
+    for (int k = cptr[s]; k < cptr[s + 1]; ++k) {
+        const int c = contrib[k];
+        const int e = c / (NPE * NPE), rem = c - e * NPE * NPE;
+        const int i = rem / NPE, j = rem - i * NPE;
+        kg += Kg[(size_t)e * Elem<NPE>::NPAIR + (i <= j ? pair_index<NPE>(i, j) : pair_index<NPE>(j, i))];
+    }
+    const int a = blk_row[s];
+    const int nb = brow[a + 1] - brow[a], ks = s - brow[a];
+    const size_t base = 9 * (size_t)brow[a] + 3 * (size_t)ks;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const size_t o = base + (size_t)c * 3 * nb + d;
+            const double g = c == d ? kg : 0.0, v = add ? vals[o] + g : g;
+            vals[o] = v;
+            vals32[o] = (float)v;
+        }
+}
+
 // ----------------------------------------------------------- block Jacobi --
 // Diagonal 3x3 blocks sum_e K_e(i,i) over the node's incidences
 // (kNodeLanes lanes per node), fixed rows/columns replaced by identity before inversion and
@@ -651,6 +684,22 @@ hipError_t launch_assemble_values_ke(jfm_ctx *ctx, const double *Ke, const doubl
     case 10: launch(Kg ? k_asm_vals_ke<10, true> : k_asm_vals_ke<10, false>); break;
     case 4: launch(Kg ? k_asm_vals_ke<4, true> : k_asm_vals_ke<4, false>); break;
     case 8: launch(Kg ? k_asm_vals_ke<8, true> : k_asm_vals_ke<8, false>); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_assemble_values_kg(jfm_ctx *ctx, const double *Kg, bool add) {
+    const int n = (int)ctx->nnzb;
+    if (n == 0) return hipSuccess;
+    auto launch = [&](auto kernel) {
+        kernel<<<nblk(n), kBlock, 0, ctx->stream>>>(n, ctx->cptr, ctx->contrib, ctx->blk_row, ctx->brow, Kg, add, ctx->vals64,
+                                                    ctx->vals32);
+    };
+    switch (ctx->npe) {
+    case 10: launch(k_asm_vals_kg<10>); break;
+    case 4: launch(k_asm_vals_kg<4>); break;
+    case 8: launch(k_asm_vals_kg<8>); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

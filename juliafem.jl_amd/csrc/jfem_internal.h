@@ -424,8 +424,7 @@ hipError_t launch_pattern_write(jfm_ctx *ctx, int32_t *scratch);
 hipError_t launch_element_matrices(jfm_ctx *ctx);
 hipError_t launch_assemble_values(jfm_ctx *ctx);
 // finite-strain element matrices Km, element-major into Ke, the factors of I of
-// Kg's blocks into Kg (when not null) and, when ye != null, f_int(u) into the
-// incidence slots
+// Kg's blocks into Kg and f_int(u) into the incidence slots ye, each when not null
 hipError_t launch_tl_element_matrices(jfm_ctx *ctx, const double *u, double *Ke, double *Kg, double *ye);
 // Values per element of the EBE matrices: 9 NPAIR rounded up to a multiple
 // of the chunk width V (2 doubles or 4 floats).
@@ -433,6 +432,8 @@ inline int64_t ke_stride(int npair, int V) { return (9 * (int64_t)npair + V - 1)
 // CSR values from element-major packed blocks Ke[(e * NPAIR + p) * 9 + m] (and Kg's
 // factors: then of the sum, and Km's and Kg's alone to vm and vg when not null)
 hipError_t launch_assemble_values_ke(jfm_ctx *ctx, const double *Ke, const double *Kg, double *vm, double *vg);
+// Kg's values alone, or (add) added to Km's, to the same bits as the sum above
+hipError_t launch_assemble_values_kg(jfm_ctx *ctx, const double *Kg, bool add);
 hipError_t launch_face_loads(jfm_ctx *ctx);
 hipError_t launch_block_jacobi(jfm_ctx *ctx, double *Minv64, float *Minv32);
 // Two-phase operators; `part` (may be null) receives one partial of

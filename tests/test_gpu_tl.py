@@ -124,3 +124,43 @@ def test_host_mirror_nonlinear_run(jf, oracle):
     assert body.assembly.Kg is not None and abs(body.assembly.Kg).max() > 0
     say(f"  {solver.iteration} iterations, |du| = {solver.u_norm_change:.2e}")
     assert np.linalg.norm(body.u - uo) / np.linalg.norm(uo) <= 1e-8
+
+
+def test_tl_where_the_workspace_of_one_pass_does_not_fit(jf):
+    """With device memory for the element blocks of Km only (what the assembly of
+    Km alone takes), Km, Kg, f and the CSR operator are those of the assembly with
+    all the memory, to the bit."""
+    import ctypes as C
+    m = box_tet10(50, 20, 16, seed=5, jitter=0.1, E_sigma=0.5)   # element blocks 380 MB, all it may take 0.9 GB
+    rng = np.random.default_rng(9)
+    u, x = 1e-3 * rng.standard_normal(m.n_dofs), rng.standard_normal(m.n_dofs)
+    ref = jf.Context(0)
+    ref.upload_mesh(m.X, m.conn, m.etype, m.E, m.nu)
+    vals, kg, f = ref.assemble_tl(u)
+    y = ref.apply(x, op="csr")
+    ref.close()
+    ctx = jf.Context(0)
+    ctx.upload_mesh(m.X, m.conn, m.etype, m.E, m.nu)
+    km0, _, f0 = ctx.assemble_tl(u, geometric=False)
+    hip = C.CDLL("libamdhip64.so.7")
+    hip.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+    hip.hipFree.argtypes = [C.c_void_p]
+    hip.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t)] * 2
+    free, total, held = C.c_size_t(), C.c_size_t(), []
+    try:
+        for size in (32 << 30, 4 << 30, 512 << 20, 64 << 20):   # until 256 MB are left
+            while hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0 and free.value >= size + (256 << 20):
+                p = C.c_void_p()
+                if hip.hipMalloc(C.byref(p), size) != 0:
+                    break
+                held.append(p)
+        say(f"tl assembly beside {len(held)} held blocks, {free.value >> 20} MB free")
+        v2, g2, f2 = ctx.assemble_tl(u)
+        y2 = ctx.apply(x, op="csr")
+        v3, _, f3 = ctx.assemble_tl(u, geometric=False)
+    finally:
+        for p in held:
+            hip.hipFree(p)
+    assert np.array_equal(v2, vals) and np.array_equal(g2, kg) and np.array_equal(f2, f) and np.array_equal(y2, y)
+    assert np.array_equal(v3, km0) and np.array_equal(f3, f0)
+    ctx.close()
