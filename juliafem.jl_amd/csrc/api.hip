@@ -352,23 +352,26 @@ extern "C" int jfm_upload_mesh(jfm_ctx *ctx, int64_t n_nodes, const double *X, i
     JFM_HIP(ctx, hipMemcpyAsync(&h_bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, s));
     if (int rc = sync(ctx)) return rc;
     if (h_bad) return jfm_fail(ctx, JFM_ENOTSPD, "element with detJ <= 0 at a Gauss point (inverted or degenerate)");
-    ctx->has_mesh = true;
     // Meshes whose iterations are launched get the patch operator with the upload,
     // so that the products of jfm_apply_noalloc, which may not allocate, take it
     // too.  It needs patches for a good part of the CUs: FP64 Tet10 13.5 against
     // 15.1 us of the two-phase form with 64 of them, 28.1 against 49.6 with 512;
     // Hex8 (eight points: more per workgroup) 18.5 against 16.2 with 86, 19.1
-    // against 19.9 with 128, 26.1 against 33.0 with 254.  Without room for it the
-    // mesh is still good for the CSR operator.
+    // against 19.9 with 128, 26.1 against 33.0 with 254.  Without room for it (or
+    // with indices that do not fit) the mesh is still good for the CSR operator;
+    // a failure of the device is one of the upload.
     const int64_t patches = (n_el + kPatchElems - 1) / kPatchElems;
     if (jfem_patch_enabled() && !jfem_persist_maybe<double>(ctx, JFM_OP_MATFREE) && patches >= (npe == 8 ? 192 : 64)) {
-        if (jfem_patch_setup(ctx) == JFM_OK) {
-            ctx->na_part = jfm_alloc<double>(ctx, 3 * (int64_t)std::max(1, ctx->nslot));
-            ctx->patch_upload = ctx->patch_ready && ctx->na_part;
-        } else {
+        const int rc = jfem_patch_setup(ctx);
+        if (rc != JFM_OK && rc != JFM_ENOMEM && rc != JFM_EINVAL) return rc;
+        if (rc == JFM_OK) ctx->na_part = jfm_alloc<double>(ctx, 3 * (int64_t)std::max(1, ctx->nslot));
+        ctx->patch_upload = ctx->patch_ready && ctx->na_part;
+        if (!ctx->patch_upload) {  // all of it or nothing
+            jfem_patch_release(ctx);
             ctx->err.clear();
         }
     }
+    ctx->has_mesh = true;
     return JFM_OK;
 }
 
