@@ -770,12 +770,6 @@ static int ensure_workspaces(jfm_ctx *ctx) {
 
 int jfem_ensure_workspaces(jfm_ctx *ctx) { return ensure_workspaces(ctx); }
 
-int jfem_apply(jfm_ctx *ctx, int op, const double *x, double *y) {
-    if (int rc = prepare_op(ctx, op)) return rc;
-    CHECK_LAUNCH(ctx, op_apply<double>(ctx, op, x, y, nullptr, nullptr, nullptr, nullptr));
-    return JFM_OK;
-}
-
 static int read_scalars(jfm_ctx *ctx);
 static int finalize_misc(jfm_ctx *ctx, int npart, int nv, int fin);
 

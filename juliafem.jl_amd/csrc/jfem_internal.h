@@ -385,7 +385,6 @@ struct jfm_ctx {
 
 // api.hip helpers used by learned.hip
 int jfem_ensure_workspaces(jfm_ctx *ctx);                                   // vectors + block Jacobi
-int jfem_apply(jfm_ctx *ctx, int op, const double *x, double *y);          // masked FP64 K.x (device)
 int jfem_dot(jfm_ctx *ctx, const double *a, const double *b, int64_t n, double *out);
 // noalloc.hip: looks up the scratch array's device address (once per device)
 int jfem_noalloc_init(jfm_ctx *ctx);
@@ -492,12 +491,12 @@ constexpr int kPersistPatches = 256;
 // latency of a load past the L2, about 0.7 us: a second or so in all);
 // JFEM_PERSIST_POLLS sets fewer.
 constexpr int kMaxPolls = 1 << 20;
-// elements of a patch, its workgroup's threads (and most nodes), the row
-// stride of its LDS image of the element terms
-// Geometric factors in the element order perm (gfQ32: folded ones too, or null).
 // Elements along a Morton curve of their centroids (cells.hip).
 std::vector<int32_t> morton_order(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int npe);
+// Geometric factors in the element order perm (gfQ32: folded ones too, or null).
 hipError_t launch_patch_factors(jfm_ctx *ctx, const int32_t *perm, double *gf64, float *gf32, float *gfQ32);
+// elements of a patch, its workgroup's threads (and most nodes), the row
+// stride of its LDS image of the element terms
 struct PersistGeometry { int elems = 0, threads = 0, stride = 0; };
 int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g);
 void jfem_cells_release(jfm_ctx *ctx);

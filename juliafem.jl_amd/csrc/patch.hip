@@ -21,7 +21,6 @@
 // loop and nodal assembly), elements per src/problems_elasticity.jl:203-451.
 #include <algorithm>
 #include <cstdlib>
-#include <numeric>
 #include <vector>
 
 #include "ebe_element.h"

@@ -100,9 +100,8 @@ template <typename T> struct PersistArgs {
     int nc, ldc;
     double *wpart;
     uint64_t *zw;
-    // nsys systems of one operator side by side: workgroups npatch s .. of the
-    // grid solve system s, its b and x ss values further, scalars at S + s
-    int nsys;
+    // systems of one operator side by side: workgroups npatch s .. of the grid
+    // solve system s, its b and x ss values further, scalars at S + s
     int64_t ss;
 };
 
@@ -1237,7 +1236,6 @@ hipError_t launch_pcg_persist(jfm_ctx *ctx, int op, const T *Minv, const T *b, c
     A.maxit = maxit;
     A.polls = ctx->persist_polls;
     A.S = nsys > 1 ? C.S : ctx->S;
-    A.nsys = nsys;
     A.ss = ss;
     const int nw = nsys * (grid_words(1, C.npatch) + grid_words(2, C.npatch));
     launch_persist_clear(ctx, nw, C.words, nz, C.zw, nsys, A.S);
