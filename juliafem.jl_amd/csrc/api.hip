@@ -1645,10 +1645,12 @@ extern "C" int jfm_postprocess(jfm_ctx *ctx, const double *u, double *strain_gp,
             if (e == hipSuccess) e = hipMemcpyAsync(outs[field[f]], J, sizeof(double) * 6 * N, hipMemcpyDeviceToHost, s);
             if (e != hipSuccess) fail_hip(e, "nodal copy");
         }
-        (void)hipStreamSynchronize(s);
+        e = hipStreamSynchronize(s);
+        if (rc == JFM_OK && e != hipSuccess) fail_hip(e, "nodal copy");
         for (void *p : {(void *)B, (void *)X, (void *)J}) jfm_free(ctx, p);
     }
-    (void)hipStreamSynchronize(s);
+    e = hipStreamSynchronize(s);
+    if (rc == JFM_OK && e != hipSuccess) fail_hip(e, "jfm_postprocess");
     cleanup();
     return rc;
 }
