@@ -880,8 +880,11 @@ extern "C" int jfm_learned_outputs(jfm_ctx *ctx, float *out, double *M) {
     return JFM_OK;
 }
 
-// residual/error pairs held on the device at a time
+// residual/error pairs held on the device at a time: at most kPairRun, fewer where
+// their vectors (r, e, z, w) and partial sums would take more than 512 MB, in which
+// a training loop keeps them; what one pair takes beyond that goes after the call
 constexpr int kPairRun = 8;
+constexpr int64_t kPairBytes = int64_t(512) << 20;
 
 void jfem_train_release(jfm_ctx *ctx) {
     auto &W = ctx->train;
@@ -906,10 +909,18 @@ extern "C" int jfm_learned_grad(jfm_ctx *ctx, int32_t n_pairs, const double *r, 
         if (int rc = jfem_patch_setup(ctx)) return rc;
     const int64_t n = ctx->ndof, N = ctx->N;
     hipStream_t s = ctx->stream;
-    // the pairs go to the device in runs of up to kPairRun; the buffers stay
-    // with the mesh (a training loop calls this once per step)
+    // the pairs go to the device in runs; the buffers stay with the mesh (a training
+    // loop calls this once per step)
     auto &W = ctx->train;
-    const int run = std::min(n_pairs, kPairRun);
+    const int64_t pair_bytes = sizeof(double) * (4 * n + 3 * (int64_t)ctx->nslot);
+    const int run = (int)std::min<int64_t>(std::min(n_pairs, kPairRun), std::max<int64_t>(1, kPairBytes / pair_bytes));
+    struct Keep {
+        jfm_ctx *ctx;
+        bool keep;
+        ~Keep() {
+            if (!keep) jfem_train_release(ctx);
+        }
+    } keep{ctx, pair_bytes <= kPairBytes};
     if (W.pairs < run) {
         jfem_train_release(ctx);
         W.r = jfm_alloc<double>(ctx, run * n);

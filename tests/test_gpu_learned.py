@@ -173,3 +173,27 @@ def test_default_network_inside_two_level_method(oracle):
         assert runs["probed"]["fallback"] == (1 if it_l > it_b else 0)
     # the recorded finding: the learned blocks lose to block Jacobi here
     assert it_l > it_b
+
+
+def test_training_buffers_on_a_large_mesh():
+    """2.6 million DOFs, eight pairs: the device memory that a gradient leaves behind
+    (the pairs' vectors at most 512 MB of it: all eight would take 0.8 GB), the loss
+    as the mean of the pairs' own, the same bits again."""
+    import jfem
+    from jfem import mesh as M
+    from jfem.learned import DEFAULT_WEIGHTS
+    m = M.box_tet10(110, 36, 26, seed=1, jitter=0.1)
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    ctx.set_learned_weights(open(DEFAULT_WEIGHTS, "rb").read())
+    R = np.random.default_rng(3).standard_normal((8, m.n_dofs)) * (1 - m.fixed_mask().ravel())
+    one = [ctx.learned_grad(R[k:k + 1], R[k:k + 1])[0] for k in range(8)]
+    before = ctx.info()["device_bytes"]
+    loss, g = ctx.learned_grad(R, R)
+    left = ctx.info()["device_bytes"] - before
+    print(f"[gpu] {m.n_dofs} DOFs, {left >> 20} MB more than for one pair", flush=True)
+    assert left <= 512 << 20
+    assert abs(loss - np.mean(one)) <= 1e-12 * abs(loss)
+    loss2, g2 = ctx.learned_grad(R, R)
+    assert loss2 == loss and np.array_equal(g2, g)
+    ctx.close()
