@@ -355,8 +355,9 @@ extern "C" int jfm_upload_mesh(jfm_ctx *ctx, int64_t n_nodes, const double *X, i
     // Meshes whose iterations are launched get the patch operator with the upload,
     // so that the products of jfm_apply_noalloc, which may not allocate, take it
     // too.  It needs patches for a good part of the CUs: FP64 Tet10 13.5 against
-    // 15.1 us of the two-phase form with 64 of them, 28.1 against 49.6 with 512;
-    // Hex8 (eight points: more per workgroup) 18.5 against 16.2 with 86, 19.1
+    // 15.1 us of the two-phase form with 64 of them, 28.1 against 49.6 with 512,
+    // curved 15.3 against 14.6 with 51, 15.5 and 15.6 with 63, 15.8 against 17.6 with
+    // 82; Hex8 (eight points: more per workgroup) 18.5 against 16.2 with 86, 19.1
     // against 19.9 with 128, 26.1 against 33.0 with 254.  Without room for it (or
     // with indices that do not fit) the mesh is still good for the CSR operator;
     // a failure of the device is one of the upload.

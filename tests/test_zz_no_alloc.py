@@ -184,3 +184,26 @@ def test_noalloc_in_place(env, op, prec, shift):
         assert np.abs(v.get()[shift:] - ref).max() <= (1e-12 if prec == 0 else 2e-6) * np.abs(ref).max()
     v.free()
     c.close()
+
+
+@pytest.mark.parametrize("g", [(30, 14, 12), (31, 14, 12)])
+def test_noalloc_at_the_forms_limit(env, g):
+    """Curved Tet10 (no resident form) on both sides of 64 patches: to the bars of
+    jfm_apply, the patch operator's own bits where it runs."""
+    jfem, lib, hip = env
+    m = box_tet10(*g, L=g, seed=1, jitter=0.1)
+    X = m.X.copy()
+    mid = np.unique(m.conn[:, 4:])
+    X[mid] += 0.005 * np.random.default_rng(5).uniform(-1.0, 1.0, (len(mid), 3))
+    c = jfem.Context(0)
+    c.upload_mesh(X, m.conn, m.etype, m.E, m.nu)
+    patches = (m.n_el + 479) // 480
+    say(f"noalloc on {patches} curved patches")
+    assert c.info()["affine"] == 0 and c.info()["n_patches"] == (patches if patches >= 64 else 0)
+    x = np.random.default_rng(3).standard_normal(m.n_dofs)
+    ref = c.apply(x, op="matfree")
+    for prec, bar in ((0, 1e-12), (1, 2e-6)):
+        rc, y = noalloc(env, c, "matfree", prec, x)
+        assert rc == 0 and np.abs(y - ref).max() <= bar * np.abs(ref).max()
+        assert np.array_equal(y, c.apply(x, op="matfree", precision=prec)) == (patches >= 64)
+    c.close()
