@@ -710,11 +710,18 @@ extern "C" int jfm_assemble_tl(jfm_ctx *ctx, int32_t geometric, const double *u,
     else JFM_HIP(ctx, hipMemsetAsync(ctx->vx64, 0, sizeof(double) * n, s));
     // Km, Kg and the element forces; f = f_ext - f_int (src/problems_elasticity.jl:432-433)
     double *const ws = ctx->tl_ws;
-    if (one_pass) {
+    auto forces = [&]() -> int {
+        CHECK_LAUNCH(ctx, launch_gather<double>(ctx, ctx->ye64, nullptr, ctx->vy64, nullptr, nullptr, nullptr, nullptr));
+        CHECK_LAUNCH(ctx, (launch_convert<double, double>(ctx, ctx->vy64, ctx->vy64, n, -1.0)));
+        CHECK_LAUNCH(ctx, launch_add(ctx, ctx->f_ext, ctx->vy64, ctx->load, n));
+        return JFM_OK;
+    };
+    if (one_pass) {  // all launches before the copies, which the host waits in
         double *Kg = geometric ? ws + least : nullptr, *vm = geometric && vals ? Kg + pairs : nullptr;
         double *vg = geometric && vals_kg ? Kg + pairs + (vals ? nv : 0) : nullptr;
         CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, ws, Kg, ctx->ye64));
         CHECK_LAUNCH(ctx, launch_assemble_values_ke(ctx, ws, Kg, vm, vg));
+        if (int rc = forces()) return rc;
         if (vals_kg) JFM_HIP(ctx, hipMemcpyAsync(vals_kg, vg, vbytes, hipMemcpyDeviceToHost, s));
         if (vals) JFM_HIP(ctx, hipMemcpyAsync(vals, vm ? vm : ctx->vals64, vbytes, hipMemcpyDeviceToHost, s));
     } else {
@@ -725,15 +732,13 @@ extern "C" int jfm_assemble_tl(jfm_ctx *ctx, int32_t geometric, const double *u,
         }
         CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, ws, nullptr, ctx->ye64));
         CHECK_LAUNCH(ctx, launch_assemble_values_ke(ctx, ws, nullptr, nullptr, nullptr));
+        if (int rc = forces()) return rc;
         if (vals) JFM_HIP(ctx, hipMemcpyAsync(vals, ctx->vals64, vbytes, hipMemcpyDeviceToHost, s));
         if (geometric) {
             CHECK_LAUNCH(ctx, launch_tl_element_matrices(ctx, ctx->vx64, nullptr, ws, nullptr));
             CHECK_LAUNCH(ctx, launch_assemble_values_kg(ctx, ws, true));
         }
     }
-    CHECK_LAUNCH(ctx, launch_gather<double>(ctx, ctx->ye64, nullptr, ctx->vy64, nullptr, nullptr, nullptr, nullptr));
-    CHECK_LAUNCH(ctx, (launch_convert<double, double>(ctx, ctx->vy64, ctx->vy64, n, -1.0)));
-    CHECK_LAUNCH(ctx, launch_add(ctx, ctx->f_ext, ctx->vy64, ctx->load, n));
     if (f) JFM_HIP(ctx, hipMemcpyAsync(f, ctx->load, sizeof(double) * n, hipMemcpyDeviceToHost, s));
     if (int rc = sync(ctx)) return rc;
     ctx->assembled = true;
