@@ -134,9 +134,11 @@ __device__ __forceinline__ double wave_total(double v) {
 // that).  One wave polls: lane 16 k + m reads value k of member m, so a sum over
 // members is a row sum.
 // FLAT: 17 to 64 workgroups store their entries once per 8 workgroups, and each
-// reads its copy of all of them, one hop (63 workgroups on the CSR matrix: 0.4 us
-// an iteration less; nothing gained with 102, and the element kernels, which have
-// no registers for it, lose 2-5%).
+// reads its copy of all of them, one hop.  On the CSR matrix an iteration with it and
+// without takes, Hex8, 5.6 and 6.4 us with 17 workgroups, 5.7 and 6.4 with 31, 5.7 and
+// 6.1 with 41, 5.9 and 6.6 with 61; Tet10 6.2 and 6.1 with 17, 6.1 and 6.8 with 23,
+// 6.1 and 6.7 with 42, 6.3 and 6.4 with 64; nothing is gained with 102, and the
+// element kernels, which have no registers for it, lose 2-5%.
 // Calls that follow each other without a block barrier use different `sh` (a
 // wave may still read it when the next one starts).
 constexpr int kGroup = 16, kCopy = 8, kFlat = 64;
