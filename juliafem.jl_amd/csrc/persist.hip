@@ -8,8 +8,8 @@
 // 139,587 DOFs 29,000 cycles, of which the element products and nodal sums take
 // 5,000, the exchanges 18,000.  Here one workgroup per patch stays
 // on its CU for the whole solve.  A patch's node vectors (r, x, z in
-// registers, p in LDS), its connectivity and its geometric factors never
-// leave the CU; what crosses workgroups in an iteration is the partial sums
+// registers, p in LDS), its connectivity and its geometric factors (but a
+// Hex8's, which are read from the L2) never leave the CU; what crosses workgroups in an iteration is the partial sums
 // of the nodes that patches share and a few scalars:
 //
 //   z = M r, partials of (r.z, r.r)           -> exchange C: beta, status
