@@ -9,6 +9,7 @@
 // sums, ascending patch.  On the host this took 7.5 ms at 12,810 Tet10 elements;
 // the kernels here take 0.13 ms.  No list depends on the order in which threads run.
 #include <algorithm>
+#include <array>
 #include <vector>
 
 #include "sort_scan.h"
@@ -209,26 +210,60 @@ static uint64_t spread16(uint64_t v) {
     return v;
 }
 
+// The axes' weights that measure long elements in their own lengths: the least mean
+// extent over the axis' own, from some thousand elements; 1 where that is less than
+// 1.3 times the least.
+static std::array<double, 3> length_weights(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int npe) {
+    std::array<double, 3> len = {0.0, 0.0, 0.0}, w;
+    const int64_t step = std::max<int64_t>(1, n_el / 1024);
+    for (int64_t e = 0; e < n_el; e += step)
+        for (int c = 0; c < 3; ++c) {
+            double l = 1e300, h = -1e300;
+            for (int i = 0; i < npe; ++i) {
+                const double x = X[3 * (size_t)conn[e * npe + i] + c];
+                l = std::min(l, x);
+                h = std::max(h, x);
+            }
+            len[c] += h - l;
+        }
+    const double least = std::min({len[0], len[1], len[2]});
+    for (int c = 0; c < 3; ++c) w[c] = least > 0.0 && len[c] > 1.3 * least ? least / len[c] : 1.0;
+    return w;
+}
+
 // Elements by the Morton code of their centroids, stable in the element id.  One
 // scale for the three axes keeps the patches compact: 35% fewer shared-node
 // partials than with each axis scaled to the bounding box at 61 x 7 x 5 hexes
-// (24,868 against 38,391), and at most 393 nodes a patch instead of 535.
-std::vector<int32_t> morton_order(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int npe) {
+// (24,868 against 38,391), and at most 393 nodes a patch instead of 535.  Long
+// elements make such patches flat: 40 x 40 x 40 hexes of 10 x 1 x 1 have 133,534
+// partials of 480-element patches, and up to 784 nodes in 256 elements, against
+// 59,000 and 486 with the axes in element lengths.  Flat patches have fewer
+// neighbours and shorter ranges of node ids, though, and were no slower but for
+// large Hex8 meshes: 500 FP32 iterations on 160 x 100 x 100 of 10 x 1 x 1 129.6 ms
+// against 124.8 in element lengths (FP64 249.8 and 240.5; bounding box 122.6 and
+// 243.9), Tet4 at 1,500,000 elements 27.0 against 28.6.  So by_length is taken by
+// the 480-element patches of Hex8, and by the resident form where it does not fit
+// without.
+std::vector<int32_t> morton_order(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int npe, bool by_length,
+                                  bool *long_elements) {
+    const std::array<double, 3> one = {1.0, 1.0, 1.0}, w = by_length ? length_weights(conn, X, n_el, npe) : one;
+    if (long_elements) *long_elements = w != one;
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
     for (size_t d = 0; d < X.size(); d += 3)
         for (int c = 0; c < 3; ++c) {
             lo[c] = std::min(lo[c], X[d + c]);
             hi[c] = std::max(hi[c], X[d + c]);
         }
-    const double side = std::max({hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]});
-    const double scale = side > 0.0 ? 65535.0 / side : 0.0;
+    double side = 0.0, scale[3];
+    for (int c = 0; c < 3; ++c) side = std::max(side, w[c] * (hi[c] - lo[c]));
+    for (int c = 0; c < 3; ++c) scale[c] = side > 0.0 ? w[c] * (65535.0 / side) : 0.0;
     std::vector<uint64_t> code(n_el);
     for (int64_t e = 0; e < n_el; ++e) {
         double s[3] = {0.0, 0.0, 0.0};
         for (int i = 0; i < npe; ++i)
             for (int c = 0; c < 3; ++c) s[c] += X[3 * (size_t)conn[e * npe + i] + c];
         uint64_t q[3];
-        for (int c = 0; c < 3; ++c) q[c] = (uint64_t)std::min(std::max((s[c] / npe - lo[c]) * scale, 0.0), 65535.0);
+        for (int c = 0; c < 3; ++c) q[c] = (uint64_t)std::min(std::max((s[c] / npe - lo[c]) * scale[c], 0.0), 65535.0);
         code[e] = spread16(q[0]) << 2 | spread16(q[1]) << 1 | spread16(q[2]);
     }
     std::vector<int32_t> perm(n_el), next(n_el);
@@ -243,20 +278,16 @@ std::vector<int32_t> morton_order(const std::vector<int32_t> &conn, const std::v
     return perm;
 }
 
-// The resident PCG's patches, once per mesh; cells.usable tells whether the
-// mesh fits.
-int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g) {
+// The resident PCG's patches from the elements' order perm; cells.usable tells
+// whether the mesh fits.
+static int cells_build(jfm_ctx *ctx, const PersistGeometry &g, const std::vector<int32_t> &perm) {
     auto &C = ctx->cells;
-    if (C.ready) return JFM_OK;
     C.ready = true;
     C.usable = false;
     const int64_t n_el = ctx->n_el, N = ctx->N;
     const int npe = ctx->npe;
     const int64_t np = (n_el + g.elems - 1) / g.elems;
-    // a node of no element is in no patch; 16-bit incidences
-    if (ctx->orphans || g.threads != kCT || g.elems * npe > kCK || npe * g.stride > 65536) return JFM_OK;
-    if ((int64_t)ctx->h_conn.size() != n_el * npe || (int64_t)ctx->h_X.size() != 3 * N) return JFM_OK;
-    std::vector<int32_t> perm = morton_order(ctx->h_conn, ctx->h_X, n_el, npe), epos(n_el);
+    std::vector<int32_t> epos(n_el);
     for (int64_t k = 0; k < n_el; ++k) epos[perm[k]] = (int32_t)k;
     hipStream_t s = ctx->stream;
     const int64_t pn = np * kCT, rows = (int64_t)ctx->ngf * GF;
@@ -302,6 +333,25 @@ int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g) {
     C.rho32 = (float)(2.0 * ctx->nu0 / (1.0 - 2.0 * ctx->nu0));
     C.usable = true;
     return JFM_OK;
+}
+
+// Once per mesh.  Long elements whose patches do not fit are cut again with the
+// axes in element lengths.
+int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g) {
+    auto &C = ctx->cells;
+    if (C.ready) return JFM_OK;
+    C.ready = true;
+    C.usable = false;
+    const int64_t n_el = ctx->n_el;
+    const int npe = ctx->npe;
+    // a node of no element is in no patch; 16-bit incidences
+    if (ctx->orphans || g.threads != kCT || g.elems * npe > kCK || npe * g.stride > 65536) return JFM_OK;
+    if ((int64_t)ctx->h_conn.size() != n_el * npe || (int64_t)ctx->h_X.size() != 3 * ctx->N) return JFM_OK;
+    if (int rc = cells_build(ctx, g, morton_order(ctx->h_conn, ctx->h_X, n_el, npe, false, nullptr))) return rc;
+    if (C.usable) return JFM_OK;
+    bool long_elements = false;
+    const std::vector<int32_t> perm = morton_order(ctx->h_conn, ctx->h_X, n_el, npe, true, &long_elements);
+    return long_elements ? cells_build(ctx, g, perm) : JFM_OK;
 }
 
 // Per patch the aggregates of its owned nodes, with those nodes, and per

@@ -224,3 +224,28 @@ def test_solves_from_several_threads(patches):
     assert all(s == [True] * 6 for s in same)
     for c in cs:
         c.close()
+
+
+@pytest.mark.parametrize("gen,g,slots", [("box_tet10", (12, 12, 12), None), ("box_tet10", (30, 12, 12), None),
+                                         ("box_hex8", (40, 40, 40), 61000)])
+def test_long_elements(gen, g, slots):
+    """Elements several times as long as wide (10 x 1 x 1): the resident form, whose
+    patches do not fit until they are cut in element lengths, and for Hex8 compact
+    480-element patches (the nodes' partial sums of the bounding box's scale within
+    2%; one scale for all axes gave 133,534)."""
+    import jfem
+    m = getattr(M, gen)(*g, seed=1, jitter=0.1)
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    say(f"long elements: {gen} {g}")
+    x = np.random.default_rng(2).normal(size=m.n_dofs)
+    y, yc = ctx.apply(x), ctx.apply(x, op="csr")
+    assert np.abs(y - yc).max() <= 1e-12 * np.abs(yc).max()
+    if slots:
+        assert ctx.info()["shared_slots"] <= slots
+    kw = dict(rtol=1e-8, coarse_nodes=300)
+    u = ctx.solve(**kw)[0]
+    assert ctx.resident_counts()[0] > 0
+    uc = ctx.solve(op="csr", op_outer="csr", **kw)[0]   # launched
+    assert np.linalg.norm(u - uc) <= 1e-6 * np.linalg.norm(uc)
+    ctx.close()
