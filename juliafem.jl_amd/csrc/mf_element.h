@@ -132,9 +132,9 @@ __host__ __device__ __forceinline__ void mf_element_x(int n_el, int e, const T *
                                                     (uint32_t)sizeof(T) * (uint32_t)(k * n_el + e));
             },
             xl, out, rho);
-    else
+    else  // q's base first: with one offset of q and k the FP32 Hex8 patches of 40 x 40 x 40 took 11.7 us, not 10.6
         mf_element_f<NPE, T, AFF, FOLD>(
-            [&](int q, int k) -> T { return gf[(size_t)(q * GF + k) * n_el + e]; }, xl, out, rho);
+            [&](int q, int k) -> T { return (gf + (size_t)q * GF * n_el + e)[(size_t)k * n_el]; }, xl, out, rho);
 }
 
 // The Gauss-point form: every element type, affine or not.
