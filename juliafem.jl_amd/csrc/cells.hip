@@ -10,6 +10,7 @@
 // the kernels here take 0.13 ms.  No list depends on the order in which threads run.
 #include <algorithm>
 #include <array>
+#include <cmath>
 #include <vector>
 
 #include "sort_scan.h"
@@ -231,23 +232,31 @@ static std::array<double, 3> length_weights(const std::vector<int32_t> &conn, co
     return w;
 }
 
+bool long_elements(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int npe) {
+    return length_weights(conn, X, n_el, npe) != std::array<double, 3>{1.0, 1.0, 1.0};
+}
+
 // Elements by the Morton code of their centroids, stable in the element id.  One
 // scale for the three axes keeps the patches compact: 35% fewer shared-node
 // partials than with each axis scaled to the bounding box at 61 x 7 x 5 hexes
 // (24,868 against 38,391), and at most 393 nodes a patch instead of 535.  Long
 // elements make such patches flat: 40 x 40 x 40 hexes of 10 x 1 x 1 have 133,534
 // partials of 480-element patches, and up to 784 nodes in 256 elements, against
-// 59,000 and 486 with the axes in element lengths.  Flat patches have fewer
-// neighbours and shorter ranges of node ids, though, and were no slower but for
-// large Hex8 meshes: 500 FP32 iterations on 160 x 100 x 100 of 10 x 1 x 1 129.6 ms
-// against 124.8 in element lengths (FP64 249.8 and 240.5; bounding box 122.6 and
-// 243.9), Tet4 at 1,500,000 elements 27.0 against 28.6.  So by_length is taken by
-// the 480-element patches of Hex8, and by the resident form where it does not fit
-// without.
-std::vector<int32_t> morton_order(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int npe, bool by_length,
-                                  bool *long_elements) {
+// 59,845 and 486 by_length, where an axis counts in element lengths and spans
+// 65,536 / 2^k, k the nearest to its length.  (Unrounded, cuts fell across the
+// grid's own: 64 x 32 x 32 hexes of 10 x 1 x 1 no longer fitted the resident form,
+// 40.4 us an FP64 iteration instead of 22.8, and 480 hexes of 100 x 25 x 26 had up
+// to 1,072 nodes, three rounds of threads instead of two.)  Per launched FP64/FP32
+// iteration, one scale, bounding box, by_length:
+//   Hex8 100 x 25 x 26             38.1/30.2   35.8/28.1   33.9/27.3 us
+//   Hex8 128 x 64 x 64, 1 x 1 x 4  178.0/90.4  172.8/84.7  170.0/82.9
+//   Tet10 90 x 30 x 30, 10 x 1 x 1 115.2/60.7  101.8/58.5  96.4/57.6
+//   Tet10 60 x 20 x 20, 10 x 1 x 1 49.5/32.1   47.6/32.3   46.2/30.6
+//   Tet4 100 x 50 x 50, 10 x 1 x 1 77.4/52.4   75.0/57.5   74.9/57.0
+// So it is taken by the 480-element patches of Hex8 and of long Tet10, and by the
+// resident form where long elements do not fit without.
+std::vector<int32_t> morton_order(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int npe, bool by_length) {
     const std::array<double, 3> one = {1.0, 1.0, 1.0}, w = by_length ? length_weights(conn, X, n_el, npe) : one;
-    if (long_elements) *long_elements = w != one;
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
     for (size_t d = 0; d < X.size(); d += 3)
         for (int c = 0; c < 3; ++c) {
@@ -256,7 +265,11 @@ std::vector<int32_t> morton_order(const std::vector<int32_t> &conn, const std::v
         }
     double side = 0.0, scale[3];
     for (int c = 0; c < 3; ++c) side = std::max(side, w[c] * (hi[c] - lo[c]));
-    for (int c = 0; c < 3; ++c) scale[c] = side > 0.0 ? w[c] * (65535.0 / side) : 0.0;
+    for (int c = 0; c < 3; ++c) {
+        const double l = w[c] * (hi[c] - lo[c]);
+        scale[c] = side > 0.0 ? w[c] * (65535.0 / side) : 0.0;
+        if (by_length && l * 32768.0 > side) scale[c] = 65535.0 / (hi[c] - lo[c]) * std::exp2(std::round(std::log2(l / side)));
+    }
     std::vector<uint64_t> code(n_el);
     for (int64_t e = 0; e < n_el; ++e) {
         double s[3] = {0.0, 0.0, 0.0};
@@ -347,11 +360,9 @@ int jfem_cells_setup(jfm_ctx *ctx, const PersistGeometry &g) {
     // a node of no element is in no patch; 16-bit incidences
     if (ctx->orphans || g.threads != kCT || g.elems * npe > kCK || npe * g.stride > 65536) return JFM_OK;
     if ((int64_t)ctx->h_conn.size() != n_el * npe || (int64_t)ctx->h_X.size() != 3 * ctx->N) return JFM_OK;
-    if (int rc = cells_build(ctx, g, morton_order(ctx->h_conn, ctx->h_X, n_el, npe, false, nullptr))) return rc;
-    if (C.usable) return JFM_OK;
-    bool long_elements = false;
-    const std::vector<int32_t> perm = morton_order(ctx->h_conn, ctx->h_X, n_el, npe, true, &long_elements);
-    return long_elements ? cells_build(ctx, g, perm) : JFM_OK;
+    if (int rc = cells_build(ctx, g, morton_order(ctx->h_conn, ctx->h_X, n_el, npe, false))) return rc;
+    if (C.usable || !long_elements(ctx->h_conn, ctx->h_X, n_el, npe)) return JFM_OK;
+    return cells_build(ctx, g, morton_order(ctx->h_conn, ctx->h_X, n_el, npe, true));
 }
 
 // Per patch the aggregates of its owned nodes, with those nodes, and per

@@ -492,9 +492,10 @@ constexpr int kPersistPatches = 256;
 // JFEM_PERSIST_POLLS sets fewer.
 constexpr int kMaxPolls = 1 << 20;
 // Elements along a Morton curve of their centroids, the axes in element lengths with
-// by_length (cells.hip); *long_elements (may be null): whether that differs.
-std::vector<int32_t> morton_order(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int npe, bool by_length,
-                                  bool *long_elements);
+// by_length (cells.hip).
+std::vector<int32_t> morton_order(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int npe, bool by_length);
+// Whether the elements' mean extents along the axes differ by more than 30%.
+bool long_elements(const std::vector<int32_t> &conn, const std::vector<double> &X, int64_t n_el, int npe);
 // Geometric factors in the element order perm (gfQ32: folded ones too, or null).
 hipError_t launch_patch_factors(jfm_ctx *ctx, const int32_t *perm, double *gf64, float *gf32, float *gfQ32);
 // elements of a patch, its workgroup's threads (and most nodes), the row

@@ -559,7 +559,8 @@ int jfem_patch_setup(jfm_ctx *ctx) {
     if ((int64_t)ctx->h_conn.size() != n_el * npe || (int64_t)ctx->h_X.size() != 3 * N)
         return jfm_fail(ctx, JFM_ESTATE, "patch setup needs the host mesh");
     const int npatch = (int)((n_el + kPatch - 1) / kPatch);
-    const std::vector<int32_t> perm = morton_order(ctx->h_conn, ctx->h_X, n_el, npe, npe == 8, nullptr);
+    const bool by_length = npe == 8 || (npe == 10 && long_elements(ctx->h_conn, ctx->h_X, n_el, npe));
+    const std::vector<int32_t> perm = morton_order(ctx->h_conn, ctx->h_X, n_el, npe, by_length);
     std::vector<int32_t> epos(n_el);
     for (int64_t k = 0; k < n_el; ++k) epos[perm[k]] = (int32_t)k;
     hipStream_t s = ctx->stream;

@@ -249,3 +249,31 @@ def test_long_elements(gen, g, slots):
     uc = ctx.solve(op="csr", op_outer="csr", **kw)[0]   # launched
     assert np.linalg.norm(u - uc) <= 1e-6 * np.linalg.norm(uc)
     ctx.close()
+
+
+@pytest.mark.parametrize("gen,g,size,slots,resident", [
+    ("box_hex8", (64, 32, 32), (10, 1, 1), 58000, True),      # 65,844 cut across the grid's halves
+    ("box_hex8", (100, 25, 26), (1, 1, 1), 66000, False),     # 66,809
+    ("box_tet10", (60, 20, 20), (10, 1, 1), 232000, False),   # 445,595 with one scale, 231,378 the bounding box's
+    ("box_tet10", (26, 25, 24), (10, 1, 1), None, False)])
+def test_patches_of_long_elements_along_the_grid(gen, g, size, slots, resident):
+    """Element lengths count in whole halvings of the mesh's extent: patches as compact
+    as those of the bounding box's scale, and resident where that fits."""
+    import jfem
+    m = getattr(M, gen)(*g, L=tuple(a * b / g[0] for a, b in zip(g, size)), seed=1, jitter=0.1)
+    ctx = jfem.Context(0)
+    ctx.upload(m)
+    say(f"long elements along the grid: {gen} {g}")
+    x = np.random.default_rng(2).normal(size=m.n_dofs)
+    yc = ctx.apply(x, op="csr")
+    for y in (ctx.apply(x), ctx.apply(x, op="ebe")):
+        assert np.abs(y - yc).max() <= 1e-12 * np.abs(yc).max()
+    if slots:
+        assert ctx.info()["shared_slots"] <= slots
+    # 30 iterations (these meshes' conditioning leaves no residual of 1e-8 to some operators)
+    kw = dict(rtol=1e-8, coarse_nodes=300, maxit=30, raise_on_noconv=False)
+    u = ctx.solve(**kw)[0]
+    assert (ctx.resident_counts()[0] > 0) == resident
+    uc = ctx.solve(op="csr", op_outer="csr", **kw)[0]
+    assert np.linalg.norm(u - uc) <= 1e-6 * np.linalg.norm(uc)
+    ctx.close()
