@@ -1557,41 +1557,29 @@ extern "C" int jfm_solve_nonlinear(jfm_ctx *ctx, const jfm_newton_opts *opts, do
 }
 
 // ========================================================= postprocessing ==
-// M x_k = b_k for the nsys right-hand sides at b + k n, x likewise (M the
-// consistent mass, Mm its inverse diagonal).
-static int mass_solves(jfm_ctx *ctx, const double *Mm, int nsys, const double *b, double *x) {
+// M x_k = b_k for the nsys right-hand sides at b + k n, x likewise, beside of them
+// side by side in the resident PCG (M the consistent mass, Mm its inverse diagonal);
+// *done: false after a give-up.
+static int mass_solves(jfm_ctx *ctx, const double *Mm, int nsys, int beside, const double *b, double *x, bool *done) {
     const int64_t n = ctx->ndof;
     hipStream_t s = ctx->stream;
-    const double rtol = 1e-13;
-    const int maxit = 2000;
-    int beside = nsys;
-    if (int rc = jfem_persist_ready<double>(ctx, kOpMass, &beside)) return rc;
-    if (beside > 1) {
-        std::vector<PcgScalars> S(beside);  // (outlives the copy into it)
-        for (int k = 0; k < nsys && beside > 1; k += beside) {
-            const ResidentHold hold(ctx, beside * ctx->cells.npatch);
-            CHECK_LAUNCH(ctx, launch_pcg_persist<double>(ctx, kOpMass, Mm, b + k * n, nullptr, nullptr, x + k * n, rtol, maxit, false, beside, n));
-            JFM_HIP(ctx, hipMemcpyAsync(S.data(), ctx->cells.S, sizeof(PcgScalars) * beside, hipMemcpyDeviceToHost, s));
-            if (int rc = sync(ctx)) return rc;
-            int failed = 0;
-            for (const PcgScalars &v : S) failed += v.fail != 0;
-            ctx->resident_solves += beside - failed;
-            if (failed) {
-                resident_gave_up(ctx, failed);
-                beside = 0;
-            }
-        }
-        if (beside) {
-            ctx->persist_fails = 0;
+    std::vector<PcgScalars> S(beside);  // (outlives the copy into it)
+    *done = false;
+    for (int k = 0; k < nsys; k += beside) {
+        const ResidentHold hold(ctx, beside * ctx->cells.npatch);
+        CHECK_LAUNCH(ctx, launch_pcg_persist<double>(ctx, kOpMass, Mm, b + k * n, nullptr, nullptr, x + k * n, 1e-13, 2000, false, beside, n));
+        JFM_HIP(ctx, hipMemcpyAsync(S.data(), ctx->cells.S, sizeof(PcgScalars) * beside, hipMemcpyDeviceToHost, s));
+        if (int rc = sync(ctx)) return rc;
+        int failed = 0;
+        for (const PcgScalars &v : S) failed += v.fail != 0;
+        ctx->resident_solves += beside - failed;
+        if (failed) {
+            resident_gave_up(ctx, failed);
             return JFM_OK;
         }
     }
-    for (int k = 0; k < nsys; ++k) {
-        JFM_HIP(ctx, hipMemcpyAsync(ctx->ws64.b, b + k * n, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-        int it = 0, status = 0;
-        if (int rc = pcg_run<double>(ctx, kOpMass, Mm, rtol, maxit, 32, &it, &status)) return rc;
-        JFM_HIP(ctx, hipMemcpyAsync(x + k * n, ctx->ws64.x, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-    }
+    ctx->persist_fails = 0;
+    *done = true;
     return JFM_OK;
 }
 
@@ -1604,8 +1592,21 @@ extern "C" int jfm_postprocess(jfm_ctx *ctx, const double *u, double *strain_gp,
     if (int rc = ensure_workspaces(ctx)) return rc;
     const int64_t n = ctx->ndof, N = ctx->N, nq = ctx->n_el * ctx->ngp * 6;
     hipStream_t s = ctx->stream;
+    // the fits are one operator with two right-hand sides per field, all of them
+    // side by side where the resident PCG takes them; their vectors are in one
+    // allocation with the diagonal (three of their own cost 0.4 ms a call, of 11
+    // at 65,000 Hex8)
+    double *outs[2] = {strain_nodal, stress_nodal};
+    int nf = 0, field[2];
+    for (int f = 0; f < 2; ++f)
+        if (outs[f]) field[nf++] = f;
+    const int nsys = 2 * nf;
+    int beside = nsys;
+    if (nsys)
+        if (int rc = jfem_persist_ready<double>(ctx, kOpMass, &beside)) return rc;
+    const int64_t kept = beside > 1 ? nsys : std::min(nsys, 1);  // solutions
     double *du = jfm_alloc<double>(ctx, n), *eps = jfm_alloc<double>(ctx, nq), *sig = jfm_alloc<double>(ctx, nq),
-           *Mm = jfm_alloc<double>(ctx, 9 * N);
+           *Mm = jfm_alloc<double>(ctx, 9 * N + (nsys ? kept * n + 6 * N : 0) + (beside > 1 ? nsys * n : 0));
     auto cleanup = [&] {
         for (void *p : {(void *)du, (void *)eps, (void *)sig, (void *)Mm}) jfm_free(ctx, p);
     };
@@ -1631,29 +1632,36 @@ extern "C" int jfm_postprocess(jfm_ctx *ctx, const double *u, double *strain_gp,
     }
     // nodal least-squares fits (src/problems_elasticity.jl:550-594): M x = b
     // per three components, PCG with the mass operator and its diagonal
-    if (rc == JFM_OK && (strain_nodal || stress_nodal)) {
+    if (rc == JFM_OK && nsys) {
         e = launch_mass_diag(ctx, Mm);
         if (e != hipSuccess) fail_hip(e, "launch_mass_diag");
-        // the fits are one operator with two right-hand sides per field, all
-        // of them side by side where the resident PCG takes them
-        double *outs[2] = {strain_nodal, stress_nodal};
-        int nf = 0, field[2];
-        for (int f = 0; f < 2; ++f)
-            if (outs[f]) field[nf++] = f;
-        const int nsys = 2 * nf;
-        double *B = jfm_alloc<double>(ctx, nsys * n), *X = jfm_alloc<double>(ctx, nsys * n), *J = jfm_alloc<double>(ctx, 6 * N);
-        if (!B || !X || !J) rc = jfm_fail(ctx, JFM_ENOMEM, "device allocation failed in jfm_postprocess");
-        for (int k = 0; k < nsys && rc == JFM_OK; ++k)
-            if ((e = launch_post_rhs(ctx, du, field[k / 2], 3 * (k % 2), B + k * n)) != hipSuccess) fail_hip(e, "launch_post_rhs");
-        if (rc == JFM_OK) rc = mass_solves(ctx, Mm, nsys, B, X);
+        double *J = Mm + 9 * N, *X = J + 6 * N, *B = X + kept * n;
+        bool done = false;
+        if (beside > 1) {
+            for (int k = 0; k < nsys && rc == JFM_OK; ++k)
+                if ((e = launch_post_rhs(ctx, du, field[k / 2], 3 * (k % 2), B + k * n)) != hipSuccess) fail_hip(e, "launch_post_rhs");
+            if (rc == JFM_OK) rc = mass_solves(ctx, Mm, nsys, beside, B, X, &done);
+        }
         for (int f = 0; f < nf && rc == JFM_OK; ++f) {
-            e = launch_post_join(ctx, X + (2 * f) * n, X + (2 * f + 1) * n, J);
+            const double *x0 = X, *x1 = (const double *)ctx->ws64.x;
+            if (done) {
+                x0 = X + 2 * f * n;
+                x1 = x0 + n;
+            }
+            for (int h = 0; h < 2 && !done && rc == JFM_OK; ++h) {
+                int it = 0, status = 0;
+                if ((e = launch_post_rhs(ctx, du, field[f], 3 * h, (double *)ctx->ws64.b)) != hipSuccess) fail_hip(e, "launch_post_rhs");
+                if (rc == JFM_OK) rc = pcg_run<double>(ctx, kOpMass, Mm, 1e-13, 2000, 32, &it, &status);
+                if (rc == JFM_OK && h == 0) {
+                    e = hipMemcpyAsync(X, ctx->ws64.x, sizeof(double) * n, hipMemcpyDeviceToDevice, s);
+                    if (e != hipSuccess) fail_hip(e, "nodal copy");
+                }
+            }
+            if (rc != JFM_OK) break;
+            e = launch_post_join(ctx, x0, x1, J);
             if (e == hipSuccess) e = hipMemcpyAsync(outs[field[f]], J, sizeof(double) * 6 * N, hipMemcpyDeviceToHost, s);
             if (e != hipSuccess) fail_hip(e, "nodal copy");
         }
-        e = hipStreamSynchronize(s);
-        if (rc == JFM_OK && e != hipSuccess) fail_hip(e, "nodal copy");
-        for (void *p : {(void *)B, (void *)X, (void *)J}) jfm_free(ctx, p);
     }
     e = hipStreamSynchronize(s);
     if (rc == JFM_OK && e != hipSuccess) fail_hip(e, "jfm_postprocess");
